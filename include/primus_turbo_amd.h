@@ -176,6 +176,18 @@ PT_API int pt_quantize_fp8_rowwise(const void *x, int x_dtype, int64_t B, int64_
 PT_API int pt_dequantize_fp8_rowwise(const void *q, int q_dtype, int64_t B, int64_t M, int64_t N,
                                      const float *scale_inv, void *y, int y_dtype, void *stream);
 
+/* The same for a reduced axis that is not the contiguous one (N > 1), dynamic scales, in two launches
+ * over a workspace (contents need no initialisation). x holds 16- / 32-bit values, or FP8 codes with
+ * one scale per row (row_scale_inv, B*M floats): the values are then the de-quantized codes rounded to
+ * hp_dtype, i.e. de-quantize along the rows + quantize along the columns in one step, same bits (what
+ * the backward of a ROWWISE product does with its forward operands, primus_turbo/pytorch/ops/
+ * gemm_fp8.py:300-330). Exactly one output: q [B, M, N] in place order, or q_t [B, N, ld_t] transposed
+ * with codes M .. ld_t zero (ld_t a multiple of 16; the only form for codes, which keep their format). */
+PT_API size_t pt_quantize_fp8_rowwise_outer_workspace_bytes(int64_t B, int64_t M, int64_t N);
+PT_API int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_scale_inv, int hp_dtype, int64_t B,
+                                         int64_t M, int64_t N, void *q, void *q_t, int64_t ld_t, int q_dtype,
+                                         float *scale_inv, void *workspace, size_t workspace_bytes, void *stream);
+
 /* FP8 128-blockwise (fp32 scales, eps 1e-4) -----------------------------------
  *
  * Numerics per block: scale = qmax / max(amax, 1e-4); the stored scale is

@@ -12,6 +12,7 @@
 #include "pt_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 // Timing probes for kernel development: a test translation unit may define this macro to record
 // timestamps; in the library it expands to nothing.
@@ -692,82 +693,9 @@ __global__ __launch_bounds__(RW_THREADS) void quant_rowwise_inner_kernel(
     }
 }
 
-// ===========================================================================
-// Rowwise, reduced axis not contiguous: x viewed as [B, M, N], one scale per (b, n)
-// ===========================================================================
-// Pass 1: column abs-max. A workgroup owns a 64-column strip of one batch and a
-// slab of rows; lanes of a wavefront read 64 consecutive columns (coalesced),
-// the 4 wavefronts take different rows. Partial maxima meet through an integer
-// atomic max on the fp32 bit pattern (amax >= 0), which is order independent.
-constexpr int CM_ROWS_PER_BLOCK = 256;
-
-template <typename T>
-__global__ __launch_bounds__(256) void colmax_kernel(const T *__restrict__ x, uint32_t *amax_bits,
-                                                     const int64_t M, const int64_t N) {
-    const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t b    = blockIdx.z;
-    const int64_t n    = static_cast<int64_t>(blockIdx.x) * 64 + lane;
-    const int64_t m0   = static_cast<int64_t>(blockIdx.y) * CM_ROWS_PER_BLOCK;
-    const int64_t m1   = (m0 + CM_ROWS_PER_BLOCK < M) ? m0 + CM_ROWS_PER_BLOCK : M;
-    __shared__ float s[4][64];
-    float            a = 0.f;
-    if (n < N) {
-        const T *p = x + b * M * N + n;
-        for (int64_t m = m0 + wave; m < m1; m += 4)
-            a = fmaxf(a, fabsf(HP<T>::to_f32(p[m * N])));
-    }
-    s[wave][lane] = a;
-    __syncthreads();
-    if (wave == 0 && n < N) {
-        a = fmaxf(fmaxf(s[0][lane], s[1][lane]), fmaxf(s[2][lane], s[3][lane]));
-        __hip_atomic_fetch_max(&amax_bits[b * N + n], __float_as_uint(a), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// Pass 2: turn the amax (held in scale_inv's storage as fp32 bits) into
-// scale_inv and quantize. Each thread handles 4 consecutive columns of a row.
-template <typename T, bool E5M2, bool DYNAMIC>
-__global__ __launch_bounds__(256) void quant_rowwise_outer_kernel(
-    const T *__restrict__ x, uint8_t *__restrict__ q, const float *__restrict__ amax_or_scale,
-    const int64_t M, const int64_t N, const float qmax) {
-    const int64_t b  = blockIdx.z;
-    const int64_t n  = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    const int64_t m0 = static_cast<int64_t>(blockIdx.y) * CM_ROWS_PER_BLOCK;
-    const int64_t m1 = (m0 + CM_ROWS_PER_BLOCK < M) ? m0 + CM_ROWS_PER_BLOCK : M;
-    if (n >= N)
-        return;
-    float scale;
-    if constexpr (DYNAMIC)
-        scale = qmax / fmaxf(amax_or_scale[b * N + n], 1e-12f);
-    else
-        scale = amax_or_scale[b * N + n];
-    const T *p = x + b * M * N + n;
-    uint8_t *o = q + b * M * N + n;
-    for (int64_t m = m0; m < m1; ++m)
-        o[m * N] = quant1<E5M2>(HP<T>::to_f32(p[m * N]), scale, qmax);
-}
-
-// amax (or given scale) -> scale_inv, in place or to a separate buffer
-template <bool DYNAMIC>
-__global__ void finish_scale_inv_kernel(const float *in, float *scale_inv, const int64_t n,
-                                        const float qmax) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) {
-        float scale;
-        if constexpr (DYNAMIC)
-            scale = qmax / fmaxf(in[i], 1e-12f);
-        else
-            scale = in[i];
-        scale_inv[i] = 1.0f / scale;
-    }
-}
-
-__global__ void zero_u32_kernel(uint32_t *p, const int64_t n) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n)
-        p[i] = 0u;
-}
+// (reduced axis not contiguous: quant_rowwise_outer.hip)
+int launch_quant_rowwise_outer(const void *x, int x_dtype, int64_t B, int64_t M, int64_t N, void *q, bool e5m2,
+                               const float *scale_in, float *scale_inv, float *ws, hipStream_t st);
 
 template <typename T, bool E5M2>
 static int launch_quant_rowwise(const void *x, int64_t B, int64_t M, int64_t N, void *q,
@@ -799,27 +727,8 @@ static int launch_quant_rowwise(const void *x, int64_t B, int64_t M, int64_t N, 
         }
         return check_launch("quant_rowwise_inner_kernel");
     }
-    const int64_t  nscale = B * N;
-    const unsigned mslabs = static_cast<unsigned>(cdiv(M, CM_ROWS_PER_BLOCK));
-    if (scale_in == nullptr) {
-        // scale_inv's storage carries the amax bit patterns between the passes
-        auto *bits = reinterpret_cast<uint32_t *>(scale_inv);
-        zero_u32_kernel<<<static_cast<unsigned>(cdiv(nscale, 256)), 256, 0, stream>>>(bits, nscale);
-        dim3 g1(static_cast<unsigned>(cdiv(N, 64)), mslabs, static_cast<unsigned>(B));
-        colmax_kernel<T><<<g1, 256, 0, stream>>>(xp, bits, M, N);
-        dim3 g2(static_cast<unsigned>(cdiv(N, 256)), mslabs, static_cast<unsigned>(B));
-        quant_rowwise_outer_kernel<T, E5M2, true>
-            <<<g2, 256, 0, stream>>>(xp, qp, scale_inv, M, N, qmax);
-        finish_scale_inv_kernel<true><<<static_cast<unsigned>(cdiv(nscale, 256)), 256, 0, stream>>>(
-            scale_inv, scale_inv, nscale, qmax);
-    } else {
-        dim3 g2(static_cast<unsigned>(cdiv(N, 256)), mslabs, static_cast<unsigned>(B));
-        quant_rowwise_outer_kernel<T, E5M2, false>
-            <<<g2, 256, 0, stream>>>(xp, qp, scale_in, M, N, qmax);
-        finish_scale_inv_kernel<false><<<static_cast<unsigned>(cdiv(nscale, 256)), 256, 0, stream>>>(
-            scale_in, scale_inv, nscale, qmax);
-    }
-    return check_launch("quant_rowwise_outer_kernel");
+    return launch_quant_rowwise_outer(x, std::is_same_v<T, bf16_t> ? PT_DTYPE_BF16 : (std::is_same_v<T, f16_t> ? PT_DTYPE_F16 : PT_DTYPE_F32),
+                                      B, M, N, q, E5M2, scale_in, scale_inv, nullptr, stream);
 }
 
 // ===========================================================================

@@ -81,6 +81,12 @@ _SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_int, c_void_p],
     ),
+    "pt_quantize_fp8_rowwise_outer_workspace_bytes": (c_size_t, [c_i64, c_i64, c_i64]),
+    "pt_quantize_fp8_rowwise_outer": (
+        c_int,
+        [c_void_p, c_int, c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_i64, c_int, c_void_p, c_void_p, c_size_t,
+         c_void_p],
+    ),
     "pt_quantize_fp8_blockwise": (
         c_int,
         [c_void_p, c_int, c_i64, c_i64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],

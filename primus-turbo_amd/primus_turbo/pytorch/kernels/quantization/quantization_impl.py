@@ -174,6 +174,18 @@ def _valid_axis(axis: int, ndim: int) -> int:
     return a
 
 
+def _rowwise_outer(x, row_scale_inv, hp_dtype, bmn, q, q_t, ld_t, scale_inv):
+    """Dynamic rowwise quantization over the middle axis of ``x`` viewed as ``bmn = (B, M, N)``."""
+    lib = N.lib()
+    ws = torch.empty(lib.pt_quantize_fp8_rowwise_outer_workspace_bytes(*bmn), dtype=torch.uint8, device=x.device)
+    N.check(
+        lib.pt_quantize_fp8_rowwise_outer(
+            N.ptr(x), N.dtype_code(x.dtype), N.ptr(row_scale_inv), N.dtype_code(hp_dtype), *bmn, N.ptr(q), N.ptr(q_t), ld_t,
+            N.dtype_code((q if q is not None else q_t).dtype), N.ptr(scale_inv), N.ptr(ws), ws.numel(), N.stream_of(x),
+        )
+    )
+
+
 def _quantize_fp8_rowwise(input: torch.Tensor, dest_dtype: torch.dtype, axis: int, scale_opt=None):
     N.require_cuda(input, scale_opt)
     _check(input.dtype in _HP_DTYPES, "input must be bfloat16, float16 or float32")
@@ -189,6 +201,9 @@ def _quantize_fp8_rowwise(input: torch.Tensor, dest_dtype: torch.dtype, axis: in
     if scale_opt is not None:
         _check(list(scale_opt.shape) == scale_shape, "scale shape must match input with size 1 along axis")
         scale_in = scale_opt.to(torch.float32).contiguous()
+    elif Nn > 1:
+        _rowwise_outer(input, None, input.dtype, (B, M, Nn), out, None, 0, scale_inv)
+        return [out, scale_inv]
     N.check(
         N.lib().pt_quantize_fp8_rowwise(
             N.ptr(input), N.dtype_code(input.dtype), B, M, Nn, N.ptr(out), N.dtype_code(dest_dtype),
@@ -272,6 +287,51 @@ def dequantize_fp8_rowwise_impl(x: torch.Tensor, out_dtype: torch.dtype, axis: i
     assert x.is_contiguous(), "The x tensor must be contiguous."
     assert scale_inv.is_contiguous(), "The scale_inv tensor must be contiguous."
     return torch.ops.primus_turbo_cpp_extension.dequantize_fp8_rowwise(x, scale_inv, axis, out_dtype)
+
+
+def _padded_rows(M: int, pad: int) -> int:
+    return -(-M // pad) * pad
+
+
+@torch.library.custom_op("primus_turbo::quant_fp8_rowwise_t_impl", mutates_args=())
+def quant_fp8_rowwise_t_impl(
+    x: torch.Tensor, row_scale_inv: Optional[torch.Tensor], hp_dtype: torch.dtype, dtype: torch.dtype, pad: int
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """ROWWISE quantization of ``x [.., M, N]`` along axis -2 with the codes emitted transposed, ``(x_fp8_t
+    [.., N, M_pad], scale_inv [.., 1, N])``, ``M_pad`` = ``M`` rounded up to ``pad`` (a multiple of 16; the
+    added codes are zero): the K-contiguous operand of the product that reduces over the rows of ``x``.
+    With ``row_scale_inv`` ``x`` holds FP8 codes of a ROWWISE quantization along axis -1, which are
+    quantized again along axis -2 from the ``hp_dtype`` values they stand for (same bits as
+    de-quantize, quantize, transpose). (No counterpart in the reference, which runs those three steps.)"""
+    N.require_cuda(x, row_scale_inv)
+    _check_fp8_out(dtype)
+    _check(x.dim() >= 2 and x.is_contiguous(), "input must be contiguous, at least 2-D")
+    _check(hp_dtype in _HP_DTYPES, "hp_dtype must be bfloat16, float16 or float32")
+    _check(pad % 16 == 0, "pad must be a multiple of 16")
+    *lead, M, Nn = x.shape
+    if row_scale_inv is None:
+        _check(x.dtype == hp_dtype, "input must be bfloat16, float16 or float32")
+    else:
+        _check(x.dtype == dtype, "codes keep their format")
+        _check(row_scale_inv.dtype == torch.float32 and row_scale_inv.is_contiguous()
+               and list(row_scale_inv.shape) == [*lead, M, 1], "row_scale_inv must hold one float32 per row")
+    Mp = _padded_rows(M, pad)
+    q_t = torch.empty((*lead, Nn, Mp), dtype=dtype, device=x.device)
+    scale_inv = torch.empty((*lead, 1, Nn), dtype=torch.float32, device=x.device)
+    B = 1
+    for d in lead:
+        B *= d
+    _rowwise_outer(x, row_scale_inv, hp_dtype, (B, M, Nn), None, q_t, Mp, scale_inv)
+    return q_t, scale_inv
+
+
+@quant_fp8_rowwise_t_impl.register_fake
+def _quant_fp8_rowwise_t_impl_fake(x, row_scale_inv, hp_dtype, dtype, pad):
+    *lead, M, Nn = x.shape
+    return (
+        torch.empty((*lead, Nn, _padded_rows(M, pad)), dtype=dtype, device=x.device),
+        torch.empty((*lead, 1, Nn), dtype=torch.float32, device=x.device),
+    )
 
 
 # ===========================================================================

@@ -38,6 +38,7 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_t_impl,
     quant_fp8_blockwise_kmajor_impl,
     quant_fp8_blockwise_for_weight_dual_impl,
+    quant_fp8_rowwise_t_impl,
 )
 from primus_turbo.pytorch.ops.quantization import dequantize_fp8, quantize_fp8, quantize_fp8_with_trans
 from primus_turbo.pytorch.ops.utils import _get_dummy_wgrad, _get_fp8_dtype, _setup_fused_grad_accum
@@ -120,36 +121,46 @@ class FP8GemmRowFunction(torch.autograd.Function):
         qa, qa_s, a_hp = _quantized_parts(a, config, True, -1)
         qb, qb_s, b_hp = _quantized_parts(b, config, True, b_axis)
 
-        def other_axis(q, q_s, hp_dtype, from_axis, given, axis):
+        def other_axis(q, q_s, hp_dtype, from_axis, given, axis, pad):
             # the operand as backward reads it: what the forward codes stand for, quantized again
-            # along the other axis
+            # along the other axis -> (codes, scales, whether the codes are stored transposed, i.e.
+            # contiguous along the axis that the backward product reduces over)
             if given is not None:
                 assert isinstance(given, QuantizedTensor)
-                return given.qdata, given.scale_inv
+                return given.qdata, given.scale_inv, False
+            if axis == -2 and pad is not None:
+                return (*quant_fp8_rowwise_t_impl(q, q_s, hp_dtype, q.dtype, pad), True)
             hp = dequantize_fp8(q, hp_dtype, gran, axis=from_axis % q.ndim, scale_inv=q_s, block_size=config.block_size)
-            return quantize_fp8(hp, q.dtype, gran, axis=axis % q.ndim, block_size=config.block_size)
+            return (*quantize_fp8(hp, q.dtype, gran, axis=axis % q.ndim, block_size=config.block_size), False)
 
         out = _gemm(qa, qa_s, trans_a, qb, qb_s, trans_b, out_dtype, False, gran)
         # the operands quantized along their other axis only feed backward: skip them when no
         # input asks for a gradient (same outputs, two quantizer passes less)
+        a_t_ready = b_t_ready = False
         if any(ctx.needs_input_grad[:2]):
-            a_c, a_cs = other_axis(qa, qa_s, a_hp, -1, a_t, -2)
-            b_c, b_cs = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1)
+            # (wgrad: both operands carry the token padding; dgrad: the gradient's rows are as they are)
+            a_c, a_cs, a_t_ready = other_axis(qa, qa_s, a_hp, -1, a_t, -2, 128)
+            b_c, b_cs, b_t_ready = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1,
+                                              16 if qb.size(-2) % 16 == 0 else None)
             ctx.save_for_backward(a_c, a_cs, b_c, b_cs)
-        ctx.meta = (trans_a, trans_b, out_dtype, config)
+        ctx.meta = (trans_a, trans_b, out_dtype, config, a_t_ready, b_t_ready)
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        trans_a, trans_b, out_dtype, config = ctx.meta
+        trans_a, trans_b, out_dtype, config, a_t_ready, b_t_ready = ctx.meta
         a_c, a_cs, b_c, b_cs = ctx.saved_tensors
         grad_out = grad_out.contiguous()
         gdt = _get_fp8_dtype(config.format, False)
         gran = config.granularity
         g_row, g_row_s = quantize_fp8(grad_out, gdt, gran, axis=1, block_size=config.block_size)
-        grad_a = _gemm(g_row, g_row_s, False, b_c, b_cs, not trans_b, out_dtype, trans_a, gran)
-        g_col, g_col_s = quantize_fp8(grad_out, gdt, gran, axis=0, block_size=config.block_size)
-        grad_b = _gemm(a_c, a_cs, not trans_a, g_col, g_col_s, False, out_dtype, trans_b, gran)
+        grad_a = _gemm(g_row, g_row_s, False, b_c, b_cs, True if b_t_ready else not trans_b, out_dtype, trans_a, gran)
+        if a_t_ready:
+            g_col, g_col_s = quant_fp8_rowwise_t_impl(grad_out, None, grad_out.dtype, gdt, 128)
+            grad_b = _gemm(a_c, a_cs, False, g_col, g_col_s, True, out_dtype, trans_b, gran)
+        else:
+            g_col, g_col_s = quantize_fp8(grad_out, gdt, gran, axis=0, block_size=config.block_size)
+            grad_b = _gemm(a_c, a_cs, not trans_a, g_col, g_col_s, False, out_dtype, trans_b, gran)
         return grad_a, grad_b, None, None, None, None, None, None
 
 

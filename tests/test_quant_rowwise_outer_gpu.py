@@ -1,0 +1,52 @@
+"""GPU parity of rowwise quantization along a non-contiguous axis vs the CPU oracle (bit-exact): codes in
+place, codes transposed, and FP8 codes quantized again along their other axis."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import FMT, bf16_randn, bits_np, codes_np, round_to, to_f32_np
+from oracle import quantize as Q
+
+pytestmark = pytest.mark.gpu
+
+# edges of the 512-column strips, of the 128 x 128 tiles and of the eight-row runs; columns that are no
+# multiple of eight take the one-column lanes
+SHAPES = [(1, 8), (7, 8), (33, 9), (128, 128), (129, 136), (257, 520), (1000, 516), (3001, 264), (3, 65, 72), (2, 5, 130, 16)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("src,dtype", [(torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float8_e5m2),
+                                       (torch.float32, torch.float8_e4m3fn)])
+def test_outer_axis(native_lib, shape, src, dtype):
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as I
+
+    x = bf16_randn(shape, seed=21, outlier_frac=0.01, dtype=src)
+    axis = len(shape) - 2
+    oq, osinv = Q.fp8_rowwise(to_f32_np(x), axis, FMT[dtype])
+    q, sinv = I.quantize_fp8_rowwise_impl(x.cuda(), dtype, axis)
+    assert np.array_equal(bits_np(sinv), osinv.view(np.uint32)) and np.array_equal(codes_np(q), oq)
+    qt, sinv = I.quant_fp8_rowwise_t_impl(x.cuda(), None, src, dtype, 128)
+    M = shape[-2]
+    assert tuple(qt.shape) == (*shape[:-2], shape[-1], -(-M // 128) * 128)
+    got = codes_np(qt)
+    assert np.array_equal(bits_np(sinv), osinv.view(np.uint32))
+    assert np.array_equal(got[..., :M], np.swapaxes(oq, -1, -2)) and not got[..., M:].any()
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("src,dtype", [(torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float8_e5m2),
+                                       (torch.float32, torch.float8_e4m3fn)])
+def test_codes_quantized_again(native_lib, shape, src, dtype):
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as I
+
+    x = bf16_randn(shape, seed=22, outlier_frac=0.01, dtype=src)
+    q1, s1 = Q.fp8_rowwise(to_f32_np(x), len(shape) - 1, FMT[dtype])
+    hp = round_to(Q.fp8_dequant(q1, s1, FMT[dtype]), src)
+    oq, osinv = Q.fp8_rowwise(to_f32_np(hp), len(shape) - 2, FMT[dtype])
+    codes = torch.from_numpy(q1).view(dtype).cuda()
+    qt, sinv = I.quant_fp8_rowwise_t_impl(codes, torch.from_numpy(s1).cuda(), src, dtype, 16)
+    M = shape[-2]
+    got = codes_np(qt)
+    assert np.array_equal(bits_np(sinv), osinv.view(np.uint32))
+    assert np.array_equal(got[..., :M], np.swapaxes(oq, -1, -2)) and not got[..., M:].any()
