@@ -292,17 +292,59 @@ template <bool ACC_IN_AGPR> __device__ __forceinline__ f32x4 read_acc(const f32x
 // Returns the number of store instructions it has issued (every one of them younger than any
 // memory operation issued before the call): what a caller may leave in flight when it next waits
 // for older operations by count.
-// `rows_left`: rows of the matrix from this lane's first row on (its row of MFMA tile i is
-// 16 i): a lane skips the loads and stores of the row groups at or beyond it, so a sub-tile that
-// hangs over the end of its matrix (the last rows of a group) still leaves in 16-byte stores.
-// (ROWCHECK = false: every row group is stored; for callers whose sub-tile is known to lie inside.)
-template <typename T, int TM, int TN, int MODE, bool ACC_IN_AGPR, bool ROWCHECK>
-__device__ __forceinline__ int epilogue_inner(T *row, int64_t step, bool accu, const f32x4 (&acc)[TM][TN],
-                                              const float (&sa)[TM], const f32x4 (&sb)[TN], const int64_t rows_left) {
+//
+// Two ways to leave out what hangs over the end of the matrix:
+//   BUF = false, sub-tiles inside the columns: stores through row pointers. `rows_left`: rows of the
+//   matrix from this lane's first row on (its row of MFMA tile i is 16 i): a lane skips the loads and
+//   stores of the row groups at or beyond it. ROWCHECK = false: every row group is stored; for callers
+//   whose sub-tile is known to lie inside.
+//   BUF = true, sub-tiles over the last columns: buffer stores from the sub-tile's first element
+//   `base`; `left` are the bytes from there to the end of the matrix' rows (of the group's rows), so a
+//   row behind the end is out of range, and a lane whose columns lie at or behind `cols` (the
+//   sub-tile's columns inside the matrix) takes an offset with its top bit set. The bounds check drops
+//   those stores; no test, no branch. 3001 x 2880 x 4096 in 256 x 256 tiles: 67 us while such sub-tiles
+//   left element by element, 48 this way. (Used for every sub-tile it costs the MX kernels 1 %, present
+//   in the grouped MX kernels, whose N is whole tiles as a rule, 2 %; the block-scaled kernels have no
+//   registers for it, 8192^3 went from 0.446 to 0.544 ms. HANG_COLS says who has it.)
+constexpr uint32_t OUT_OF_RANGE = 0x80000000u;
+template <typename T, int TM, int TN, int MODE, bool ACC_IN_AGPR, bool BUF, bool ROWCHECK>
+__device__ __forceinline__ int epilogue_inner(uint8_t *base, uint32_t left, const int64_t row_bytes, const int cols,
+                                              const int64_t rows_left, bool accu, const f32x4 (&acc)[TM][TN],
+                                              const float (&sa)[TM], const f32x4 (&sb)[TN], int lane) {
+    constexpr bool F32 = sizeof(T) == 4;
+    // (the lane number is made opaque: the compiler would otherwise compute the offsets of every output
+    // type ahead of the K loop and hold them there)
+    if constexpr (BUF)
+        asm volatile("" : "+v"(lane));
+    const int      lm = lane & 15, lg = lane >> 4;
+    const int      c0    = F32 ? 4 * lg : 16 * (lg & 1) + 8 * (lg >> 1);
+    const uint32_t row16 = 16u * static_cast<uint32_t>(row_bytes);
+    [[maybe_unused]] const uint32_t voff0 = static_cast<uint32_t>(lm) * static_cast<uint32_t>(row_bytes) + c0 * static_cast<uint32_t>(sizeof(T));
+    [[maybe_unused]] auto voff = [&](int j) { return (c0 + j * (F32 ? 16 : 32) < cols ? voff0 : OUT_OF_RANGE) + j * 64; };
+    [[maybe_unused]] uint8_t *row = base + lm * row_bytes + c0 * static_cast<int>(sizeof(T));
     int stores = 0;
     static_for<0, TM>([&](auto ic) {
         constexpr int i = ic;
-        const bool    live = !ROWCHECK || 16 * i < rows_left;
+        const bool    live = BUF || !ROWCHECK || 16 * i < rows_left;
+        // 16 bytes of the row: lane's group j (64 bytes apart)
+#if defined(__HIP_DEVICE_COMPILE__) // the buffer resource type only exists in the device pass
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, left, 0x00020000);
+        auto load = [&](int j) {
+            if constexpr (BUF)
+                return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff(j), 0, 0));
+            else
+                return *reinterpret_cast<const u32x4 *>(row + j * 64);
+        };
+        auto store = [&](int j, u32x4 v) { // (streaming stores measured no faster here)
+            if constexpr (BUF)
+                __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff(j), 0, 0);
+            else
+                *reinterpret_cast<u32x4 *>(row + j * 64) = v;
+        };
+#else
+        auto load  = [&](int) { return u32x4{0, 0, 0, 0}; };
+        auto store = [&](int, u32x4) {};
+#endif
         if constexpr (sizeof(T) == 4) {
             // accumulating: the old values of four tiles are requested together, then used (one
             // load at a time would pay the memory latency TN times per row)
@@ -325,21 +367,22 @@ __device__ __forceinline__ int epilogue_inner(T *row, int64_t step, bool accu, c
                     return v;
                 };
                 if (accu && live) {
-                    f32x4 old[JB];
+                    u32x4 old[JB];
 #pragma unroll
                     for (int jj = 0; jj < JB; ++jj)
-                        old[jj] = *reinterpret_cast<const f32x4 *>(row + (j0 + jj) * 16);
+                        old[jj] = load(j0 + jj);
                     __builtin_amdgcn_sched_barrier(0);
                     static_for<0, JB>([&](auto jjc) {
                         constexpr int j = j0 + jjc;
-                        *reinterpret_cast<f32x4 *>(row + j * 16) = tile_value(std::integral_constant<int, j>{}) + old[j - j0];
+                        store(j, __builtin_bit_cast(u32x4, tile_value(std::integral_constant<int, j>{}) +
+                                                               __builtin_bit_cast(f32x4, old[j - j0])));
                         // keep each accumulator's read next to its store (register pressure)
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 } else if (live) {
                     static_for<0, JB>([&](auto jjc) {
                         constexpr int j = j0 + jjc;
-                        *reinterpret_cast<f32x4 *>(row + j * 16) = tile_value(std::integral_constant<int, j>{});
+                        store(j, __builtin_bit_cast(u32x4, tile_value(std::integral_constant<int, j>{})));
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 }
@@ -368,7 +411,7 @@ __device__ __forceinline__ int epilogue_inner(T *row, int64_t step, bool accu, c
                     u32x4 old[TN / 2];
 #pragma unroll
                     for (int jj = 0; jj < TN / 2; ++jj)
-                        old[jj] = *reinterpret_cast<const u32x4 *>(row + jj * 32);
+                        old[jj] = load(jj);
                     __builtin_amdgcn_sched_barrier(0);
                     static_for<0, TN / 2>([&](auto jc) {
                         constexpr int j = 2 * jc;
@@ -387,8 +430,7 @@ __device__ __forceinline__ int epilogue_inner(T *row, int64_t step, bool accu, c
                         unpack2<T>(o.y, o0, o1); x[2] += o0; x[3] += o1;
                         unpack2<T>(o.z, o0, o1); y[0] += o0; y[1] += o1;
                         unpack2<T>(o.w, o0, o1); y[2] += o0; y[3] += o1;
-                        *reinterpret_cast<u32x4 *>(row + j * 16) =
-                            u32x4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
+                        store(jc, u32x4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])});
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 } else {
@@ -400,14 +442,19 @@ __device__ __forceinline__ int epilogue_inner(T *row, int64_t step, bool accu, c
                         swap16(w0, w2);
                         swap16(w1, w3);
                         asm volatile("s_nop 1" ::: "memory");
-                        *reinterpret_cast<u32x4 *>(row + j * 16) = u32x4{w0, w1, w2, w3}; // (streaming stores measured no faster here)
+                        store(jc, u32x4{w0, w1, w2, w3});
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 }
             }
             stores += TN / 2;
         }
-        row += step;
+        if constexpr (BUF) {
+            base += row16;
+            left = left > row16 ? left - row16 : 0u;
+        } else {
+            row += row16;
+        }
     });
     return stores; // (a compile-time constant after unrolling: TM * TN, or TM * TN / 2 for 16-bit outputs)
 }
@@ -425,6 +472,23 @@ __device__ __forceinline__ void store_elem(float f, uint8_t *q, int out_dtype, b
     }
 }
 
+// Four consecutive values of one row (8 or 16 bytes, aligned): what a lane holds of an MFMA tile.
+template <typename T> __device__ __forceinline__ void store_quad(f32x4 v, uint8_t *q, bool accu) {
+    if constexpr (sizeof(T) == 4) {
+        f32x4 *p = reinterpret_cast<f32x4 *>(q);
+        *p       = accu ? v + *p : v;
+    } else {
+        u32x2 *p = reinterpret_cast<u32x2 *>(q);
+        if (accu) {
+            const u32x2 o = *p;
+            float       o0, o1;
+            unpack2<T>(o.x, o0, o1); v[0] += o0; v[1] += o1;
+            unpack2<T>(o.y, o0, o1); v[2] += o0; v[3] += o1;
+        }
+        *p = u32x2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+    }
+}
+
 // `Cm` / `sAm` / `sBm` / `m_end` describe the matrix the tile belongs to (the whole problem,
 // or one group's share of it).
 // Returns (uniform over the wavefront) how many of the vector-memory operations it issued are
@@ -432,10 +496,11 @@ __device__ __forceinline__ void store_elem(float f, uint8_t *q, int out_dtype, b
 // return: the store count of the straight-line path, 0 for the generic path. Kernels that wait
 // for older direct-to-LDS copies by count (memory operations retire in order) leave exactly
 // that many operations outstanding instead of waiting for the stores to be acknowledged.
+// HANG_COLS: sub-tiles over the last columns leave in 16-byte buffer stores (see epilogue_inner).
 // ROWCHECK = false keeps the 16-byte stores for sub-tiles that lie wholly inside the matrix only
 // (a hanging one takes the generic path): for kernels that cannot afford the registers of the
 // row test around their epilogue.
-template <int TM, int TN, int MODE, bool ACC_IN_AGPR, bool ROWCHECK = true>
+template <int TM, int TN, int MODE, bool ACC_IN_AGPR, bool ROWCHECK = true, bool HANG_COLS = false>
 __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM][TN], uint8_t *Cm,
                                          const float *sAm, const float *sBm, int64_t m_end,
                                          int64_t wm_base, int64_t wn_base, int lane) {
@@ -471,27 +536,35 @@ __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM
         for (int j = 0; j < TN; ++j)
             asm volatile("" ::"v"(sb[j]));
     }
-    // all columns of the sub-tile inside the matrix and every 16-byte group aligned: 16-byte stores,
-    // with the row groups beyond the end of the matrix (the end of a group's rows) left out
-    // (only a sub-tile that lies wholly inside is certain to have issued every store it counts)
-    const bool whole = wm_base + TM * 16 <= m_end;
-    const bool fast  = (ROWCHECK || whole) && wn_base + TN * 16 <= a.N && (a.N & 7) == 0 &&
-                      (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+    // 16-byte stores where every 16-byte group of a row is aligned and wholly inside or outside the
+    // matrix (only a sub-tile that lies wholly inside is certain to have issued every store it counts)
+    const bool whole_m = wm_base + TM * 16 <= m_end, whole_n = wn_base + TN * 16 <= a.N;
+    const bool aligned = (a.N & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
     uint8_t      *row  = C + (m0 * a.N + n0) * ES;
     const int64_t step = 16 * a.N;
+    uint8_t      *base = C + (wm_base * a.N + wn_base) * ES;
     const int64_t rows_left = m_end - m0;
-    if (fast) {
-        // 16-bit outputs: the lane's eight columns after the exchange between tile pairs
-        uint8_t *rowp = C + (m0 * a.N + wn_base + 16 * (lg & 1) + 8 * (lg >> 1)) * 2;
-        int stores;
+    auto by_type = [&](auto buf, uint32_t left, int cols) {
+        constexpr bool BUF = decltype(buf)::value;
         if (a.out_dtype == PT_DTYPE_BF16)
-            stores = epilogue_inner<bf16_t, TM, TN, MODE, ACC_IN_AGPR, ROWCHECK>(reinterpret_cast<bf16_t *>(rowp), step, accu, acc, sa, sb, rows_left);
-        else if (a.out_dtype == PT_DTYPE_F16)
-            stores = epilogue_inner<f16_t, TM, TN, MODE, ACC_IN_AGPR, ROWCHECK>(reinterpret_cast<f16_t *>(rowp), step, accu, acc, sa, sb, rows_left);
-        else
-            stores = epilogue_inner<float, TM, TN, MODE, ACC_IN_AGPR, ROWCHECK>(reinterpret_cast<float *>(row), step, accu, acc, sa, sb, rows_left);
-        return whole ? stores : 0;
+            return epilogue_inner<bf16_t, TM, TN, MODE, ACC_IN_AGPR, BUF, ROWCHECK>(base, left, a.N * 2, cols, rows_left, accu, acc, sa, sb, lane);
+        if (a.out_dtype == PT_DTYPE_F16)
+            return epilogue_inner<f16_t, TM, TN, MODE, ACC_IN_AGPR, BUF, ROWCHECK>(base, left, a.N * 2, cols, rows_left, accu, acc, sa, sb, lane);
+        return epilogue_inner<float, TM, TN, MODE, ACC_IN_AGPR, BUF, ROWCHECK>(base, left, a.N * 4, cols, rows_left, accu, acc, sa, sb, lane);
+    };
+    if (aligned && (ROWCHECK || whole_m) && whole_n) {
+        const int stores = by_type(std::false_type{}, 0u, 0);
+        return whole_m ? stores : 0;
+    }
+    // (a sub-tile's rows are addressed with 31-bit offsets)
+    if (HANG_COLS && aligned && a.N < (1 << 22)) {
+        if constexpr (HANG_COLS) {
+            const int64_t bytes = ((m_end - wm_base) * a.N - wn_base) * ES;
+            by_type(std::true_type{}, bytes < 0 ? 0u : (bytes > 0xffffffffll ? 0xffffffffu : static_cast<uint32_t>(bytes)),
+                    static_cast<int>(a.N - wn_base < TN * 16 ? a.N - wn_base : TN * 16));
+        }
     } else {
+        const bool quads = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
         static_for<0, TM>([&](auto ic) {
             constexpr int i = ic;
             static_for<0, TN>([&](auto jc) {
@@ -502,11 +575,26 @@ __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM
                     for (int e = 0; e < 4; ++e)
                         v[e] = v[e] * sa[i] * sb[j][e];
                 }
+                // A sub-tile over the last columns of a matrix whose rows are whole 4-column groups: the
+                // lane's four values are wholly in or out and leave in one store (block-scaled
+                // 286 x 1440 x 1792: 16.1 us element by element, 13.6 this way).
                 if (m0 + i * 16 < m_end) {
+                    if (quads) {
+                        if (n0 + j * 16 < a.N) {
+                            uint8_t *q = row + j * 16 * ES;
+                            if (a.out_dtype == PT_DTYPE_BF16)
+                                store_quad<bf16_t>(v, q, accu);
+                            else if (a.out_dtype == PT_DTYPE_F16)
+                                store_quad<f16_t>(v, q, accu);
+                            else
+                                store_quad<float>(v, q, accu);
+                        }
+                    } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n0 + j * 16 + e < a.N)
-                            store_elem(v[e], row + (j * 16 + e) * ES, a.out_dtype, accu);
+                        for (int e = 0; e < 4; ++e)
+                            if (n0 + j * 16 + e < a.N)
+                                store_elem(v[e], row + (j * 16 + e) * ES, a.out_dtype, accu);
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -1187,7 +1275,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
                 asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
             PT_GEMM_TRACE_POINT(5);
             // (0, ST16 or ST32: the stores of the epilogue's straight-line path)
-            pending = __builtin_amdgcn_readfirstlane(epilogue<TM, TN, MODE, MODE != SCALE_BLOCK>(
+            pending = __builtin_amdgcn_readfirstlane(epilogue<TM, TN, MODE, MODE != SCALE_BLOCK, true, MODE != SCALE_BLOCK && GMODE == GROUP_NONE>(
                 a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane));
         } else {
             const int ES     = a.out_dtype == PT_DTYPE_F32 ? 4 : 2;

@@ -271,7 +271,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_mx8_kernel(const GemmArgs a) 
         // tracking does not see: let the last MFMA's write-back finish first
         asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
         const int64_t wm_base = cur_t.m0 + wm * (TM * 16), wn_base = cur_t.n0 + wn * (TN * 16);
-        epilogue<TM, TN, SCALE_MX, true>(a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane);
+        epilogue<TM, TN, SCALE_MX, true, true, GMODE == GROUP_NONE>(a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane);
 
         if (next_tile >= total)
             break;

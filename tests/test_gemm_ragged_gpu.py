@@ -1,0 +1,50 @@
+"""GPU parity of the GEMM kernels at sizes that hang over a tile: columns, rows and K that are no multiple of
+anything a tile is made of. Operands hold small whole numbers, so every product is exact in fp32 and the
+result is the whole-number product rounded once to the output type."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+G = None
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _impl(native_lib):
+    global G, impl
+    from primus_turbo.pytorch.core.low_precision import ScalingGranularity as G
+    from primus_turbo.pytorch.kernels.gemm import gemm_fp8_impl as impl
+
+
+def _whole(rows, cols, seed):
+    """fp8 codes of whole numbers in [-4, 4] and the numbers."""
+    g = torch.Generator().manual_seed(seed)
+    v = torch.randint(-4, 5, (rows, cols), generator=g).float()
+    return v.to(torch.float8_e4m3fn).cuda(), v
+
+
+def _vec(M, N, K, out_dtype, accumulate, cfg, seed=0):
+    (a, av), (b, bv) = _whole(M, K, seed), _whole(N, K, seed + 1)
+    sa = 2.0 ** torch.randint(-2, 3, (M, 1)).float()
+    sb = 2.0 ** torch.randint(-2, 3, (N, 1)).float()
+    ref = (av.double() * sa.double()) @ (bv.double() * sb.double()).T
+    old = torch.randint(-8, 9, (M, N)).to(out_dtype)
+    out = old.cuda().clone()
+    impl.TILE_CFG = cfg
+    try:
+        impl._launch(a, sa.cuda(), False, b, sb.cuda(), True, out, False, G.ROWWISE, accumulate)
+    finally:
+        impl.TILE_CFG = 0
+    want = (ref + old.double() if accumulate else ref).float().to(out_dtype)
+    return out.cpu(), want
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("N", [264, 268, 262, 40, 7])  # 8-, 4- and 2-column groups at the edge; less than a sub-tile
+@pytest.mark.parametrize("cfg", [1, 2, 3])
+def test_ragged_columns(out_dtype, accumulate, N, cfg):
+    got, want = _vec(333, N, 512, out_dtype, accumulate, cfg)
+    assert torch.equal(got, want), f"{(got != want).sum().item()} of {got.numel()} differ"
