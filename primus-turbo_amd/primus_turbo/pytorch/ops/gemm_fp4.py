@@ -73,6 +73,9 @@ class FP4GemmMXFunction(torch.autograd.Function):
             what a pre-quantized operand must carry (the reference's recipes, shuffle flags included)."""
             if isinstance(x, QuantizedTensor):
                 check_quantized_tensor(x, config, scaling_recipe=recipe)
+                # (a pre-shuffled operand's column form has size limits of its own: made, and so checked, always)
+                if x_t is None and not need_bwd and not pre:
+                    return x.qdata, x.scale_inv, None, None
                 if x_t is None:
                     x_t = QuantizedTensor.quantize(x.dequantize(), x.real_dtype, gran, axis=-2, block_size=bs,
                                                    scaling_recipe=recipe_t)
@@ -86,7 +89,7 @@ class FP4GemmMXFunction(torch.autograd.Function):
             if not need_bwd:
                 # the transposed copies only feed backward: skip them when nothing asks for a gradient
                 q, sc = quantize_mxfp4_impl(x, dt, x.dim() - 1, bs, scaling_recipe=recipe)
-                return q, sc, q, sc
+                return q, sc, None, None
             return quantize_fp4_with_trans(x, dt, gran, block_size=bs, scaling_recipe=recipe,
                                            scaling_recipe_for_trans=recipe_t)
 
@@ -96,7 +99,8 @@ class FP4GemmMXFunction(torch.autograd.Function):
                                                    ScalingRecipe(use_rht=True, shuffle_scale=pre, shuffle_out=pre))
         b_row, b_row_s, b_col, b_col_s = both_ways(b, b_t, w_recipe, w_recipe)
         out = gemm_fp4_impl(a_row, a_row_s, False, b_row, b_row_s, True, out_dtype, False, gran.value, _NATIVE)
-        ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s)
+        if need_bwd:
+            ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s)
         ctx.meta = (out_dtype, config, fuse, main_grad)
         return out
 

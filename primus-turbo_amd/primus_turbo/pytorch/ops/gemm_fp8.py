@@ -83,9 +83,12 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         qb, qb_s, _ = _quantized_parts(b, config, True, -1)
         out = _gemm(qa, qa_s, trans_a, qb, qb_s, trans_b, out_dtype, False, config.granularity)
         # NT forward: keep physically transposed fp8 copies so that both backward GEMMs
-        # are NT as well (contiguous-K operands need no transposition pass inside the GEMM)
+        # are NT as well (contiguous-K operands need no transposition pass inside the GEMM);
+        # they only feed backward: skipped when nothing asks for a gradient
         nt_bwd = (not trans_a) and trans_b
-        if nt_bwd:
+        if not any(ctx.needs_input_grad[:2]):
+            pass
+        elif nt_bwd:
             # a tensorwise transpose moves the codes and shares the scalar scale
             sa, sa_s = (a_t.qdata, a_t.scale_inv) if isinstance(a_t, QuantizedTensor) else (transpose_last_two(qa), qa_s)
             sb, sb_s = (b_t.qdata, b_t.scale_inv) if isinstance(b_t, QuantizedTensor) else (transpose_last_two(qb), qb_s)
@@ -254,6 +257,8 @@ class FP8GemmMXFunction(torch.autograd.Function):
         def both_ways(x, x_t, recipe):
             if isinstance(x, QuantizedTensor):
                 check_quantized_tensor(x, config, axis=-1, scaling_recipe=recipe)
+                if not need_bwd:
+                    return x.qdata, x.scale_inv, None, None
                 if x_t is None:
                     x_t = QuantizedTensor.quantize(x.dequantize(), x.real_dtype, gran, axis=-2, block_size=bs,
                                                    scaling_recipe=recipe)
@@ -261,14 +266,15 @@ class FP8GemmMXFunction(torch.autograd.Function):
             if not need_bwd:
                 # the transposed copies only feed backward: skip them when nothing asks for a gradient
                 q, sc = quantize_mxfp8_impl(x, fdt, x.dim() - 1, bs, scaling_recipe=recipe)
-                return q, sc, q, sc
+                return q, sc, None, None
             return quantize_mxfp8_impl(x, fdt, None, bs, with_trans=True, scaling_recipe=recipe,
                                        scaling_recipe_for_trans=recipe)
 
         a_row, a_row_s, a_col, a_col_s = both_ways(a, a_t, ScalingRecipe())
         b_row, b_row_s, b_col, b_col_s = both_ways(b, b_t, ScalingRecipe(use_2d_block=True))
         out = _gemm(a_row, a_row_s, False, b_row, b_row_s, True, out_dtype, False, gran)
-        ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s)
+        if need_bwd:
+            ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s)
         ctx.meta = (out_dtype, config, fuse, main_grad)
         return out
 
