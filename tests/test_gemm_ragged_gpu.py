@@ -48,3 +48,10 @@ def _vec(M, N, K, out_dtype, accumulate, cfg, seed=0):
 def test_ragged_columns(out_dtype, accumulate, N, cfg):
     got, want = _vec(333, N, 512, out_dtype, accumulate, cfg)
     assert torch.equal(got, want), f"{(got != want).sum().item()} of {got.numel()} differ"
+
+
+@pytest.mark.parametrize("M,N", [(1, 16), (333, 264)])
+@pytest.mark.parametrize("K", [16, 144, 272, 2000, 40, 257])  # padded in 16-byte groups, byte by byte
+def test_ragged_reduction(M, N, K):
+    got, want = _vec(M, N, K, torch.float32, False, 0)
+    assert torch.equal(got, want), f"{(got != want).sum().item()} of {got.numel()} differ"
