@@ -60,6 +60,17 @@ def test_preprocessing_matches_oracle(T, E, K, kind, pad):
     assert int(got[2].item()) == overflow == 0 and int(got[3].item()) == nd == T - empty
 
 
+@pytest.mark.parametrize("T,E,K", [(300, 16, 8), (257, 240, 255), (64, 8, 256)])
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_preprocessing_repeated_choices(T, E, K, dtype):
+    """An expert named twice by a token counts once, with its first slot; more slots than a byte holds."""
+    emap = np.random.default_rng(K).integers(-2, E + 2, (T, K)).astype(dtype)
+    got = ext.permute_preprocessing(torch.from_numpy(emap).cuda(), E, K, 16, -1, K)
+    rmap, tpe, _, nd = P.preprocess(emap, E, 16, topk_aligned_probs=True)
+    assert np.array_equal(got[0].cpu().numpy(), rmap)
+    assert np.array_equal(got[1].cpu().numpy(), tpe) and int(got[3].item()) == nd
+
+
 @pytest.mark.parametrize("limit", [1, 1500, 4096, 8191, 8192, 9000])
 def test_preprocessing_overflow(limit):
     T, E, K, pad = 2048, 16, 4, 32
