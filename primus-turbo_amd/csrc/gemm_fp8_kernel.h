@@ -27,6 +27,7 @@
 //     neighbourhoods of the tile grid.
 #pragma once
 #include "pt_common.h"
+#include "store_window.h"
 
 #include <atomic>
 #include <type_traits>
@@ -299,14 +300,13 @@ template <bool ACC_IN_AGPR> __device__ __forceinline__ f32x4 read_acc(const f32x
 //   stores of the row groups at or beyond it. ROWCHECK = false: every row group is stored; for callers
 //   whose sub-tile is known to lie inside.
 //   BUF = true, sub-tiles over the last columns: buffer stores from the sub-tile's first element
-//   `base`; `left` are the bytes from there to the end of the matrix' rows (of the group's rows), so a
-//   row behind the end is out of range, and a lane whose columns lie at or behind `cols` (the
-//   sub-tile's columns inside the matrix) takes an offset with its top bit set. The bounds check drops
-//   those stores; no test, no branch. 3001 x 2880 x 4096 in 256 x 256 tiles: 67 us while such sub-tiles
+//   `base` through a window of `left` bytes (store_window.h): a row behind the end of the matrix (of the
+//   group) is out of range, and a lane whose columns lie at or behind `cols` (the sub-tile's columns
+//   inside the matrix) takes an offset behind every window. The bounds check drops those stores; no
+//   test, no branch. 3001 x 2880 x 4096 in 256 x 256 tiles: 67 us while such sub-tiles
 //   left element by element, 48 this way. (Used for every sub-tile it costs the MX kernels 1 %, present
 //   in the grouped MX kernels, whose N is whole tiles as a rule, 2 %; the block-scaled kernels have no
 //   registers for it, 8192^3 went from 0.446 to 0.544 ms. HANG_COLS says who has it.)
-constexpr uint32_t OUT_OF_RANGE = 0x80000000u;
 template <typename T, int TM, int TN, int MODE, bool ACC_IN_AGPR, bool BUF, bool ROWCHECK>
 __device__ __forceinline__ int epilogue_inner(uint8_t *base, uint32_t left, const int64_t row_bytes, const int cols,
                                               const int64_t rows_left, bool accu, const f32x4 (&acc)[TM][TN],
@@ -320,7 +320,8 @@ __device__ __forceinline__ int epilogue_inner(uint8_t *base, uint32_t left, cons
     const int      c0    = F32 ? 4 * lg : 16 * (lg & 1) + 8 * (lg >> 1);
     const uint32_t row16 = 16u * static_cast<uint32_t>(row_bytes);
     [[maybe_unused]] const uint32_t voff0 = static_cast<uint32_t>(lm) * static_cast<uint32_t>(row_bytes) + c0 * static_cast<uint32_t>(sizeof(T));
-    [[maybe_unused]] auto voff = [&](int j) { return (c0 + j * (F32 ? 16 : 32) < cols ? voff0 : OUT_OF_RANGE) + j * 64; };
+    [[maybe_unused]] auto voff = [&](int j) { return window_offset(voff0, c0 + j * (F32 ? 16 : 32), cols, j * 64); };
+    static_assert(!BUF || TM <= WINDOW_MAX_GROUPS, "row groups of a window");
     [[maybe_unused]] uint8_t *row = base + lm * row_bytes + c0 * static_cast<int>(sizeof(T));
     int stores = 0;
     static_for<0, TM>([&](auto ic) {
@@ -451,7 +452,7 @@ __device__ __forceinline__ int epilogue_inner(uint8_t *base, uint32_t left, cons
         }
         if constexpr (BUF) {
             base += row16;
-            left = left > row16 ? left - row16 : 0u;
+            left = window_next(left, row16);
         } else {
             row += row16;
         }
@@ -556,13 +557,10 @@ __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM
         const int stores = by_type(std::false_type{}, 0u, 0);
         return whole_m ? stores : 0;
     }
-    // (a sub-tile's rows are addressed with 31-bit offsets)
-    if (HANG_COLS && aligned && a.N < (1 << 22)) {
-        if constexpr (HANG_COLS) {
-            const int64_t bytes = ((m_end - wm_base) * a.N - wn_base) * ES;
-            by_type(std::true_type{}, bytes < 0 ? 0u : (bytes > 0xffffffffll ? 0xffffffffu : static_cast<uint32_t>(bytes)),
+    if (HANG_COLS && aligned && a.N < WINDOW_MAX_N) {
+        if constexpr (HANG_COLS)
+            by_type(std::true_type{}, window_bytes(m_end, wm_base, wn_base, a.N, ES),
                     static_cast<int>(a.N - wn_base < TN * 16 ? a.N - wn_base : TN * 16));
-        }
     } else {
         const bool quads = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
         static_for<0, TM>([&](auto ic) {
