@@ -168,7 +168,8 @@ PT_API int pt_dequantize_fp8_tensorwise(const void *q, int q_dtype, int64_t nume
  * axis is the last, contiguous one). One scale per (b, n): scale_inv holds B*N
  * floats; numerics per scale as tensorwise (eps 1e-12).
  *
- * scale_in : optional precomputed scales (B*N floats); NULL = dynamic amax.
+ * scale_in : optional precomputed scales (B*N floats); NULL = dynamic amax. With N > 1 it may be
+ *            scale_inv's own storage, which then holds the inverses.
  */
 PT_API int pt_quantize_fp8_rowwise(const void *x, int x_dtype, int64_t B, int64_t M, int64_t N,
                                    void *q, int q_dtype, const float *scale_in, float *scale_inv,

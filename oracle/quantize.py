@@ -113,11 +113,14 @@ def fp8_tensorwise(x: np.ndarray, fmt="e4m3", scale: np.ndarray | None = None):
     return _cast_fp8(x, scale_v, fmt), np.asarray(scale_inv, dtype=F32).reshape(())
 
 
-def fp8_rowwise(x: np.ndarray, axis: int, fmt="e4m3"):
+def fp8_rowwise(x: np.ndarray, axis: int, fmt="e4m3", scale: np.ndarray | None = None):
     """One scale per slice along ``axis`` -> (codes, scale_inv with that axis kept as 1)."""
     fmt = _fmt(fmt)
     x = np.asarray(x, dtype=F32)
     axis = axis if axis >= 0 else x.ndim + axis
+    if scale is not None:
+        scale = np.asarray(scale, dtype=F32)
+        return _cast_fp8(x, scale, fmt), (F32(1.0) / scale).astype(F32)
     amax = _abs_max(x, axis=axis, keepdims=True)
     scale, scale_inv = _scale_from_amax(amax, fmt.max_finite, 1e-12)
     return _cast_fp8(x, scale, fmt), scale_inv

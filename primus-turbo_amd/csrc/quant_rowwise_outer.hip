@@ -153,7 +153,7 @@ __device__ __forceinline__ float outer_scale(const float *__restrict__ amax_or_s
     return qmax / fmaxf(a, 1e-12f);
 }
 
-// Codes in place. scale_inv == nullptr: another launch writes it (the maxima sit in its storage).
+// Codes in place. scale_inv == nullptr: another launch writes it (the maxima or scales sit in its storage).
 template <typename SRC, bool E5M2, int VEC>
 __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t *__restrict__ q,
                                                           const float *__restrict__ amax_or_scale, const bool dynamic,
@@ -296,11 +296,12 @@ __global__ void zero_u32_kernel(uint32_t *p, const int64_t n) {
         p[i] = 0u;
 }
 
-// column maxima -> scale_inv in place, for the form without a workspace
-__global__ void finish_scale_inv_kernel(float *scale_inv, const int64_t n, const float qmax) {
+// column maxima (dynamic) or given scales -> scale_inv in place: for the form without a workspace, and for
+// scales that are given in scale_inv's own storage
+__global__ void finish_scale_inv_kernel(float *scale_inv, const bool dynamic, const int64_t n, const float qmax) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n)
-        scale_inv[i] = 1.0f / (qmax / fmaxf(scale_inv[i], 1e-12f));
+        scale_inv[i] = 1.0f / (dynamic ? qmax / fmaxf(scale_inv[i], 1e-12f) : scale_inv[i]);
 }
 
 // Row chunks per column strip: about four workgroups per CU over all strips, at least 32 rows each (a
@@ -353,7 +354,7 @@ static int launch_outer(const SRC &src, bool vec, int64_t B, int64_t M, int64_t 
         else
             quant_outer_kernel<SRC, E5M2, 1><<<g, 256, 0, st>>>(src, q, from, dynamic, n, to, M, N, rows_per, qmax);
         if (to == nullptr)
-            finish_scale_inv_kernel<<<gs, 256, 0, st>>>(scale_inv, B * N, qmax);
+            finish_scale_inv_kernel<<<gs, 256, 0, st>>>(scale_inv, dynamic, B * N, qmax);
     }
     return check_launch("quant_outer_kernel");
 }
