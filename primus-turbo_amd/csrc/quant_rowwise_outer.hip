@@ -230,7 +230,9 @@ __global__ __launch_bounds__(256) void quant_outer_t_kernel(const SRC src, uint8
     __shared__ uint32_t t[128 * P];
     __shared__ float    s[128];
     const int           tid = threadIdx.x;
-    const int64_t       b = blockIdx.z, n0 = static_cast<int64_t>(blockIdx.x) * 128, m0 = static_cast<int64_t>(blockIdx.y) * 128;
+    // (tiles numbered along x, columns first: the y extent of a grid ends at 65535, 8.4 million rows)
+    const uint32_t      nt = static_cast<uint32_t>((N + 127) / 128), tn = blockIdx.x % nt, tm = blockIdx.x / nt;
+    const int64_t       b = blockIdx.z, n0 = static_cast<int64_t>(tn) * 128, m0 = static_cast<int64_t>(tm) * 128;
     const int           cc = tid & 15, rg = tid >> 4; // eight columns, four rows (two rounds of 64 rows)
     const int64_t       n = n0 + cc * 8;
     typename SRC::Raw   raw[VEC8 ? 8 : 1];
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(256) void quant_outer_t_kernel(const SRC src, uint8
         float sc = 0.f;
         if (n0 + tid < N) {
             sc = outer_scale(part, true, b, n0 + tid, N, chunks, qmax);
-            if (blockIdx.y == 0)
+            if (tm == 0)
                 scale_inv[b * N + n0 + tid] = 1.0f / sc;
         }
         s[tid] = sc;
@@ -329,7 +331,7 @@ static int launch_outer(const SRC &src, bool vec, int64_t B, int64_t M, int64_t 
             col_amax_kernel<SRC, 1, false><<<g, 256, 0, st>>>(src, ws, M, N, rows_per);
     }
     if (qt != nullptr) {
-        const dim3 gt(static_cast<unsigned>(cdiv(N, 128)), static_cast<unsigned>(cdiv(ldt, 128)), static_cast<unsigned>(B));
+        const dim3 gt(static_cast<unsigned>(cdiv(N, 128) * cdiv(ldt, 128)), 1, static_cast<unsigned>(B));
         if (vec)
             quant_outer_t_kernel<SRC, E5M2, true><<<gt, 256, 0, st>>>(src, qt, ws, parts, scale_inv, M, N, ldt, qmax);
         else
@@ -421,7 +423,9 @@ int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_s
     PT_REQUIRE(x && scale_inv, "NULL tensor pointer");
     PT_REQUIRE(q_t == nullptr || (ld_t >= M && ld_t % 16 == 0 && aligned_to(q_t, 16)),
                "transposed rows must be 16-byte aligned and hold M codes");
-    PT_REQUIRE(B < 65536 && cdiv(q_t != nullptr ? ld_t : M, 128) < 65536, "grid dimension out of range");
+    // (the rows that pt_quantize_fp8_rowwise takes; transposed, 2^32 threads along x)
+    PT_REQUIRE(B < 65536 && cdiv(M, 256) < 65536 && (q_t == nullptr || cdiv(N, 128) * cdiv(ld_t, 128) < (1LL << 24)),
+               "grid dimension out of range");
     if (workspace == nullptr || workspace_bytes < pt_quantize_fp8_rowwise_outer_workspace_bytes(B, M, N) || !aligned_to(workspace, 16))
         return fail(PT_ERR_WORKSPACE, "pt_quantize_fp8_rowwise_outer: workspace missing, too small or misaligned");
     auto       st = static_cast<hipStream_t>(stream);

@@ -69,3 +69,23 @@ def test_given_scales(native_lib, shape, in_place):
     N.check(native_lib.pt_quantize_fp8_rowwise(N.ptr(xd), N.dtype_code(xd.dtype), B, M, n, N.ptr(q), N.dtype_code(q.dtype),
                                                N.ptr(given), N.ptr(sinv), N.stream_of(xd)))
     assert np.array_equal(bits_np(sinv), osinv.view(np.uint32)) and np.array_equal(codes_np(q), oq)
+
+
+def test_more_rows_than_a_grid_has_blocks_along_y(native_lib):
+    """128 rows for each of 65535 blocks and a few more: the scales are the columns' maxima, the codes those of
+    the same rows under given scales, and the transposed codes the same codes."""
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as I
+
+    M, n = 128 * 65535 + 200, 8
+    x = torch.randn(M, n, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda", dtype=torch.bfloat16)
+    amax = to_f32_np(x.abs().amax(0, keepdim=True))
+    _, osinv = Q.fp8_rowwise(amax, 0, "e4m3")
+    scale = torch.from_numpy(np.float32(448) / amax).cuda()
+    q, sinv = I.quantize_fp8_rowwise_impl(x, torch.float8_e4m3fn, 0)
+    assert np.array_equal(bits_np(sinv), osinv.view(np.uint32))
+    for m in (0, M // 2, M - 1000):
+        part, _ = torch.ops.primus_turbo_cpp_extension.quantize_fp8_rowwise(x[m : m + 1000].contiguous(), torch.float8_e4m3fn, 0, scale)
+        assert torch.equal(q[m : m + 1000].view(torch.uint8), part.view(torch.uint8))
+    qt, sinv_t = I.quant_fp8_rowwise_t_impl(x, None, x.dtype, torch.float8_e4m3fn, 128)
+    assert torch.equal(sinv_t, sinv) and torch.equal(qt[:, :M].view(torch.uint8), q.view(torch.uint8).t())
+    assert not qt[:, M:].view(torch.uint8).any()
