@@ -178,7 +178,7 @@ PT_API int pt_dequantize_fp8_rowwise(const void *q, int q_dtype, int64_t B, int6
                                      const float *scale_inv, void *y, int y_dtype, void *stream);
 
 /* The same for a reduced axis that is not the contiguous one (N > 1), dynamic scales, in two launches
- * over a workspace (contents need no initialisation). x holds 16- / 32-bit values, or FP8 codes with
+ * (three for a tall, narrow matrix) over a workspace (contents need no initialisation). x holds 16- / 32-bit values, or FP8 codes with
  * one scale per row (row_scale_inv, B*M floats): the values are then the de-quantized codes rounded to
  * hp_dtype, i.e. de-quantize along the rows + quantize along the columns in one step, same bits (what
  * the backward of a ROWWISE product does with its forward operands, primus_turbo/pytorch/ops/

@@ -3,9 +3,11 @@
 // axis != -1, csrc/pytorch/quantization/quantization.cpp:110-208).
 //
 // Two launches: column abs-max of row chunks into a small array of partial maxima, then scale and
-// cast. Both walk rows with 64 lanes x 8 columns, eight rows requested back to back per lane; the
-// second launch reads its columns' partial maxima (at most 64 x 512 floats from the L2) and so needs
-// neither a zero-fill and atomics before it nor a scale_inv pass behind it.
+// cast. Both walk rows with 8 columns per lane, eight rows requested back to back; the second launch
+// reads its columns' partial maxima (at most 64 x 512 floats from the L2) and so needs neither a
+// zero-fill and atomics before it nor a scale_inv pass behind it. A wavefront covers 512 columns of one
+// row or, in a narrower matrix, several rows; a matrix with more rows than 64 chunks are good for takes a
+// third launch, after which the maxima of any number of chunks meet by atomics (outer_plan).
 //
 // What it reads and how it writes are template choices:
 //   * the source is the 16- / 32-bit tensor, or FP8 codes with a scale per row: the value is then the
@@ -82,25 +84,26 @@ template <typename T, bool SRC_E5M2> struct OuterSrcCodes {
 
 constexpr int RO_ROWS = 8; // rows a lane requests back to back
 
-// Abs-max of a row chunk for 64 * VEC columns: part[(b * chunks + chunk) * N + n], or, without a
-// workspace, an integer atomic max into amax[b * N + n] (non-negative floats order like integers).
+// Abs-max of a row chunk for VEC << lc columns: part[(b * chunks + chunk) * N + n], or an integer atomic
+// max into amax[b * N + n] (non-negative floats order like integers). 1 << lc lanes share a row, so a
+// wavefront covers 64 >> lc rows at once.
 template <typename SRC, int VEC, bool ATOMIC>
 __global__ __launch_bounds__(256) void col_amax_kernel(const SRC src, float *__restrict__ out, const int64_t M, const int64_t N,
-                                                       const int64_t rows_per) {
-    constexpr int    W = 64 * VEC;
-    __shared__ float s[4][W];
+                                                       const int64_t rows_per, const int lc) {
+    __shared__ float s[4][64 * VEC];
     const int        lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t    b = blockIdx.z, n = static_cast<int64_t>(blockIdx.x) * W + lane * VEC;
+    const int        W = VEC << lc, col = (lane & ((1 << lc) - 1)) * VEC, rows = 64 >> lc; // rows of a wavefront
+    const int64_t    b = blockIdx.z, n = static_cast<int64_t>(blockIdx.x) * W + col;
     const int64_t    m0 = blockIdx.y * rows_per, m1 = (m0 + rows_per < M) ? m0 + rows_per : M;
     float            a[VEC] = {};
     if (n < N) {
-        for (int64_t m = m0 + wave; m < m1; m += 4 * RO_ROWS) {
+        for (int64_t m = m0 + wave * rows + (lane >> lc); m < m1; m += 4 * RO_ROWS * rows) {
             // (a row behind the chunk's end re-reads the first one of the run: the maximum is the same)
             if constexpr (VEC == 8) {
                 typename SRC::Raw r[RO_ROWS];
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k) {
-                    const int64_t row = b * M + (m + 4 * k < m1 ? m + 4 * k : m);
+                    const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
                     r[k]              = src.load8(row, row * N + n);
                 }
 #pragma unroll
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const SRC src, float *__r
                 float f[RO_ROWS];
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k) {
-                    const int64_t row = b * M + (m + 4 * k < m1 ? m + 4 * k : m);
+                    const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
                     f[k]              = src.get1(row, row * N + n);
                 }
 #pragma unroll
@@ -124,9 +127,14 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const SRC src, float *__r
             }
         }
     }
+    for (int d = 1 << lc; d < 64; d <<= 1) // the rows of the wavefront
 #pragma unroll
-    for (int e = 0; e < VEC; ++e)
-        s[wave][lane * VEC + e] = a[e];
+        for (int e = 0; e < VEC; ++e)
+            a[e] = fmaxf(a[e], __shfl_xor(a[e], d));
+    if (lane < 1 << lc)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            s[wave][col + e] = a[e];
     __syncthreads();
     for (int c = threadIdx.x; c < W; c += 256) {
         const int64_t nc = static_cast<int64_t>(blockIdx.x) * W + c;
@@ -158,10 +166,11 @@ template <typename SRC, bool E5M2, int VEC>
 __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t *__restrict__ q,
                                                           const float *__restrict__ amax_or_scale, const bool dynamic,
                                                           const int chunks, float *__restrict__ scale_inv, const int64_t M,
-                                                          const int64_t N, const int64_t rows_per, const float qmax) {
-    constexpr int    W = 64 * VEC;
-    __shared__ float s[W];
+                                                          const int64_t N, const int64_t rows_per, const int lc,
+                                                          const float qmax) {
+    __shared__ float s[64 * VEC];
     const int        lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int        W = VEC << lc, col = (lane & ((1 << lc) - 1)) * VEC, rows = 64 >> lc; // (as col_amax_kernel)
     const int64_t    b = blockIdx.z, nb = static_cast<int64_t>(blockIdx.x) * W;
     for (int c = threadIdx.x; c < W; c += 256) {
         if (nb + c < N) {
@@ -172,20 +181,20 @@ __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t
         }
     }
     __syncthreads();
-    const int64_t n  = nb + lane * VEC;
+    const int64_t n  = nb + col;
     const int64_t m0 = blockIdx.y * rows_per, m1 = (m0 + rows_per < M) ? m0 + rows_per : M;
     if (n >= N)
         return;
     float sc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e)
-        sc[e] = s[lane * VEC + e];
-    for (int64_t m = m0 + wave; m < m1; m += 4 * RO_ROWS) {
+        sc[e] = s[col + e];
+    for (int64_t m = m0 + wave * rows + (lane >> lc); m < m1; m += 4 * RO_ROWS * rows) {
         if constexpr (VEC == 8) {
             typename SRC::Raw r[RO_ROWS];
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k) {
-                const int64_t row = b * M + (m + 4 * k < m1 ? m + 4 * k : m);
+                const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
                 r[k]              = src.load8(row, row * N + n);
             }
 #pragma unroll
@@ -195,21 +204,21 @@ __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     f[e] = scale_clamp(f[e], sc[e], qmax);
-                if (m + 4 * k < m1)
-                    st64_nt(q + (b * M + m + 4 * k) * N + n,
+                if (m + 4 * k * rows < m1)
+                    st64_nt(q + (b * M + m + 4 * k * rows) * N + n,
                             u32x2{cvt4_fp8<E5M2>(f[0], f[1], f[2], f[3]), cvt4_fp8<E5M2>(f[4], f[5], f[6], f[7])});
             }
         } else {
             float f[RO_ROWS];
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k) {
-                const int64_t row = b * M + (m + 4 * k < m1 ? m + 4 * k : m);
+                const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
                 f[k]              = src.get1(row, row * N + n);
             }
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k)
-                if (m + 4 * k < m1)
-                    q[(b * M + m + 4 * k) * N + n] =
+                if (m + 4 * k * rows < m1)
+                    q[(b * M + m + 4 * k * rows) * N + n] =
                         static_cast<uint8_t>(cvt_pk_fp8<E5M2>(scale_clamp(f[k], sc[0], qmax), 0.f, 0u, false));
         }
     }
@@ -306,55 +315,83 @@ __global__ void finish_scale_inv_kernel(float *scale_inv, const bool dynamic, co
         scale_inv[i] = 1.0f / (dynamic ? qmax / fmaxf(scale_inv[i], 1e-12f) : scale_inv[i]);
 }
 
-// Row chunks per column strip: about four workgroups per CU over all strips, at least 32 rows each (a
-// wavefront's one round of requests), at most 64 (the second launch reads that many maxima per column).
-static int outer_chunks(int64_t B, int64_t M, int64_t strips) {
-    int64_t c = cdiv(4 * 256, strips * B);
-    if (c > cdiv(M, 32))
-        c = cdiv(M, 32);
-    return static_cast<int>(c < 1 ? 1 : (c > 64 ? 64 : c));
+// How a problem is split: 1 << lc lanes across a row (as many as its columns need, at most 64), strips of
+// columns, row chunks for about OUTER_BLOCKS workgroups over all strips; a chunk is at least one round of
+// requests of its workgroup. The second launch reads each chunk's maxima for every column, so there are
+// at most OUTER_PARTS of them, unless a matrix is so tall and narrow that twice as many would pay (lanes
+// that request two bytes need more workgroups than those that request sixteen) and each of OUTER_PARTS
+// chunks had more than 12 (32) rounds: then the maxima meet by atomics behind a zero-fill, one launch more,
+// and the cast is split as if there were none to read. bf16 from memory, in place / transposed, us:
+//   512 columns    16384 rows (8 rounds): two launches 29 / 23, three 25 / 28; 32768 (16): two 54 / 37, three 31 / 34
+//   33 columns, one per lane    32768 rows (16 rounds): two 27 / 25, three 26 / 32; 130, 70000 (34): 67 / 55, 36 / 45
+//   64 columns, 1048576 rows: 64 lanes across a row and two launches 2410 / 834, eight lanes and three 89 / 97
+constexpr int64_t OUTER_BLOCKS = 1024, OUTER_PARTS = 64;
+struct OuterPlan {
+    int     lc;
+    int64_t strips;                 // workgroups along the columns
+    int64_t chunks, rows;           // chunks of the maxima, rows of each
+    int64_t cast_chunks, cast_rows; // the same of a cast behind one maximum (or given scale) per column
+    bool    meet;
+};
+static OuterPlan outer_plan(int64_t B, int64_t M, int64_t N, int vec) {
+    OuterPlan p{};
+    while (p.lc < 6 && (int64_t{vec} << p.lc) < N)
+        ++p.lc;
+    p.strips            = cdiv(N, int64_t{vec} << p.lc);
+    const int64_t round = 4 * RO_ROWS * (64 >> p.lc), most = cdiv(M, round), across = p.strips * B;
+    auto          split = [&](int64_t want, int64_t &chunks, int64_t &rows) {
+        const int64_t c = want < most ? want : most;
+        rows            = cdiv(M, c < 1 ? 1 : c);
+        chunks          = cdiv(M, rows);
+    };
+    const int64_t blocks = cdiv(OUTER_BLOCKS, across), tall = cdiv(vec == 1 ? 1024 : 256, across);
+    p.meet               = tall >= 2 * OUTER_PARTS && cdiv(M, OUTER_PARTS) > (vec == 1 ? 32 : 12) * round;
+    split(p.meet ? tall : (blocks < OUTER_PARTS ? blocks : OUTER_PARTS), p.chunks, p.rows);
+    split(blocks, p.cast_chunks, p.cast_rows);
+    return p;
 }
 
 template <typename SRC, bool E5M2>
 static int launch_outer(const SRC &src, bool vec, int64_t B, int64_t M, int64_t N, [[maybe_unused]] uint8_t *q, uint8_t *qt,
                         int64_t ldt, [[maybe_unused]] const float *scale_in, float *scale_inv, float *ws, hipStream_t st) {
-    const float   qmax     = E5M2 ? 57344.0f : 448.0f;
-    const int64_t strips   = cdiv(N, vec ? 512 : 64);
-    const int     chunks   = outer_chunks(B, M, strips);
-    const int64_t rows_per = cdiv(M, chunks);
-    const dim3    g(static_cast<unsigned>(strips), static_cast<unsigned>(cdiv(M, rows_per)), static_cast<unsigned>(B));
-    const int     parts = static_cast<int>(g.y);
-    if (ws != nullptr) {
-        if (vec)
-            col_amax_kernel<SRC, 8, false><<<g, 256, 0, st>>>(src, ws, M, N, rows_per);
-        else
-            col_amax_kernel<SRC, 1, false><<<g, 256, 0, st>>>(src, ws, M, N, rows_per);
+    const float     qmax    = E5M2 ? 57344.0f : 448.0f;
+    const OuterPlan p       = outer_plan(B, M, N, vec ? 8 : 1);
+    const bool      dynamic = scale_in == nullptr, meet = p.meet || ws == nullptr;
+    float          *amax    = ws != nullptr ? ws : scale_inv; // (without a workspace the maxima meet in scale_inv's storage)
+    const int       parts   = meet ? 1 : static_cast<int>(p.chunks);
+    const dim3      g(static_cast<unsigned>(p.strips), static_cast<unsigned>(p.chunks), static_cast<unsigned>(B));
+    const unsigned  gs = static_cast<unsigned>(cdiv(B * N, 256));
+    if (dynamic) {
+        if (meet) {
+            zero_u32_kernel<<<gs, 256, 0, st>>>(reinterpret_cast<uint32_t *>(amax), B * N);
+            if (vec)
+                col_amax_kernel<SRC, 8, true><<<g, 256, 0, st>>>(src, amax, M, N, p.rows, p.lc);
+            else
+                col_amax_kernel<SRC, 1, true><<<g, 256, 0, st>>>(src, amax, M, N, p.rows, p.lc);
+        } else if (vec) {
+            col_amax_kernel<SRC, 8, false><<<g, 256, 0, st>>>(src, amax, M, N, p.rows, p.lc);
+        } else {
+            col_amax_kernel<SRC, 1, false><<<g, 256, 0, st>>>(src, amax, M, N, p.rows, p.lc);
+        }
     }
     if (qt != nullptr) {
         const dim3 gt(static_cast<unsigned>(cdiv(N, 128) * cdiv(ldt, 128)), 1, static_cast<unsigned>(B));
         if (vec)
-            quant_outer_t_kernel<SRC, E5M2, true><<<gt, 256, 0, st>>>(src, qt, ws, parts, scale_inv, M, N, ldt, qmax);
+            quant_outer_t_kernel<SRC, E5M2, true><<<gt, 256, 0, st>>>(src, qt, amax, parts, scale_inv, M, N, ldt, qmax);
         else
-            quant_outer_t_kernel<SRC, E5M2, false><<<gt, 256, 0, st>>>(src, qt, ws, parts, scale_inv, M, N, ldt, qmax);
+            quant_outer_t_kernel<SRC, E5M2, false><<<gt, 256, 0, st>>>(src, qt, amax, parts, scale_inv, M, N, ldt, qmax);
         return check_launch("quant_outer_t_kernel");
     }
     if constexpr (SRC::IN_PLACE) {
-        const bool     dynamic = scale_in == nullptr;
-        const unsigned gs      = static_cast<unsigned>(cdiv(B * N, 256));
-        if (dynamic && ws == nullptr) { // the maxima meet in scale_inv's storage
-            zero_u32_kernel<<<gs, 256, 0, st>>>(reinterpret_cast<uint32_t *>(scale_inv), B * N);
-            if (vec)
-                col_amax_kernel<SRC, 8, true><<<g, 256, 0, st>>>(src, scale_inv, M, N, rows_per);
-            else
-                col_amax_kernel<SRC, 1, true><<<g, 256, 0, st>>>(src, scale_inv, M, N, rows_per);
-        }
-        const float *from = dynamic ? (ws != nullptr ? ws : scale_inv) : scale_in;
+        const float *from = dynamic ? amax : scale_in;
         float       *to   = from != scale_inv ? scale_inv : nullptr;
-        const int    n    = ws != nullptr ? parts : 1;
+        const bool   one  = !dynamic || meet;
+        const dim3   gc(g.x, static_cast<unsigned>(one ? p.cast_chunks : p.chunks), g.z);
+        const int64_t rows = one ? p.cast_rows : p.rows;
         if (vec)
-            quant_outer_kernel<SRC, E5M2, 8><<<g, 256, 0, st>>>(src, q, from, dynamic, n, to, M, N, rows_per, qmax);
+            quant_outer_kernel<SRC, E5M2, 8><<<gc, 256, 0, st>>>(src, q, from, dynamic, parts, to, M, N, rows, p.lc, qmax);
         else
-            quant_outer_kernel<SRC, E5M2, 1><<<g, 256, 0, st>>>(src, q, from, dynamic, n, to, M, N, rows_per, qmax);
+            quant_outer_kernel<SRC, E5M2, 1><<<gc, 256, 0, st>>>(src, q, from, dynamic, parts, to, M, N, rows, p.lc, qmax);
         if (to == nullptr)
             finish_scale_inv_kernel<<<gs, 256, 0, st>>>(scale_inv, dynamic, B * N, qmax);
     }
@@ -402,8 +439,14 @@ extern "C" {
 size_t pt_quantize_fp8_rowwise_outer_workspace_bytes(int64_t B, int64_t M, int64_t N) {
     if (B <= 0 || M <= 0 || N <= 0)
         return 0;
-    const int c8 = outer_chunks(B, M, cdiv(N, 512)), c1 = outer_chunks(B, M, cdiv(N, 64));
-    return static_cast<size_t>(B * (c8 > c1 ? c8 : c1) * N) * sizeof(float);
+    // (the wider lanes' plan may not be taken, so the workspace serves either)
+    int64_t parts = 1;
+    for (const int vec : {8, 1}) {
+        const OuterPlan p = outer_plan(B, M, N, vec);
+        if (!p.meet && p.chunks > parts)
+            parts = p.chunks;
+    }
+    return static_cast<size_t>(B * parts * N) * sizeof(float);
 }
 
 int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_scale_inv, int hp_dtype, int64_t B, int64_t M,

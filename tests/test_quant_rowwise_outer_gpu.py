@@ -13,9 +13,12 @@ pytestmark = pytest.mark.gpu
 # edges of the 512-column strips, of the 128 x 128 tiles and of the eight-row runs; columns that are no
 # multiple of eight take the one-column lanes
 SHAPES = [(1, 8), (7, 8), (33, 9), (128, 128), (129, 136), (257, 520), (1000, 516), (3001, 264), (3, 65, 72), (2, 5, 130, 16)]
+# a wavefront over several rows, with whole and with idle lanes, and with more rows than one round of a
+# workgroup; rows for more than 64 chunks, whose maxima meet by atomics
+SPLITS = [(300, 1), (300, 3), (4099, 16), (700, 24), (1000, 40), (70, 33, 24), (25000, 264), (66000, 33)]
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + SPLITS)
 @pytest.mark.parametrize("src,dtype", [(torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float8_e5m2),
                                        (torch.float32, torch.float8_e4m3fn)])
 def test_outer_axis(native_lib, shape, src, dtype):
@@ -52,7 +55,25 @@ def test_codes_quantized_again(native_lib, shape, src, dtype):
     assert np.array_equal(got[..., :M], np.swapaxes(oq, -1, -2)) and not got[..., M:].any()
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SPLITS)
+@pytest.mark.parametrize("src,dtype", [(torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float8_e5m2),
+                                       (torch.float32, torch.float8_e4m3fn)])
+def test_codes_quantized_again_is_three_steps(native_lib, shape, src, dtype):
+    """The same bits as de-quantize, quantize, transpose. (Against those launches and not the oracle's rounding:
+    over ten million fp16 elements a dozen de-quantized values differ from it in their last bit, the GPU
+    rounding code times scale once where the oracle rounds to fp32 and then to fp16.)"""
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as I
+
+    nd, M = len(shape), shape[-2]
+    codes, s1 = I.quantize_fp8_rowwise_impl(bf16_randn(shape, seed=22, outlier_frac=0.01, dtype=src).cuda(), dtype, nd - 1)
+    want, sinv = I.quantize_fp8_rowwise_impl(I.dequantize_fp8_rowwise_impl(codes, src, nd - 1, s1), dtype, nd - 2)
+    qt, sinv_t = I.quant_fp8_rowwise_t_impl(codes, s1, src, dtype, 16)
+    qt = qt.view(torch.uint8)
+    assert torch.equal(sinv_t, sinv) and torch.equal(qt[..., :M], want.view(torch.uint8).transpose(-1, -2))
+    assert not qt[..., M:].any()
+
+
+@pytest.mark.parametrize("shape", SHAPES + SPLITS)
 @pytest.mark.parametrize("in_place", [False, True])
 def test_given_scales(native_lib, shape, in_place):
     """Scales given by the caller, in a buffer of their own or in scale_inv's."""
