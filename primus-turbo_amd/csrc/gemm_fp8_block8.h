@@ -313,7 +313,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         const int64_t wm_base = cur_t.m0 + wm * (TM * 16), wn_base = cur_t.n0 + wn * (TN * 16);
         // stores of the epilogue's straight-line path (0, 16 or 32: the cases of the barrier's wait)
         pending = __builtin_amdgcn_readfirstlane(
-            epilogue<TM, TN, SCALE_BLOCK, false>(a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane));
+            epilogue<TM, TN, SCALE_BLOCK, false, true, false, false>(a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane));
         static_assert(TM * TN == 32, "the barrier's wait distinguishes 16 and 32 stores in flight");
 
         if (next_tile >= total)

@@ -460,17 +460,9 @@ __device__ __forceinline__ int epilogue_inner(uint8_t *base, uint32_t left, cons
     return stores; // (a compile-time constant after unrolling: TM * TN, or TM * TN / 2 for 16-bit outputs)
 }
 
-__device__ __forceinline__ void store_elem(float f, uint8_t *q, int out_dtype, bool accu) {
-    if (out_dtype == PT_DTYPE_F32) {
-        float *p = reinterpret_cast<float *>(q);
-        *p       = accu ? f + *p : f;
-    } else if (out_dtype == PT_DTYPE_BF16) {
-        bf16_t *p = reinterpret_cast<bf16_t *>(q);
-        *p        = HP<bf16_t>::from_f32(accu ? f + HP<bf16_t>::to_f32(*p) : f);
-    } else {
-        f16_t *p = reinterpret_cast<f16_t *>(q);
-        *p       = HP<f16_t>::from_f32(accu ? f + HP<f16_t>::to_f32(*p) : f);
-    }
+template <typename T> __device__ __forceinline__ void store_elem(float f, uint8_t *q, bool accu) {
+    T *p = reinterpret_cast<T *>(q);
+    *p   = HP<T>::from_f32(accu ? f + HP<T>::to_f32(*p) : f);
 }
 
 // Four consecutive values of one row (8 or 16 bytes, aligned): what a lane holds of an MFMA tile.
@@ -490,6 +482,42 @@ template <typename T> __device__ __forceinline__ void store_quad(f32x4 v, uint8_
     }
 }
 
+// A sub-tile whose rows are no aligned 16-byte groups, or that hangs over the last columns of a kernel
+// without a window: a lane's four values of each MFMA tile by themselves, with a test of row and column.
+// QUADS: the matrix' rows are whole 4-column groups, so the four are wholly in or out and leave in one
+// store (block-scaled 286 x 1440 x 1792: 16.1 us element by element, 13.6 this way).
+// `row` is the lane's first value; rows / cols are what is left of the matrix from there.
+template <typename T, bool QUADS, int TM, int TN, int MODE, bool ACC_IN_AGPR>
+__device__ __forceinline__ void epilogue_pieces(uint8_t *row, const int64_t step, const int64_t rows, const int64_t cols,
+                                                const bool accu, const f32x4 (&acc)[TM][TN], const float (&sa)[TM],
+                                                const f32x4 (&sb)[TN]) {
+    static_for<0, TM>([&](auto ic) {
+        constexpr int i = ic;
+        static_for<0, TN>([&](auto jc) {
+            constexpr int j = jc;
+            f32x4         v = read_acc<ACC_IN_AGPR>(acc[i][j]);
+            if constexpr (MODE == SCALE_VECTOR) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = v[e] * sa[i] * sb[j][e];
+            }
+            if (i * 16 < rows) {
+                if constexpr (QUADS) {
+                    if (j * 16 < cols)
+                        store_quad<T>(v, row + j * 16 * sizeof(T), accu);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (j * 16 + e < cols)
+                            store_elem<T>(v[e], row + (j * 16 + e) * sizeof(T), accu);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        row += step;
+    });
+}
+
 // `Cm` / `sAm` / `sBm` / `m_end` describe the matrix the tile belongs to (the whole problem,
 // or one group's share of it).
 // Returns (uniform over the wavefront) how many of the vector-memory operations it issued are
@@ -501,7 +529,12 @@ template <typename T> __device__ __forceinline__ void store_quad(f32x4 v, uint8_
 // ROWCHECK = false keeps the 16-byte stores for sub-tiles that lie wholly inside the matrix only
 // (a hanging one takes the generic path): for kernels that cannot afford the registers of the
 // row test around their epilogue.
-template <int TM, int TN, int MODE, bool ACC_IN_AGPR, bool ROWCHECK = true, bool HANG_COLS = false>
+// PIECES_APART: the sub-tiles that leave by pieces have code of their own for each output type and width.
+// Where both are chosen at each piece (false), the ways not taken lie between the stores and the 256 x 256
+// vector-scale kernel spills: 3001 x 2882 x 1024 took 83 us, and takes 37. The eight-wavefront block-scaled
+// kernels have no registers for it: the variable-K one spilled four more in its K loop and the 32-expert
+// training step went from 4.54 to 5.02 ms.
+template <int TM, int TN, int MODE, bool ACC_IN_AGPR, bool ROWCHECK = true, bool HANG_COLS = false, bool PIECES_APART = true>
 __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM][TN], uint8_t *Cm,
                                          const float *sAm, const float *sBm, int64_t m_end,
                                          int64_t wm_base, int64_t wn_base, int lane) {
@@ -563,41 +596,61 @@ __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM
                     static_cast<int>(a.N - wn_base < TN * 16 ? a.N - wn_base : TN * 16));
     } else {
         const bool quads = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
-        static_for<0, TM>([&](auto ic) {
-            constexpr int i = ic;
-            static_for<0, TN>([&](auto jc) {
-                constexpr int j = jc;
-                f32x4         v = read_acc<ACC_IN_AGPR>(acc[i][j]);
-                if constexpr (MODE == SCALE_VECTOR) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        v[e] = v[e] * sa[i] * sb[j][e];
-                }
-                // A sub-tile over the last columns of a matrix whose rows are whole 4-column groups: the
-                // lane's four values are wholly in or out and leave in one store (block-scaled
-                // 286 x 1440 x 1792: 16.1 us element by element, 13.6 this way).
-                if (m0 + i * 16 < m_end) {
-                    if (quads) {
-                        if (n0 + j * 16 < a.N) {
-                            uint8_t *q = row + j * 16 * ES;
-                            if (a.out_dtype == PT_DTYPE_BF16)
-                                store_quad<bf16_t>(v, q, accu);
-                            else if (a.out_dtype == PT_DTYPE_F16)
-                                store_quad<f16_t>(v, q, accu);
-                            else
-                                store_quad<float>(v, q, accu);
-                        }
-                    } else {
+        auto by_type_apart = [&](auto tag) {
+            using T = decltype(tag);
+            if (quads)
+                epilogue_pieces<T, true, TM, TN, MODE, ACC_IN_AGPR>(row, step * ES, rows_left, a.N - n0, accu, acc, sa, sb);
+            else
+                epilogue_pieces<T, false, TM, TN, MODE, ACC_IN_AGPR>(row, step * ES, rows_left, a.N - n0, accu, acc, sa, sb);
+        };
+        if constexpr (PIECES_APART) {
+            if (a.out_dtype == PT_DTYPE_BF16)
+                by_type_apart(bf16_t{});
+            else if (a.out_dtype == PT_DTYPE_F16)
+                by_type_apart(f16_t{});
+            else
+                by_type_apart(0.f);
+        } else {
+            static_for<0, TM>([&](auto ic) {
+                constexpr int i = ic;
+                static_for<0, TN>([&](auto jc) {
+                    constexpr int j = jc;
+                    f32x4         v = read_acc<ACC_IN_AGPR>(acc[i][j]);
+                    if constexpr (MODE == SCALE_VECTOR) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            if (n0 + j * 16 + e < a.N)
-                                store_elem(v[e], row + (j * 16 + e) * ES, a.out_dtype, accu);
+                            v[e] = v[e] * sa[i] * sb[j][e];
                     }
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                    if (m0 + i * 16 < m_end) {
+                        if (quads) {
+                            if (n0 + j * 16 < a.N) {
+                                uint8_t *q = row + j * 16 * ES;
+                                if (a.out_dtype == PT_DTYPE_BF16)
+                                    store_quad<bf16_t>(v, q, accu);
+                                else if (a.out_dtype == PT_DTYPE_F16)
+                                    store_quad<f16_t>(v, q, accu);
+                                else
+                                    store_quad<float>(v, q, accu);
+                            }
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (n0 + j * 16 + e < a.N) {
+                                    uint8_t *q = row + (j * 16 + e) * ES;
+                                    if (a.out_dtype == PT_DTYPE_F32)
+                                        store_elem<float>(v[e], q, accu);
+                                    else if (a.out_dtype == PT_DTYPE_BF16)
+                                        store_elem<bf16_t>(v[e], q, accu);
+                                    else
+                                        store_elem<f16_t>(v[e], q, accu);
+                                }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                row += step * ES;
             });
-            row += step * ES;
-        });
+        }
     }
     return 0;
 }
@@ -749,6 +802,9 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     constexpr int NSTAGE = gemm_stages(TM, TN, FA == 4);
     constexpr int LA = BM / 8 / GEMM_WAVES, LB = BN / 8 / GEMM_WAVES; // data copies per wave and slab
     constexpr int NLD = LA + LB;
+    // (see epilogue. Nor have the block-scaled kernels with vectors of B scales or the largest tile: with it the
+    // training step of an 8192 x 8192 x 8192 layer took 1781 us, without 1752)
+    constexpr bool PIECES_APART = MODE != SCALE_BLOCK || (!SB_VEC && TM * TN < 64);
     // MXFP4: a 128-byte slab row holds 256 E2M1 codes, i.e. two MFMAs' worth of K; a lane's two
     // 16-byte fragment reads (chunks g and 4 + g) then feed one MFMA each instead of one together
     constexpr bool F4 = FA == 4;
@@ -1273,7 +1329,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
                 asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
             PT_GEMM_TRACE_POINT(5);
             // (0, ST16 or ST32: the stores of the epilogue's straight-line path)
-            pending = __builtin_amdgcn_readfirstlane(epilogue<TM, TN, MODE, MODE != SCALE_BLOCK, true, MODE != SCALE_BLOCK && GMODE == GROUP_NONE>(
+            pending = __builtin_amdgcn_readfirstlane(epilogue<TM, TN, MODE, MODE != SCALE_BLOCK, true, MODE != SCALE_BLOCK && GMODE == GROUP_NONE, PIECES_APART>(
                 a, acc, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane));
         } else {
             const int ES     = a.out_dtype == PT_DTYPE_F32 ? 4 : 2;
@@ -1304,7 +1360,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
                 uint8_t *Cg = cur_t.C + static_cast<int64_t>(g) * a.c_gstride * ES;
                 // (the stores of a group's result are waited for at the next barrier here: leaving them in
                 // flight, as the row-group mode does, measured no faster in this mode)
-                epilogue<TM, TN, MODE, MODE != SCALE_BLOCK>(a, acc, Cg, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane);
+                epilogue<TM, TN, MODE, MODE != SCALE_BLOCK, true, false, PIECES_APART>(a, acc, Cg, cur_t.sA, cur_t.sB, cur_t.m_end, wm_base, wn_base, lane);
             }
             if (cur_t.g0 >= cur_t.g1 && next_tile < total && nxt_t.KT > 0)
                 request_first_slabs(nxt_t); // (an empty chunk: nothing was in flight)
