@@ -37,6 +37,14 @@ def test_forward_only(native_lib, recipe, quantized, M, N, K):
     assert torch.equal(plain, out.detach()) and not plain.requires_grad
     (gx,) = torch.autograd.grad(out, (xg,), torch.ones_like(out))
     ref = torch.ones(M, N) @ (w.dequantize() if quantized else w).float().cpu()
-    err = (gx.float().cpu() - ref).norm() / ref.norm()
     # E4M3 carries 4 significant bits, E2M1 two: operands rounded to half a unit, both operands
-    assert err < (2 ** -2 if recipe == "mxfp4" else 2 ** -4)
+    bound = 2 ** -2 if recipe == "mxfp4" else 2 ** -4
+    assert (gx.float().cpu() - ref).norm() / ref.norm() < bound
+    if quantized:
+        return
+    wg = w.clone().requires_grad_(True)  # the weight alone
+    out = op(x, wg, trans_b=True, config=cfg)
+    assert torch.equal(plain, out.detach())
+    (gw,) = torch.autograd.grad(out, (wg,), torch.ones_like(out))
+    ref = torch.ones(N, M) @ x.float().cpu()
+    assert (gw.float().cpu() - ref).norm() / ref.norm() < bound

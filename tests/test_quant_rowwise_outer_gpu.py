@@ -74,19 +74,22 @@ def test_codes_quantized_again_is_three_steps(native_lib, shape, src, dtype):
 
 
 @pytest.mark.parametrize("shape", SHAPES + SPLITS)
-@pytest.mark.parametrize("in_place", [False, True])
-def test_given_scales(native_lib, shape, in_place):
-    """Scales given by the caller, in a buffer of their own or in scale_inv's."""
+@pytest.mark.parametrize("src,dtype", [(torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float8_e5m2),
+                                       (torch.float32, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("scales", ["dynamic", "given", "given in place"])
+def test_entry_without_workspace(native_lib, shape, src, dtype, scales):
+    """pt_quantize_fp8_rowwise: scales from the columns' maxima, which meet in scale_inv's storage, or given by
+    the caller in a buffer of their own or in scale_inv's."""
     from primus_turbo import _native as N
 
-    x = bf16_randn(shape, seed=23)
+    x = bf16_randn(shape, seed=23, outlier_frac=0.01, dtype=src)
     axis = len(shape) - 2
     B, M, n = int(np.prod(shape[:-2])), shape[-2], shape[-1]
     scale = torch.rand(*shape[:-2], 1, n, generator=torch.Generator().manual_seed(5)) * 60 + 0.5
-    oq, osinv = Q.fp8_rowwise(to_f32_np(x), axis, "e4m3", scale=scale.numpy())
+    oq, osinv = Q.fp8_rowwise(to_f32_np(x), axis, FMT[dtype], scale=None if scales == "dynamic" else scale.numpy())
     xd, sinv = x.cuda(), scale.cuda()
-    given = sinv if in_place else sinv.clone()
-    q = torch.empty(shape, dtype=torch.float8_e4m3fn, device="cuda")
+    given = {"dynamic": None, "given": sinv.clone(), "given in place": sinv if n > 1 else sinv.clone()}[scales]
+    q = torch.empty(shape, dtype=dtype, device="cuda")
     N.check(native_lib.pt_quantize_fp8_rowwise(N.ptr(xd), N.dtype_code(xd.dtype), B, M, n, N.ptr(q), N.dtype_code(q.dtype),
                                                N.ptr(given), N.ptr(sinv), N.stream_of(xd)))
     assert np.array_equal(bits_np(sinv), osinv.view(np.uint32)) and np.array_equal(codes_np(q), oq)
