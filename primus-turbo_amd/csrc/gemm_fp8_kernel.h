@@ -802,9 +802,11 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     constexpr int NSTAGE = gemm_stages(TM, TN, FA == 4);
     constexpr int LA = BM / 8 / GEMM_WAVES, LB = BN / 8 / GEMM_WAVES; // data copies per wave and slab
     constexpr int NLD = LA + LB;
-    // (see epilogue. Nor have the block-scaled kernels with vectors of B scales or the largest tile: with it the
-    // training step of an 8192 x 8192 x 8192 layer took 1781 us, without 1752)
-    constexpr bool PIECES_APART = MODE != SCALE_BLOCK || (!SB_VEC && TM * TN < 64);
+    // (see epilogue. Nor have registers for it the block-scaled kernels with vectors of B scales or the largest
+    // tile, 8192 x 8192 x 8192 training step 1781 us with it, 1752 without, and the MX kernels of variable K, an
+    // expert layer's weight gradient 275 us with it, 267 without. Of variable K the vector-scale ones gain: 57 -> 50)
+    constexpr bool PIECES_APART = MODE == SCALE_VECTOR || (MODE == SCALE_MX && GMODE != GROUP_K) ||
+                                  (MODE == SCALE_BLOCK && !SB_VEC && TM * TN < 64);
     // MXFP4: a 128-byte slab row holds 256 E2M1 codes, i.e. two MFMAs' worth of K; a lane's two
     // 16-byte fragment reads (chunks g and 4 + g) then feed one MFMA each instead of one together
     constexpr bool F4 = FA == 4;
