@@ -17,11 +17,11 @@
 //   * the codes leave in place ([B, M, N]) or transposed ([B, N, ldt], rows M .. ldt zero): the
 //     transposed form is the K-contiguous operand of the products that reduce over M.
 //
-// Bound by memory traffic. 3001 x 4096 bf16 (24.6 MB in, 12.3 MB out), same box: the launches before
-// these (one 2-byte load in flight per lane, four rows of 64 columns per workgroup and step, 12 row
-// chunks) took 29.6 us for the maxima and 66.3 us for the cast, plus 8.6 us of zero-fill and scale
-// launches; these take 6.2 and 9.1 us. 16384 x 16384: 116 + 174 us (4.6 TB/s over both reads and the
-// write).
+// Bound by memory traffic. 3001 x 4096 bf16 (24.6 MB in, 12.3 MB out) from memory, same box: the launches
+// before these (one 2-byte load in flight per lane, four rows of 64 columns per workgroup and step, 12 row
+// chunks) took 33.6 us for the maxima and 66.7 us for the cast, plus 9.5 us of zero-fill and scale
+// launches; these take 10.1 and 9.3 us. 16384 x 16384: 307 + 326 us, now 151 + 174 (4.1 TB/s over both
+// reads and the write).
 #include "pt_common.h"
 
 namespace pt {
