@@ -129,7 +129,8 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     g.ldb        = need;
     g.sa_m       = sa_ld;
     g.sb_n       = sb_ld;
-    g.kb_valid   = static_cast<int>(kblocks);
+    // whole words of four blocks: the scales travel in words, and the last row's last one ends the array
+    g.kb_valid   = static_cast<int>(round_up(kblocks, 4));
     g.out_dtype  = c_dtype;
     g.accumulate = accumulate;
     if (fp4)

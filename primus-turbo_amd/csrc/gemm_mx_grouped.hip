@@ -124,7 +124,7 @@ int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, int64_t 
         g.ldb            = ldb;
         g.sa_m           = sa_ld;
         g.sb_n           = sb_ld;
-        g.kb_valid       = static_cast<int>(K / 32);
+        g.kb_valid       = static_cast<int>(round_up(K / 32, 4)); // (whole words, see pt_gemm_mx)
         g.out_dtype      = c_dtype;
         g.G              = static_cast<int>(G);
         g.group_offs     = group_offs;

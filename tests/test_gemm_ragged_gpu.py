@@ -68,6 +68,23 @@ def test_ragged_reduction(M, N, K):
     assert torch.equal(got, want), f"{(got != want).sum().item()} of {got.numel()} differ"
 
 
+@pytest.mark.parametrize("cfg", [1, 2, 3, 4])
+@pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4"])
+def test_blocks_that_end_inside_a_scale_word(recipe, cfg):
+    """38 blocks of 32: the last word of the last row of either operand holds two of them."""
+    M, N, K = 333, 264, 1216
+    (a, sa, av), (b, sb, bv) = (_exact_operand(recipe, rows, K, seed, True) for rows, seed in ((M, 0), (N, 1)))
+    sa, sb = (torch.nn.functional.pad(s, (0, 2)) for s in (sa, sb))
+    out = torch.empty(M, N, dtype=torch.float32, device="cuda")
+    impl.TILE_CFG = cfg
+    try:
+        impl._launch(a, sa, False, b, sb, True, out, False, GRAN[recipe], False)
+    finally:
+        impl.TILE_CFG = 0
+    want = (av.double() @ bv.double().T).float()
+    assert torch.equal(out, want), f"{(out != want).sum().item()} of {out.numel()} differ"
+
+
 @pytest.mark.parametrize("recipe,out_dtype,accumulate", [("rowwise", torch.bfloat16, False), ("rowwise", torch.float32, True),
                                                          ("mxfp8", torch.bfloat16, False), ("mxfp4", torch.bfloat16, False)])
 def test_output_above_2_gib(recipe, out_dtype, accumulate):
