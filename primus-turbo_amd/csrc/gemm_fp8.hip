@@ -322,7 +322,10 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     }
 
     const int64_t  Kp  = padded_k(K);
-    const bool     pad = Kp != K;
+    // few output tiles: a kernel that reads rows as they are (gemm_direct.h)
+    const int      direct    = tile_cfg == 0 ? gemm_direct_tile(M, N, K, scale_mode, false) : -1;
+    const bool     unpadded  = direct >= 0 && !trans_a && trans_b && K % 16 == 0;
+    const bool     pad       = Kp != K;
     const uint8_t *A   = static_cast<const uint8_t *>(a);
     const uint8_t *B   = static_cast<const uint8_t *>(b);
     // workspace layout: [scale area of block_scale_copy_pays problems][operand copies]
@@ -343,6 +346,8 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
             return fail(PT_ERR_WORKSPACE, "pt_gemm_fp8: workspace missing, too small or misaligned");
         uint8_t *ws = static_cast<uint8_t *>(workspace) + scale_area;
         if (trans_a || pad) {
+    }
+    if ((trans_a || !trans_b || pad) && !unpadded) {
             if (M * Kp > 0) {
                 if (trans_a) // stored [K, M] -> [M, Kp]
                     launch_transpose(A, ws, 1, K, M, Kp, st);
@@ -386,6 +391,12 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     const int fa = a_dtype == PT_DTYPE_E5M2 ? 1 : 0, fb = b_dtype == PT_DTYPE_E5M2 ? 1 : 0;
     if (scale_mode == SCALE_VECTOR)
         return launch_gemm_vector(g, fa, fb, tile_cfg, st);
+    if (direct >= 0) {
+        g.K = unpadded ? K : round_up(K, KSTEP); // (a padded copy may hold whole slabs of zeros, which have no scales)
+        if (unpadded)
+            g.lda = g.ldb = K;
+        return launch_gemm_direct_mode(g, scale_mode, sb_block == 1, fa, fb, direct, st);
+    }
     return launch_gemm_block(g, fa, fb, sb_block == 1, tile_cfg, st);
 }
 

@@ -1478,3 +1478,7 @@ int launch_transpose_words(const uint32_t *in, uint32_t *out, int64_t R, int64_t
 int  launch_gemm_block(const GemmArgs &a, int fa, int fb, bool sb_vec, int tile_cfg, hipStream_t stream);
 
 } // namespace pt
+// The GEMM for few output tiles (gemm_direct.hip): its tile for an M x N product over rows of row_bytes, or -1
+// where the tiled kernel is the faster one; rows need whole 16-byte groups and pitches below 2^24, no padding.
+int gemm_direct_tile(int64_t M, int64_t N, int64_t row_bytes, int mode, bool fp4);
+int launch_gemm_direct_mode(const GemmArgs &a, int mode, bool sb_vec, int fa, int fb, int tile, hipStream_t stream);

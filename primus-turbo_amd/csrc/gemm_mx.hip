@@ -87,9 +87,11 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
                            aligned_to(a_scale, 4) && aligned_to(b_scale, 4) && sa_ld >= mx_scale_words(K) * 4 &&
                            sb_ld >= mx_scale_words(K) * 4;
     const void *sa_use = a_scale, *sb_use = b_scale;
-    if (copies || wordmajor) {
-        if (workspace == nullptr || workspace_bytes < want_copy || !aligned_to(workspace, 16))
-            return fail(PT_ERR_WORKSPACE, "pt_gemm_mx: workspace missing, too small or misaligned");
+    if ((copies || wordmajor) && (workspace == nullptr || workspace_bytes < want_copy || !aligned_to(workspace, 16)))
+        return fail(PT_ERR_WORKSPACE, "pt_gemm_mx: workspace missing, too small or misaligned");
+    // few output tiles: a kernel that reads rows and scales as they are (gemm_direct.h)
+    const int direct = tile_cfg == 0 && lda < (1LL << 24) && ldb < (1LL << 24) ? gemm_direct_tile(M, N, kbytes, SCALE_MX, fp4) : -1;
+    if ((copies || wordmajor) && direct < 0) {
         uint8_t *ws = static_cast<uint8_t *>(workspace);
         if (wordmajor) {
             const int64_t W = mx_scale_words(K);
@@ -137,6 +139,16 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
         return launch_mx_tiles<4, 4>(g, tile_cfg, st);
     if (!a_e5m2 && !b_e5m2)
         return launch_mx_tiles<0, 0>(g, tile_cfg, st);
+    if (direct >= 0) {
+        if (sa_ld % 4 != 0 || sb_ld % 4 != 0 || !aligned_to(a_scale, 4) || !aligned_to(b_scale, 4)) // (as the tiled kernel)
+            return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
+        g.sa_wpitch = g.sb_wpitch = 0; // (A, B and the scales are the caller's)
+        g.kb_valid = static_cast<int>(kblocks); // (reads byte by byte)
+        g.K   = kbytes;
+        g.lda = lda;
+        g.ldb = ldb;
+        return launch_gemm_direct_mode(g, SCALE_MX, false, fp4 ? 4 : a_e5m2 != 0, b_e5m2 != 0, direct, st);
+    }
     if (!a_e5m2 && b_e5m2)
         return launch_mx_tiles<0, 1>(g, tile_cfg, st);
     if (a_e5m2 && !b_e5m2)
