@@ -181,6 +181,8 @@ static int launch_vector_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stre
         return launch_gemm_cfg<8, 8, SCALE_VECTOR, false, FA, FB>(a, stream);
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_VECTOR, false, FA, FB>(a, stream);
+    if (one_tile_per_cu(a.M, a.N))
+        return launch_gemm_cfg<4, 4, SCALE_VECTOR, false, FA, FB, GROUP_NONE, 4>(a, stream);
     return launch_gemm_cfg<4, 4, SCALE_VECTOR, false, FA, FB>(a, stream);
 }
 
@@ -344,10 +346,10 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     if (trans_a || !trans_b || pad) {
         if (!have_ws)
             return fail(PT_ERR_WORKSPACE, "pt_gemm_fp8: workspace missing, too small or misaligned");
-        uint8_t *ws = static_cast<uint8_t *>(workspace) + scale_area;
-        if (trans_a || pad) {
     }
     if ((trans_a || !trans_b || pad) && !unpadded) {
+        uint8_t *ws = static_cast<uint8_t *>(workspace) + scale_area;
+        if (trans_a || pad) {
             if (M * Kp > 0) {
                 if (trans_a) // stored [K, M] -> [M, Kp]
                     launch_transpose(A, ws, 1, K, M, Kp, st);
@@ -389,14 +391,14 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     g.out_dtype = c_dtype;
     g.accumulate = accumulate;
     const int fa = a_dtype == PT_DTYPE_E5M2 ? 1 : 0, fb = b_dtype == PT_DTYPE_E5M2 ? 1 : 0;
-    if (scale_mode == SCALE_VECTOR)
-        return launch_gemm_vector(g, fa, fb, tile_cfg, st);
     if (direct >= 0) {
         g.K = unpadded ? K : round_up(K, KSTEP); // (a padded copy may hold whole slabs of zeros, which have no scales)
         if (unpadded)
             g.lda = g.ldb = K;
         return launch_gemm_direct_mode(g, scale_mode, sb_block == 1, fa, fb, direct, st);
     }
+    if (scale_mode == SCALE_VECTOR)
+        return launch_gemm_vector(g, fa, fb, tile_cfg, st);
     return launch_gemm_block(g, fa, fb, sb_block == 1, tile_cfg, st);
 }
 

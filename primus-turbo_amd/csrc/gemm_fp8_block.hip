@@ -23,6 +23,10 @@ static int launch_block_tiles(const GemmArgs &a, int tile_cfg, hipStream_t strea
         else
             return launch_gemm_block8<FA, FB>(a, stream);
     }
+    if constexpr (!SB_VEC) {
+        if (tile_cfg == 3 && one_tile_per_cu(a.M, a.N))
+            return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB, GROUP_NONE, 4>(a, stream);
+    }
     if (tile_cfg == 3)
         return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
     if (tile_cfg == 1)

@@ -794,12 +794,12 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 //   * tile boundaries do not drain the pipeline: while a tile's result is written out, the
 //     fragments of the next tile's first slab are already in registers and its second slab is
 //     in flight.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE>
 __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     static_assert(TN % 4 == 0 && TM % 4 == 0, "sub-tiles are multiples of 64 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
-    constexpr int NSTAGE = gemm_stages(TM, TN, FA == 4);
+    constexpr int AHEAD = NSTAGE < 4 ? 2 : NSTAGE - 1; // slabs the copies run ahead of the MFMAs
     constexpr int LA = BM / 8 / GEMM_WAVES, LB = BN / 8 / GEMM_WAVES; // data copies per wave and slab
     constexpr int NLD = LA + LB;
     // (see epilogue. Nor have registers for it the block-scaled kernels with vectors of B scales or the largest
@@ -889,9 +889,9 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     } else {
         total = a.tiles_m * a.tiles_n;
     }
-    const int KT_ALL = static_cast<int>(a.K / KSTEP); // XPIPE: every tile has this many slabs (> 2)
+    const int KT_ALL = static_cast<int>(a.K / KSTEP); // XPIPE: every tile has this many slabs (> AHEAD)
     int       tile   = blockIdx.x;
-    if (tile >= total || (XPIPE && KT_ALL <= 2))
+    if (tile >= total || (XPIPE && KT_ALL <= AHEAD))
         return;
     int     g_cur = 0, g_nxt = 0;
     TileCtx cur_t = make_tile<BM, BN, GMODE, FA == 4>(a, tile, prefix, g_cur);
@@ -1096,7 +1096,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     // which nobody may still be reading) ...
     auto request_first_slabs = [&](const TileCtx &t) {
         loader_to(t);
-        static_for<0, 2>([&](auto st) {
+        static_for<0, AHEAD>([&](auto st) {
             static_for<0, NB>([&](auto c) { issue_part_b(c, st); });
             static_for<0, LA>([&](auto c) { issue_copy(c, st); });
             advance_loader();
@@ -1107,7 +1107,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     // previous tile), the copies of slab 0 are older than the NL copies of slab 1 and copies
     // complete in order, so none of them can be among the NL youngest.
     auto take_first_slab = [&]() {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NL) : "memory");
         __builtin_amdgcn_s_barrier();
         buf = 0;
         read_scales(smem);
@@ -1227,6 +1227,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
             constexpr int COL = NH * TM, SLOTS = TN * COL;
             constexpr int S_B0 = NSTAGE == 2 ? COL : 0, S_B1 = NSTAGE == 2 ? JY * COL : SLOTS * NB / NL;
             constexpr int S_A0 = S_B1, S_A1 = SLOTS;
+            constexpr int LATER = (AHEAD - 2) * NL; // copies of the slabs between the next and the one requested now
             // copies of this slab's schedule issued before slot s
             constexpr auto issued_before = [](int s) {
                 const int b = s <= S_B0 ? 0 : (s >= S_B1 ? NB : (s - S_B0) * NB / (S_B1 - S_B0));
@@ -1259,9 +1260,9 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
                     if constexpr (GMODE == GROUP_NONE) {
                         // (dense problems: few tiles per workgroup, and the case distinction costs
                         // about 1 % of a long K loop: the plain wait)
-                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LA + issued_before(COL)) : "memory");
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LA + LATER + issued_before(COL)) : "memory");
                     } else {
-                        constexpr int W = LA + issued_before(COL);
+                        constexpr int W = LA + LATER + issued_before(COL);
                         asm volatile("s_cmp_eq_u32 %0, 0\n\t"
                                      "s_cbranch_scc1 .Lx0_%=\n\t"
                                      "s_cmp_eq_u32 %0, %4\n\t"
@@ -1286,9 +1287,9 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
                 if constexpr (j == JY - 1) {
                     // ---- barrier Y: the next slab's A part has landed ----
                     if constexpr (GMODE == GROUP_NONE) {
-                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(issued_before(JY * COL)) : "memory");
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER + issued_before(JY * COL)) : "memory");
                     } else {
-                        constexpr int W = issued_before(JY * COL);
+                        constexpr int W = LATER + issued_before(JY * COL);
                         asm volatile("s_cmp_eq_u32 %0, 0\n\t"
                                      "s_cbranch_scc1 .Ly0_%=\n\t"
                                      "s_cmp_eq_u32 %0, %4\n\t"
@@ -1400,10 +1401,10 @@ static inline int vk_pick_chunks(int64_t positions, int64_t grid, int64_t groups
 
 // Upper bound on the number of tiles (exact for the ungrouped case): GROUP_ROWS cannot know
 // the per-group row counts on the host, but every group adds at most one partial tile row.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4)>
 static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
-    constexpr int STAGES  = gemm_stages(TM, TN, FA == 4) * gemm_stage_bytes(TM, TN, MODE, FA == 4);
+    constexpr int STAGES  = NSTAGE * gemm_stage_bytes(TM, TN, MODE, FA == 4);
     // groups whose tile prefix sums fit into the LDS next to the stages
     constexpr int MAX_G   = (160 * 1024 - STAGES) / 4 - 2 < 2048 ? 1024 : 2048;
     constexpr int LDS_MAX = STAGES + (GMODE == GROUP_ROWS ? (MAX_G + 2) * 4 : GMODE == GROUP_K ? (VK_MAX_CHUNKS + 2) * 4 : 0);
@@ -1421,7 +1422,7 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
                              (a.sa_wpitch != 0) != (a.sb_wpitch != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
                              reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
-    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE>;
+    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE>;
     // the attribute belongs to the (kernel, device) pair: one bit per device, set once
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
@@ -1457,6 +1458,16 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
 }
 
 // ---- host helpers shared by the translation units that instantiate the kernel ----
+// 128 x 128 tiles, at most one for each CU: the second workgroup that would share a CU, and hide this one's
+// waits, does not exist, so the LDS it would have held goes into four stages and the copies run three slabs
+// ahead instead of two. 777 x 4096 x 7168 (224 tiles, 56 slabs), vector scales: 42.6 us with two stages, 28.8
+// with four; 256 x 4096 x 4096 18.5 -> 15.4. With more tiles than CUs two workgroups on two stages each are the
+// better use of the LDS: 1400 x 4096 x 4096 (352 tiles) 28.7 us, with four stages 31.6. MXFP8 777 x 4096 x 7168
+// 54.3 -> 45.1, block scales 46.2 -> 41.5; no gain, and two stages, for vectors of scales on both operands (51.2
+// against 50.0) and MXFP4 (1024 x 1024 x 16384 50.3 against 52.9), whose slabs take longer to issue than to fetch.
+static inline bool one_tile_per_cu(int64_t M, int64_t N) {
+    return (M + 127) / 128 * ((N + 127) / 128) <= device_cu_count();
+}
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;
 }
@@ -1476,9 +1487,9 @@ void launch_pad_rows2(const uint8_t *in, uint8_t *out, int64_t R, int64_t C, int
 int launch_transpose_words(const uint32_t *in, uint32_t *out, int64_t R, int64_t W, int64_t pitch, hipStream_t st,
                             int64_t batch = 1);
 int  launch_gemm_block(const GemmArgs &a, int fa, int fb, bool sb_vec, int tile_cfg, hipStream_t stream);
-
-} // namespace pt
 // The GEMM for few output tiles (gemm_direct.hip): its tile for an M x N product over rows of row_bytes, or -1
 // where the tiled kernel is the faster one; rows need whole 16-byte groups and pitches below 2^24, no padding.
 int gemm_direct_tile(int64_t M, int64_t N, int64_t row_bytes, int mode, bool fp4);
 int launch_gemm_direct_mode(const GemmArgs &a, int mode, bool sb_vec, int fa, int fb, int tile, hipStream_t stream);
+
+} // namespace pt

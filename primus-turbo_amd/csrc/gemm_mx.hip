@@ -17,6 +17,10 @@ template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile
         return launch_gemm_cfg<8, 8, SCALE_MX, false, FA, FB>(a, stream);
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_MX, false, FA, FB>(a, stream);
+    if constexpr (FA != 4) {
+        if (one_tile_per_cu(a.M, a.N))
+            return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB, GROUP_NONE, 4>(a, stream);
+    }
     return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB>(a, stream);
 }
 
@@ -135,10 +139,6 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     g.kb_valid   = static_cast<int>(round_up(kblocks, 4));
     g.out_dtype  = c_dtype;
     g.accumulate = accumulate;
-    if (fp4)
-        return launch_mx_tiles<4, 4>(g, tile_cfg, st);
-    if (!a_e5m2 && !b_e5m2)
-        return launch_mx_tiles<0, 0>(g, tile_cfg, st);
     if (direct >= 0) {
         if (sa_ld % 4 != 0 || sb_ld % 4 != 0 || !aligned_to(a_scale, 4) || !aligned_to(b_scale, 4)) // (as the tiled kernel)
             return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
@@ -149,6 +149,10 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
         g.ldb = ldb;
         return launch_gemm_direct_mode(g, SCALE_MX, false, fp4 ? 4 : a_e5m2 != 0, b_e5m2 != 0, direct, st);
     }
+    if (fp4)
+        return launch_mx_tiles<4, 4>(g, tile_cfg, st);
+    if (!a_e5m2 && !b_e5m2)
+        return launch_mx_tiles<0, 0>(g, tile_cfg, st);
     if (!a_e5m2 && b_e5m2)
         return launch_mx_tiles<0, 1>(g, tile_cfg, st);
     if (a_e5m2 && !b_e5m2)
