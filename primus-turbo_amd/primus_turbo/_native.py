@@ -265,13 +265,15 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on ``t``'s device. Kernels are launched on the
-    current device, so that has to be the tensor's."""
-    if t.device.index != torch.cuda.current_device():
+    current device, so that has to be the tensor's. (Without the Stream object that
+    ``torch.cuda.current_stream`` builds: 2.2 -> 0.5 us.)"""
+    index = t.device.index
+    if index != torch.cuda.current_device():
         raise RuntimeError(
             f"primus_turbo: tensor on {t.device} but the current device is cuda:{torch.cuda.current_device()}; "
             "wrap the call in torch.cuda.device(tensor.device)"
         )
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_cuda(*tensors: torch.Tensor) -> None:

@@ -16,6 +16,7 @@ from typing import Any, Callable, Dict, NamedTuple, Optional, Tuple, Union
 import torch
 
 from primus_turbo import _native as N
+from primus_turbo.pytorch.core.native_op import native_op
 from primus_turbo.pytorch.core.low_precision import (
     MXFP4_BLOCK_SIZE,
     MXFP8_BLOCK_SIZE,
@@ -51,7 +52,7 @@ def _is_fp4(dtype) -> bool:
     return float4_e2m1fn_x2 is not None and dtype == float4_e2m1fn_x2
 
 
-@torch.library.custom_op("primus_turbo::transpose_last_two", mutates_args=())
+@native_op("primus_turbo::transpose_last_two")
 def transpose_last_two(t: torch.Tensor) -> torch.Tensor:
     """Physical transpose of the last two dimensions of a contiguous 1-byte tensor (fp8 codes)."""
     assert t.element_size() == 1 and t.is_contiguous() and t.dim() in (2, 3)

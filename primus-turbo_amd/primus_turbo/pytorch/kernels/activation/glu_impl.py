@@ -9,6 +9,7 @@ from typing import Optional, Tuple
 import torch
 
 from primus_turbo import _native as N
+from primus_turbo.pytorch.core.native_op import native_op
 
 ACT_SILU, ACT_GELU = 0, 1
 
@@ -30,7 +31,7 @@ def _common(x, probs, row_mask):
     return x.contiguous(), probs.contiguous().view(-1), row_mask
 
 
-@torch.library.custom_op("primus_turbo::glu_fwd_with_probs", mutates_args=())
+@native_op("primus_turbo::glu_fwd_with_probs")
 def glu_fwd_with_probs(x: torch.Tensor, probs: torch.Tensor, row_mask: Optional[torch.Tensor], act: int) -> torch.Tensor:
     """``out[t] = act(x[t, :H]) * x[t, H:] * probs[t]``; rows with ``row_mask == 0`` come out as zeros."""
     x, probs, row_mask = _common(x, probs, row_mask)
@@ -46,7 +47,7 @@ def _glu_fwd_with_probs_fake(x, probs, row_mask, act):
     return torch.empty((x.shape[0], x.shape[1] // 2), dtype=x.dtype, device=x.device)
 
 
-@torch.library.custom_op("primus_turbo::glu_bwd_with_probs", mutates_args=())
+@native_op("primus_turbo::glu_bwd_with_probs")
 def glu_bwd_with_probs(grad_out: torch.Tensor, x: torch.Tensor, probs: torch.Tensor, row_mask: Optional[torch.Tensor],
                        act: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """-> ``(grad_x [tokens, 2 H], grad_probs`` shaped like ``probs)``."""

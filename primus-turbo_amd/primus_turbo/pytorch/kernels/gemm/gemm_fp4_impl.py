@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 
 from primus_turbo.pytorch.core.low_precision import ScalingGranularity
+from primus_turbo.pytorch.core.native_op import native_op
 from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import _check, launch_mx
 
 
@@ -33,7 +34,7 @@ def _validate(a, trans_a, b, trans_b, granularity, preshuffled):
     _check(fp4 is not None and a.dtype == fp4 and b.dtype == fp4, "operands must be float4_e2m1fn_x2")
 
 
-@torch.library.custom_op("primus_turbo::gemm_fp4_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::gemm_fp4_impl", device_types="cuda")
 def gemm_fp4_impl(
     a: torch.Tensor,
     a_scale_inv: torch.Tensor,

@@ -14,6 +14,7 @@ from typing import Tuple
 import torch
 
 from primus_turbo import _native as N
+from primus_turbo.pytorch.core.native_op import native_op
 from primus_turbo.pytorch.core.low_precision import ScalingGranularity
 
 _FP8 = (torch.float8_e4m3fn, torch.float8_e5m2)
@@ -155,7 +156,7 @@ def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, gran
     return out
 
 
-@torch.library.custom_op("primus_turbo::gemm_fp8_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::gemm_fp8_impl", device_types="cuda")
 def gemm_fp8_impl(
     a: torch.Tensor,
     a_scale_inv: torch.Tensor,

@@ -14,6 +14,7 @@ from typing import Optional
 import torch
 
 from primus_turbo.pytorch.core.low_precision import ScalingGranularity
+from primus_turbo.pytorch.core.native_op import native_op
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import _grouped_mx, _variable_k_mx
 
 _FP4X2 = getattr(torch, "float4_e2m1fn_x2", None)
@@ -27,7 +28,7 @@ def _check_mx(granularity: int, *ts) -> None:
             raise RuntimeError(f"operands must be float4_e2m1fn_x2, got {t.dtype}")
 
 
-@torch.library.custom_op("primus_turbo::grouped_gemm_fp4_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::grouped_gemm_fp4_impl", device_types="cuda")
 def grouped_gemm_fp4_impl(
     a: torch.Tensor,
     b: torch.Tensor,
@@ -67,7 +68,7 @@ def _variable_k_out(a, b, group_offs, trans_c, out_dtype):
     return torch.empty((G, Ml, Nr), dtype=out_dtype, device=a.device)
 
 
-@torch.library.custom_op("primus_turbo::grouped_gemm_fp4_variable_k_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::grouped_gemm_fp4_variable_k_impl", device_types="cuda")
 def grouped_gemm_fp4_variable_k_impl(
     a: torch.Tensor,
     b: torch.Tensor,

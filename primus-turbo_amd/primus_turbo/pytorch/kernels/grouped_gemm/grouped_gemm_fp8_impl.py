@@ -17,6 +17,7 @@ import torch
 
 from primus_turbo import _native as N
 from primus_turbo.pytorch.core.low_precision import ScalingGranularity
+from primus_turbo.pytorch.core.native_op import native_op
 
 _FP8 = (torch.float8_e4m3fn, torch.float8_e5m2)
 
@@ -211,7 +212,7 @@ def _variable_k_mx(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans
     return out
 
 
-@torch.library.custom_op("primus_turbo::grouped_gemm_fp8_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::grouped_gemm_fp8_impl", device_types="cuda")
 def grouped_gemm_fp8_impl(
     a: torch.Tensor,
     b: torch.Tensor,
@@ -317,7 +318,7 @@ def _variable_k(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans_c,
     return out
 
 
-@torch.library.custom_op("primus_turbo::grouped_gemm_fp8_variable_k_impl", mutates_args=(), device_types="cuda")
+@native_op("primus_turbo::grouped_gemm_fp8_variable_k_impl", device_types="cuda")
 def grouped_gemm_fp8_variable_k_impl(
     a: torch.Tensor,
     b: torch.Tensor,

@@ -17,6 +17,7 @@ from typing import List, Optional, Tuple
 import torch
 
 from primus_turbo import _native as N
+from primus_turbo.pytorch.core.native_op import native_op
 
 _HP_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 _FP8_DTYPES = (torch.float8_e4m3fn, torch.float8_e5m2)
@@ -293,7 +294,7 @@ def _padded_rows(M: int, pad: int) -> int:
     return -(-M // pad) * pad
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_rowwise_t_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_rowwise_t_impl")
 def quant_fp8_rowwise_t_impl(
     x: torch.Tensor, row_scale_inv: Optional[torch.Tensor], hp_dtype: torch.dtype, dtype: torch.dtype, pad: int
 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -367,7 +368,7 @@ def _blockwise_launch(x, dtype, want_row: bool, want_col: bool):
     return q_row, s_row, q_col, s_col
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_impl")
 def quant_fp8_blockwise_impl(
     x: torch.Tensor, dtype: torch.dtype, axis: int, block_size: int = 128
 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -397,7 +398,7 @@ def _quant_fp8_blockwise_impl_fake(x, dtype, axis, block_size=128):
     )
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_dual_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_dual_impl")
 def quant_fp8_blockwise_dual_impl(
     x: torch.Tensor, dtype: torch.dtype, block_size: int = 128
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -422,7 +423,7 @@ def _quant_fp8_blockwise_dual_impl_fake(x, dtype, block_size=128):
     )
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_dual_t_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_dual_t_impl")
 def quant_fp8_blockwise_dual_t_impl(
     x: torch.Tensor, dtype: torch.dtype, block_size: int = 128
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -463,7 +464,7 @@ def _quant_fp8_blockwise_dual_t_impl_fake(x, dtype, block_size=128):
     )
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_kmajor_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_kmajor_impl")
 def quant_fp8_blockwise_kmajor_impl(
     x: torch.Tensor, dtype: torch.dtype, block_size: int, with_col_t: bool
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -552,7 +553,7 @@ _ext.impl("quantize_fp8_blockwise_for_weight", _quantize_fp8_blockwise_for_weigh
 _ext.impl("quantize_fp8_blockwise_for_weight", _quantize_fp8_blockwise_for_weight_meta, "Meta")
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_for_weight_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_for_weight_impl")
 def quant_fp8_blockwise_for_weight_impl(
     w: torch.Tensor, dtype: torch.dtype, block_size: int = 128
 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -569,7 +570,7 @@ def _quant_fp8_blockwise_for_weight_impl_fake(w, dtype, block_size=128):
     return q, s
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_for_weight_dual_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_for_weight_dual_impl")
 def quant_fp8_blockwise_for_weight_dual_impl(
     w: torch.Tensor, dtype: torch.dtype, block_size: int = 128
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -623,7 +624,7 @@ def _dequant_block(q: torch.Tensor, scale_inv: torch.Tensor, out_dtype, B, M, Nn
     return out
 
 
-@torch.library.custom_op("primus_turbo::dequant_fp8_blockwise_impl", mutates_args=())
+@native_op("primus_turbo::dequant_fp8_blockwise_impl")
 def dequant_fp8_blockwise_impl(
     x_fp8: torch.Tensor, scale_inv: torch.Tensor, out_dtype: torch.dtype, axis: int, block_size: int = 128
 ) -> torch.Tensor:
@@ -641,7 +642,7 @@ def _dequant_fp8_blockwise_impl_fake(x_fp8, scale_inv, out_dtype, axis, block_si
     return torch.empty(x_fp8.shape, dtype=out_dtype, device=x_fp8.device)
 
 
-@torch.library.custom_op("primus_turbo::dequant_fp8_blockwise_for_weight_impl", mutates_args=())
+@native_op("primus_turbo::dequant_fp8_blockwise_for_weight_impl")
 def dequant_fp8_blockwise_for_weight_impl(
     w_fp8: torch.Tensor, scale_inv: torch.Tensor, out_dtype: torch.dtype, block_size: int = 128
 ) -> torch.Tensor:
@@ -747,7 +748,7 @@ _ext.impl("quantize_fp8_blockwise_segment_m_row_col", _quantize_fp8_blockwise_se
 _ext.impl("quantize_fp8_blockwise_segment_m_row_col", _quantize_fp8_blockwise_segment_m_row_col_meta, "Meta")
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_segment_m_row_col_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_segment_m_row_col_impl")
 def quant_fp8_blockwise_segment_m_row_col_impl(
     x: torch.Tensor,
     dtype: torch.dtype,
@@ -780,7 +781,7 @@ def _segment_t_pitch(M: int, G: int, block_size: int) -> int:
     return ceil_div(M + G * block_size, block_size) * block_size
 
 
-@torch.library.custom_op("primus_turbo::quant_fp8_blockwise_segment_m_row_col_t_impl", mutates_args=())
+@native_op("primus_turbo::quant_fp8_blockwise_segment_m_row_col_t_impl")
 def quant_fp8_blockwise_segment_m_row_col_t_impl(
     x: torch.Tensor, dtype: torch.dtype, block_size: int, group_lens: torch.Tensor, group_offs: torch.Tensor
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -831,7 +832,7 @@ def _quant_fp8_blockwise_segment_m_row_col_t_impl_fake(x, dtype, block_size, gro
 _GLU_ACT = {"silu": 0, "gelu": 1}
 
 
-@torch.library.custom_op("primus_turbo::glu_quant_fp8_blockwise_segment_m_row_col_impl", mutates_args=())
+@native_op("primus_turbo::glu_quant_fp8_blockwise_segment_m_row_col_impl")
 def glu_quant_fp8_blockwise_segment_m_row_col_impl(
     x: torch.Tensor, probs: torch.Tensor, row_mask: Optional[torch.Tensor], act: str, dtype: torch.dtype,
     block_size: int, group_lens: torch.Tensor, group_offs: torch.Tensor, transposed_col: bool,
@@ -1055,7 +1056,7 @@ def mx_plain_layout(q: torch.Tensor, scale: torch.Tensor, shuffled_out: bool, sh
     return q, scale
 
 
-@torch.library.custom_op("primus_turbo::shuffle_mx_codes_impl", mutates_args=())
+@native_op("primus_turbo::shuffle_mx_codes_impl")
 def _shuffle_codes_op(codes: torch.Tensor, inverse: bool) -> torch.Tensor:
     N.require_cuda(codes)
     _check(codes.dim() in (2, 3), "codes must be 2-D or 3-D")
@@ -1142,7 +1143,7 @@ def _mx_quantize(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, want_c
     return rq, rs, cq, cs
 
 
-@torch.library.custom_op("primus_turbo::quantize_mx", mutates_args=())
+@native_op("primus_turbo::quantize_mx")
 def _quantize_mx_op(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, want_col: bool, row_flags: int,
                     col_flags: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """The four outputs of ``_mx_quantize`` with an empty tensor for an unwanted direction (an
@@ -1221,7 +1222,7 @@ def quantize_mxfp4_impl(x, out_dtype, axis, block_size, with_trans=False, scalin
     return _quantize_mx_impl(x, out_dtype, axis, block_size, with_trans, scaling_recipe, scaling_recipe_for_trans, "MXFP4")
 
 
-@torch.library.custom_op("primus_turbo::dequantize_mx", mutates_args=())
+@native_op("primus_turbo::dequantize_mx")
 def _dequantize_mx_op(x: torch.Tensor, scale_inv: torch.Tensor, out_dtype: torch.dtype, rows: int, cols: int,
                       rowwise: bool) -> torch.Tensor:
     """``[rows, cols]`` codes with ``[rows, cols / 32]`` E8M0 scales -> ``[rows, cols]`` values, or
@@ -1315,7 +1316,7 @@ def _grouped_mx_dims(M, Nn, G, fp4):
     return ra, ca, m_pad_row, m_pad_col, n_pad
 
 
-@torch.library.custom_op("primus_turbo::grouped_quantize_mx", mutates_args=())
+@native_op("primus_turbo::grouped_quantize_mx")
 def _grouped_quantize_mx_op(
     x: torch.Tensor, out_dtype: torch.dtype, group_lens: torch.Tensor, group_offs: torch.Tensor, want_row: bool,
     want_col: bool, row_flags: int, col_flags: int,
@@ -1381,7 +1382,7 @@ def _grouped_quantize_mx_op_fake(x, out_dtype, group_lens, group_offs, want_row,
             i64(0 if fp4 else G), i64(0 if fp4 else G + 1), i64(G), i64(G + 1))
 
 
-@torch.library.custom_op("primus_turbo::glu_grouped_quantize_mx", mutates_args=())
+@native_op("primus_turbo::glu_grouped_quantize_mx")
 def glu_grouped_quantize_mx_impl(
     x: torch.Tensor, probs: torch.Tensor, row_mask: Optional[torch.Tensor], act: str, out_dtype: torch.dtype,
     group_lens: torch.Tensor, group_offs: torch.Tensor, with_trans: bool, col_flags: int = 0,
