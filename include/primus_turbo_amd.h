@@ -252,6 +252,10 @@ PT_API int pt_quantize_fp8_blockwise_weight_dual(const void *w, int w_dtype, int
  * (csrc/kernels/quantization/quantization_blockwise.cu:18-48). All int64, on device. */
 PT_API int pt_compute_group_offs(const int64_t *group_lens, int64_t num_groups, int64_t align,
                                  int64_t *padded_lens, int64_t *group_offs, void *stream);
+/* The same for two alignments in one launch (the row and column paddings of one quantizer). */
+PT_API int pt_compute_group_offs2(const int64_t *group_lens, int64_t num_groups, int64_t align_a,
+                                  int64_t *padded_lens_a, int64_t *group_offs_a, int64_t align_b,
+                                  int64_t *padded_lens_b, int64_t *group_offs_b, void *stream);
 
 /* Replaces torch.ops.primus_turbo_cpp_extension.quantize_fp8_blockwise_segment_m_row_col
  * (csrc/pytorch/quantization/quantization.cpp:1384-1441,

@@ -67,6 +67,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     int *prefix = reinterpret_cast<int *>(smem + NSTAGE * STAGE); // GROUP_ROWS: tiles before group g
     int  total;
     if constexpr (GMODE == GROUP_ROWS) {
+        zero_tail_rows(a, B8_THREADS);
         for (int g = tid; g < a.G; g += B8_THREADS) {
             const int64_t *o   = a.group_offs_out != nullptr ? a.group_offs_out : a.group_offs;
             const int64_t rows = o[g + 1] - o[g];

@@ -51,26 +51,15 @@ static int launch_grouped(const GemmArgs &a, int fa, int fb, int tile_cfg, hipSt
     return launch_grouped_tiles<GMODE, SB_VEC, 1, 1>(a, tile_cfg, stream);
 }
 
-// rows [offs[G], rows) of a [rows, row_bytes] matrix := 0 (16-byte stores; row_bytes % 16 == 0
-// is not required: the tail is a contiguous byte range)
-__global__ __launch_bounds__(256) void zero_tail_rows_kernel(uint8_t *c, const int64_t *group_offs, int G,
-                                                             int64_t rows, int64_t row_bytes) {
-    const int64_t first = group_offs[G];
-    if (first >= rows)
-        return;
-    uint8_t      *p     = c + first * row_bytes;
-    const int64_t bytes = (rows - first) * row_bytes;
-    const int64_t head  = (16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15; // bytes up to alignment
-    const int64_t tid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, nthr = static_cast<int64_t>(gridDim.x) * 256;
-    const int64_t h   = head < bytes ? head : bytes;
-    for (int64_t i = tid; i < h; i += nthr)
-        p[i] = 0;
-    const int64_t n16 = (bytes - h) / 16;
-    u32x4        *q   = reinterpret_cast<u32x4 *>(p + h);
-    for (int64_t i = tid; i < n16; i += nthr)
-        q[i] = u32x4{0u, 0u, 0u, 0u};
-    for (int64_t i = h + n16 * 16 + tid; i < bytes; i += nthr)
-        p[i] = 0;
+__global__ __launch_bounds__(256) void zero_rows_kernel(uint8_t *c, const int64_t *offs, int G, int64_t rows, int64_t row_bytes) {
+    const int64_t first = offs[G];
+    if (first < rows)
+        zero_bytes(c + first * row_bytes, (rows - first) * row_bytes, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x,
+                   static_cast<int64_t>(gridDim.x) * 256);
+}
+int launch_zero_rows(void *c, const int64_t *offs, int64_t G, int64_t rows, int64_t row_bytes, hipStream_t st) {
+    zero_rows_kernel<<<256, 256, 0, st>>>(static_cast<uint8_t *>(c), offs, static_cast<int>(G), rows, row_bytes);
+    return check_launch("zero_rows_kernel");
 }
 
 } // namespace pt
@@ -159,18 +148,9 @@ int pt_grouped_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const 
     g.sb_gstride = nb * kb;
     g.c_gstride  = 0;
     const int fa = a_dtype == PT_DTYPE_E5M2 ? 1 : 0, fb = b_dtype == PT_DTYPE_E5M2 ? 1 : 0;
-    if (G > 0 && M > 0) {
-        const int rc = launch_grouped<GROUP_ROWS, false>(g, fa, fb, tile_cfg, st);
-        if (rc != PT_OK)
-            return rc;
-    }
-    // rows past the last routed token (over-allocated outputs) read as zero
-    if (out_rows > 0) {
-        zero_tail_rows_kernel<<<256, 256, 0, st>>>(static_cast<uint8_t *>(c), group_offs, static_cast<int>(G), out_rows,
-                                                   N * ES);
-        return check_launch("zero_tail_rows_kernel");
-    }
-    return PT_OK;
+    g.out_rows = out_rows; // (rows past the last routed token read as zero)
+    return G > 0 && M > 0 ? launch_grouped<GROUP_ROWS, false>(g, fa, fb, tile_cfg, st)
+                          : launch_zero_rows(c, group_offs, G, out_rows, N * ES, st);
 }
 
 size_t pt_grouped_gemm_fp8_variable_k_workspace_bytes(int64_t Mp, int64_t Ml, int64_t Nr) {

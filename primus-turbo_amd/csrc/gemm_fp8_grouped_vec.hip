@@ -122,18 +122,6 @@ __global__ __launch_bounds__(256) void transpose_grouped_pad_kernel(const uint8_
     }
 }
 
-__global__ __launch_bounds__(256) void zero_rows_from2_kernel(uint8_t *c, const int64_t *offs, int G, int64_t rows,
-                                                              int64_t row_bytes) {
-    const int64_t first = offs[G];
-    if (first >= rows)
-        return;
-    uint8_t      *p     = c + first * row_bytes;
-    const int64_t bytes = (rows - first) * row_bytes;
-    const int64_t tid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, nthr = static_cast<int64_t>(gridDim.x) * 256;
-    for (int64_t i = tid; i < bytes; i += nthr)
-        p[i] = 0;
-}
-
 } // namespace pt
 
 using namespace pt;
@@ -206,14 +194,13 @@ int pt_grouped_gemm_fp8_vec(const void *a, int a_dtype, const float *a_scale, in
         g.group_offs = group_offs;
         g.b_gstride  = N * Kp;
         g.sb_gstride = sb_gstride;
-        const int rc = launch_gvec<GROUP_ROWS>(g, a_dtype == PT_DTYPE_E5M2, b_dtype == PT_DTYPE_E5M2, tile_cfg, st);
-        if (rc != PT_OK)
-            return rc;
-    } else if (K == 0 && M > 0) {
-        zero_rows_from2_kernel<<<256, 256, 0, st>>>(static_cast<uint8_t *>(c), group_offs, 0, M, N * ES); // offs[0] = 0
+        g.out_rows   = out_rows; // (rows past the last routed token read as zero)
+        return launch_gvec<GROUP_ROWS>(g, a_dtype == PT_DTYPE_E5M2, b_dtype == PT_DTYPE_E5M2, tile_cfg, st);
     }
-    zero_rows_from2_kernel<<<256, 256, 0, st>>>(static_cast<uint8_t *>(c), group_offs, static_cast<int>(G), out_rows, N * ES);
-    return check_launch("pt_grouped_gemm_fp8_vec");
+    if (K == 0 && M > 0) // (offs[0] = 0)
+        if (const int rc = launch_zero_rows(c, group_offs, 0, M, N * ES, st))
+            return rc;
+    return launch_zero_rows(c, group_offs, G, out_rows, N * ES, st);
 }
 
 size_t pt_grouped_gemm_fp8_vec_variable_k_workspace_bytes(int64_t G, int64_t M, int64_t Ml, int64_t Nr) {

@@ -58,7 +58,7 @@ struct GemmArgs {
     // VECTOR: sA[m * sa_m], sB[n * sb_n]                      (stride 0 = one scalar)
     // BLOCK : sA[(m >> sa_shift) * sa_m + kb * sa_k], sB[(n >> sb_shift) * sb_n + kb * sb_k]
     // MX    : sA / sB point at E8M0 bytes, byte[m * sa_m + kb] and byte[n * sb_n + kb];
-    //         or, "word-major" (sa_wpitch, sb_wpitch != 0): the 32-bit word w of row m (its K blocks
+    //         or, "word-major" (sa_wpitch / sb_wpitch != 0, each operand for itself): the 32-bit word w of row m (its K blocks
     //         4 w .. 4 w + 3) at byte m * 4 + w * sa_wpitch, i.e. the words of one K position of all
     //         rows are contiguous and a scale copy fetches two cache lines instead of sixty-four
     int64_t sa_m, sa_k, sb_n, sb_k;
@@ -83,6 +83,7 @@ struct GemmArgs {
     // GROUP_ROWS only, optional: row offsets of the groups in C when they differ from those in A
     // (A in a per-group padded layout, C packed tight); NULL = the same offsets
     const int64_t *group_offs_out;
+    int64_t        out_rows; // GROUP_ROWS: rows of C; those behind the last group's are set to zero
     int64_t        b_gstride;  // bytes
     int64_t        sb_gstride; // floats
     int64_t        c_gstride;  // elements
@@ -655,6 +656,19 @@ __device__ __forceinline__ int epilogue(const GemmArgs &a, const f32x4 (&acc)[TM
     return 0;
 }
 
+// bytes [0, bytes) from p := 0, by thread `tid` of `threads`
+__device__ __forceinline__ void zero_bytes(uint8_t *p, const int64_t bytes, const int64_t tid, const int64_t threads) {
+    const int64_t to_aligned = (16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15;
+    const int64_t head = to_aligned < bytes ? to_aligned : bytes, n16 = (bytes - head) / 16;
+    u32x4        *q = reinterpret_cast<u32x4 *>(p + head);
+    for (int64_t i = tid; i < n16; i += threads)
+        q[i] = u32x4{0u, 0u, 0u, 0u};
+    if (tid < head)
+        p[tid] = 0;
+    if (tid < bytes - head - n16 * 16)
+        p[head + n16 * 16 + tid] = 0;
+}
+
 // Wavefront-uniform 64-bit loads of values written before the launch (group offsets), through the
 // scalar cache. Left to the compiler these are vector loads -- the kernel also stores to global
 // memory, so it cannot prove the location unclobbered -- and the wait for a vector load is also a
@@ -685,6 +699,19 @@ __device__ __forceinline__ int64_t uniform_load(const int64_t *p) {
     v = p[0];
 #endif
     return v;
+}
+
+// GROUP_ROWS: rows of C behind the last group's (over-allocated outputs) read as zero. Written by the product's
+// own workgroups before their first copy: a launch of its own for it is 4.7 to 5.5 us of an otherwise idle GPU
+// behind every grouped product, here it passes under the first slabs' latency. (The stores are older than every
+// copy that a wait counts, so the waits stay on the safe side.)
+__device__ __forceinline__ void zero_tail_rows(const GemmArgs &a, const int threads) {
+    const int64_t first = uniform_load((a.group_offs_out != nullptr ? a.group_offs_out : a.group_offs) + a.G);
+    if (first >= a.out_rows)
+        return;
+    const int64_t row_bytes = a.N * (a.out_dtype == PT_DTYPE_F32 ? 4 : 2);
+    zero_bytes(static_cast<uint8_t *>(a.C) + first * row_bytes, (a.out_rows - first) * row_bytes,
+               static_cast<int64_t>(blockIdx.x) * threads + threadIdx.x, static_cast<int64_t>(gridDim.x) * threads);
 }
 
 // Where a workgroup's tile lives. The second half only varies between tiles of grouped
@@ -852,6 +879,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     int *prefix = reinterpret_cast<int *>(smem + NSTAGE * STAGE);
     int  total;
     if constexpr (GMODE == GROUP_ROWS) {
+        zero_tail_rows(a, 256);
         for (int g = tid; g < a.G; g += 256) {
             const int64_t *o   = a.group_offs_out != nullptr ? a.group_offs_out : a.group_offs;
             const int64_t rows = o[g + 1] - o[g];
@@ -907,11 +935,11 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     // cross-tile pipelining it stops at the tile's last slab and keeps re-reading that one.
     // scale addressing in bytes: from one row (column) to the next, and (MX) from one 32-bit word
     // of a row to its next
-    [[maybe_unused]] const bool     mx_wordmajor = MODE == SCALE_MX && a.sa_wpitch != 0;
-    [[maybe_unused]] const uint32_t sa_rowp  = mx_wordmajor ? 4u : static_cast<uint32_t>(a.sa_m) * (MODE == SCALE_MX ? 1 : 4);
-    [[maybe_unused]] const uint32_t sb_rowp  = mx_wordmajor ? 4u : static_cast<uint32_t>(a.sb_n) * (MODE == SCALE_MX ? 1 : 4);
-    [[maybe_unused]] const uint32_t sa_wordp = mx_wordmajor ? static_cast<uint32_t>(a.sa_wpitch) : 4u;
-    [[maybe_unused]] const uint32_t sb_wordp = mx_wordmajor ? static_cast<uint32_t>(a.sb_wpitch) : 4u;
+    [[maybe_unused]] const bool     words_a = MODE == SCALE_MX && a.sa_wpitch != 0, words_b = MODE == SCALE_MX && a.sb_wpitch != 0;
+    [[maybe_unused]] const uint32_t sa_rowp  = words_a ? 4u : static_cast<uint32_t>(a.sa_m) * (MODE == SCALE_MX ? 1 : 4);
+    [[maybe_unused]] const uint32_t sb_rowp  = words_b ? 4u : static_cast<uint32_t>(a.sb_n) * (MODE == SCALE_MX ? 1 : 4);
+    [[maybe_unused]] const uint32_t sa_wordp = words_a ? static_cast<uint32_t>(a.sa_wpitch) : 4u;
+    [[maybe_unused]] const uint32_t sb_wordp = words_b ? static_cast<uint32_t>(a.sb_wpitch) : 4u;
     uint32_t off[NL];
     {
         const int lrow = lane >> 3, pchk = lane & 7;
@@ -943,10 +971,10 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     // arrays (reads beyond return zero; they only ever meet rows that are never stored)
     [[maybe_unused]] const uint8_t *ld_sa = nullptr, *ld_sb = nullptr, *ld_sa_end = nullptr, *ld_sb_end = nullptr;
     [[maybe_unused]] const int64_t  sa_extent =
-        MODE == SCALE_MX ? (mx_wordmajor ? static_cast<int64_t>((a.kb_valid + 3) / 4) * a.sa_wpitch : (a.M - 1) * a.sa_m + a.kb_valid)
+        MODE == SCALE_MX ? (words_a ? static_cast<int64_t>((a.kb_valid + 3) / 4) * a.sa_wpitch : (a.M - 1) * a.sa_m + a.kb_valid)
                          : (((a.M - 1) >> a.sa_shift) * a.sa_m + (a.kb_valid - 1) * a.sa_k + 1) * 4;
     [[maybe_unused]] const int64_t sb_extent =
-        MODE == SCALE_MX ? (mx_wordmajor ? static_cast<int64_t>((a.kb_valid + 3) / 4) * a.sb_wpitch : (a.N - 1) * a.sb_n + a.kb_valid)
+        MODE == SCALE_MX ? (words_b ? static_cast<int64_t>((a.kb_valid + 3) / 4) * a.sb_wpitch : (a.N - 1) * a.sb_n + a.kb_valid)
                          : (((a.N - 1) >> a.sb_shift) * a.sb_n + (a.kb_valid - 1) * a.sb_k + 1) * 4;
     [[maybe_unused]] const int64_t sa_step = MODE == SCALE_MX ? static_cast<int64_t>(NW) * sa_wordp : a.sa_k * 4; // bytes per slab
     [[maybe_unused]] const int64_t sb_step = MODE == SCALE_MX ? static_cast<int64_t>(NW) * sb_wordp : a.sb_k * 4;
@@ -1418,8 +1446,8 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     if (MODE == SCALE_BLOCK && ((!SB_VEC && a.sb_shift != 7) || (GMODE == GROUP_ROWS && a.sa_shift != 0)))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_fp8: unsupported block-scale layout");
     // MX scale words are fetched as aligned 32-bit units
-    if (MODE == SCALE_MX && (a.sa_shift != 0 || a.sb_shift != 0 || (a.sa_wpitch == 0 && (a.sa_m % 4 != 0 || a.sb_n % 4 != 0)) ||
-                             (a.sa_wpitch != 0) != (a.sb_wpitch != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
+    if (MODE == SCALE_MX && (a.sa_shift != 0 || a.sb_shift != 0 || (a.sa_wpitch == 0 && a.sa_m % 4 != 0) ||
+                             (a.sb_wpitch == 0 && a.sb_n % 4 != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
                              reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
     auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE>;
@@ -1484,6 +1512,8 @@ void launch_pad_rows(const uint8_t *in, uint8_t *out, int64_t R, int64_t C, int6
 // in[R, C] with row pitch ldi -> out[R, ldo] (columns [C, ldo) zero-filled)
 void launch_pad_rows2(const uint8_t *in, uint8_t *out, int64_t R, int64_t C, int64_t ldi, int64_t ldo, hipStream_t st);
 // out[b][w * R + r] = in[b][r * pitch + w] for w < W (32-bit words): scale arrays made contiguous along their rows
+// rows [offs[G], rows) of c := 0, in a launch of its own: for a grouped product of nothing
+int launch_zero_rows(void *c, const int64_t *offs, int64_t G, int64_t rows, int64_t row_bytes, hipStream_t st);
 int launch_transpose_words(const uint32_t *in, uint32_t *out, int64_t R, int64_t W, int64_t pitch, hipStream_t st,
                             int64_t batch = 1);
 int  launch_gemm_block(const GemmArgs &a, int fa, int fb, bool sb_vec, int tile_cfg, hipStream_t stream);

@@ -47,6 +47,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_mx8_kernel(const GemmArgs a) 
     int *prefix = reinterpret_cast<int *>(smem + B8_NSTAGE * STAGE);
     int  total;
     if constexpr (GMODE == GROUP_ROWS) {
+        zero_tail_rows(a, B8_THREADS);
         for (int g = tid; g < a.G; g += B8_THREADS) {
             const int64_t *o   = a.group_offs_out != nullptr ? a.group_offs_out : a.group_offs;
             const int64_t rows = o[g + 1] - o[g];
@@ -78,8 +79,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_mx8_kernel(const GemmArgs a) 
     // ---- loader ----
     // scale addressing in bytes: from one row (column) to the next, and from one 32-bit word of a
     // row to its next (row-major arrays, or the word-major copy)
-    const bool     wordmajor = a.sa_wpitch != 0;
     const bool     sc_is_a   = wave < 4;
+    const bool     wordmajor = (sc_is_a ? a.sa_wpitch : a.sb_wpitch) != 0;
     const uint32_t sc_rowp   = wordmajor ? 4u : static_cast<uint32_t>(sc_is_a ? a.sa_m : a.sb_n);
     const uint32_t sc_wordp  = wordmajor ? static_cast<uint32_t>(sc_is_a ? a.sa_wpitch : a.sb_wpitch) : 4u;
     uint32_t       off[NL];
@@ -293,8 +294,8 @@ template <int FA, int FB, int GMODE = GROUP_NONE> static int launch_gemm_mx8(con
     a.tiles_n  = static_cast<int>(cdiv(a.N, B8_BN));
     if (GMODE != GROUP_NONE && a.G > MAX_G)
         return fail(PT_ERR_INVALID_ARGUMENT, "grouped gemm_mx: too many groups for this tile configuration");
-    if (a.sa_shift != 0 || a.sb_shift != 0 || (a.sa_wpitch == 0 && (a.sa_m % 4 != 0 || a.sb_n % 4 != 0)) ||
-        (a.sa_wpitch != 0) != (a.sb_wpitch != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
+    if (a.sa_shift != 0 || a.sb_shift != 0 || (a.sa_wpitch == 0 && a.sa_m % 4 != 0) || (a.sb_wpitch == 0 && a.sb_n % 4 != 0) ||
+        a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
         reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0)
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
     if (a.K / KSTEP < 2)

@@ -45,25 +45,6 @@ template <int GMODE> static int launch_mxg(const GemmArgs &a, int fa, int fb, in
     return launch_mxg_tiles<GMODE, 1, 1>(a, tile_cfg, stream);
 }
 
-// rows [first, rows) of a [rows, row_bytes] matrix := 0, first = offs[G]
-__global__ __launch_bounds__(256) void zero_rows_from_kernel(uint8_t *c, const int64_t *offs, int G, int64_t rows,
-                                                             int64_t row_bytes) {
-    const int64_t first = offs[G];
-    if (first >= rows)
-        return;
-    uint8_t      *p     = c + first * row_bytes;
-    const int64_t bytes = (rows - first) * row_bytes;
-    const int64_t tid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, nthr = static_cast<int64_t>(gridDim.x) * 256;
-    if ((reinterpret_cast<uintptr_t>(p) & 15) == 0 && (bytes & 15) == 0) {
-        u32x4 *q = reinterpret_cast<u32x4 *>(p);
-        for (int64_t i = tid; i < bytes / 16; i += nthr)
-            q[i] = u32x4{0u, 0u, 0u, 0u};
-    } else {
-        for (int64_t i = tid; i < bytes; i += nthr)
-            p[i] = 0;
-    }
-}
-
 } // namespace pt
 
 using namespace pt;
@@ -148,15 +129,10 @@ int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, int64_t 
             g.sb_wpitch  = N * 4;
             g.sb_gstride = W * N;
         }
-        const int rc = launch_mxg<GROUP_ROWS>(g, fp4 ? 4 : a_dtype == PT_DTYPE_E5M2, b_dtype == PT_DTYPE_E5M2, tile_cfg, st);
-        if (rc != PT_OK)
-            return rc;
+        g.out_rows = out_rows; // (rows past the last routed token, in an over-allocated output, read as zero)
+        return launch_mxg<GROUP_ROWS>(g, fp4 ? 4 : a_dtype == PT_DTYPE_E5M2, b_dtype == PT_DTYPE_E5M2, tile_cfg, st);
     }
-    // rows past the last routed token (over-allocated outputs) read as zero
-    const int64_t ES = c_dtype == PT_DTYPE_F32 ? 4 : 2;
-    zero_rows_from_kernel<<<256, 256, 0, st>>>(static_cast<uint8_t *>(c), group_offs_out ? group_offs_out : group_offs,
-                                               static_cast<int>(G), out_rows, N * ES);
-    return check_launch("zero_rows_from_kernel");
+    return launch_zero_rows(c, group_offs_out ? group_offs_out : group_offs, G, out_rows, N * (c_dtype == PT_DTYPE_F32 ? 4 : 2), st);
 }
 
 int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lhs_scale, const void *rhs, int rhs_dtype,

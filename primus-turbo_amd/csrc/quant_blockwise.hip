@@ -603,12 +603,19 @@ __global__ __launch_bounds__(256) void dequant_block_vec_kernel(
 
 // ---------------------------------------------------------------------------
 // Group offsets: offs[0] = 0, offs[i+1] = offs[i] + round_up(lens[i], align).
-// One wavefront; each lane owns a strided slice, partial sums meet in LDS.
+// One wavefront for each alignment; each lane owns a strided slice, partial sums meet in LDS. Bound by its own
+// launch (4.7 us of GPU time for a few hundred bytes), which is why the two paddings that a quantizer needs
+// come from one.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void group_offs_kernel(const int64_t *__restrict__ lens,
-                                                        int64_t *__restrict__ padded_lens,
-                                                        int64_t *__restrict__ offs, const int G,
-                                                        const int64_t align) {
+struct GroupOffsOut {
+    int64_t *padded_lens, *offs;
+    int64_t  align;
+};
+__global__ __launch_bounds__(64) void group_offs_kernel(const int64_t *__restrict__ lens, const int G, const GroupOffsOut first,
+                                                        const GroupOffsOut second) {
+    int64_t *const     padded_lens = blockIdx.x == 0 ? first.padded_lens : second.padded_lens;
+    int64_t *const     offs        = blockIdx.x == 0 ? first.offs : second.offs;
+    const int64_t      align       = blockIdx.x == 0 ? first.align : second.align;
     __shared__ int64_t s_sum[64];
     const int          lane  = threadIdx.x;
     const int          chunk = (G + 63) / 64;
@@ -777,8 +784,19 @@ int pt_compute_group_offs(const int64_t *group_lens, int64_t num_groups, int64_t
     PT_REQUIRE(align >= 1, "align must be >= 1");
     PT_REQUIRE(group_offs != nullptr && (num_groups == 0 || group_lens != nullptr),
                "NULL tensor pointer");
-    group_offs_kernel<<<1, 64, 0, static_cast<hipStream_t>(stream)>>>(
-        group_lens, padded_lens, group_offs, static_cast<int>(num_groups), align);
+    const GroupOffsOut out{padded_lens, group_offs, align};
+    group_offs_kernel<<<1, 64, 0, static_cast<hipStream_t>(stream)>>>(group_lens, static_cast<int>(num_groups), out, out);
+    return check_launch("group_offs_kernel");
+}
+
+int pt_compute_group_offs2(const int64_t *group_lens, int64_t num_groups, int64_t align_a, int64_t *padded_lens_a,
+                           int64_t *group_offs_a, int64_t align_b, int64_t *padded_lens_b, int64_t *group_offs_b, void *stream) {
+    PT_REQUIRE(num_groups >= 0 && num_groups < (1LL << 31), "num_groups out of range");
+    PT_REQUIRE(align_a >= 1 && align_b >= 1, "align must be >= 1");
+    PT_REQUIRE(group_offs_a != nullptr && group_offs_b != nullptr && (num_groups == 0 || group_lens != nullptr), "NULL tensor pointer");
+    group_offs_kernel<<<2, 64, 0, static_cast<hipStream_t>(stream)>>>(group_lens, static_cast<int>(num_groups),
+                                                                      GroupOffsOut{padded_lens_a, group_offs_a, align_a},
+                                                                      GroupOffsOut{padded_lens_b, group_offs_b, align_b});
     return check_launch("group_offs_kernel");
 }
 

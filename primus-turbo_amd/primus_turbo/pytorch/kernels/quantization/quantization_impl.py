@@ -676,6 +676,19 @@ def _group_offs(group_lens: torch.Tensor, align: int, want_padded_lens: bool):
     return padded, offs
 
 
+def _group_offs_pair(group_lens: torch.Tensor, align_a: int, align_b: int):
+    """``(padded_lens, offs)`` for both alignments, from one launch."""
+    N.require_cuda(group_lens)
+    _check(group_lens.dtype == torch.int64 and group_lens.dim() == 1, "group_lens must be a 1-D int64 tensor")
+    gl = group_lens.contiguous()
+    G = gl.numel()
+    lens_a, lens_b = (torch.empty(G, dtype=torch.int64, device=gl.device) for _ in range(2))
+    offs_a, offs_b = (torch.empty(G + 1, dtype=torch.int64, device=gl.device) for _ in range(2))
+    N.check(N.lib().pt_compute_group_offs2(N.ptr(gl), G, align_a, N.ptr(lens_a), N.ptr(offs_a), align_b, N.ptr(lens_b),
+                                           N.ptr(offs_b), N.stream_of(gl)))
+    return lens_a, offs_a, lens_b, offs_b
+
+
 def _grouped_gemm_compute_offs(group_lens: torch.Tensor) -> torch.Tensor:
     return _group_offs(group_lens, 1, False)[1]
 
@@ -777,18 +790,29 @@ def _quant_fp8_blockwise_segment_m_row_col_impl_fake(x, dtype, block_size, group
     return r[0], r[1], r[2], r[3], r[4], r[5]
 
 
+def _known_offs(offs: Optional[torch.Tensor], G: int) -> bool:
+    """Whether a caller hands in padded offsets of the same groups (a backward pass those of its forward)."""
+    if offs is None:
+        return False
+    _check(offs.dtype == torch.int64 and offs.is_contiguous() and offs.numel() == G + 1 and offs.is_cuda,
+           "padded offsets must be contiguous int64 [G + 1]")
+    return True
+
+
 def _segment_t_pitch(M: int, G: int, block_size: int) -> int:
     return ceil_div(M + G * block_size, block_size) * block_size
 
 
 @native_op("primus_turbo::quant_fp8_blockwise_segment_m_row_col_t_impl")
 def quant_fp8_blockwise_segment_m_row_col_t_impl(
-    x: torch.Tensor, dtype: torch.dtype, block_size: int, group_lens: torch.Tensor, group_offs: torch.Tensor
+    x: torch.Tensor, dtype: torch.dtype, block_size: int, group_lens: torch.Tensor, group_offs: torch.Tensor,
+    padded_offs: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """:func:`quant_fp8_blockwise_segment_m_row_col_impl` with the segment-padded column codes
     emitted transposed: ``x_fp8_col_t [N, Mp]`` (``Mp`` = ``M + G * b`` rounded up to ``b``), the
     K-contiguous operand of the variable-K wgrad product; everything else (row codes, both scale
-    tensors, padded lens / offs) as there. (No counterpart in the reference, whose GEMM backends
+    tensors, padded lens / offs) as there. Given the ``padded_offs`` of an earlier call for the same
+    groups, both come back empty. (No counterpart in the reference, whose GEMM backends
     read the untransposed layout.)"""
     N.require_cuda(x, group_lens, group_offs)
     _check(x.dtype in _HP_DTYPES, "input must be bfloat16, float16 or float32")
@@ -803,30 +827,34 @@ def quant_fp8_blockwise_segment_m_row_col_t_impl(
     _, rs_shape, cs_shape = _segment_shapes(M, Nn, G, block_size)
     ldt = _segment_t_pitch(M, G, block_size)
     dev = x.device
-    padded_lens, padded_offs = _group_offs(group_lens, block_size, True)
+    known = _known_offs(padded_offs, G)
+    padded_lens, offs = (None, padded_offs) if known else _group_offs(group_lens, block_size, True)
     q_row = torch.empty((M, Nn), dtype=dtype, device=dev)
     q_col_t = torch.empty((Nn, ldt), dtype=dtype, device=dev)
     s_row = torch.empty(rs_shape, dtype=torch.float32, device=dev)
     s_col = torch.empty(cs_shape, dtype=torch.float32, device=dev)
     N.check(
         N.lib().pt_quantize_fp8_blockwise_segment_m_row_col_t(
-            N.ptr(x), N.dtype_code(x.dtype), M, Nn, N.dtype_code(dtype), N.ptr(group_offs), N.ptr(padded_offs), G,
+            N.ptr(x), N.dtype_code(x.dtype), M, Nn, N.dtype_code(dtype), N.ptr(group_offs), N.ptr(offs), G,
             N.ptr(q_row), N.ptr(s_row), None, N.ptr(q_col_t), ldt, N.ptr(s_col), N.stream_of(x),
         )
     )
-    return q_row, q_col_t, s_row, s_col, padded_lens, padded_offs
+    if known:
+        padded_lens, offs = (torch.empty(0, dtype=torch.int64, device=dev) for _ in range(2))
+    return q_row, q_col_t, s_row, s_col, padded_lens, offs
 
 
 @quant_fp8_blockwise_segment_m_row_col_t_impl.register_fake
-def _quant_fp8_blockwise_segment_m_row_col_t_impl_fake(x, dtype, block_size, group_lens, group_offs):
+def _quant_fp8_blockwise_segment_m_row_col_t_impl_fake(x, dtype, block_size, group_lens, group_offs, padded_offs=None):
     M, Nn = x.shape
     G = group_lens.numel()
     _, rs_shape, cs_shape = _segment_shapes(M, Nn, G, block_size)
     dev = x.device
+    n_lens, n_offs = (G, G + 1) if padded_offs is None else (0, 0)
     return (torch.empty((M, Nn), dtype=dtype, device=dev),
             torch.empty((Nn, _segment_t_pitch(M, G, block_size)), dtype=dtype, device=dev),
             torch.empty(rs_shape, dtype=torch.float32, device=dev), torch.empty(cs_shape, dtype=torch.float32, device=dev),
-            torch.empty(G, dtype=torch.int64, device=dev), torch.empty(G + 1, dtype=torch.int64, device=dev))
+            torch.empty(n_lens, dtype=torch.int64, device=dev), torch.empty(n_offs, dtype=torch.int64, device=dev))
 
 
 _GLU_ACT = {"silu": 0, "gelu": 1}
@@ -1290,19 +1318,23 @@ MXFP4_GROUP_K_DIM_PADDING_ALIGN_SIZE = 256
 
 
 def _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, want_row: bool, want_col: bool, row_flags: int = 0,
-                         col_flags: int = 0):
+                         col_flags: int = 0, known=None):
     """MXFP8: rows of every group padded to 32, transposed columns to 128. MXFP4: rows stay
     where they are in ``x`` (their "padded" lens / offs are the originals), transposed columns
     padded to 256 per group.
     -> (row_q, row_scale, col_q, col_scale, lens_row, offs_row, lens_col, offs_col); the pair of an
-    unwanted direction is None."""
-    rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_quantize_mx_op(x, out_dtype, group_lens, group_offs, want_row, want_col,
-                                                                 int(row_flags), int(col_flags))
+    unwanted direction is None. ``known``: the last four of an earlier call for the same groups."""
+    fp4 = _FP4X2 is not None and out_dtype == _FP4X2
+    rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_quantize_mx_op(
+        x, out_dtype, group_lens, group_offs, want_row, want_col, int(row_flags), int(col_flags),
+        *((None, None) if known is None else (None if fp4 else known[1], known[3])))
+    if known is not None:
+        lr, orow, lc, ocol = known
     if not want_row:
         rq = rs = None
     if not want_col:
         cq = cs = None
-    if _FP4X2 is not None and out_dtype == _FP4X2:
+    if fp4:
         lr, orow = group_lens, group_offs
     return rq, rs, cq, cs, lr, orow, lc, ocol
 
@@ -1316,13 +1348,22 @@ def _grouped_mx_dims(M, Nn, G, fp4):
     return ra, ca, m_pad_row, m_pad_col, n_pad
 
 
+def _grouped_mx_offs(group_lens, ra, ca, fp4):
+    """-> (lens_row, offs_row, lens_col, offs_col); MXFP4 keeps the rows where they are: None for theirs."""
+    if fp4:
+        return (None, None, *_group_offs(group_lens, ca, True))
+    return _group_offs_pair(group_lens, ra, ca)
+
+
 @native_op("primus_turbo::grouped_quantize_mx")
 def _grouped_quantize_mx_op(
     x: torch.Tensor, out_dtype: torch.dtype, group_lens: torch.Tensor, group_offs: torch.Tensor, want_row: bool,
-    want_col: bool, row_flags: int, col_flags: int,
+    want_col: bool, row_flags: int, col_flags: int, known_offs_row: Optional[torch.Tensor] = None,
+    known_offs_col: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """The outputs of ``_grouped_mx_quantize`` with an empty tensor where that returns None, and
-    empty row lens / offs for MXFP4 (an operator may not hand its inputs back)."""
+    empty lens / offs where they are not new: the rows' for MXFP4, all of them with ``known_offs_*``
+    (an operator may not hand its inputs back)."""
     N.require_cuda(x, group_lens, group_offs)
     if x.dtype not in (torch.bfloat16, torch.float16):
         raise RuntimeError("Input must be BFloat16 or Half")
@@ -1341,8 +1382,9 @@ def _grouped_quantize_mx_op(
     ra, ca, m_pad_row, m_pad_col, n_pad = _grouped_mx_dims(M, Nn, G, fp4)
     dev = x.device
     group_offs = group_offs.contiguous()
-    lens_row, offs_row = (group_lens, group_offs) if fp4 else _group_offs(group_lens, ra, True)
-    lens_col, offs_col = _group_offs(group_lens, ca, True)
+    known = _known_offs(known_offs_col, G) and (fp4 or _known_offs(known_offs_row, G))
+    lens_row, offs_row, lens_col, offs_col = (
+        (None, known_offs_row, None, known_offs_col) if known else _grouped_mx_offs(group_lens, ra, ca, fp4))
     row_q = row_s = col_q = col_s = None
     if want_row:
         row_q = torch.empty((m_pad_row, n_pad // pack), dtype=torch.uint8, device=dev)
@@ -1360,14 +1402,17 @@ def _grouped_quantize_mx_op(
     )
     empty = lambda dt=torch.uint8: torch.empty(0, dtype=dt, device=dev)  # noqa: E731
     view = lambda t, dt: (empty() if t is None else t).view(dt)  # noqa: E731
-    if fp4:
+    if fp4 or known:
         lens_row, offs_row = empty(torch.int64), empty(torch.int64)
+    if known:
+        lens_col, offs_col = empty(torch.int64), empty(torch.int64)
     return (view(row_q, out_dtype), view(row_s, _E8M0), view(col_q, out_dtype), view(col_s, _E8M0),
             lens_row, offs_row, lens_col, offs_col)
 
 
 @_grouped_quantize_mx_op.register_fake
-def _grouped_quantize_mx_op_fake(x, out_dtype, group_lens, group_offs, want_row, want_col, row_flags, col_flags):
+def _grouped_quantize_mx_op_fake(x, out_dtype, group_lens, group_offs, want_row, want_col, row_flags, col_flags,
+                                 known_offs_row=None, known_offs_col=None):
     fp4 = _FP4X2 is not None and out_dtype == _FP4X2
     M, Nn = x.shape
     G = group_lens.numel()
@@ -1379,7 +1424,8 @@ def _grouped_quantize_mx_op_fake(x, out_dtype, group_lens, group_offs, want_row,
             mk((m_pad_row, n_pad // 32) if want_row else (0,), _E8M0),
             mk((Nn, m_pad_col // pack) if want_col else (0,), out_dtype),
             mk((Nn, m_pad_col // 32) if want_col else (0,), _E8M0),
-            i64(0 if fp4 else G), i64(0 if fp4 else G + 1), i64(G), i64(G + 1))
+            *((i64(0) for _ in range(4)) if known_offs_col is not None else
+              (i64(0 if fp4 else G), i64(0 if fp4 else G + 1), i64(G), i64(G + 1))))
 
 
 @native_op("primus_turbo::glu_grouped_quantize_mx")
@@ -1419,8 +1465,7 @@ def glu_grouped_quantize_mx_impl(
     ra, ca, m_pad_row, m_pad_col, n_pad = _grouped_mx_dims(M, Nn, G, fp4)
     dev = x.device
     group_offs = group_offs.contiguous()
-    lens_row, offs_row = (group_lens, group_offs) if fp4 else _group_offs(group_lens, ra, True)
-    lens_col, offs_col = _group_offs(group_lens, ca, True)
+    lens_row, offs_row, lens_col, offs_col = _grouped_mx_offs(group_lens, ra, ca, fp4)
     row_q = torch.empty((m_pad_row, n_pad // pack), dtype=torch.uint8, device=dev)
     row_s = torch.empty((m_pad_row, n_pad // 32), dtype=torch.uint8, device=dev)
     col_q = col_s = None
@@ -1449,7 +1494,7 @@ def _glu_grouped_quantize_mx_impl_fake(x, probs, row_mask, act, out_dtype, group
 
 
 def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, group_offs, with_trans=False,
-                                scaling_recipe=None, scaling_recipe_for_trans=None):
+                                scaling_recipe=None, scaling_recipe_for_trans=None, known=None):
     """MXFP8 quantization of the packed rows of G groups, each virtually zero-padded along M.
 
     ``with_trans`` -> ``(row_q [M_pad_row, N_pad], row_scale [M_pad_row, N_pad/32], col_q [N, M_pad_col],
@@ -1457,12 +1502,13 @@ def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, grou
     otherwise ``(q, scale, group_lens_padded, group_offs_padded)`` of the direction ``axis`` asks
     for (1 = rows padded to 32 per group, 0 = transposed columns padded to 128 per group).
     ``M_pad_row`` / ``M_pad_col`` = ``total_M + G * align`` rounded up to ``align``; what lies
-    beyond ``offs_padded[G]`` is unspecified."""
+    beyond ``offs_padded[G]`` is unspecified. ``known`` (with ``with_trans``): the four lens / offs of an
+    earlier call for the same groups, which are then not computed again."""
     assert block_size == 32, "The block size must be 32 for MXFP8 quantization"
     r, rt = _mx_recipes(with_trans, scaling_recipe, scaling_recipe_for_trans, "MXFP8")
     if with_trans:
         rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, True,
-                                                                  _mx_flags(r), _mx_flags(rt))
+                                                                  _mx_flags(r), _mx_flags(rt), known)
         rq, rs = _apply_mx_shuffles(rq, rs, r, "rowwise")
         cq, cs = _apply_mx_shuffles(cq, cs, rt, "colwise")
         return rq, rs, cq, cs, lr, orow, lc, ocol
@@ -1495,7 +1541,7 @@ def grouped_dequantize_mxfp8_impl(x, out_dtype, axis, block_size, scale_inv, gro
 
 
 def grouped_quantize_mxfp4_impl(x, out_dtype, axis, block_size, group_lens, group_offs, with_trans=False,
-                                scaling_recipe=None, scaling_recipe_for_trans=None):
+                                scaling_recipe=None, scaling_recipe_for_trans=None, known=None):
     """MXFP4 quantization of the packed rows of G groups (reference: quantization_impl.py:657-811,
     layout of its default dispatch flydsl/quantization/mxfp4_grouped_quant.py:320-349).
 
@@ -1508,13 +1554,14 @@ def grouped_quantize_mxfp4_impl(x, out_dtype, axis, block_size, group_lens, grou
     16-point Hadamard transform along that direction (within each group's padded rows for the
     column direction), ``use_sr`` rounds the codes stochastically, ``use_2d_block`` shares one
     exponent per 32 x 32 block counted from the group's first row, ``shuffle_out`` /
-    ``shuffle_scale`` give the pre-shuffled forms of the outputs (a pass over the plain ones)."""
+    ``shuffle_scale`` give the pre-shuffled forms of the outputs (a pass over the plain ones).
+    ``known`` as in :func:`grouped_quantize_mxfp8_impl`."""
     assert block_size == 32, "The block size must be 32 for MXFP4 quantization"
     assert _FP4X2 is not None and out_dtype == _FP4X2, "The out_dtype must be float4_e2m1fn_x2 for MXFP4 quantization"
     r, rt = _mx_recipes(with_trans, scaling_recipe, scaling_recipe_for_trans, "MXFP4")
     if with_trans:
         rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, True,
-                                                                  _mx_flags(r), _mx_flags(rt))
+                                                                  _mx_flags(r), _mx_flags(rt), known)
         rq, rs = _apply_mx_shuffles(rq, rs, r, "rowwise")
         cq, cs = _apply_mx_shuffles(cq, cs, rt, "colwise")
         return rq, rs, cq, cs, lr, orow, lc, ocol

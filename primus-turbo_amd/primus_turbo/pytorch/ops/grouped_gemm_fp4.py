@@ -41,6 +41,7 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp4_impl import (
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     glu_grouped_quantize_mx_impl,
+    grouped_quantize_mxfp4_impl,
     quantize_mxfp4_impl,
 )
 from primus_turbo.pytorch.ops.quantization import (
@@ -98,14 +99,15 @@ def _fp4_weight_operands(b, b_t, config, need_bwd):
     return b_row, b_row_s, b_col, b_col_s
 
 
-def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, config, dgrad_dtype,
-                           wgrad_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad):
-    """dgrad and wgrad of the MXFP4 grouped product from the saved column-direction operands."""
+def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col, offs_col, config,
+                           dgrad_dtype, wgrad_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad):
+    """dgrad and wgrad of the MXFP4 grouped product from the saved column-direction operands; the padded
+    offsets are the forward quantizer's (None: the caller quantized the activation)."""
     gran = config.granularity
-    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_fp4_with_trans(
-        grad_out, float4_e2m1fn_x2, gran, group_lens, group_offs, block_size=config.block_size,
-        scaling_recipe=ScalingRecipe(use_sr=config.use_gradient_sr),
-        scaling_recipe_for_trans=ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True))
+    known = None if offs_col is None else (None, None, lens_col, offs_col)
+    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mxfp4_impl(
+        grad_out, float4_e2m1fn_x2, None, config.block_size, group_lens, group_offs, True,
+        ScalingRecipe(use_sr=config.use_gradient_sr), ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), known)
     # dgrad: grad_a = grad_out @ b as an NT product with the transposed weight quantization [G, K, N]
     grad_a = grouped_gemm_fp4_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
                                    gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
@@ -139,6 +141,7 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
         gran, bs = config.granularity, config.block_size
         need_bwd = any(ctx.needs_input_grad[:2])
         a_recipe, a_t_recipe = ScalingRecipe(), ScalingRecipe(use_rht=True)
+        lens_col = offs_col = None
         if isinstance(a, QuantizedTensor):
             # a grouped (packed rows) quantization made by the caller
             check_quantized_tensor(a, config, axis=-1, scaling_recipe=a_recipe)
@@ -152,7 +155,7 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
                 check_quantized_tensor(a_t, config, scaling_recipe=a_t_recipe)
                 a_col, a_col_s = a_t.qdata, a_t.scale_inv
         elif need_bwd:
-            a_row, a_row_s, a_col, a_col_s, _, offs_row, _, _ = grouped_quantize_fp4_with_trans(
+            a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_fp4_with_trans(
                 a.contiguous(), float4_e2m1fn_x2, gran, group_lens, group_offs, block_size=bs,
                 scaling_recipe=a_recipe, scaling_recipe_for_trans=a_t_recipe)
         else:
@@ -165,17 +168,16 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
                                     gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
         if need_bwd:
-            ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s, group_lens, group_offs)
+            ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col, offs_col)
         ctx.meta = (config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad)
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
         grad_out = _ensure_contiguous_grad_out(grad_out)
-        a_col, a_col_s, b_col, b_col_s, group_lens, group_offs = ctx.saved_tensors
         config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad = ctx.meta
-        grad_a, grad_b = _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, config,
-                                                out_dtype, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad)
+        grad_a, grad_b = _fp4_backward_products(grad_out, *ctx.saved_tensors, config, out_dtype, out_dtype, num_cu, total_m,
+                                                fuse_bgrad_accum, main_grad)
         return grad_a, grad_b, None, None, None, None, None, None, None, None, None
 
 
@@ -203,13 +205,14 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
         total_m = int(x.size(0))
         need_bwd = any(ctx.needs_input_grad[i] for i in (0, 1, 4))
         x2, p1 = x.contiguous(), probs.reshape(-1).contiguous()
-        a_row, a_row_s, a_col, a_col_s, _, _, _, _ = glu_grouped_quantize_mx_impl(
+        a_row, a_row_s, a_col, a_col_s, _, _, lens_col, offs_col = glu_grouped_quantize_mx_impl(
             x2, p1, row_mask, act_type, float4_e2m1fn_x2, group_lens, group_offs, need_bwd, 2)
         b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, None, config, need_bwd)
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, group_offs, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]
         if need_bwd:
-            ctx.save_for_backward(x2, p1, row_mask, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs)
+            ctx.save_for_backward(x2, p1, row_mask, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col,
+                                  offs_col)
         ctx.meta = (config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs.shape)
         return out
 
@@ -218,10 +221,10 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
         from primus_turbo.pytorch.kernels.activation.glu_impl import ACT_GELU, ACT_SILU, glu_bwd_with_probs
 
         grad_out = _ensure_contiguous_grad_out(grad_out)
-        x2, p1, row_mask, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs = ctx.saved_tensors
+        x2, p1, row_mask, *operands = ctx.saved_tensors
         config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs_shape = ctx.meta
-        grad_act, grad_b = _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, config,
-                                                  x2.dtype, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad)
+        grad_act, grad_b = _fp4_backward_products(grad_out, *operands, config, x2.dtype, out_dtype, num_cu, total_m,
+                                                  fuse_bgrad_accum, main_grad)
         grad_x, grad_probs = glu_bwd_with_probs(grad_act.contiguous(), x2, p1, row_mask,
                                                 ACT_SILU if act_type == "silu" else ACT_GELU)
         return grad_x, grad_probs.view(probs_shape), None, None, grad_b, None, None, None, None, None, None, None
