@@ -329,7 +329,9 @@ PT_API int pt_dequantize_fp8_block(const void *q, int q_dtype, int64_t B, int64_
  * "RHT" of the two wgrad operands, which cancels in their product. Bit 2 (MXFP4 only) rounds
  * the codes stochastically (unbiased; scales unchanged) from sr_seed, which the caller changes
  * from launch to launch (mxfp4_quant_kernel.py:48-75: random by design, not reproducible bit
- * for bit against the reference).
+ * for bit against the reference). Bit 3 stores the direction's scales word-major, as the GEMMs read
+ * them: row_scale [B, Npad / 128, M, 4], col_scale [B, Mpad / 128, N, 4] (the four bytes of one
+ * 128-wide stretch of all rows side by side).
  *
  * pt_dequantize_mx replaces dequantize_mxfp8 / dequantize_mxfp4 (quantization.cpp:285-359,
  * 436-508; kernels dequantization_mxfp8.cu:29-113, dequantization_mxfp4.cu:28-160):
@@ -394,7 +396,8 @@ PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const v
  * (both K-contiguous) with row pitches lda / ldb in BYTES; ab_dtype PT_DTYPE_E4M3 / PT_DTYPE_E5M2
  * selects MXFP8 (a_e5m2 / b_e5m2 give each operand's format), PT_DTYPE_E2M1X2 selects MXFP4 (two
  * codes per byte, K counts codes). a_scale [M, >= K / 32] and b_scale [N, >= K / 32] are E8M0
- * bytes with row pitches sa_ld / sb_ld. K % 32 == 0; bytes of a row behind K must be zero
+ * bytes with row pitches sa_ld / sb_ld, or with pitch 0 word-major [K / 128, M, 4] / [K / 128, N, 4]
+ * (K % 128 == 0; either operand by itself). K % 32 == 0; bytes of a row behind K must be zero
  * codes, as the MX quantizers leave them. Rows that are not whole 128-byte slabs (at least
  * four) are first copied into `workspace` (16-byte aligned); a workspace of
  * pt_gemm_mx_workspace_bytes also receives, for large problems, a copy of both scale arrays with
@@ -517,7 +520,8 @@ PT_API int pt_grouped_gemm_fp8_vec_variable_k(const void *lhs, int lhs_dtype, co
  * quantization.cpp:1209-1378; default dispatch flydsl/quantization/mxfp4_grouped_quant.py:320-349):
  * two codes per byte, rows kept tight (row_offs_padded NULL) and column groups padded to 256;
  * row_flags / col_flags / sr_seed as for pt_quantize_mx; a direction's 32 x 32 blocks (bit 0) are
- * counted from its group's first row, the rows behind the group's end being zeros.
+ * counted from its group's first row, the rows behind the group's end being zeros. Word-major row
+ * scales (bit 3) are [Npad / 128, R, 4] with R = M, or M + 32 G rounded up to 32 with padded rows.
  *
  * pt_grouped_gemm_mx replaces primus_turbo::grouped_gemm_fp8_impl for MX_BLOCKWISE
  * (kernels/grouped_gemm/grouped_gemm_fp8_impl.py:888-930 with group_offs_out; caller
@@ -530,7 +534,7 @@ PT_API int pt_grouped_gemm_fp8_vec_variable_k(const void *lhs, int lhs_dtype, co
  * padded row layout above), oo = group_offs_out (rows of the output, packed tight; NULL = the
  * same as o); len_g = oo[g + 1] - oo[g] when oo is given. K counts elements (a multiple of 32);
  * lda == ldb is a multiple of 128 bytes, at least 512, and the bytes of a row behind its K
- * codes are zero.
+ * codes are zero. sa_ld / sb_ld 0: word-major scales [K / 128, a_rows, 4] / [G, K / 128, N, 4].
  *
  * pt_grouped_gemm_mx_variable_k replaces primus_turbo::grouped_gemm_fp8_variable_k_impl for
  * MX_BLOCKWISE (grouped_gemm_fp8_impl.py:933-974; caller ops/grouped_gemm_fp8.py:809-825) and
@@ -560,7 +564,8 @@ PT_API int pt_grouped_quantize_mx(const void *x, int x_dtype, int64_t M, int64_t
  * without y travelling through HBM; bit-identical with running the two steps of this library one
  * after the other. The reference has no fused form. Round to nearest, 1-D blocks; row_q /
  * row_scale are required (fc2's forward operand), col_q / col_scale (its wgrad operand) optional;
- * col_flags: 0, or 2 = Hadamard-transformed column direction (MXFP4's wgrad recipe). probs is
+ * col_flags: bit 1 = Hadamard-transformed column direction (MXFP4's wgrad recipe), bit 3 = word-major
+ * scales in both directions. probs is
  * fp32 [M], row_mask optional int64 [M]. */
 PT_API int pt_glu_grouped_quantize_mx(const void *x, int x_dtype, const float *probs, const int64_t *row_mask,
                                       int act, int64_t M, int64_t N, int q_dtype, const int64_t *group_offs,
@@ -580,6 +585,11 @@ PT_API int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const v
                                          int c_dtype, const int64_t *group_offs, int64_t G, int64_t Ml,
                                          int64_t Nr, int64_t ld, int accumulate, void *workspace,
                                          size_t workspace_bytes, int tile_cfg, void *stream);
+/* The same for word-major scales [ld / 128, Ml, 4] / [ld / 128, Nr, 4]. */
+PT_API int pt_grouped_gemm_mx_variable_k_words(const void *lhs, int lhs_dtype, const void *lhs_scale,
+                                               const void *rhs, int rhs_dtype, const void *rhs_scale, void *c,
+                                               int c_dtype, const int64_t *group_offs, int64_t G, int64_t Ml,
+                                               int64_t Nr, int64_t ld, int accumulate, int tile_cfg, void *stream);
 
 /* Gated activation of an MoE expert MLP with the router probability folded in -------------
  *

@@ -75,20 +75,25 @@ __global__ __launch_bounds__(W * 64) void gemm_direct_kernel(const GemmArgs a) {
         for (int i = 0; i < RM; ++i)
             s.fa[i] = frag(ra, row_a + 16 * i * static_cast<uint32_t>(a.lda));
         if constexpr (MODE == SCALE_MX) {
-            const uint32_t kb = kt * (4 * NH), nkb = static_cast<uint32_t>(a.kb_valid);
-            const uint8_t *sA = reinterpret_cast<const uint8_t *>(a.sA) + m0 * a.sa_m, *sB = reinterpret_cast<const uint8_t *>(a.sB) + n0 * a.sb_n;
-            const __amdgpu_buffer_rsrc_t qa = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sA), 0, on ? static_cast<uint32_t>((rows_a - 1) * a.sa_m) + nkb : 0u, RSRC_FLAGS);
-            const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sB), 0, on ? static_cast<uint32_t>((rows_b - 1) * a.sb_n) + nkb : 0u, RSRC_FLAGS);
+            // row-major or word-major scales, each operand for itself (see GemmArgs)
+            const uint32_t nkb   = static_cast<uint32_t>(a.kb_valid);
+            const uint32_t rowpa = a.sa_wpitch != 0 ? 4u : static_cast<uint32_t>(a.sa_m), rowpb = a.sb_wpitch != 0 ? 4u : static_cast<uint32_t>(a.sb_n);
+            const int64_t  wordpa = a.sa_wpitch != 0 ? a.sa_wpitch : 4, wordpb = a.sb_wpitch != 0 ? a.sb_wpitch : 4;
 #pragma unroll
             for (int h = 0; h < NH; ++h) {
-                const uint32_t b   = kb + 4 * h + lg;
-                const uint32_t off = b < nkb ? b : NOWHERE;
+                const uint32_t word = on ? kt * NH + h : 0u;
+                const bool     some = on && 4 * word < nkb;
+                const uint8_t *sA = reinterpret_cast<const uint8_t *>(a.sA) + m0 * rowpa + word * wordpa;
+                const uint8_t *sB = reinterpret_cast<const uint8_t *>(a.sB) + n0 * rowpb + word * wordpb;
+                const __amdgpu_buffer_rsrc_t qa = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sA), 0, some ? (rows_a - 1) * rowpa + 4u : 0u, RSRC_FLAGS);
+                const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(sB), 0, some ? (rows_b - 1) * rowpb + 4u : 0u, RSRC_FLAGS);
+                const uint32_t off = 4 * word + lg < nkb ? static_cast<uint32_t>(lg) : NOWHERE;
 #pragma unroll
                 for (int i = 0; i < RM; ++i)
-                    s.sa[i][h] = __builtin_amdgcn_raw_buffer_load_b8(qa, (16 * i + lm) * static_cast<uint32_t>(a.sa_m) + off, 0, 0);
+                    s.sa[i][h] = __builtin_amdgcn_raw_buffer_load_b8(qa, (16 * i + lm) * rowpa + off, 0, 0);
 #pragma unroll
                 for (int j = 0; j < RN; ++j)
-                    s.sb[j][h] = __builtin_amdgcn_raw_buffer_load_b8(qb, (16 * j + lm) * static_cast<uint32_t>(a.sb_n) + off, 0, 0);
+                    s.sb[j][h] = __builtin_amdgcn_raw_buffer_load_b8(qb, (16 * j + lm) * rowpb + off, 0, 0);
             }
         }
         if constexpr (MODE == SCALE_BLOCK) {

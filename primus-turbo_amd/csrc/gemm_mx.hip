@@ -67,7 +67,9 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     PT_REQUIRE(M >= 0 && N >= 0 && K > 0 && K % 32 == 0, "K must be a positive multiple of 32");
     PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= 4, "tile_cfg must be 0..4");
     const int64_t kbytes = fp4 ? K / 2 : K, kblocks = K / 32;
-    PT_REQUIRE(lda >= kbytes && ldb >= kbytes && sa_ld >= kblocks && sb_ld >= kblocks, "row pitches too small");
+    const bool    words_a = sa_ld == 0, words_b = sb_ld == 0; // word-major scales
+    PT_REQUIRE(lda >= kbytes && ldb >= kbytes && (words_a || sa_ld >= kblocks) && (words_b || sb_ld >= kblocks), "row pitches too small");
+    PT_REQUIRE((!words_a && !words_b) || K % 128 == 0, "word-major scales need K to be a multiple of 128");
     PT_REQUIRE(kbytes < (1LL << 24), "K too large");
     if (M == 0 || N == 0)
         return PT_OK;
@@ -80,30 +82,32 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     // that carry anything but zeros behind K, into zero-padded rows
     const int64_t  need = mx_row_bytes(K, fp4);
     const uint8_t *A = static_cast<const uint8_t *>(a), *B = static_cast<const uint8_t *>(b);
-    // word-major scales need whole 32-bit words per row in the source, and room in the workspace:
-    // without it (a caller that passes only what the operand copies need, or nothing) the scales
-    // are read in place
+    // word-major copies of scales that are not word-major already need whole 32-bit words per row in the
+    // source, and room in the workspace: without it (a caller that passes only what the operand copies
+    // need, or nothing) the scales are read in place
     const bool     copies    = lda != need || ldb != need;
     const size_t   want_copy = static_cast<size_t>((lda != need ? round_up(M * need, 256) : 0) + (ldb != need ? round_up(N * need, 256) : 0));
     const size_t   want_all  = pt_gemm_mx_workspace_bytes(M, N, K, lda, ldb, fp4);
     const bool     have_all  = workspace != nullptr && workspace_bytes >= want_all && aligned_to(workspace, 16);
-    const bool     wordmajor = have_all && mx_wordmajor_pays(M, N, K) && sa_ld % 4 == 0 && sb_ld % 4 == 0 &&
-                           aligned_to(a_scale, 4) && aligned_to(b_scale, 4) && sa_ld >= mx_scale_words(K) * 4 &&
-                           sb_ld >= mx_scale_words(K) * 4;
+    const bool     pays = have_all && mx_wordmajor_pays(M, N, K);
+    const bool     copy_sa = pays && !words_a && sa_ld % 4 == 0 && aligned_to(a_scale, 4) && sa_ld >= mx_scale_words(K) * 4;
+    const bool     copy_sb = pays && !words_b && sb_ld % 4 == 0 && aligned_to(b_scale, 4) && sb_ld >= mx_scale_words(K) * 4;
     const void *sa_use = a_scale, *sb_use = b_scale;
-    if ((copies || wordmajor) && (workspace == nullptr || workspace_bytes < want_copy || !aligned_to(workspace, 16)))
+    if (copies && (workspace == nullptr || workspace_bytes < want_copy || !aligned_to(workspace, 16)))
         return fail(PT_ERR_WORKSPACE, "pt_gemm_mx: workspace missing, too small or misaligned");
     // few output tiles: a kernel that reads rows and scales as they are (gemm_direct.h)
     const int direct = tile_cfg == 0 && lda < (1LL << 24) && ldb < (1LL << 24) ? gemm_direct_tile(M, N, kbytes, SCALE_MX, fp4) : -1;
-    if ((copies || wordmajor) && direct < 0) {
-        uint8_t *ws = static_cast<uint8_t *>(workspace);
-        if (wordmajor) {
-            const int64_t W = mx_scale_words(K);
-            // in: [rows, sa_ld / 4] words (the first W of every row are used) -> out: [W, rows]
+    if ((copies || copy_sa || copy_sb) && direct < 0) {
+        uint8_t      *ws = static_cast<uint8_t *>(workspace);
+        const int64_t W  = mx_scale_words(K);
+        // in: [rows, sa_ld / 4] words (the first W of every row are used) -> out: [W, rows]
+        if (copy_sa) {
             if (const int rc = launch_transpose_words(static_cast<const uint32_t *>(a_scale), reinterpret_cast<uint32_t *>(ws), M, W, sa_ld / 4, st))
                 return rc;
             sa_use = ws;
             ws += round_up(M * W * 4, 256);
+        }
+        if (copy_sb) {
             if (const int rc = launch_transpose_words(static_cast<const uint32_t *>(b_scale), reinterpret_cast<uint32_t *>(ws), N, W, sb_ld / 4, st))
                 return rc;
             sb_use = ws;
@@ -126,8 +130,8 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     g.C          = c;
     g.sA         = reinterpret_cast<const float *>(sa_use); // E8M0 bytes in this mode
     g.sB         = reinterpret_cast<const float *>(sb_use);
-    g.sa_wpitch  = wordmajor ? M * 4 : 0;
-    g.sb_wpitch  = wordmajor ? N * 4 : 0;
+    g.sa_wpitch  = words_a || (copy_sa && direct < 0) ? M * 4 : 0;
+    g.sb_wpitch  = words_b || (copy_sb && direct < 0) ? N * 4 : 0;
     g.M          = M;
     g.N          = N;
     g.K          = need;
@@ -142,7 +146,6 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     if (direct >= 0) {
         if (sa_ld % 4 != 0 || sb_ld % 4 != 0 || !aligned_to(a_scale, 4) || !aligned_to(b_scale, 4)) // (as the tiled kernel)
             return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
-        g.sa_wpitch = g.sb_wpitch = 0; // (A, B and the scales are the caller's)
         g.kb_valid = static_cast<int>(kblocks); // (reads byte by byte)
         g.K   = kbytes;
         g.lda = lda;

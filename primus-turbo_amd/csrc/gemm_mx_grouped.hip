@@ -82,8 +82,10 @@ int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, int64_t 
                "row pitches must be equal multiples of 128 bytes, at least 512, that hold K");
     PT_REQUIRE(lda < (1LL << 24), "K must be below 2^24");
     PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= 4, "tile_cfg must be 0..4");
-    PT_REQUIRE(sa_ld >= K / 32 && sb_ld >= K / 32 && sa_ld % 4 == 0 && sb_ld % 4 == 0,
+    const bool words_a = sa_ld == 0, words_b = sb_ld == 0; // word-major scales
+    PT_REQUIRE((words_a || (sa_ld >= K / 32 && sa_ld % 4 == 0)) && (words_b || (sb_ld >= K / 32 && sb_ld % 4 == 0)),
                "scale rows must hold K / 32 bytes and be 4-byte multiples");
+    PT_REQUIRE((!words_a && !words_b) || K % 128 == 0, "word-major scales need K to be a multiple of 128");
     auto st = static_cast<hipStream_t>(stream);
     if (out_rows == 0 || N == 0)
         return PT_OK;
@@ -112,20 +114,28 @@ int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, int64_t 
         g.group_offs_out = group_offs_out;
         g.b_gstride      = N * ldb;
         g.sb_gstride     = N * sb_ld / 4; // the kernel steps a 4-byte pointer
-        // with a workspace: scale words of one K position of all rows contiguous (two cache lines
-        // per scale copy of the kernel instead of sixty-four)
-        const int64_t W = mxg_words(K / 32);
-        if (workspace != nullptr && aligned_to(workspace, 16) && aligned_to(a_scale, 4) && aligned_to(b_scale, 4) &&
-            workspace_bytes >= pt_grouped_gemm_mx_workspace_bytes(G, a_rows, N, K) && sa_ld >= 4 * W && sb_ld >= 4 * W) {
-            uint32_t *wa = static_cast<uint32_t *>(workspace);
-            uint32_t *wb = wa + round_up(a_rows * W * 4, 256) / 4;
+        // word-major scales, made with a workspace where they do not come so: the words of one K position of all
+        // rows contiguous (two cache lines per scale copy of the kernel instead of sixty-four)
+        const int64_t W    = mxg_words(K / 32);
+        const bool    room = workspace != nullptr && aligned_to(workspace, 16) &&
+                          workspace_bytes >= pt_grouped_gemm_mx_workspace_bytes(G, a_rows, N, K);
+        const bool copy_sa = !words_a && room && aligned_to(a_scale, 4) && sa_ld >= 4 * W;
+        const bool copy_sb = !words_b && room && aligned_to(b_scale, 4) && sb_ld >= 4 * W;
+        uint32_t  *wa      = static_cast<uint32_t *>(workspace);
+        if (copy_sa) {
             if (const int rc = launch_transpose_words(static_cast<const uint32_t *>(a_scale), wa, a_rows, W, sa_ld / 4, st))
                 return rc;
+            g.sA = reinterpret_cast<const float *>(wa);
+        }
+        if (copy_sb) {
+            uint32_t *wb = wa + round_up(a_rows * W * 4, 256) / 4;
             if (const int rc = launch_transpose_words(static_cast<const uint32_t *>(b_scale), wb, N, W, sb_ld / 4, st, G))
                 return rc;
-            g.sA         = reinterpret_cast<const float *>(wa);
-            g.sB         = reinterpret_cast<const float *>(wb);
-            g.sa_wpitch  = a_rows * 4;
+            g.sB = reinterpret_cast<const float *>(wb);
+        }
+        if (words_a || copy_sa)
+            g.sa_wpitch = a_rows * 4;
+        if (words_b || copy_sb) {
             g.sb_wpitch  = N * 4;
             g.sb_gstride = W * N;
         }
@@ -135,10 +145,10 @@ int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, int64_t 
     return launch_zero_rows(c, group_offs_out ? group_offs_out : group_offs, G, out_rows, N * (c_dtype == PT_DTYPE_F32 ? 4 : 2), st);
 }
 
-int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lhs_scale, const void *rhs, int rhs_dtype,
-                                  const void *rhs_scale, void *c, int c_dtype, const int64_t *group_offs, int64_t G,
-                                  int64_t Ml, int64_t Nr, int64_t ld, int accumulate, void *workspace,
-                                  size_t workspace_bytes, int tile_cfg, void *stream) {
+static int mxg_variable_k(const void *lhs, int lhs_dtype, const void *lhs_scale, const void *rhs, int rhs_dtype,
+                          const void *rhs_scale, bool words, void *c, int c_dtype, const int64_t *group_offs, int64_t G,
+                          int64_t Ml, int64_t Nr, int64_t ld, int accumulate, void *workspace, size_t workspace_bytes,
+                          int tile_cfg, void *stream) {
     const bool fp4 = lhs_dtype == PT_DTYPE_E2M1X2;
     PT_REQUIRE(fp4 ? rhs_dtype == PT_DTYPE_E2M1X2 : (is_fp8_dtype(lhs_dtype) && is_fp8_dtype(rhs_dtype)),
                "operands must both be fp8 (e4m3 / e5m2) or both e2m1x2");
@@ -173,8 +183,9 @@ int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lh
     g.group_offs = group_offs;
     g.c_gstride  = Ml * Nr;
     const int64_t W = mxg_words(ld / 32);
-    if (workspace != nullptr && aligned_to(workspace, 16) && aligned_to(lhs_scale, 4) && aligned_to(rhs_scale, 4) &&
-        workspace_bytes >= pt_grouped_gemm_mx_variable_k_workspace_bytes(Ml, Nr, ld) && (ld / 32) % 4 == 0) {
+    const bool    copy = !words && workspace != nullptr && aligned_to(workspace, 16) && aligned_to(lhs_scale, 4) && aligned_to(rhs_scale, 4) &&
+                      workspace_bytes >= pt_grouped_gemm_mx_variable_k_workspace_bytes(Ml, Nr, ld) && (ld / 32) % 4 == 0;
+    if (copy) {
         auto      st = static_cast<hipStream_t>(stream);
         uint32_t *wa = static_cast<uint32_t *>(workspace);
         uint32_t *wb = wa + round_up(Ml * W * 4, 256) / 4;
@@ -184,6 +195,8 @@ int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lh
             return rc;
         g.sA        = reinterpret_cast<const float *>(wa);
         g.sB        = reinterpret_cast<const float *>(wb);
+    }
+    if (words || copy) {
         g.sa_wpitch = Ml * 4;
         g.sb_wpitch = Nr * 4;
         g.sa_k      = (fp4 ? 2 : 1) * Ml; // a slab's scale words of all rows, in steps of the kernel's 4-byte scale pointer
@@ -191,6 +204,21 @@ int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lh
     }
     return launch_mxg<GROUP_K>(g, fp4 ? 4 : lhs_dtype == PT_DTYPE_E5M2, rhs_dtype == PT_DTYPE_E5M2, tile_cfg,
                                static_cast<hipStream_t>(stream));
+}
+
+int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lhs_scale, const void *rhs, int rhs_dtype,
+                                  const void *rhs_scale, void *c, int c_dtype, const int64_t *group_offs, int64_t G,
+                                  int64_t Ml, int64_t Nr, int64_t ld, int accumulate, void *workspace,
+                                  size_t workspace_bytes, int tile_cfg, void *stream) {
+    return mxg_variable_k(lhs, lhs_dtype, lhs_scale, rhs, rhs_dtype, rhs_scale, false, c, c_dtype, group_offs, G, Ml, Nr, ld,
+                          accumulate, workspace, workspace_bytes, tile_cfg, stream);
+}
+
+int pt_grouped_gemm_mx_variable_k_words(const void *lhs, int lhs_dtype, const void *lhs_scale, const void *rhs, int rhs_dtype,
+                                        const void *rhs_scale, void *c, int c_dtype, const int64_t *group_offs, int64_t G,
+                                        int64_t Ml, int64_t Nr, int64_t ld, int accumulate, int tile_cfg, void *stream) {
+    return mxg_variable_k(lhs, lhs_dtype, lhs_scale, rhs, rhs_dtype, rhs_scale, true, c, c_dtype, group_offs, G, Ml, Nr, ld,
+                          accumulate, nullptr, 0, tile_cfg, stream);
 }
 
 } // extern "C"

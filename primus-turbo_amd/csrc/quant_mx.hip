@@ -161,9 +161,13 @@ struct MxArgs {
     const void *x; // [B, M, N] bf16 / fp16
     int64_t     B, M, N, Mpad, Npad;
     uint8_t    *row_q; // [B, M, Npad] (FP4: Npad / 2 bytes per row) or NULL
-    uint8_t    *row_s; // [B, M, Npad / 32] or NULL
+    uint8_t    *row_s; // [B, M, Npad / 32] or NULL; word-major: [B, Npad / 128, rows, 4]
     uint8_t    *col_q; // [B, N, Mpad] (FP4: Mpad / 2) or NULL
-    uint8_t    *col_s; // [B, N, Mpad / 32] or NULL
+    uint8_t    *col_s; // [B, N, Mpad / 32] or NULL; word-major: [B, Mpad / 128, N, 4]
+    // Bytes from the scale word of a row (column) to the next one's, and to the row's next word. Word-major
+    // scales are what the GEMM reads (gemm_fp8_kernel.h): a tile's 128 words leave side by side, 512 bytes,
+    // instead of one word into each of 128 rows, and no product transposes them first.
+    int64_t row_s_row, row_s_word, col_s_row, col_s_word;
     // Grouped mode (B = 1, group_offs != NULL): the rows of x belong to G groups; the tile grid
     // runs over the row space in which every group is padded to a multiple of 128 rows
     // (col_offs_pad, Mpad = its allocated extent): the column-direction output lives there, pad
@@ -536,7 +540,7 @@ __global__ __launch_bounds__(256) void mx_quant_kernel(const MxArgs a) {
         } // the row pass through the LDS
         // the four scale bytes of a tile row leave as one word (Npad / 32 is a multiple of 4)
         if (tid < MX_TILE && tid < row_cnt)
-            *reinterpret_cast<uint32_t *>(a.row_s + (row_dst0 + tid) * (a.Npad >> 5) + (n0 >> 5)) =
+            *reinterpret_cast<uint32_t *>(a.row_s + b * a.M * (a.Npad >> 5) + (row_dst0 - b * a.M + tid) * a.row_s_row + (n0 >> 7) * a.row_s_word) =
                 *reinterpret_cast<const uint32_t *>(&sbytes[tid * 4]);
     }
 
@@ -626,7 +630,7 @@ __global__ __launch_bounds__(256) void mx_quant_kernel(const MxArgs a) {
             }
         }
         if (tid < MX_TILE && n0 + tid < a.N)
-            *reinterpret_cast<uint32_t *>(a.col_s + (b * a.N + n0 + tid) * (a.Mpad >> 5) + (m0 >> 5)) =
+            *reinterpret_cast<uint32_t *>(a.col_s + b * a.N * (a.Mpad >> 5) + (n0 + tid) * a.col_s_row + (m0 >> 7) * a.col_s_word) =
                 *reinterpret_cast<const uint32_t *>(&sbytes[tid * 4]);
     }
     PT_MX_TRACE(7);
@@ -741,10 +745,19 @@ __global__ __launch_bounds__(256) void mx_quant_rows_kernel(const MxArgs a, cons
     }
 }
 
+// rows: of the row direction's output
+static void mx_scale_layout(MxArgs &a, int row_flags, int col_flags, int64_t rows) {
+    const bool wr = (row_flags & 8) != 0, wc = (col_flags & 8) != 0;
+    a.row_s_row  = wr ? 4 : a.Npad / 32;
+    a.row_s_word = wr ? rows * 4 : 4;
+    a.col_s_row  = wc ? 4 : a.Mpad / 32;
+    a.col_s_word = wc ? a.N * 4 : 4;
+}
+
 // The streaming row kernel serves an ungrouped launch when only the row direction is asked for,
-// with 1-D blocks and no transform, and the rows are whole 16-byte pieces.
+// with 1-D blocks, no transform and row-major scales, and the rows are whole 16-byte pieces.
 static bool mx_rows_stream_ok(const MxArgs &a, bool row2d, bool rht) {
-    return a.col_q == nullptr && a.row_q != nullptr && !row2d && !rht && (a.N & 7) == 0 &&
+    return a.row_s_word == 4 && a.col_q == nullptr && a.row_q != nullptr && !row2d && !rht && (a.N & 7) == 0 &&
            (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && a.group_offs == nullptr;
 }
 template <typename T> static void launch_mx_rows(const MxArgs &a, int fmt, hipStream_t st) {
@@ -992,9 +1005,9 @@ using namespace pt;
 extern "C" {
 
 // direction flags: bit 0 = 2-D (32 x 32) blocks, bit 1 = Hadamard transform (MXFP4, 1-D blocks),
-// bit 2 = stochastic rounding (MXFP4)
+// bit 2 = stochastic rounding (MXFP4), bit 3 = word-major scales
 static int check_mx_flags(int fmt, int row_flags, int col_flags) {
-    PT_REQUIRE((row_flags & ~7) == 0 && (col_flags & ~7) == 0, "unknown direction flags");
+    PT_REQUIRE((row_flags & ~15) == 0 && (col_flags & ~15) == 0, "unknown direction flags");
     const bool rht = ((row_flags | col_flags) & 2) != 0;
     PT_REQUIRE(!rht || fmt == MX_E2M1, "the Hadamard transform belongs to the MXFP4 recipe");
     PT_REQUIRE(((row_flags | col_flags) & 4) == 0 || fmt == MX_E2M1, "stochastic rounding belongs to the MXFP4 recipe");
@@ -1037,6 +1050,7 @@ int pt_quantize_mx(const void *x, int x_dtype, int64_t B, int64_t M, int64_t N, 
     a.row_mask   = nullptr;
     a.sr_mask    = ((row_q && (row_flags & 4)) ? 1 : 0) | ((col_q && (col_flags & 4)) ? 2 : 0);
     a.sr_seed    = sr_seed;
+    mx_scale_layout(a, row_flags, col_flags, M);
     PT_REQUIRE(a.Mpad / 128 < 65536 && B < 65536, "grid dimension out of range");
     dim3 grid(static_cast<unsigned>(a.Npad / 128), static_cast<unsigned>(a.Mpad / 128), static_cast<unsigned>(B));
     auto st = static_cast<hipStream_t>(stream);
@@ -1109,6 +1123,7 @@ static int grouped_quantize_mx(const void *x, int x_dtype, const float *probs, c
     a.sr_seed      = sr_seed;
     a.probs        = probs;
     a.row_mask     = row_mask;
+    mx_scale_layout(a, row_flags, col_flags, row_offs_padded != nullptr ? cdiv(M + 32 * G, 32) * 32 : M);
     PT_REQUIRE(col_ld / 128 < 65536, "grid dimension out of range");
     dim3 grid(static_cast<unsigned>(a.Npad / 128), static_cast<unsigned>(col_ld / 128), 1);
     auto st = static_cast<hipStream_t>(stream);
@@ -1146,8 +1161,8 @@ int pt_glu_grouped_quantize_mx(const void *x, int x_dtype, const float *probs, c
                                void *col_scale, int col_flags, int64_t col_ld, void *stream) {
     PT_REQUIRE(act == ACT_SILU || act == ACT_GELU, "act must be 0 (SiLU) or 1 (GELU)");
     return grouped_quantize_mx(x, x_dtype, probs, row_mask, 1 + act, M, N, q_dtype, group_offs,
-                               row_offs_padded, col_offs_padded, G, row_q, row_scale, 0, col_q, col_scale, col_flags, col_ld,
-                               0u, stream);
+                               row_offs_padded, col_offs_padded, G, row_q, row_scale, col_flags & 8, col_q, col_scale, col_flags,
+                               col_ld, 0u, stream);
 }
 
 int pt_dequantize_mx(const void *q, int q_dtype, const void *scale, int64_t rows, int64_t cols, void *y, int y_dtype,

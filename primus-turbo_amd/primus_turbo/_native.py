@@ -212,6 +212,11 @@ _SIGNATURES = {
         [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_i64, c_i64, c_i64, c_i64, c_int,
          c_void_p, c_size_t, c_int, c_void_p],
     ),
+    "pt_grouped_gemm_mx_variable_k_words": (
+        c_int,
+        [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_i64, c_i64, c_i64, c_i64, c_int,
+         c_int, c_void_p],
+    ),
     "pt_dequantize_fp8_block": (
         c_int,
         [c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_i64, c_i64, c_void_p, c_int, c_void_p],

@@ -69,9 +69,21 @@ def _scale_desc(granularity, a_scale_inv, b_scale_inv, trans_a, trans_b, M, Nn, 
     raise NotImplementedError(f"granularity {granularity} is handled by the MX GEMM entry points")
 
 
+def _mx_scale_pitch(scale, rows, K):
+    """Bytes from one row's scales to the next row's; 0 for word-major ones."""
+    if scale.dtype == torch.int32:
+        _check(tuple(scale.shape) == (K // 128, rows) and K % 128 == 0, "word-major scales must be [K / 128, rows]")
+        return 0
+    _check(scale.shape[0] == rows, "scale rows must match operand rows")
+    _check(scale.shape[1] >= K // 32, "scales must hold K / 32 blocks per row")
+    _check(scale.element_size() == 1, "scales must be E8M0 bytes")
+    return scale.shape[1]
+
+
 def launch_mx(a, a_scale, b, b_scale, out, trans_c, accumulate):
     """NT GEMM with E8M0 block scales on MX-quantized operands: ``a`` ``[M, K]`` and ``b`` ``[N, K]``
-    codes (fp8, or ``float4_e2m1fn_x2`` with two codes per byte), scales ``[rows, K / 32]``."""
+    codes (fp8, or ``float4_e2m1fn_x2`` with two codes per byte), scales ``[rows, K / 32]`` or, of either
+    operand, int32 words ``[K / 128, rows]``."""
     N.require_cuda(a, b, a_scale, b_scale, out)
     fp4 = hasattr(torch, "float4_e2m1fn_x2") and a.dtype == torch.float4_e2m1fn_x2
     _check(a.dim() == 2 and b.dim() == 2, "MX GEMM expects 2-D operands")
@@ -85,21 +97,21 @@ def launch_mx(a, a_scale, b, b_scale, out, trans_c, accumulate):
     K = a.shape[1] * pack
     _check(b.shape[1] * pack == K, f"reduction dims differ: {K} vs {b.shape[1] * pack}")
     _check(K % 32 == 0, "K must be a multiple of 32")
-    _check(a_scale.shape[0] == M and b_scale.shape[0] == Nn, "scale rows must match operand rows")
-    _check(a_scale.shape[1] >= K // 32 and b_scale.shape[1] >= K // 32, "scales must hold K / 32 blocks per row")
-    _check(a_scale.element_size() == 1 and b_scale.element_size() == 1, "scales must be E8M0 bytes")
+    sa_ld, sb_ld = _mx_scale_pitch(a_scale, M, K), _mx_scale_pitch(b_scale, Nn, K)
     _check(tuple(out.shape) == (M, Nn) and out.is_contiguous(), f"out must be a contiguous {(M, Nn)} tensor")
     lib = N.lib()
     lda = ldb = K // pack
     ws = None
-    ws_bytes = lib.pt_gemm_mx_workspace_bytes(M, Nn, K, lda, ldb, int(fp4))
+    # (rows of whole slabs with word-major scales need no copy of anything)
+    ready = sa_ld == 0 and sb_ld == 0 and lda % 128 == 0 and lda >= 512
+    ws_bytes = 0 if ready else lib.pt_gemm_mx_workspace_bytes(M, Nn, K, lda, ldb, int(fp4))
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
     N.check(
         lib.pt_gemm_mx(
             N.ptr(a), N.ptr(a_scale), N.ptr(b), N.ptr(b_scale), N.dtype_code(a.dtype),
             int(a.dtype == torch.float8_e5m2), int(b.dtype == torch.float8_e5m2),
-            N.ptr(out), N.dtype_code(out.dtype), M, Nn, K, lda, ldb, a_scale.shape[1], b_scale.shape[1],
+            N.ptr(out), N.dtype_code(out.dtype), M, Nn, K, lda, ldb, sa_ld, sb_ld,
             int(accumulate), N.ptr(ws), ws_bytes, TILE_CFG, N.stream_of(a),
         )
     )

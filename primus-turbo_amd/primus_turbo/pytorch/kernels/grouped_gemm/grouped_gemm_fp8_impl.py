@@ -118,8 +118,27 @@ def _is_mx(granularity: int) -> bool:
     return ScalingGranularity(granularity) == ScalingGranularity.MX_BLOCKWISE
 
 
+def _mx_group_scales(scales, lead, rows, K, what):
+    """-> (contiguous scales, bytes from one row's to the next row's, 0 for word-major int32 ``[.., K / 128, rows]``)"""
+    if scales.dtype == torch.int32:
+        _check(tuple(scales.shape) == (*lead, K // 128, rows) and K % 128 == 0, f"word-major {what} must be [.., K / 128, rows]")
+        return scales.contiguous(), 0
+    s = _u8(scales)
+    _check(s.dim() == len(lead) + 2 and tuple(s.shape[:-1]) == (*lead, rows) and s.shape[-1] >= K // 32,
+           f"{what} must be {[*lead, rows]} rows of K/32")
+    _check(s.shape[-1] % 4 == 0, "scale rows must be multiples of 4 bytes")
+    return s, s.shape[-1]
+
+
 def _u8(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous().view(torch.uint8)
+
+
+def _row_major_scales(scales: torch.Tensor) -> torch.Tensor:
+    """E8M0 bytes ``[rows, K / 32]`` (an operand that the caller quantized meets one quantized here)."""
+    if scales.dtype != torch.int32:
+        return _u8(scales)
+    return scales.t().clone(memory_format=torch.contiguous_format).view(torch.uint8)
 
 
 _FP4X2 = getattr(torch, "float4_e2m1fn_x2", None)
@@ -155,20 +174,20 @@ def _grouped_mx(a, b, a_scales, b_scales, group_offs, group_offs_out, trans_a, t
     # csrc/pytorch/quantization/quantization.cpp:971-1100)
     _check(K % 32 == 0, "MX grouped GEMM needs K to be a multiple of 32")
     _check(group_offs.dtype == torch.int64 and group_offs.numel() == G + 1, "group_offs must be int64 [G + 1]")
-    a_s, b_s = _u8(a_scales), _u8(b_scales)
-    _check(a_s.dim() == 2 and a_s.shape[0] == rows and a_s.shape[1] >= K // 32, "a_scales must be [rows, K/32]")
-    _check(b_s.dim() == 3 and tuple(b_s.shape[:2]) == (G, Nn) and b_s.shape[2] >= K // 32, "b_scales must be [G, N, K/32]")
-    _check(a_s.shape[1] % 4 == 0 and b_s.shape[2] % 4 == 0, "scale rows must be multiples of 4 bytes")
+    a_s, sa_ld = _mx_group_scales(a_scales, (), rows, K, "a_scales")
+    b_s, sb_ld = _mx_group_scales(b_scales, (G,), Nn, K, "b_scales")
     da, db = N.dtype_code(a.dtype), N.dtype_code(b.dtype)
     a, b = _mx_pitch(_u8(a), kb), _mx_pitch(_u8(b), kb)
     out = torch.empty((rows, Nn), dtype=out_dtype, device=a.device)
     oo = None if group_offs_out is None else group_offs_out.contiguous()
-    # word-major scale copies pay once the K loop is long (measured: MXFP8 from K = 4096, MXFP4 from K = 2048)
-    ws_bytes = N.lib().pt_grouped_gemm_mx_workspace_bytes(G, rows, Nn, K) if K >= (2048 if fp4 else 4096) else 0
+    # word-major copies of scales that are not pay once the K loop is long (measured: MXFP8 from K = 4096, MXFP4 from
+    # K = 2048)
+    copy = (sa_ld != 0 or sb_ld != 0) and K >= (2048 if fp4 else 4096)
+    ws_bytes = N.lib().pt_grouped_gemm_mx_workspace_bytes(G, rows, Nn, K) if copy else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     N.check(
         N.lib().pt_grouped_gemm_mx(
-            N.ptr(a), da, N.ptr(a_s), a.shape[1], a_s.shape[1], N.ptr(b), db, N.ptr(b_s), b.shape[2], b_s.shape[2], N.ptr(out),
+            N.ptr(a), da, N.ptr(a_s), a.shape[1], sa_ld, N.ptr(b), db, N.ptr(b_s), b.shape[2], sb_ld, N.ptr(out),
             N.dtype_code(out.dtype), N.ptr(group_offs.contiguous()), N.ptr(oo), G, rows, rows, Nn, K, N.ptr(ws), ws_bytes,
             MX_TILE_CFG, N.stream_of(a),
         )
@@ -195,11 +214,22 @@ def _variable_k_mx(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans
     Nr = b.shape[0]
     G = group_offs.numel() - 1
     _check(ld % (256 if fp4 else 128) == 0, "the padded length must be a multiple of 128 (MXFP4: 256)")
-    a_s, b_s = _u8(a_scales), _u8(b_scales)
-    _check(tuple(a_s.shape) == (Ml, ld // 32) and tuple(b_s.shape) == (Nr, ld // 32), "scales must be [rows, padded length / 32]")
     _check(tuple(out.shape) == (G, Ml, Nr) and out.is_contiguous(), f"out must be a contiguous {(G, Ml, Nr)} tensor")
     da, db = N.dtype_code(a.dtype), N.dtype_code(b.dtype)
     a, b = _u8(a), _u8(b)
+    if a_scales.dtype == torch.int32 and b_scales.dtype == torch.int32:
+        a_s, b_s = a_scales.contiguous(), b_scales.contiguous()
+        _check(tuple(a_s.shape) == (ld // 128, Ml) and tuple(b_s.shape) == (ld // 128, Nr),
+               "word-major scales must be [padded length / 128, rows]")
+        N.check(
+            N.lib().pt_grouped_gemm_mx_variable_k_words(
+                N.ptr(a), da, N.ptr(a_s), N.ptr(b), db, N.ptr(b_s), N.ptr(out), N.dtype_code(out.dtype),
+                N.ptr(group_offs.contiguous()), G, Ml, Nr, ld, int(accumulate), _cfg_without_eight_waves(), N.stream_of(a),
+            )
+        )
+        return out
+    a_s, b_s = (_row_major_scales(s) for s in (a_scales, b_scales))
+    _check(tuple(a_s.shape) == (Ml, ld // 32) and tuple(b_s.shape) == (Nr, ld // 32), "scales must be [rows, padded length / 32]")
     ws_bytes = N.lib().pt_grouped_gemm_mx_variable_k_workspace_bytes(Ml, Nr, ld) if ld >= 1024 else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
     N.check(

@@ -1160,6 +1160,27 @@ def _mx_shapes(x, out_dtype, want_row, want_col):
             lead + (Nn, Mp // pack) if want_col else none, lead + (Nn, Mp // 32) if want_col else none)
 
 
+#: direction flag of the native quantizers: scales stored word-major
+_MX_WORDS = 8
+
+
+def _mx_scales(lead, rows, width, flags, device):
+    """The scale tensor of one direction: E8M0 bytes ``[.., rows, width / 32]``, or word-major, int32 words
+    ``[.., width / 128, rows]`` of four bytes each: the layout the products read (``launch_mx``)."""
+    if flags & _MX_WORDS:
+        return torch.empty((*lead, width // 128, rows), dtype=torch.int32, device=device)
+    return torch.empty((*lead, rows, width // 32), dtype=torch.uint8, device=device).view(_E8M0)
+
+
+def quantize_mx_operands(x, out_dtype, recipe, recipe_t, what):
+    """Both directions of an operand for this package's own products, ``(q_row, words_row, q_col, words_col)``:
+    the codes of ``quantize_mxfp8_impl`` / ``quantize_mxfp4_impl`` with ``with_trans``, the same scale bytes
+    word-major. For scales that stay between a quantizer and a product; what a caller may see is row-major."""
+    r, rt = _mx_recipes(True, recipe, recipe_t, what)
+    _check(not (r.shuffle_out or r.shuffle_scale or rt.shuffle_out or rt.shuffle_scale), "operands have the plain layout")
+    return _mx_quantize(x, out_dtype, True, True, _mx_flags(r) | _MX_WORDS, _mx_flags(rt) | _MX_WORDS)
+
+
 def _mx_quantize(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, want_col: bool, row_flags: int, col_flags: int):
     """-> (row_q, row_scale, col_q, col_scale); the pair of an unwanted direction is None.
     ``row_flags`` / ``col_flags``: see ``_mx_flags``."""
@@ -1196,10 +1217,10 @@ def _quantize_mx_op(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, wan
     row_q = row_s = col_q = col_s = None
     if want_row:
         row_q = torch.empty(lead + (M, Np // pack), dtype=torch.uint8, device=dev)
-        row_s = torch.empty(lead + (M, Np // 32), dtype=torch.uint8, device=dev)
+        row_s = _mx_scales(lead, M, Np, row_flags, dev)
     if want_col:
         col_q = torch.empty(lead + (Nn, Mp // pack), dtype=torch.uint8, device=dev)
-        col_s = torch.empty(lead + (Nn, Mp // 32), dtype=torch.uint8, device=dev)
+        col_s = _mx_scales(lead, Nn, Mp, col_flags, dev)
     N.check(
         N.lib().pt_quantize_mx(
             N.ptr(x), N.dtype_code(x.dtype), B, M, Nn, N.dtype_code(out_dtype),
@@ -1209,14 +1230,18 @@ def _quantize_mx_op(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, wan
     )
     empty = lambda: torch.empty(0, dtype=torch.uint8, device=dev)  # noqa: E731
     view = lambda t, dt: (empty() if t is None else t).view(dt)  # noqa: E731
-    return view(row_q, out_dtype), view(row_s, _E8M0), view(col_q, out_dtype), view(col_s, _E8M0)
+    scales = lambda t: empty().view(_E8M0) if t is None else t  # noqa: E731
+    return view(row_q, out_dtype), scales(row_s), view(col_q, out_dtype), scales(col_s)
 
 
 @_quantize_mx_op.register_fake
 def _quantize_mx_op_fake(x, out_dtype, want_row, want_col, row_flags, col_flags):
     shapes = _mx_shapes(x, out_dtype, want_row, want_col)
     mk = lambda shp, dt: torch.empty(shp, dtype=torch.uint8, device=x.device).view(dt)  # noqa: E731
-    return mk(shapes[0], out_dtype), mk(shapes[1], _E8M0), mk(shapes[2], out_dtype), mk(shapes[3], _E8M0)
+    lead, M, Nn = tuple(x.shape[:-2]), x.shape[-2], x.shape[-1]
+    Mp, Np = -(-M // _MX_PAD) * _MX_PAD, -(-Nn // _MX_PAD) * _MX_PAD
+    return (mk(shapes[0], out_dtype), _mx_scales(lead, M, Np, row_flags, x.device) if want_row else mk((0,), _E8M0),
+            mk(shapes[2], out_dtype), _mx_scales(lead, Nn, Mp, col_flags, x.device) if want_col else mk((0,), _E8M0))
 
 
 def _quantize_mx_impl(x, out_dtype, axis, block_size, with_trans, scaling_recipe, scaling_recipe_for_trans, what):
@@ -1388,10 +1413,10 @@ def _grouped_quantize_mx_op(
     row_q = row_s = col_q = col_s = None
     if want_row:
         row_q = torch.empty((m_pad_row, n_pad // pack), dtype=torch.uint8, device=dev)
-        row_s = torch.empty((m_pad_row, n_pad // 32), dtype=torch.uint8, device=dev)
+        row_s = _mx_scales((), m_pad_row, n_pad, row_flags, dev)
     if want_col:
         col_q = torch.empty((Nn, m_pad_col // pack), dtype=torch.uint8, device=dev)
-        col_s = torch.empty((Nn, m_pad_col // 32), dtype=torch.uint8, device=dev)
+        col_s = _mx_scales((), Nn, m_pad_col, col_flags, dev)
     N.check(
         N.lib().pt_grouped_quantize_mx(
             N.ptr(x), N.dtype_code(x.dtype), M, Nn, N.dtype_code(out_dtype), N.ptr(group_offs),
@@ -1406,8 +1431,8 @@ def _grouped_quantize_mx_op(
         lens_row, offs_row = empty(torch.int64), empty(torch.int64)
     if known:
         lens_col, offs_col = empty(torch.int64), empty(torch.int64)
-    return (view(row_q, out_dtype), view(row_s, _E8M0), view(col_q, out_dtype), view(col_s, _E8M0),
-            lens_row, offs_row, lens_col, offs_col)
+    scales = lambda t: empty().view(_E8M0) if t is None else t  # noqa: E731
+    return (view(row_q, out_dtype), scales(row_s), view(col_q, out_dtype), scales(col_s), lens_row, offs_row, lens_col, offs_col)
 
 
 @_grouped_quantize_mx_op.register_fake
@@ -1421,9 +1446,9 @@ def _grouped_quantize_mx_op_fake(x, out_dtype, group_lens, group_offs, want_row,
     mk = lambda shp, dt: torch.empty(shp, dtype=torch.uint8, device=x.device).view(dt)  # noqa: E731
     i64 = lambda n: torch.empty(n, dtype=torch.int64, device=x.device)  # noqa: E731
     return (mk((m_pad_row, n_pad // pack) if want_row else (0,), out_dtype),
-            mk((m_pad_row, n_pad // 32) if want_row else (0,), _E8M0),
+            _mx_scales((), m_pad_row, n_pad, row_flags, x.device) if want_row else mk((0,), _E8M0),
             mk((Nn, m_pad_col // pack) if want_col else (0,), out_dtype),
-            mk((Nn, m_pad_col // 32) if want_col else (0,), _E8M0),
+            _mx_scales((), Nn, m_pad_col, col_flags, x.device) if want_col else mk((0,), _E8M0),
             *((i64(0) for _ in range(4)) if known_offs_col is not None else
               (i64(0 if fp4 else G), i64(0 if fp4 else G + 1), i64(G), i64(G + 1))))
 
@@ -1439,8 +1464,9 @@ def glu_grouped_quantize_mx_impl(
     which never travels through HBM here. Outputs as ``primus_turbo::grouped_quantize_mx`` on the
     stored activation with round-to-nearest 1-D blocks, bit for bit: ``(row_q, row_scale, col_q,
     col_scale, lens_row, offs_row, lens_col, offs_col)``, the column pair empty unless ``with_trans``,
-    row lens / offs empty for MXFP4 (its rows stay in place); ``col_flags=2`` transforms the MXFP4
-    column direction (``use_rht``). (No counterpart in the reference.)"""
+    row lens / offs empty for MXFP4 (its rows stay in place); ``col_flags`` bit 1 transforms the MXFP4
+    column direction (``use_rht``), bit 3 stores the scales of both directions word-major (``_mx_scales``). (No
+    counterpart in the reference.)"""
     N.require_cuda(x, probs, row_mask, group_lens, group_offs)
     _check(act in _GLU_ACT, "act must be 'silu' or 'gelu'")
     _check(x.dtype in (torch.bfloat16, torch.float16), "input must be bfloat16 or float16")
@@ -1467,34 +1493,36 @@ def glu_grouped_quantize_mx_impl(
     group_offs = group_offs.contiguous()
     lens_row, offs_row, lens_col, offs_col = _grouped_mx_offs(group_lens, ra, ca, fp4)
     row_q = torch.empty((m_pad_row, n_pad // pack), dtype=torch.uint8, device=dev)
-    row_s = torch.empty((m_pad_row, n_pad // 32), dtype=torch.uint8, device=dev)
+    row_s = _mx_scales((), m_pad_row, n_pad, col_flags, dev)
     col_q = col_s = None
     if with_trans:
         col_q = torch.empty((Nn, m_pad_col // pack), dtype=torch.uint8, device=dev)
-        col_s = torch.empty((Nn, m_pad_col // 32), dtype=torch.uint8, device=dev)
+        col_s = _mx_scales((), Nn, m_pad_col, col_flags, dev)
     N.check(
         N.lib().pt_glu_grouped_quantize_mx(
             N.ptr(x), N.dtype_code(x.dtype), N.ptr(p32), N.ptr(mask), _GLU_ACT[act], M, Nn, N.dtype_code(out_dtype),
             N.ptr(group_offs), None if fp4 else N.ptr(offs_row), N.ptr(offs_col), G, N.ptr(row_q), N.ptr(row_s),
-            N.ptr(col_q), N.ptr(col_s), int(col_flags) if with_trans else 0, m_pad_col, N.stream_of(x),
+            N.ptr(col_q), N.ptr(col_s), int(col_flags) if with_trans else int(col_flags) & _MX_WORDS, m_pad_col,
+            N.stream_of(x),
         )
     )
     empty = lambda dt=torch.uint8: torch.empty(0, dtype=dt, device=dev)  # noqa: E731
     view = lambda t, dt: (empty() if t is None else t).view(dt)  # noqa: E731
     if fp4:
         lens_row, offs_row = empty(torch.int64), empty(torch.int64)
-    return (view(row_q, out_dtype), view(row_s, _E8M0), view(col_q, out_dtype), view(col_s, _E8M0),
+    return (view(row_q, out_dtype), row_s, view(col_q, out_dtype), empty().view(_E8M0) if col_s is None else col_s,
             lens_row, offs_row, lens_col, offs_col)
 
 
 @glu_grouped_quantize_mx_impl.register_fake
 def _glu_grouped_quantize_mx_impl_fake(x, probs, row_mask, act, out_dtype, group_lens, group_offs, with_trans, col_flags=0):
     half = x.new_empty((x.shape[0], x.shape[1] // 2))
-    return _grouped_quantize_mx_op_fake(half, out_dtype, group_lens, group_offs, True, with_trans, 0, 0)
+    words = col_flags & _MX_WORDS
+    return _grouped_quantize_mx_op_fake(half, out_dtype, group_lens, group_offs, True, with_trans, words, words)
 
 
 def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, group_offs, with_trans=False,
-                                scaling_recipe=None, scaling_recipe_for_trans=None, known=None):
+                                scaling_recipe=None, scaling_recipe_for_trans=None):
     """MXFP8 quantization of the packed rows of G groups, each virtually zero-padded along M.
 
     ``with_trans`` -> ``(row_q [M_pad_row, N_pad], row_scale [M_pad_row, N_pad/32], col_q [N, M_pad_col],
@@ -1502,13 +1530,12 @@ def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, grou
     otherwise ``(q, scale, group_lens_padded, group_offs_padded)`` of the direction ``axis`` asks
     for (1 = rows padded to 32 per group, 0 = transposed columns padded to 128 per group).
     ``M_pad_row`` / ``M_pad_col`` = ``total_M + G * align`` rounded up to ``align``; what lies
-    beyond ``offs_padded[G]`` is unspecified. ``known`` (with ``with_trans``): the four lens / offs of an
-    earlier call for the same groups, which are then not computed again."""
+    beyond ``offs_padded[G]`` is unspecified."""
     assert block_size == 32, "The block size must be 32 for MXFP8 quantization"
     r, rt = _mx_recipes(with_trans, scaling_recipe, scaling_recipe_for_trans, "MXFP8")
     if with_trans:
         rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, True,
-                                                                  _mx_flags(r), _mx_flags(rt), known)
+                                                                  _mx_flags(r), _mx_flags(rt))
         rq, rs = _apply_mx_shuffles(rq, rs, r, "rowwise")
         cq, cs = _apply_mx_shuffles(cq, cs, rt, "colwise")
         return rq, rs, cq, cs, lr, orow, lc, ocol
@@ -1520,6 +1547,16 @@ def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, grou
         return rq, rs, lr, orow
     cq, cs = _apply_mx_shuffles(cq, cs, r, "colwise")
     return cq, cs, lc, ocol
+
+
+def grouped_quantize_mx_operands(x, out_dtype, group_lens, group_offs, recipe, recipe_t, what, with_col=True, known=None):
+    """:func:`quantize_mx_operands` for the packed rows of groups: the eight outputs of
+    ``grouped_quantize_mxfp8_impl`` / ``grouped_quantize_mxfp4_impl`` with ``with_trans`` (the column pair None
+    without ``with_col``), scales word-major. ``known``: the last four of an earlier call for the same groups,
+    which are then not computed again."""
+    r, rt = _mx_recipes(True, recipe, recipe_t, what)
+    return _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, with_col, _mx_flags(r) | _MX_WORDS,
+                                _mx_flags(rt) | _MX_WORDS, known)
 
 
 def grouped_dequantize_mxfp8_impl(x, out_dtype, axis, block_size, scale_inv, group_offs, group_offs_padded,
@@ -1541,7 +1578,7 @@ def grouped_dequantize_mxfp8_impl(x, out_dtype, axis, block_size, scale_inv, gro
 
 
 def grouped_quantize_mxfp4_impl(x, out_dtype, axis, block_size, group_lens, group_offs, with_trans=False,
-                                scaling_recipe=None, scaling_recipe_for_trans=None, known=None):
+                                scaling_recipe=None, scaling_recipe_for_trans=None):
     """MXFP4 quantization of the packed rows of G groups (reference: quantization_impl.py:657-811,
     layout of its default dispatch flydsl/quantization/mxfp4_grouped_quant.py:320-349).
 
@@ -1554,14 +1591,13 @@ def grouped_quantize_mxfp4_impl(x, out_dtype, axis, block_size, group_lens, grou
     16-point Hadamard transform along that direction (within each group's padded rows for the
     column direction), ``use_sr`` rounds the codes stochastically, ``use_2d_block`` shares one
     exponent per 32 x 32 block counted from the group's first row, ``shuffle_out`` /
-    ``shuffle_scale`` give the pre-shuffled forms of the outputs (a pass over the plain ones).
-    ``known`` as in :func:`grouped_quantize_mxfp8_impl`."""
+    ``shuffle_scale`` give the pre-shuffled forms of the outputs (a pass over the plain ones)."""
     assert block_size == 32, "The block size must be 32 for MXFP4 quantization"
     assert _FP4X2 is not None and out_dtype == _FP4X2, "The out_dtype must be float4_e2m1fn_x2 for MXFP4 quantization"
     r, rt = _mx_recipes(with_trans, scaling_recipe, scaling_recipe_for_trans, "MXFP4")
     if with_trans:
         rq, rs, cq, cs, lr, orow, lc, ocol = _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, True,
-                                                                  _mx_flags(r), _mx_flags(rt), known)
+                                                                  _mx_flags(r), _mx_flags(rt))
         rq, rs = _apply_mx_shuffles(rq, rs, r, "rowwise")
         cq, cs = _apply_mx_shuffles(cq, cs, rt, "colwise")
         return rq, rs, cq, cs, lr, orow, lc, ocol

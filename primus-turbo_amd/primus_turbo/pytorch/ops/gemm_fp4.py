@@ -32,8 +32,11 @@ from primus_turbo.pytorch.core.quantized_tensor import (
     check_quantized_tensor,
 )
 from primus_turbo.pytorch.kernels.gemm.gemm_fp4_impl import gemm_fp4_accum_impl, gemm_fp4_impl
-from primus_turbo.pytorch.kernels.quantization.quantization_impl import mx_plain_layout, quantize_mxfp4_impl
-from primus_turbo.pytorch.ops.quantization import quantize_fp4_with_trans
+from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
+    mx_plain_layout,
+    quantize_mx_operands,
+    quantize_mxfp4_impl,
+)
 from primus_turbo.pytorch.ops.utils import _get_dummy_wgrad, _setup_fused_grad_accum
 
 __all__ = ["gemm_fp4"]
@@ -90,8 +93,8 @@ class FP4GemmMXFunction(torch.autograd.Function):
                 # the transposed copies only feed backward: skip them when nothing asks for a gradient
                 q, sc = quantize_mxfp4_impl(x, dt, x.dim() - 1, bs, scaling_recipe=recipe)
                 return q, sc, None, None
-            return quantize_fp4_with_trans(x, dt, gran, block_size=bs, scaling_recipe=recipe,
-                                           scaling_recipe_for_trans=recipe_t)
+            assert bs == 32, "The block size must be 32 for MXFP4 quantization"
+            return quantize_mx_operands(x, dt, recipe, recipe_t, "MXFP4")
 
         # reference lines 112-160: the second operand of each product is the one held pre-shuffled
         w_recipe = ScalingRecipe(use_2d_block=True, shuffle_scale=pre, shuffle_out=pre)
@@ -111,10 +114,9 @@ class FP4GemmMXFunction(torch.autograd.Function):
         dt = FP4GemmMXFunction.get_fp4_dtype(config.format)
         gran = config.granularity
         g = grad_out.reshape(grad_out.shape[0], -1).contiguous()
-        g_row, g_row_s, g_col, g_col_s = quantize_fp4_with_trans(
-            g, dt, gran, block_size=config.block_size, scaling_recipe=ScalingRecipe(use_sr=config.use_gradient_sr),
-            scaling_recipe_for_trans=ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True),  # pairs with a_col
-        )
+        g_row, g_row_s, g_col, g_col_s = quantize_mx_operands(
+            g, dt, ScalingRecipe(use_sr=config.use_gradient_sr),
+            ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), "MXFP4")  # pairs with a_col
         # both directions are stored transposed, so dgrad and wgrad are NT products as well
         grad_a = gemm_fp4_impl(g_row, g_row_s, False, b_col, b_col_s, True, out_dtype, False, gran.value, _NATIVE)
         grad_b = _bgrad_gemm_fp4_impl_wrapper(g_col, g_col_s, False, a_col, a_col_s, True, out_dtype, False, gran.value,

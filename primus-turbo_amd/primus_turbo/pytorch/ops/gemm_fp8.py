@@ -39,6 +39,7 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_kmajor_impl,
     quant_fp8_blockwise_for_weight_dual_impl,
     quant_fp8_rowwise_t_impl,
+    quantize_mx_operands,
 )
 from primus_turbo.pytorch.ops.quantization import dequantize_fp8, quantize_fp8, quantize_fp8_with_trans
 from primus_turbo.pytorch.ops.utils import _get_dummy_wgrad, _get_fp8_dtype, _setup_fused_grad_accum
@@ -267,8 +268,8 @@ class FP8GemmMXFunction(torch.autograd.Function):
                 # the transposed copies only feed backward: skip them when nothing asks for a gradient
                 q, sc = quantize_mxfp8_impl(x, fdt, x.dim() - 1, bs, scaling_recipe=recipe)
                 return q, sc, None, None
-            return quantize_mxfp8_impl(x, fdt, None, bs, with_trans=True, scaling_recipe=recipe,
-                                       scaling_recipe_for_trans=recipe)
+            assert bs == 32, "The block size must be 32 for MXFP8 quantization"
+            return quantize_mx_operands(x, fdt, recipe, recipe, "MXFP8")
 
         a_row, a_row_s, a_col, a_col_s = both_ways(a, a_t, ScalingRecipe())
         b_row, b_row_s, b_col, b_col_s = both_ways(b, b_t, ScalingRecipe(use_2d_block=True))
@@ -280,16 +281,12 @@ class FP8GemmMXFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        from primus_turbo.pytorch.kernels.quantization.quantization_impl import quantize_mxfp8_impl
-
         out_dtype, config, fuse, main_grad = ctx.meta
         a_col, a_col_s, b_col, b_col_s = ctx.saved_tensors
         gran = config.granularity
         g = grad_out.reshape(grad_out.shape[0], -1).contiguous()
-        g_row, g_row_s, g_col, g_col_s = quantize_mxfp8_impl(
-            g, _get_fp8_dtype(config.format, False), None, config.block_size, with_trans=True,
-            scaling_recipe=ScalingRecipe(), scaling_recipe_for_trans=ScalingRecipe(),
-        )
+        g_row, g_row_s, g_col, g_col_s = quantize_mx_operands(g, _get_fp8_dtype(config.format, False), ScalingRecipe(),
+                                                              ScalingRecipe(), "MXFP8")
         # the two-direction casts are stored transposed, so dgrad and wgrad are NT GEMMs too
         grad_a = _gemm(g_row, g_row_s, False, b_col, b_col_s, True, out_dtype, False, gran)
         grad_b = _wgrad_gemm(g_col, g_col_s, False, a_col, a_col_s, True, out_dtype, False, gran,

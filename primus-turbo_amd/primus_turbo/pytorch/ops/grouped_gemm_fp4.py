@@ -40,14 +40,11 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp4_impl import (
 )
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
+    _MX_WORDS,
     glu_grouped_quantize_mx_impl,
-    grouped_quantize_mxfp4_impl,
+    grouped_quantize_mx_operands,
+    quantize_mx_operands,
     quantize_mxfp4_impl,
-)
-from primus_turbo.pytorch.ops.quantization import (
-    grouped_quantize_fp4,
-    grouped_quantize_fp4_with_trans,
-    quantize_fp4_with_trans,
 )
 from primus_turbo.pytorch.ops.utils import (
     _ensure_contiguous_grad_out,
@@ -91,9 +88,8 @@ def _fp4_weight_operands(b, b_t, config, need_bwd):
             assert isinstance(b_t, QuantizedTensor)
             b_col, b_col_s = b_t.qdata, b_t.scale_inv
     elif need_bwd:
-        b_row, b_row_s, b_col, b_col_s = quantize_fp4_with_trans(
-            b.contiguous(), float4_e2m1fn_x2, gran, block_size=bs, scaling_recipe=w_recipe,
-            scaling_recipe_for_trans=w_recipe)
+        assert bs == 32, "The block size must be 32 for MXFP4 quantization"
+        b_row, b_row_s, b_col, b_col_s = quantize_mx_operands(b.contiguous(), float4_e2m1fn_x2, w_recipe, w_recipe, "MXFP4")
     else:
         b_row, b_row_s = quantize_mxfp4_impl(b.contiguous(), float4_e2m1fn_x2, 2, bs, scaling_recipe=w_recipe)
     return b_row, b_row_s, b_col, b_col_s
@@ -105,9 +101,9 @@ def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens,
     offsets are the forward quantizer's (None: the caller quantized the activation)."""
     gran = config.granularity
     known = None if offs_col is None else (None, None, lens_col, offs_col)
-    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mxfp4_impl(
-        grad_out, float4_e2m1fn_x2, None, config.block_size, group_lens, group_offs, True,
-        ScalingRecipe(use_sr=config.use_gradient_sr), ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), known)
+    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
+        grad_out, float4_e2m1fn_x2, group_lens, group_offs, ScalingRecipe(use_sr=config.use_gradient_sr),
+        ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), "MXFP4", known=known)
     # dgrad: grad_a = grad_out @ b as an NT product with the transposed weight quantization [G, K, N]
     grad_a = grouped_gemm_fp4_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
                                    gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
@@ -155,13 +151,13 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
                 check_quantized_tensor(a_t, config, scaling_recipe=a_t_recipe)
                 a_col, a_col_s = a_t.qdata, a_t.scale_inv
         elif need_bwd:
-            a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_fp4_with_trans(
-                a.contiguous(), float4_e2m1fn_x2, gran, group_lens, group_offs, block_size=bs,
-                scaling_recipe=a_recipe, scaling_recipe_for_trans=a_t_recipe)
+            assert bs == 32, "The block size must be 32 for MXFP4 quantization"
+            a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
+                a.contiguous(), float4_e2m1fn_x2, group_lens, group_offs, a_recipe, a_t_recipe, "MXFP4")
         else:
-            a_row, a_row_s, _, offs_row = grouped_quantize_fp4(
-                a.contiguous(), float4_e2m1fn_x2, gran, group_lens, group_offs, block_size=bs, axis=1)
-            a_col = a_col_s = None
+            assert bs == 32, "The block size must be 32 for MXFP4 quantization"
+            a_row, a_row_s, a_col, a_col_s, _, offs_row, _, _ = grouped_quantize_mx_operands(
+                a.contiguous(), float4_e2m1fn_x2, group_lens, group_offs, a_recipe, a_t_recipe, "MXFP4", with_col=False)
 
         b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, b_t, config, need_bwd)
 
@@ -206,7 +202,7 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
         need_bwd = any(ctx.needs_input_grad[i] for i in (0, 1, 4))
         x2, p1 = x.contiguous(), probs.reshape(-1).contiguous()
         a_row, a_row_s, a_col, a_col_s, _, _, lens_col, offs_col = glu_grouped_quantize_mx_impl(
-            x2, p1, row_mask, act_type, float4_e2m1fn_x2, group_lens, group_offs, need_bwd, 2)
+            x2, p1, row_mask, act_type, float4_e2m1fn_x2, group_lens, group_offs, need_bwd, 2 | _MX_WORDS)
         b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, None, config, need_bwd)
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, group_offs, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]

@@ -40,13 +40,15 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import (
 )
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
+    _MX_WORDS,
     glu_grouped_quantize_mx_impl,
     glu_quant_fp8_blockwise_segment_m_row_col_impl,
-    grouped_quantize_mxfp8_impl,
+    grouped_quantize_mx_operands,
     quant_fp8_blockwise_for_weight_dual_impl,
     quant_fp8_blockwise_for_weight_impl,
     quant_fp8_blockwise_kmajor_impl,
     quant_fp8_blockwise_segment_m_row_col_t_impl,
+    quantize_mx_operands,
     quantize_mxfp8_impl,
 )
 from primus_turbo.pytorch.ops.quantization import dequantize_fp8, quantize_fp8
@@ -330,8 +332,8 @@ def _mx_weight_operands(b, b_t, config, need_bwd):
             assert isinstance(b_t, QuantizedTensor)
             b_col, b_col_s = b_t.qdata, b_t.scale_inv
     elif need_bwd:
-        b_row, b_row_s, b_col, b_col_s = quantize_mxfp8_impl(
-            b.contiguous(), fdt, None, bs, with_trans=True, scaling_recipe=w_recipe, scaling_recipe_for_trans=w_recipe)
+        assert bs == 32, "The block size must be 32 for MXFP8 quantization"
+        b_row, b_row_s, b_col, b_col_s = quantize_mx_operands(b.contiguous(), fdt, w_recipe, w_recipe, "MXFP8")
     else:
         b_row, b_row_s = quantize_mxfp8_impl(b.contiguous(), fdt, 2, bs, scaling_recipe=w_recipe)
     return b_row, b_row_s, b_col, b_col_s
@@ -344,8 +346,8 @@ def _mx_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, 
     gdt = _get_fp8_dtype(config.format, False)
     gran = config.granularity.value
     known = None if offs_col is None else (None, offs_row, lens_col, offs_col)
-    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mxfp8_impl(
-        grad_out, gdt, None, config.block_size, group_lens, group_offs, with_trans=True, known=known)
+    g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
+        grad_out, gdt, group_lens, group_offs, None, None, "MXFP8", known=known)
     # dgrad: grad_a = grad_out @ b, as an NT product with the transposed weight quantization [G, K, N]
     grad_a = grouped_gemm_fp8_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
                                    gran, num_cu, _NATIVE, False, group_offs)[:total_m]
@@ -386,10 +388,13 @@ class FP8GroupedGemmMXFunc(torch.autograd.Function):
                 assert isinstance(a_t, QuantizedTensor)
                 a_col, a_col_s = a_t.qdata, a_t.scale_inv
         elif need_bwd:
-            a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mxfp8_impl(
-                a.contiguous(), fdt, None, bs, group_lens, group_offs, with_trans=True)
+            assert bs == 32, "The block size must be 32 for MXFP8 quantization"
+            a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
+                a.contiguous(), fdt, group_lens, group_offs, None, None, "MXFP8")
         else:
-            a_row, a_row_s, _, offs_row = grouped_quantize_mxfp8_impl(a.contiguous(), fdt, 1, bs, group_lens, group_offs)
+            assert bs == 32, "The block size must be 32 for MXFP8 quantization"
+            a_row, a_row_s, _, _, _, offs_row, _, _ = grouped_quantize_mx_operands(
+                a.contiguous(), fdt, group_lens, group_offs, None, None, "MXFP8", with_col=False)
         b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, b_t, config, need_bwd)
         # the padded row layout is read through offs_row, the result is packed by group_offs
         # into an output over-allocated to the padded rows
@@ -427,7 +432,7 @@ class FP8GluGroupedGemmMXFunc(torch.autograd.Function):
         need_bwd = any(ctx.needs_input_grad[i] for i in (0, 1, 4))
         x2, p1 = x.contiguous(), probs.reshape(-1).contiguous()
         a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = glu_grouped_quantize_mx_impl(
-            x2, p1, row_mask, act_type, _get_fp8_dtype(config.format, True), group_lens, group_offs, need_bwd)
+            x2, p1, row_mask, act_type, _get_fp8_dtype(config.format, True), group_lens, group_offs, need_bwd, _MX_WORDS)
         b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, None, config, need_bwd)
         out = grouped_gemm_fp8_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]
