@@ -128,6 +128,14 @@ PT_API int pt_quantize_fp8_tensorwise_static(const void *x, int x_dtype, int64_t
                                              int q_dtype, const float *scale_in, float *scale_inv,
                                              int32_t *status, void *stream);
 
+/* pt_quantize_fp8_tensorwise of a matrix x [R, C] (both multiples of 16) with the codes emitted transposed as
+ * well, q_t [C, R]: both from one read, same bytes as the cast followed by pt_transpose_u8 (the reference keeps
+ * the two steps, ops/gemm_fp8.py:96-276). workspace as for pt_quantize_fp8_tensorwise, or NULL: the static
+ * scratch of pt_quantize_fp8_tensorwise_static, with its conditions. */
+PT_API int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t C, void *q, void *q_t,
+                                        int q_dtype, float *scale_inv, void *workspace,
+                                        size_t workspace_bytes, void *stream);
+
 /* Gives the slot set that pt_quantize_fp8_tensorwise_static keeps for `stream` on the current
  * device back, so that another stream handle can take it (a process that cycles through
  * stream handles would otherwise run out of the PT_TENSORWISE_STATIC_MAX_STREAMS sets). Every

@@ -132,6 +132,41 @@ _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise, "CUDA")
 _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise, "CPU")  # raises: no CPU path
 _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise_meta, "Meta")
 
+
+@native_op("primus_turbo::quantize_fp8_tensorwise_t")
+def quantize_fp8_tensorwise_t_impl(x: torch.Tensor, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """TENSORWISE quantization of a contiguous matrix ``x [R, C]`` with the codes emitted transposed as well,
+    ``(x_fp8 [R, C], x_fp8_t [C, R], scale_inv)``, same bytes as the cast followed by a transposition. One launch
+    where the plain cast is one (eager calls in the fused mode) and both sizes are multiples of 16; else those two
+    steps. (No counterpart in the reference, which runs them.)"""
+    _check(x.dim() == 2 and x.is_contiguous(), "input must be a contiguous matrix")
+    R, C = x.shape
+    one_launch = (
+        R % 16 == 0 and C % 16 == 0 and x.numel() > 0 and x.dtype in _HP_DTYPES and x.is_cuda and x.data_ptr() % 16 == 0
+        and _tensorwise_mode != "two_pass" and not torch.cuda.is_current_stream_capturing())
+    if one_launch:
+        _check_fp8_out(dtype)
+        q = torch.empty_like(x, dtype=dtype)
+        q_t = torch.empty((C, R), dtype=dtype, device=x.device)
+        scale_inv = torch.empty((), dtype=torch.float32, device=x.device)
+        status = N.lib().pt_quantize_fp8_tensorwise_t(
+            N.ptr(x), N.dtype_code(x.dtype), R, C, N.ptr(q), N.ptr(q_t), N.dtype_code(dtype), N.ptr(scale_inv), None, 0,
+            N.stream_of(x))
+        if status != N.PT_ERR_WORKSPACE:  # (more stream handles than the static scratch has slot sets for)
+            N.check(status)
+            return q, q_t, scale_inv
+    q, scale_inv = _quantize_fp8_tensorwise(x, dtype)
+    q_t = torch.empty((C, R), dtype=dtype, device=x.device)
+    N.check(N.lib().pt_transpose_u8(N.ptr(q), N.ptr(q_t), 1, R, C, N.stream_of(q)))
+    return q, q_t, scale_inv
+
+
+@quantize_fp8_tensorwise_t_impl.register_fake
+def _quantize_fp8_tensorwise_t_impl_fake(x, dtype):
+    return (torch.empty_like(x, dtype=dtype), torch.empty((x.shape[1], x.shape[0]), dtype=dtype, device=x.device),
+            torch.empty((), dtype=torch.float32, device=x.device))
+
+
 # ---------------------------------------------------------------------------
 # dequantize_fp8_tensorwise(Tensor input, Tensor scale_inv, ScalarType dest_dtype) -> Tensor
 # ---------------------------------------------------------------------------

@@ -39,6 +39,7 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_kmajor_impl,
     quant_fp8_blockwise_for_weight_dual_impl,
     quant_fp8_rowwise_t_impl,
+    quantize_fp8_tensorwise_t_impl,
     quantize_mx_operands,
 )
 from primus_turbo.pytorch.ops.quantization import dequantize_fp8, quantize_fp8, quantize_fp8_with_trans
@@ -80,19 +81,29 @@ class FP8GemmTensorFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum_pattern=None):
         fuse, main_grad = _setup_fused_grad_accum(b, fuse_bgrad_accum_pattern)
-        qa, qa_s, _ = _quantized_parts(a, config, True, -1)
-        qb, qb_s, _ = _quantized_parts(b, config, True, -1)
-        out = _gemm(qa, qa_s, trans_a, qb, qb_s, trans_b, out_dtype, False, config.granularity)
         # NT forward: keep physically transposed fp8 copies so that both backward GEMMs
         # are NT as well (contiguous-K operands need no transposition pass inside the GEMM);
-        # they only feed backward: skipped when nothing asks for a gradient
+        # they only feed backward: skipped when nothing asks for a gradient. A tensorwise transpose
+        # shares the scalar scale; the cast of a plain operand emits it from the same read
         nt_bwd = (not trans_a) and trans_b
-        if not any(ctx.needs_input_grad[:2]):
+        need_bwd = any(ctx.needs_input_grad[:2])
+
+        def operand(x, x_t):
+            want_t = need_bwd and nt_bwd and not isinstance(x_t, QuantizedTensor)
+            if want_t and not isinstance(x, QuantizedTensor):
+                q, q_t, q_s = quantize_fp8_tensorwise_t_impl(x.contiguous(), _get_fp8_dtype(config.format, True))
+                return q, q_s, q_t, q_s
+            q, q_s, _ = _quantized_parts(x, config, True, -1)
+            if want_t:
+                return q, q_s, transpose_last_two(q), q_s
+            return (q, q_s, x_t.qdata, x_t.scale_inv) if isinstance(x_t, QuantizedTensor) else (q, q_s, None, None)
+
+        qa, qa_s, sa, sa_s = operand(a, a_t)
+        qb, qb_s, sb, sb_s = operand(b, b_t)
+        out = _gemm(qa, qa_s, trans_a, qb, qb_s, trans_b, out_dtype, False, config.granularity)
+        if not need_bwd:
             pass
         elif nt_bwd:
-            # a tensorwise transpose moves the codes and shares the scalar scale
-            sa, sa_s = (a_t.qdata, a_t.scale_inv) if isinstance(a_t, QuantizedTensor) else (transpose_last_two(qa), qa_s)
-            sb, sb_s = (b_t.qdata, b_t.scale_inv) if isinstance(b_t, QuantizedTensor) else (transpose_last_two(qb), qb_s)
             ctx.save_for_backward(sa, sa_s, sb, sb_s)
         else:
             ctx.save_for_backward(qa, qa_s, qb, qb_s)
@@ -104,13 +115,15 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         trans_a, trans_b, out_dtype, config, nt_bwd, fuse, main_grad = ctx.meta
         sa, sa_s, sb, sb_s = ctx.saved_tensors
         gran = config.granularity
-        g, g_s = quantize_fp8(grad_out.contiguous(), _get_fp8_dtype(config.format, False), gran)
+        gdt = _get_fp8_dtype(config.format, False)
         acc = main_grad if fuse else None
         if nt_bwd:
             # saved: A^T [K, M], B^T [K, N]
+            g, g_t, g_s = quantize_fp8_tensorwise_t_impl(grad_out.contiguous(), gdt)
             grad_a = _gemm(g, g_s, False, sb, sb_s, True, out_dtype, False, gran)
-            grad_b = _wgrad_gemm(sa, sa_s, False, transpose_last_two(g), g_s, True, out_dtype, trans_b, gran, acc)
+            grad_b = _wgrad_gemm(sa, sa_s, False, g_t, g_s, True, out_dtype, trans_b, gran, acc)
         else:
+            g, g_s = quantize_fp8(grad_out.contiguous(), gdt, gran)
             grad_a = _gemm(g, g_s, False, sb, sb_s, not trans_b, out_dtype, trans_a, gran)
             grad_b = _wgrad_gemm(sa, sa_s, not trans_a, g, g_s, False, out_dtype, trans_b, gran, acc)
         return grad_a, grad_b, None, None, None, None, None, None, None

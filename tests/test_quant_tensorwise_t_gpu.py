@@ -1,0 +1,36 @@
+"""The tensorwise cast that emits the codes transposed as well: the same bytes as the cast and a transposition, at
+the edges of its 128 x 128 tiles, beyond what its registers hold, and where it takes the two steps."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,C", [(16, 16), (16, 2048), (128, 128), (144, 272), (1040, 112), (4096, 4096), (8208, 4112), (40, 64), (64, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_same_bytes_as_two_steps(native_lib, R, C, dtype, fp8):
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as impl
+
+    x = torch.randn(R, C, generator=torch.Generator(device="cuda").manual_seed(R + C), device="cuda", dtype=dtype)
+    x[R // 2, C // 3] = 37.0  # the maximum, in one place
+    q, scale_inv = impl._quantize_fp8_tensorwise(x, fp8)
+    for mode in ("auto", "two_pass"):
+        before = impl.set_tensorwise_mode(mode)
+        try:
+            got, got_t, got_scale = impl.quantize_fp8_tensorwise_t_impl(x, fp8)
+        finally:
+            impl.set_tensorwise_mode(before)
+        assert torch.equal(got_scale, scale_inv)
+        assert torch.equal(got.view(torch.uint8), q.view(torch.uint8))
+        assert torch.equal(got_t.view(torch.uint8), q.view(torch.uint8).t())
+
+
+def test_one_launch_needs_an_aligned_tensor(native_lib):
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as impl
+
+    x = torch.randn(64 * 64 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(64, 64)
+    q, q_t, _ = impl.quantize_fp8_tensorwise_t_impl(x, torch.float8_e4m3fn)
+    assert torch.equal(q.view(torch.uint8), impl._quantize_fp8_tensorwise(x, torch.float8_e4m3fn)[0].view(torch.uint8))
+    assert torch.equal(q_t.view(torch.uint8), q.view(torch.uint8).t())
