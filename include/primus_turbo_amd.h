@@ -128,12 +128,13 @@ PT_API int pt_quantize_fp8_tensorwise_static(const void *x, int x_dtype, int64_t
                                              int q_dtype, const float *scale_in, float *scale_inv,
                                              int32_t *status, void *stream);
 
-/* pt_quantize_fp8_tensorwise of a matrix x [R, C] (both multiples of 16) with the codes emitted transposed as
- * well, q_t [C, R]: both from one read, same bytes as the cast followed by pt_transpose_u8 (the reference keeps
- * the two steps, ops/gemm_fp8.py:96-276). workspace as for pt_quantize_fp8_tensorwise, or NULL: the static
+/* pt_quantize_fp8_tensorwise of a matrix x [R, C] (C a multiple of 16) with the codes emitted transposed as
+ * well: q [R, ldq] and q_t [C, ldt] from one read, the bytes of the cast followed by pt_transpose_u8 and zeros
+ * behind the end of a row; pitches are multiples of 16 that pad to the next multiple of 128 at most (the
+ * reference keeps the two steps, ops/gemm_fp8.py:96-276). workspace as for pt_quantize_fp8_tensorwise, or NULL: the static
  * scratch of pt_quantize_fp8_tensorwise_static, with its conditions. */
-PT_API int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t C, void *q, void *q_t,
-                                        int q_dtype, float *scale_inv, void *workspace,
+PT_API int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t C, void *q, int64_t ldq,
+                                        void *q_t, int64_t ldt, int q_dtype, float *scale_inv, void *workspace,
                                         size_t workspace_bytes, void *stream);
 
 /* Gives the slot set that pt_quantize_fp8_tensorwise_static keeps for `stream` on the current
@@ -196,6 +197,15 @@ PT_API size_t pt_quantize_fp8_rowwise_outer_workspace_bytes(int64_t B, int64_t M
 PT_API int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_scale_inv, int hp_dtype, int64_t B,
                                          int64_t M, int64_t N, void *q, void *q_t, int64_t ld_t, int q_dtype,
                                          float *scale_inv, void *workspace, size_t workspace_bytes, void *stream);
+/* The same for FP8 codes in rows of ld_x >= N bytes. */
+PT_API int pt_quantize_fp8_rowwise_outer_ld(const void *x, int64_t ld_x, int x_dtype, const float *row_scale_inv,
+                                            int hp_dtype, int64_t B, int64_t M, int64_t N, void *q, void *q_t,
+                                            int64_t ld_t, int q_dtype, float *scale_inv, void *workspace,
+                                            size_t workspace_bytes, void *stream);
+/* pt_quantize_fp8_rowwise of the rows of x [rows, cols] with codes in rows of ldq >= cols bytes, zeros behind cols:
+ * the form a product reads without a padding copy when cols is no multiple of 128. */
+PT_API int pt_quantize_fp8_rowwise_padded(const void *x, int x_dtype, int64_t rows, int64_t cols, void *q, int64_t ldq,
+                                          int q_dtype, float *scale_inv, void *stream);
 
 /* FP8 128-blockwise (fp32 scales, eps 1e-4) -----------------------------------
  *

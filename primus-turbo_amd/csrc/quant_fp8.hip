@@ -322,8 +322,9 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_kernel(
     }
 }
 
-// The same with the codes of x [R, C] emitted transposed as well, q_t [C, R]: the operand of the product that
-// reduces over the rows. Bound by memory traffic and the grid exchange, like the plain form; the transposition
+// The same with the codes of x [R, C] emitted transposed as well, q_t [C, ldt]: the operand of the product that
+// reduces over the rows. Either output's rows may be longer than the matrix is wide (ldq, ldt): the codes behind
+// the end are zero, which is the form the products read without a padding copy. Bound by memory traffic and the grid exchange, like the plain form; the transposition
 // passes through the LDS while the row codes leave, where a launch of its own read and wrote every code once
 // more (4096 x 4096 bf16 within a training step: 14.1 + 6.7 us in two launches, 17.3 in this one).
 //
@@ -331,11 +332,13 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_kernel(
 // of row t / 8 of each, so a tile is read and its codes leave in whole 256- and 128-byte rows. The codes of a
 // tile lie in the LDS as 128 rows of 32 words, word w of row r at w ^ 8 ((r / 16) % 4): the eight 16-row chunks
 // that a wavefront collects for an output row then come from different banks, without padding that would not
-// leave room for four tiles. R and C are multiples of 16 (the host checks): every 16-byte group is in or out.
+// leave room for four tiles. C and both pitches are multiples of 16 (the host checks): every 16-byte group is in
+// or out.
 template <typename T, bool E5M2>
 __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
                                                                         uint8_t *__restrict__ q_t, const int64_t R,
-                                                                        const int64_t C, float *__restrict__ scale_inv_out,
+                                                                        const int64_t C, const int64_t ldq, const int64_t ldt,
+                                                                        float *__restrict__ scale_inv_out,
                                                                         const GridWait gw, const float qmax) {
     constexpr int       TILES = 4, TILE = 128, WORDS = TILE / 4;
     __shared__ uint32_t codes[TILES][TILE * WORDS] __attribute__((aligned(16)));
@@ -343,19 +346,19 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T 
     __shared__ uint32_t s_tag[3];
     const uint32_t      gen  = grid_generation(gw);
     const int           row  = threadIdx.x >> 3, chunk = threadIdx.x & 7;
-    const int64_t       across = (C + TILE - 1) / TILE, total = (R + TILE - 1) / TILE * across;
+    const int64_t       across = (ldq + TILE - 1) / TILE, total = (R + TILE - 1) / TILE * across;
     const int64_t       step = static_cast<int64_t>(gridDim.x);
 
-    // offset of this thread's unit of a tile, -1 outside the matrix
-    auto unit_of = [&](const int64_t tile) -> int64_t {
+    // offset of this thread's unit of a tile in rows of `ld`, -1 outside the `width` columns
+    auto unit_of = [&](const int64_t tile, const int64_t width, const int64_t ld) -> int64_t {
         const int64_t tr = tile / across, r = tr * TILE + row, c = (tile - tr * across) * TILE + chunk * 16;
-        return tile < total && r < R && c < C ? r * C + c : -1;
+        return tile < total && r < R && c < width ? r * ld + c : -1;
     };
     Unit16<T> held[TILES];
     auto load = [&](const int64_t first) {
 #pragma unroll
         for (int k = 0; k < TILES; ++k) {
-            const int64_t u = unit_of(first + k * step);
+            const int64_t u = unit_of(first + k * step, C, C);
             if (u >= 0)
                 held[k].load(x + u);
             else
@@ -368,7 +371,7 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T 
     for (int k = 0; k < TILES; ++k)
         amax = fmaxf(amax, held[k].amax());
     for (int64_t tile = blockIdx.x + TILES * step; tile < total; tile += step) {
-        const int64_t u = unit_of(tile);
+        const int64_t u = unit_of(tile, C, C);
         if (u >= 0) {
             Unit16<T> t;
             t.load(x + u);
@@ -389,7 +392,7 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T 
 #pragma unroll
         for (int k = 0; k < TILES; ++k) {
             const u32x4   c = held[k].template quant<E5M2>(scale, qmax);
-            const int64_t u = unit_of(first + k * step);
+            const int64_t u = unit_of(first + k * step, ldq, ldq);
             if (u >= 0)
                 st128_nt(q + u, c);
             *reinterpret_cast<u32x4 *>(&codes[k][row * WORDS + ((chunk * 4) ^ (((row >> 4) & 3) * 8))]) = c;
@@ -400,7 +403,7 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T 
         const int     k = threadIdx.x >> 8, j = threadIdx.x & 7, w = (threadIdx.x & 255) >> 3;
         const int64_t tile = first + k * step, tr = tile / across;
         const int64_t r0 = tr * TILE + j * 16, c0 = (tile - tr * across) * TILE + w * 4;
-        if (tile < total && r0 < R && c0 < C) {
+        if (tile < total && r0 < ldt && c0 < C) {
             u32x4 out[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -417,21 +420,22 @@ __global__ __launch_bounds__(TW_THREADS) void quant_tensorwise_t_kernel(const T 
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                st128(q_t + (c0 + e) * R + r0, out[e]);
+                st128(q_t + (c0 + e) * ldt + r0, out[e]);
         }
     }
 }
 
 template <typename T, bool E5M2>
-static int launch_quant_tensorwise_t(const void *x, int64_t R, int64_t C, void *q, void *q_t, float *scale_inv, uint64_t *ws,
-                                     hipStream_t stream) {
-    const int64_t tiles = cdiv(R, 128) * cdiv(C, 128);
+static int launch_quant_tensorwise_t(const void *x, int64_t R, int64_t C, void *q, int64_t ldq, void *q_t, int64_t ldt,
+                                     float *scale_inv, uint64_t *ws, hipStream_t stream) {
+    const int64_t tiles = cdiv(R, 128) * cdiv(ldq, 128);
     int64_t       grid  = device_cu_count(); // (one workgroup per CU, resident at the exchange, as the plain form)
     grid                = grid > WS_MAX_BLOCKS ? WS_MAX_BLOCKS : grid;
     grid                = grid > tiles ? tiles : grid;
     const GridWait gw{ws, nullptr, GRID_WAIT_MAX_PROBES, static_cast<uint32_t>(grid)};
     quant_tensorwise_t_kernel<T, E5M2><<<static_cast<unsigned>(grid), TW_THREADS, 0, stream>>>(
-        static_cast<const T *>(x), static_cast<uint8_t *>(q), static_cast<uint8_t *>(q_t), R, C, scale_inv, gw, E5M2 ? 57344.0f : 448.0f);
+        static_cast<const T *>(x), static_cast<uint8_t *>(q), static_cast<uint8_t *>(q_t), R, C, ldq, ldt, scale_inv, gw,
+        E5M2 ? 57344.0f : 448.0f);
     return check_launch("quant_tensorwise_t_kernel");
 }
 
@@ -738,13 +742,15 @@ template <typename T> struct Vec8 {
 
 template <typename T, bool E5M2, bool VEC8, bool DYNAMIC, int HOLD>
 __global__ __launch_bounds__(RW_THREADS) void quant_rowwise_inner_kernel(
-    const T *__restrict__ x, uint8_t *__restrict__ q, const int64_t inner,
+    const T *__restrict__ x, uint8_t *__restrict__ q, const int64_t inner, const int64_t ldq,
     const float *__restrict__ scale_in, float *__restrict__ scale_inv_out, const float qmax) {
     __shared__ float s_red[RW_THREADS / 64];
     const int64_t    row = blockIdx.x;
     const T         *xr  = x + row * inner;
-    uint8_t         *qr  = q + row * inner;
+    uint8_t         *qr  = q + row * ldq;
     float            scale;
+    for (int64_t i = inner + threadIdx.x; i < ldq; i += RW_THREADS) // (zero codes behind the row)
+        qr[i] = 0;
     if constexpr (VEC8) {
         const int64_t units = inner / 8; // inner % 8 == 0 on this path
         Vec8<T>       held[HOLD];
@@ -811,7 +817,7 @@ int launch_quant_rowwise_outer(const void *x, int x_dtype, int64_t B, int64_t M,
                                const float *scale_in, float *scale_inv, float *ws, hipStream_t st);
 
 template <typename T, bool E5M2>
-static int launch_quant_rowwise(const void *x, int64_t B, int64_t M, int64_t N, void *q,
+static int launch_quant_rowwise(const void *x, int64_t B, int64_t M, int64_t N, void *q, int64_t ldq,
                                 const float *scale_in, float *scale_inv, hipStream_t stream) {
     const float qmax = E5M2 ? 57344.0f : 448.0f;
     const T    *xp   = static_cast<const T *>(x);
@@ -819,24 +825,24 @@ static int launch_quant_rowwise(const void *x, int64_t B, int64_t M, int64_t N, 
     if (B * M * N == 0)
         return PT_OK;
     if (N == 1) {
-        // contiguous rows: B rows of M elements
+        // contiguous rows: B rows of M elements, codes in rows of ldq
         constexpr int HOLD = sizeof(T) == 4 ? 4 : 8;
-        const bool    vec  = (M % 8 == 0) && aligned_to(x, 16) && aligned_to(q, 8);
+        const bool    vec  = (M % 8 == 0) && ldq % 8 == 0 && aligned_to(x, 16) && aligned_to(q, 8);
         dim3          g(static_cast<unsigned>(B)), b(RW_THREADS);
         if (scale_in == nullptr) {
             if (vec)
                 quant_rowwise_inner_kernel<T, E5M2, true, true, HOLD>
-                    <<<g, b, 0, stream>>>(xp, qp, M, nullptr, scale_inv, qmax);
+                    <<<g, b, 0, stream>>>(xp, qp, M, ldq, nullptr, scale_inv, qmax);
             else
                 quant_rowwise_inner_kernel<T, E5M2, false, true, 1>
-                    <<<g, b, 0, stream>>>(xp, qp, M, nullptr, scale_inv, qmax);
+                    <<<g, b, 0, stream>>>(xp, qp, M, ldq, nullptr, scale_inv, qmax);
         } else {
             if (vec)
                 quant_rowwise_inner_kernel<T, E5M2, true, false, 1>
-                    <<<g, b, 0, stream>>>(xp, qp, M, scale_in, scale_inv, qmax);
+                    <<<g, b, 0, stream>>>(xp, qp, M, ldq, scale_in, scale_inv, qmax);
             else
                 quant_rowwise_inner_kernel<T, E5M2, false, false, 1>
-                    <<<g, b, 0, stream>>>(xp, qp, M, scale_in, scale_inv, qmax);
+                    <<<g, b, 0, stream>>>(xp, qp, M, ldq, scale_in, scale_inv, qmax);
         }
         return check_launch("quant_rowwise_inner_kernel");
     }
@@ -1041,14 +1047,16 @@ int pt_quantize_fp8_tensorwise_static(const void *x, int x_dtype, int64_t numel,
                                           status, 0, 0, static_cast<hipStream_t>(stream));
 }
 
-int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t C, void *q, void *q_t, int q_dtype,
-                                 float *scale_inv, void *workspace, size_t workspace_bytes, void *stream) {
+int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t C, void *q, int64_t ldq, void *q_t, int64_t ldt,
+                                 int q_dtype, float *scale_inv, void *workspace, size_t workspace_bytes, void *stream) {
     PT_REQUIRE(is_hp_dtype(x_dtype), "input must be bf16, fp16 or fp32");
     PT_REQUIRE(is_fp8_dtype(q_dtype), "output must be e4m3 or e5m2");
-    PT_REQUIRE(R > 0 && C > 0 && R % 16 == 0 && C % 16 == 0, "rows and columns must be positive multiples of 16");
+    PT_REQUIRE(R > 0 && C > 0 && C % 16 == 0, "rows and columns must be positive, columns a multiple of 16");
+    PT_REQUIRE(ldq >= C && ldt >= R && ldq % 16 == 0 && ldt % 16 == 0 && ldq - C < 128 && ldt <= cdiv(R, 128) * 128,
+               "pitches must be multiples of 16 that hold a row and pad it to 128 at most");
     PT_REQUIRE(x && q && q_t && scale_inv, "NULL tensor pointer");
     PT_REQUIRE(aligned_to(x, 16) && aligned_to(q, 16) && aligned_to(q_t, 16), "tensors must be 16-byte aligned");
-    PT_REQUIRE(R * C <= PT_TENSORWISE_STATIC_MAX_NUMEL, "too many elements");
+    PT_REQUIRE(R <= PT_TENSORWISE_STATIC_MAX_NUMEL / C, "too many elements");
     auto  st = static_cast<hipStream_t>(stream);
     auto *ws = static_cast<uint64_t *>(workspace);
     if (workspace == nullptr) {
@@ -1057,7 +1065,7 @@ int pt_quantize_fp8_tensorwise_t(const void *x, int x_dtype, int64_t R, int64_t 
     } else if (workspace_bytes < pt_quantize_fp8_tensorwise_workspace_bytes() || !aligned_to(workspace, 16)) {
         return fail(PT_ERR_WORKSPACE, "pt_quantize_fp8_tensorwise_t: workspace too small or misaligned");
     }
-#define CALL(T, E5) return launch_quant_tensorwise_t<T, E5>(x, R, C, q, q_t, scale_inv, ws, st)
+#define CALL(T, E5) return launch_quant_tensorwise_t<T, E5>(x, R, C, q, ldq, q_t, ldt, scale_inv, ws, st)
     PT_DISPATCH_HP_FP8(x_dtype, q_dtype, CALL);
 #undef CALL
 }
@@ -1107,7 +1115,19 @@ int pt_quantize_fp8_rowwise(const void *x, int x_dtype, int64_t B, int64_t M, in
     PT_REQUIRE(N == 1 ? B < (1LL << 31) : (B < 65536 && cdiv(M, 256) < 65536),
                "grid dimension out of range");
     auto st = static_cast<hipStream_t>(stream);
-#define CALL(T, E5) return launch_quant_rowwise<T, E5>(x, B, M, N, q, scale_in, scale_inv, st)
+#define CALL(T, E5) return launch_quant_rowwise<T, E5>(x, B, M, N, q, M, scale_in, scale_inv, st)
+    PT_DISPATCH_HP_FP8(x_dtype, q_dtype, CALL);
+#undef CALL
+}
+
+int pt_quantize_fp8_rowwise_padded(const void *x, int x_dtype, int64_t rows, int64_t cols, void *q, int64_t ldq, int q_dtype,
+                                   float *scale_inv, void *stream) {
+    PT_REQUIRE(is_hp_dtype(x_dtype), "input must be bf16, fp16 or fp32");
+    PT_REQUIRE(is_fp8_dtype(q_dtype), "output must be e4m3 or e5m2");
+    PT_REQUIRE(rows >= 0 && rows < (1LL << 31) && cols >= 0 && ldq >= cols, "bad dimensions");
+    PT_REQUIRE(rows * cols == 0 || (x && q && scale_inv), "NULL tensor pointer");
+    auto st = static_cast<hipStream_t>(stream);
+#define CALL(T, E5) return launch_quant_rowwise<T, E5>(x, rows, cols, 1, q, ldq, nullptr, scale_inv, st)
     PT_DISPATCH_HP_FP8(x_dtype, q_dtype, CALL);
 #undef CALL
 }

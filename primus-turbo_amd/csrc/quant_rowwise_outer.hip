@@ -30,6 +30,7 @@ namespace pt {
 template <typename T> struct OuterSrcHP {
     static constexpr bool IN_PLACE = true; // codes may also leave untransposed
     const T              *x;
+    int64_t               ld; // elements from one row to the next
     struct Raw {
         u32x4 v[sizeof(T) / 2];
     };
@@ -59,6 +60,7 @@ template <typename T> struct OuterSrcHP {
 template <typename T, bool SRC_E5M2> struct OuterSrcCodes {
     static constexpr bool IN_PLACE = false;
     const uint8_t        *q;
+    int64_t               ld;
     const float          *row_scale; // scale_inv of row b * M + m
     struct Raw {
         u32x2 v;
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const SRC src, float *__r
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k) {
                     const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
-                    r[k]              = src.load8(row, row * N + n);
+                    r[k]              = src.load8(row, row * src.ld + n);
                 }
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k) {
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const SRC src, float *__r
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k) {
                     const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
-                    f[k]              = src.get1(row, row * N + n);
+                    f[k]              = src.get1(row, row * src.ld + n);
                 }
 #pragma unroll
                 for (int k = 0; k < RO_ROWS; ++k)
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k) {
                 const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
-                r[k]              = src.load8(row, row * N + n);
+                r[k]              = src.load8(row, row * src.ld + n);
             }
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k) {
@@ -213,7 +215,7 @@ __global__ __launch_bounds__(256) void quant_outer_kernel(const SRC src, uint8_t
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k) {
                 const int64_t row = b * M + (m + 4 * k * rows < m1 ? m + 4 * k * rows : m);
-                f[k]              = src.get1(row, row * N + n);
+                f[k]              = src.get1(row, row * src.ld + n);
             }
 #pragma unroll
             for (int k = 0; k < RO_ROWS; ++k)
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(256) void quant_outer_t_kernel(const SRC src, uint8
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int64_t m = m0 + (k >> 2) * 64 + rg * 4 + (k & 3), row = b * M + (m < M ? m : 0);
-            raw[k] = src.load8(row, row * N + nn);
+            raw[k] = src.load8(row, row * src.ld + nn);
         }
     }
     if (tid < 128) {
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void quant_outer_t_kernel(const SRC src, uint8
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    f[k][e] = (m < M && n + e < N) ? src.get1(b * M + m, (b * M + m) * N + n + e) : 0.f;
+                    f[k][e] = (m < M && n + e < N) ? src.get1(b * M + m, (b * M + m) * src.ld + n + e) : 0.f;
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) // (rows behind the end: code 0)
@@ -401,7 +403,7 @@ static int launch_outer(const SRC &src, bool vec, int64_t B, int64_t M, int64_t 
 template <typename T>
 static int launch_outer_hp(const void *x, int64_t B, int64_t M, int64_t N, void *q, void *qt, int64_t ldt, bool e5m2,
                            const float *scale_in, float *scale_inv, float *ws, hipStream_t st) {
-    const OuterSrcHP<T> src{static_cast<const T *>(x)};
+    const OuterSrcHP<T> src{static_cast<const T *>(x), N};
     const bool          vec = N % 8 == 0 && aligned_to(x, 16) && (q == nullptr || aligned_to(q, 8));
     auto *qp = static_cast<uint8_t *>(q), *tp = static_cast<uint8_t *>(qt);
     return e5m2 ? launch_outer<OuterSrcHP<T>, true>(src, vec, B, M, N, qp, tp, ldt, scale_in, scale_inv, ws, st)
@@ -410,14 +412,14 @@ static int launch_outer_hp(const void *x, int64_t B, int64_t M, int64_t N, void 
 
 // codes quantized again keep their format
 template <typename T>
-static int launch_outer_codes(const void *x, const float *row_scale, int64_t B, int64_t M, int64_t N, void *qt, int64_t ldt,
-                              bool e5m2, float *scale_inv, float *ws, hipStream_t st) {
-    const bool vec = N % 8 == 0 && aligned_to(x, 8);
+static int launch_outer_codes(const void *x, int64_t ld, const float *row_scale, int64_t B, int64_t M, int64_t N, void *qt,
+                              int64_t ldt, bool e5m2, float *scale_inv, float *ws, hipStream_t st) {
+    const bool vec = N % 8 == 0 && ld % 8 == 0 && aligned_to(x, 8);
     auto      *xp  = static_cast<const uint8_t *>(x);
     auto      *tp  = static_cast<uint8_t *>(qt);
     if (e5m2)
-        return launch_outer<OuterSrcCodes<T, true>, true>({xp, row_scale}, vec, B, M, N, nullptr, tp, ldt, nullptr, scale_inv, ws, st);
-    return launch_outer<OuterSrcCodes<T, false>, false>({xp, row_scale}, vec, B, M, N, nullptr, tp, ldt, nullptr, scale_inv, ws, st);
+        return launch_outer<OuterSrcCodes<T, true>, true>({xp, ld, row_scale}, vec, B, M, N, nullptr, tp, ldt, nullptr, scale_inv, ws, st);
+    return launch_outer<OuterSrcCodes<T, false>, false>({xp, ld, row_scale}, vec, B, M, N, nullptr, tp, ldt, nullptr, scale_inv, ws, st);
 }
 
 // the form behind pt_quantize_fp8_rowwise (quant_fp8.hip); ws may be NULL
@@ -452,11 +454,19 @@ size_t pt_quantize_fp8_rowwise_outer_workspace_bytes(int64_t B, int64_t M, int64
 int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_scale_inv, int hp_dtype, int64_t B, int64_t M,
                                   int64_t N, void *q, void *q_t, int64_t ld_t, int q_dtype, float *scale_inv, void *workspace,
                                   size_t workspace_bytes, void *stream) {
+    return pt_quantize_fp8_rowwise_outer_ld(x, N, x_dtype, row_scale_inv, hp_dtype, B, M, N, q, q_t, ld_t, q_dtype, scale_inv,
+                                            workspace, workspace_bytes, stream);
+}
+
+int pt_quantize_fp8_rowwise_outer_ld(const void *x, int64_t ld_x, int x_dtype, const float *row_scale_inv, int hp_dtype,
+                                     int64_t B, int64_t M, int64_t N, void *q, void *q_t, int64_t ld_t, int q_dtype,
+                                     float *scale_inv, void *workspace, size_t workspace_bytes, void *stream) {
     const bool codes = is_fp8_dtype(x_dtype);
     PT_REQUIRE(codes || is_hp_dtype(x_dtype), "input must be bf16, fp16, fp32 or fp8 codes");
     PT_REQUIRE(is_fp8_dtype(q_dtype), "output must be e4m3 or e5m2");
     PT_REQUIRE(B >= 0 && M >= 0 && N >= 0, "dimensions must be non-negative");
     PT_REQUIRE((q != nullptr) != (q_t != nullptr), "one of q and q_t is written");
+    PT_REQUIRE(codes ? ld_x >= N : ld_x == N, "only rows of codes may be longer than the matrix is wide");
     if (codes) {
         PT_REQUIRE(row_scale_inv != nullptr && is_hp_dtype(hp_dtype), "codes need their row scales and the type they stand for");
         PT_REQUIRE(q_t != nullptr && q_dtype == x_dtype, "codes are quantized again into their own format, transposed");
@@ -477,10 +487,10 @@ int pt_quantize_fp8_rowwise_outer(const void *x, int x_dtype, const float *row_s
     const int  hp = codes ? hp_dtype : x_dtype;
     if (codes) {
         if (hp == PT_DTYPE_BF16)
-            return launch_outer_codes<bf16_t>(x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
+            return launch_outer_codes<bf16_t>(x, ld_x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
         if (hp == PT_DTYPE_F16)
-            return launch_outer_codes<f16_t>(x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
-        return launch_outer_codes<float>(x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
+            return launch_outer_codes<f16_t>(x, ld_x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
+        return launch_outer_codes<float>(x, ld_x, row_scale_inv, B, M, N, q_t, ld_t, e5, scale_inv, ws, st);
     }
     if (hp == PT_DTYPE_BF16)
         return launch_outer_hp<bf16_t>(x, B, M, N, q, q_t, ld_t, e5, nullptr, scale_inv, ws, st);

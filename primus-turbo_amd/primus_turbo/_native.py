@@ -69,7 +69,16 @@ _SIGNATURES = {
     ),
     "pt_quantize_fp8_tensorwise_t": (
         c_int,
-        [c_void_p, c_int, c_i64, c_i64, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_void_p],
+        [c_void_p, c_int, c_i64, c_i64, c_void_p, c_i64, c_void_p, c_i64, c_int, c_void_p, c_void_p, c_size_t, c_void_p],
+    ),
+    "pt_quantize_fp8_rowwise_padded": (
+        c_int,
+        [c_void_p, c_int, c_i64, c_i64, c_void_p, c_i64, c_int, c_void_p, c_void_p],
+    ),
+    "pt_quantize_fp8_rowwise_outer_ld": (
+        c_int,
+        [c_void_p, c_i64, c_int, c_void_p, c_int, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_i64, c_int, c_void_p, c_void_p,
+         c_size_t, c_void_p],
     ),
     "pt_tensorwise_static_release": (c_int, [c_void_p]),
     "pt_quantize_fp8_tensorwise_two_pass": (

@@ -134,36 +134,46 @@ _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise_meta, "Meta")
 
 
 @native_op("primus_turbo::quantize_fp8_tensorwise_t")
-def quantize_fp8_tensorwise_t_impl(x: torch.Tensor, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """TENSORWISE quantization of a contiguous matrix ``x [R, C]`` with the codes emitted transposed as well,
-    ``(x_fp8 [R, C], x_fp8_t [C, R], scale_inv)``, same bytes as the cast followed by a transposition. One launch
-    where the plain cast is one (eager calls in the fused mode) and both sizes are multiples of 16; else those two
-    steps. (No counterpart in the reference, which runs them.)"""
+def quantize_fp8_tensorwise_t_impl(x: torch.Tensor, dtype: torch.dtype, width: int, width_t: int
+                                   ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """TENSORWISE quantization of a contiguous matrix ``x [R, C]`` with the codes emitted transposed as well:
+    ``(x_fp8 [R, width], x_fp8_t [C, width_t], scale_inv)``, the bytes of the cast and of its transposition and
+    zeros behind them (``width`` = C or C rounded up to 128, ``width_t`` likewise for R: rows that a product reads
+    without a padding copy). One launch where the plain cast is one (eager calls in the fused mode) and C and both
+    widths are multiples of 16; else those steps. (No counterpart in the reference, which runs them.)"""
     _check(x.dim() == 2 and x.is_contiguous(), "input must be a contiguous matrix")
     R, C = x.shape
+    _check(width in (C, _padded_rows(C, 128)) and width_t in (R, _padded_rows(R, 128)), "a width is the size or padded to 128")
     one_launch = (
-        R % 16 == 0 and C % 16 == 0 and x.numel() > 0 and x.dtype in _HP_DTYPES and x.is_cuda and x.data_ptr() % 16 == 0
-        and _tensorwise_mode != "two_pass" and not torch.cuda.is_current_stream_capturing())
+        C % 16 == 0 and width % 16 == 0 and width_t % 16 == 0 and x.numel() > 0 and x.dtype in _HP_DTYPES and x.is_cuda
+        and x.data_ptr() % 16 == 0 and _tensorwise_mode != "two_pass" and not torch.cuda.is_current_stream_capturing())
     if one_launch:
         _check_fp8_out(dtype)
-        q = torch.empty_like(x, dtype=dtype)
-        q_t = torch.empty((C, R), dtype=dtype, device=x.device)
+        q = torch.empty((R, width), dtype=dtype, device=x.device)
+        q_t = torch.empty((C, width_t), dtype=dtype, device=x.device)
         scale_inv = torch.empty((), dtype=torch.float32, device=x.device)
         status = N.lib().pt_quantize_fp8_tensorwise_t(
-            N.ptr(x), N.dtype_code(x.dtype), R, C, N.ptr(q), N.ptr(q_t), N.dtype_code(dtype), N.ptr(scale_inv), None, 0,
-            N.stream_of(x))
+            N.ptr(x), N.dtype_code(x.dtype), R, C, N.ptr(q), width, N.ptr(q_t), width_t, N.dtype_code(dtype), N.ptr(scale_inv),
+            None, 0, N.stream_of(x))
         if status != N.PT_ERR_WORKSPACE:  # (more stream handles than the static scratch has slot sets for)
             N.check(status)
             return q, q_t, scale_inv
     q, scale_inv = _quantize_fp8_tensorwise(x, dtype)
     q_t = torch.empty((C, R), dtype=dtype, device=x.device)
     N.check(N.lib().pt_transpose_u8(N.ptr(q), N.ptr(q_t), 1, R, C, N.stream_of(q)))
-    return q, q_t, scale_inv
+    return _zero_padded(q, width), _zero_padded(q_t, width_t), scale_inv
+
+
+def _zero_padded(q: torch.Tensor, width: int) -> torch.Tensor:
+    if q.shape[-1] == width:
+        return q
+    return torch.nn.functional.pad(q.view(torch.uint8), (0, width - q.shape[-1])).view(q.dtype)
 
 
 @quantize_fp8_tensorwise_t_impl.register_fake
-def _quantize_fp8_tensorwise_t_impl_fake(x, dtype):
-    return (torch.empty_like(x, dtype=dtype), torch.empty((x.shape[1], x.shape[0]), dtype=dtype, device=x.device),
+def _quantize_fp8_tensorwise_t_impl_fake(x, dtype, width, width_t):
+    return (torch.empty((x.shape[0], width), dtype=dtype, device=x.device),
+            torch.empty((x.shape[1], width_t), dtype=dtype, device=x.device),
             torch.empty((), dtype=torch.float32, device=x.device))
 
 
@@ -211,12 +221,13 @@ def _valid_axis(axis: int, ndim: int) -> int:
 
 
 def _rowwise_outer(x, row_scale_inv, hp_dtype, bmn, q, q_t, ld_t, scale_inv):
-    """Dynamic rowwise quantization over the middle axis of ``x`` viewed as ``bmn = (B, M, N)``."""
+    """Dynamic rowwise quantization over the middle axis of ``x`` viewed as ``bmn = (B, M, N)``, the first N of
+    longer rows where ``x`` holds codes."""
     lib = N.lib()
     ws = torch.empty(lib.pt_quantize_fp8_rowwise_outer_workspace_bytes(*bmn), dtype=torch.uint8, device=x.device)
     N.check(
-        lib.pt_quantize_fp8_rowwise_outer(
-            N.ptr(x), N.dtype_code(x.dtype), N.ptr(row_scale_inv), N.dtype_code(hp_dtype), *bmn, N.ptr(q), N.ptr(q_t), ld_t,
+        lib.pt_quantize_fp8_rowwise_outer_ld(
+            N.ptr(x), bmn[2] if row_scale_inv is None else x.shape[-1], N.dtype_code(x.dtype), N.ptr(row_scale_inv), N.dtype_code(hp_dtype), *bmn, N.ptr(q), N.ptr(q_t), ld_t,
             N.dtype_code((q if q is not None else q_t).dtype), N.ptr(scale_inv), N.ptr(ws), ws.numel(), N.stream_of(x),
         )
     )
@@ -331,20 +342,24 @@ def _padded_rows(M: int, pad: int) -> int:
 
 @native_op("primus_turbo::quant_fp8_rowwise_t_impl")
 def quant_fp8_rowwise_t_impl(
-    x: torch.Tensor, row_scale_inv: Optional[torch.Tensor], hp_dtype: torch.dtype, dtype: torch.dtype, pad: int
+    x: torch.Tensor, row_scale_inv: Optional[torch.Tensor], hp_dtype: torch.dtype, dtype: torch.dtype, pad: int,
+    cols: Optional[int] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """ROWWISE quantization of ``x [.., M, N]`` along axis -2 with the codes emitted transposed, ``(x_fp8_t
     [.., N, M_pad], scale_inv [.., 1, N])``, ``M_pad`` = ``M`` rounded up to ``pad`` (a multiple of 16; the
     added codes are zero): the K-contiguous operand of the product that reduces over the rows of ``x``.
     With ``row_scale_inv`` ``x`` holds FP8 codes of a ROWWISE quantization along axis -1, which are
     quantized again along axis -2 from the ``hp_dtype`` values they stand for (same bits as
-    de-quantize, quantize, transpose). (No counterpart in the reference, which runs those three steps.)"""
+    de-quantize, quantize, transpose), the first ``cols`` of a row where rows are padded. (No counterpart in the reference, which runs those three steps.)"""
     N.require_cuda(x, row_scale_inv)
     _check_fp8_out(dtype)
     _check(x.dim() >= 2 and x.is_contiguous(), "input must be contiguous, at least 2-D")
     _check(hp_dtype in _HP_DTYPES, "hp_dtype must be bfloat16, float16 or float32")
     _check(pad % 16 == 0, "pad must be a multiple of 16")
     *lead, M, Nn = x.shape
+    if cols is not None:
+        _check(row_scale_inv is not None and 0 <= cols <= Nn, "cols belongs to padded rows of codes")
+        Nn = cols
     if row_scale_inv is None:
         _check(x.dtype == hp_dtype, "input must be bfloat16, float16 or float32")
     else:
@@ -362,12 +377,35 @@ def quant_fp8_rowwise_t_impl(
 
 
 @quant_fp8_rowwise_t_impl.register_fake
-def _quant_fp8_rowwise_t_impl_fake(x, row_scale_inv, hp_dtype, dtype, pad):
+def _quant_fp8_rowwise_t_impl_fake(x, row_scale_inv, hp_dtype, dtype, pad, cols=None):
     *lead, M, Nn = x.shape
+    Nn = Nn if cols is None else cols
     return (
         torch.empty((*lead, Nn, _padded_rows(M, pad)), dtype=dtype, device=x.device),
         torch.empty((*lead, 1, Nn), dtype=torch.float32, device=x.device),
     )
+
+
+@native_op("primus_turbo::quant_fp8_rowwise_padded_impl")
+def quant_fp8_rowwise_padded_impl(x: torch.Tensor, dtype: torch.dtype, width: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """ROWWISE quantization of a contiguous matrix ``x [M, N]`` along its rows with zero codes behind them:
+    ``(x_fp8 [M, width], scale_inv [M, 1])``, rows that a product reads without a padding copy. (No counterpart in
+    the reference.)"""
+    N.require_cuda(x)
+    _check(x.dtype in _HP_DTYPES, "input must be bfloat16, float16 or float32")
+    _check_fp8_out(dtype)
+    _check(x.dim() == 2 and x.is_contiguous() and width >= x.shape[1], "input must be a contiguous matrix, at most width wide")
+    q = torch.empty((x.shape[0], width), dtype=dtype, device=x.device)
+    scale_inv = torch.empty((x.shape[0], 1), dtype=torch.float32, device=x.device)
+    N.check(N.lib().pt_quantize_fp8_rowwise_padded(N.ptr(x), N.dtype_code(x.dtype), x.shape[0], x.shape[1], N.ptr(q), width,
+                                                   N.dtype_code(dtype), N.ptr(scale_inv), N.stream_of(x)))
+    return q, scale_inv
+
+
+@quant_fp8_rowwise_padded_impl.register_fake
+def _quant_fp8_rowwise_padded_impl_fake(x, dtype, width):
+    return (torch.empty((x.shape[0], width), dtype=dtype, device=x.device),
+            torch.empty((x.shape[0], 1), dtype=torch.float32, device=x.device))
 
 
 # ===========================================================================

@@ -38,6 +38,7 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_t_impl,
     quant_fp8_blockwise_kmajor_impl,
     quant_fp8_blockwise_for_weight_dual_impl,
+    quant_fp8_rowwise_padded_impl,
     quant_fp8_rowwise_t_impl,
     quantize_fp8_tensorwise_t_impl,
     quantize_mx_operands,
@@ -77,6 +78,11 @@ def _quantized_parts(x, config, fwd: bool, axis):
     return q, s, x.dtype
 
 
+def _whole_slabs(n: int) -> int:
+    """``n`` codes padded to what the products read as they are: whole 128-byte slabs of a row."""
+    return -(-n // 128) * 128
+
+
 class FP8GemmTensorFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum_pattern=None):
@@ -87,11 +93,16 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         # shares the scalar scale; the cast of a plain operand emits it from the same read
         nt_bwd = (not trans_a) and trans_b
         need_bwd = any(ctx.needs_input_grad[:2])
+        # (rows are padded to whole slabs of the products where both operands of a product are made here, in
+        # one launch each: codes in 16-byte groups along K and N)
+        plain = not any(isinstance(t, QuantizedTensor) for t in (a, b, a_t, b_t)) and b.shape[0] % 16 == 0 and b.shape[1] % 16 == 0
 
         def operand(x, x_t):
             want_t = need_bwd and nt_bwd and not isinstance(x_t, QuantizedTensor)
             if want_t and not isinstance(x, QuantizedTensor):
-                q, q_t, q_s = quantize_fp8_tensorwise_t_impl(x.contiguous(), _get_fp8_dtype(config.format, True))
+                pad = _whole_slabs if plain else (lambda n: n)
+                q, q_t, q_s = quantize_fp8_tensorwise_t_impl(x.contiguous(), _get_fp8_dtype(config.format, True),
+                                                             pad(x.shape[1]), pad(x.shape[0]))
                 return q, q_s, q_t, q_s
             q, q_s, _ = _quantized_parts(x, config, True, -1)
             if want_t:
@@ -118,8 +129,8 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         gdt = _get_fp8_dtype(config.format, False)
         acc = main_grad if fuse else None
         if nt_bwd:
-            # saved: A^T [K, M], B^T [K, N]
-            g, g_t, g_s = quantize_fp8_tensorwise_t_impl(grad_out.contiguous(), gdt)
+            # saved: A^T [K, M], B^T [K, N] (rows as long as the gradient's have to be)
+            g, g_t, g_s = quantize_fp8_tensorwise_t_impl(grad_out.contiguous(), gdt, sb.shape[1], sa.shape[1])
             grad_a = _gemm(g, g_s, False, sb, sb_s, True, out_dtype, False, gran)
             grad_b = _wgrad_gemm(sa, sa_s, False, g_t, g_s, True, out_dtype, trans_b, gran, acc)
         else:
@@ -135,8 +146,18 @@ class FP8GemmRowFunction(torch.autograd.Function):
         assert trans_a == False, "trans_a has to be False"  # noqa: E712
         gran = config.granularity
         b_axis = -1 if trans_b else -2
-        qa, qa_s, a_hp = _quantized_parts(a, config, True, -1)
-        qb, qb_s, b_hp = _quantized_parts(b, config, True, b_axis)
+        # operands made here have rows of whole slabs: no product copies them to pad them
+        plain = trans_b and not any(isinstance(t, QuantizedTensor) for t in (a, b))
+        K = a.shape[1]
+
+        def along_rows(x, axis):
+            if not plain or K % 128 == 0:
+                return _quantized_parts(x, config, True, axis)
+            return (*quant_fp8_rowwise_padded_impl(x.contiguous(), _get_fp8_dtype(config.format, True), _whole_slabs(K)), x.dtype)
+
+        qa, qa_s, a_hp = along_rows(a, -1)
+        qb, qb_s, b_hp = along_rows(b, b_axis)
+        cols = K if qa.shape[1] != K else None
 
         def other_axis(q, q_s, hp_dtype, from_axis, given, axis, pad):
             # the operand as backward reads it: what the forward codes stand for, quantized again
@@ -146,7 +167,9 @@ class FP8GemmRowFunction(torch.autograd.Function):
                 assert isinstance(given, QuantizedTensor)
                 return given.qdata, given.scale_inv, False
             if axis == -2 and pad is not None:
-                return (*quant_fp8_rowwise_t_impl(q, q_s, hp_dtype, q.dtype, pad), True)
+                return (*quant_fp8_rowwise_t_impl(q, q_s, hp_dtype, q.dtype, pad, cols), True)
+            if cols is not None:
+                q = q[:, :cols].contiguous()
             hp = dequantize_fp8(q, hp_dtype, gran, axis=from_axis % q.ndim, scale_inv=q_s, block_size=config.block_size)
             return (*quantize_fp8(hp, q.dtype, gran, axis=axis % q.ndim, block_size=config.block_size), False)
 
@@ -155,10 +178,9 @@ class FP8GemmRowFunction(torch.autograd.Function):
         # input asks for a gradient (same outputs, two quantizer passes less)
         a_t_ready = b_t_ready = False
         if any(ctx.needs_input_grad[:2]):
-            # (wgrad: both operands carry the token padding; dgrad: the gradient's rows are as they are)
+            # (both operands of a product carry the padding of its reduction: tokens in wgrad, N in dgrad)
             a_c, a_cs, a_t_ready = other_axis(qa, qa_s, a_hp, -1, a_t, -2, 128)
-            b_c, b_cs, b_t_ready = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1,
-                                              16 if qb.size(-2) % 16 == 0 else None)
+            b_c, b_cs, b_t_ready = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1, 128)
             ctx.save_for_backward(a_c, a_cs, b_c, b_cs)
         ctx.meta = (trans_a, trans_b, out_dtype, config, a_t_ready, b_t_ready)
         return out
@@ -170,7 +192,10 @@ class FP8GemmRowFunction(torch.autograd.Function):
         grad_out = grad_out.contiguous()
         gdt = _get_fp8_dtype(config.format, False)
         gran = config.granularity
-        g_row, g_row_s = quantize_fp8(grad_out, gdt, gran, axis=1, block_size=config.block_size)
+        if b_t_ready:
+            g_row, g_row_s = quant_fp8_rowwise_padded_impl(grad_out, gdt, b_c.shape[1])
+        else:
+            g_row, g_row_s = quantize_fp8(grad_out, gdt, gran, axis=1, block_size=config.block_size)
         grad_a = _gemm(g_row, g_row_s, False, b_c, b_cs, True if b_t_ready else not trans_b, out_dtype, trans_a, gran)
         if a_t_ready:
             g_col, g_col_s = quant_fp8_rowwise_t_impl(grad_out, None, grad_out.dtype, gdt, 128)
