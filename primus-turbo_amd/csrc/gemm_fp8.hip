@@ -176,7 +176,7 @@ template <int FA, int FB>
 static int launch_vector_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
     // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128
     if (tile_cfg == 0)
-        tile_cfg = (a.M >= 2048 && a.N >= 2048) ? 1 : 3;
+        tile_cfg = dense_tile<SCALE_VECTOR>(a.M, a.N, a.K / KSTEP, true);
     if (tile_cfg == 1 || tile_cfg == 4)
         return launch_gemm_cfg<8, 8, SCALE_VECTOR, false, FA, FB>(a, stream);
     if (tile_cfg == 2)

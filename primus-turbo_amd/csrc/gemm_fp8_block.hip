@@ -9,29 +9,25 @@ namespace pt {
 
 template <bool SB_VEC, int FA, int FB>
 static int launch_block_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
-    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128 (two workgroups per CU),
-    // 4 = 256x256 with eight wavefronts (2-D B scales only)
-    if (tile_cfg == 0) {
-        tile_cfg = (a.M >= 2048 && a.N >= 1024) ? 2 : 3;
-        // 256x256 with eight wavefronts once both dimensions fill the machine with such tiles
-        if (!SB_VEC && a.M >= 2048 && a.N >= 2048 && cdiv(a.M, 256) * cdiv(a.N, 256) >= device_cu_count())
-            tile_cfg = 4;
-    }
-    if (tile_cfg == 4) {
-        if constexpr (SB_VEC)
-            tile_cfg = 2;
-        else
-            return launch_gemm_block8<FA, FB>(a, stream);
-    }
+    // tile_cfg: 0 = auto, 1 and 4 = 256x256 with eight wavefronts, 2 = 256x128 (per-column B scales: as 3),
+    // 3 = 128x128 (two workgroups per CU)
+    // (Per-column B scales, the weight gradient of the blockwise recipe, us: 256x256 with eight wavefronts /
+    // 256x128 / 128x128: 8192^3 522 / 651 / 661, 4096 x 7168 x 4096 127 / 164 / 144, 2048 x 2048 x 8192 106 / 81
+    // / 59, 5120 x 4096 x 2048 66 / 68 / 54; 128 x 128 B blocks: 454 / 566 / 574, 112 / 142 / 131, 87 / 64 / 48,
+    // 57 / 56 / 49.)
+    if (tile_cfg == 0)
+        tile_cfg = dense_tile<SCALE_BLOCK>(a.M, a.N, a.K / KSTEP, !SB_VEC);
+    if (tile_cfg == 1 || tile_cfg == 4)
+        return launch_gemm_block8<FA, FB, GROUP_NONE, SB_VEC>(a, stream);
     if constexpr (!SB_VEC) {
         if (tile_cfg == 3 && one_tile_per_cu(a.M, a.N))
             return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB, GROUP_NONE, 4>(a, stream);
     }
-    if (tile_cfg == 3)
-        return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
-    if (tile_cfg == 1)
-        return launch_gemm_cfg<8, 8, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
-    return launch_gemm_cfg<8, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
+    if constexpr (!SB_VEC) {
+        if (tile_cfg == 2)
+            return launch_gemm_cfg<8, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
+    }
+    return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
 }
 
 template <bool SB_VEC>

@@ -23,6 +23,10 @@
 //     rows, scales, A rows) go into the stage just freed during row groups 6 and 7: every
 //     copy a barrier waits for is then older than the stores of a result tile written in
 //     between, which is what lets that wait leave the stores in flight;
+//   * SB_VEC: a scale per row of both operands (the weight gradient of the blockwise recipe, whose reduction
+//     runs over the tokens). The column scales travel like the row scales, the fold costs a multiply more
+//     for each value (bound by it: 8192^3 takes 522 us, without the multiply 434) and the 24 scales are read as
+//     the slab starts, for want of registers. Still a fifth faster than 256 x 128 with four wavefronts (651 us);
 //   * the slab sequence runs across tile boundaries (persistent grid), the loader changing
 //     tile by swapping uniform values as in the four-wavefront kernel.
 #pragma once
@@ -46,9 +50,10 @@ constexpr int B8_LA = B8_BM / 8 / B8_WAVES, B8_LB = B8_BN / 8 / B8_WAVES; // row
 constexpr int B8_NL = B8_LA + B8_LB + 1;                                  // + one scale copy
 constexpr int B8_P1 = B8_LB + 1; // copies of a slab issued in row groups 6, 7 (B rows, scales)
 
-template <int FA, int FB, int GMODE>
+template <int FA, int FB, int GMODE, bool SB_VEC>
 __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmArgs a) {
     static_assert(GMODE == GROUP_NONE || GMODE == GROUP_ROWS, "row groups or none");
+    static_assert(!SB_VEC || GMODE == GROUP_NONE, "a scale per column: dense products");
     constexpr int TM = B8_TM, TN = B8_TN, BM = B8_BM, BN = B8_BN;
     constexpr int A_BYTES = B8_A_BYTES, STAGE = B8_STAGE, NSTAGE = B8_NSTAGE;
     constexpr int LA = B8_LA, LB = B8_LB, NL = B8_NL;
@@ -109,6 +114,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         }
         if (wave < 4) // scale of tile row 64 wave + lane
             off[NL - 1] = static_cast<uint32_t>((wave * 64 + lane) >> a.sa_shift) * static_cast<uint32_t>(a.sa_m) * 4u;
+        else if constexpr (SB_VEC) // scale of tile column 64 (wave - 4) + lane
+            off[NL - 1] = static_cast<uint32_t>((wave - 4) * 64 + lane) * static_cast<uint32_t>(a.sb_n) * 4u;
         else          // scale of the tile's column block `lane` (two blocks; the other lanes read nothing)
             off[NL - 1] = lane < BN / 128 ? static_cast<uint32_t>(lane) * static_cast<uint32_t>(a.sb_n) * 4u : 0x7ffffff0u;
     }
@@ -176,7 +183,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     f32x4 acc[TM][TN];
     i32x8 fb[TN], fa[4];
     float sn[TM], sbn; // scales of the next slab as read from its stage
-    float sc[TM];      // sA[row] * sB of the slab being multiplied
+    float sc[TM];      // sA[row] * sB of the slab being multiplied (SB_VEC: sA[row])
+    f32x4 sb_cur[TN];  // SB_VEC: sB of the lane's columns
     int   buf = 0;
 
     auto ldfrag = [&](const uint8_t *part, int f) {
@@ -215,7 +223,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     // copies the next barrier waits for: memory operations retire in order, and leaving that many
     // outstanding waits for the copies without waiting for the stores to be acknowledged.
     int pending = 0;
-    read_scales(smem);
+    if constexpr (!SB_VEC)
+        read_scales(smem);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
         fb[j] = ldfrag(smem + b_part, j);
@@ -238,9 +247,21 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         for (int kt = 0; kt < KT_ALL; ++kt) {
             const uint8_t *cur = smem + buf * STAGE;
             const uint8_t *nxt = smem + (buf ^ 1) * STAGE;
+            if constexpr (SB_VEC) {
+                // (24 values a slab instead of 9: read when the slab starts, there are no registers to hold two slabs')
+                const float *sa = reinterpret_cast<const float *>(cur + B8_SC_A) + wm * (TM * 16) + lm;
+                const float *sb = reinterpret_cast<const float *>(cur + B8_SC_B) + wn * (TN * 16) + lg * 4;
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-                sc[i] = sn[i] * sbn;
+                for (int i = 0; i < TM; ++i)
+                    sc[i] = sa[i * 16];
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    sb_cur[j] = *reinterpret_cast<const f32x4 *>(sb + j * 16);
+            } else {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    sc[i] = sn[i] * sbn;
+            }
 
             constexpr int DEPTH = 3, RING = DEPTH + 1, TILES = TM * TN;
             f32x4         ring[RING];
@@ -249,7 +270,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
                 const f32x4 &p = ring[t % RING];
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    acc[i][j][e] = fmaf(p[e], sc[i], acc[i][j][e]);
+                    acc[i][j][e] = fmaf(p[e], SB_VEC ? sc[i] * sb_cur[j][e] : sc[i], acc[i][j][e]);
             };
 
             static_for<0, TM>([&](auto ic) {
@@ -276,7 +297,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
                                  : "memory", "scc");
                     pending = 0;
                     __builtin_amdgcn_s_barrier();
-                    read_scales(nxt);
+                    if constexpr (!SB_VEC)
+                        read_scales(nxt);
                 }
                 // A fragment two row groups ahead
                 if constexpr (i + 2 < TM)
@@ -326,7 +348,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int FA, int FB, int GMODE = GROUP_NONE>
+template <int FA, int FB, int GMODE = GROUP_NONE, bool SB_VEC = false>
 static int launch_gemm_block8(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int STAGES  = B8_NSTAGE * B8_STAGE;
     constexpr int MAX_G   = 2048;
@@ -338,11 +360,11 @@ static int launch_gemm_block8(const GemmArgs &args_in, hipStream_t stream) {
     a.tiles_n  = static_cast<int>(cdiv(a.N, B8_BN));
     if (GMODE != GROUP_NONE && a.G > MAX_G)
         return fail(PT_ERR_INVALID_ARGUMENT, "grouped gemm: too many groups for this tile configuration");
-    if (a.sb_shift != 7 || (GMODE == GROUP_ROWS && a.sa_shift != 0))
+    if (a.sb_shift != (SB_VEC ? 0 : 7) || (GMODE == GROUP_ROWS && a.sa_shift != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_fp8: unsupported block-scale layout for the 256x256 tile");
     if (a.K / KSTEP < 2)
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_fp8: K too short for the 256x256 tile");
-    auto kern = gemm_fp8_block8_kernel<FA, FB, GMODE>;
+    auto kern = gemm_fp8_block8_kernel<FA, FB, GMODE, SB_VEC>;
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)

@@ -1496,6 +1496,35 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
 static inline bool one_tile_per_cu(int64_t M, int64_t N) {
     return (M + 127) / 128 * ((N + 127) / 128) <= device_cu_count();
 }
+// The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128. A large tile multiplies more for each
+// byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
+// how the tiles divide among the CUs. The time of a round for one slab, in 64ths of what a 256 x 256 tile takes:
+//                     256x256   256x128   2 of 128x128   1 of 128x128     (256 x 256: us)
+//   vector scales        64        36          42             23                1.50
+//   MXFP8                64        37          42             23                1.64
+//   MXFP4                64        38          40             26                2.1 (256 codes)
+//   block scales         64        40          41             27                1.75 (a scale per column 2.0)
+// and a tile spends about the time of two slabs on its first copies and its result, the 256 x 256 one, whose CU has
+// nothing else to do meanwhile, that of three or four. (Medians over products of 26 sizes with every tile, 512 to
+// 28672 wide, K 512 to 8192.) Taking 256 x 256 wherever both sides reach 2048, and 128 x 128 elsewhere, lost 6 to
+// 13 % against the best tile on average: vector scales 2048 x 2048 x 8192 72 us, 128 x 128 32 (MXFP8 82 / 40);
+// 4096 x 2048 x 4096 43.8, 256 x 128 31.1; 16384 x 1024 x 4096 61.5, 256 x 256 51.9. This rule loses 0.3 %, at
+// most 5 %, and nowhere to that one.
+// middle: 256 x 128 may be taken (for MXFP4 and a scale per column it is nowhere more than 3 % ahead).
+template <int MODE, bool F4 = false> static inline int dense_tile(int64_t M, int64_t N, int64_t slabs, bool middle) {
+    constexpr int64_t PAIR = MODE == SCALE_VECTOR ? 42 : 41, SINGLE = MODE == SCALE_VECTOR ? 28 : 27;
+    constexpr int64_t HALF_SLABS = MODE == SCALE_VECTOR ? 8 : MODE == SCALE_MX && !F4 ? 7 : 6; // half slabs beside the K loop
+    const int64_t cus = device_cu_count();
+    auto up = [](int64_t x, int64_t m) { return (x + m - 1) / m; };
+    const int64_t m2 = up(M, 256), n2 = up(N, 256), m1 = up(M, 128), n1 = up(N, 128);
+    const int64_t pairs = m1 * n1 / (2 * cus), rest = m1 * n1 % (2 * cus);
+    const int64_t t3 = (PAIR * pairs + (rest == 0 ? 0 : rest <= cus ? SINGLE : PAIR)) * (slabs + 2);
+    const int64_t t2 = PAIR * up(m2 * n1, cus) * (slabs + 2);
+    const int64_t t1 = 32 * up(m2 * n2, cus) * (2 * slabs + HALF_SLABS);
+    if (t1 <= t3 && (!middle || t1 <= t2))
+        return 1;
+    return middle && t2 <= t3 ? 2 : 3;
+}
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;
 }

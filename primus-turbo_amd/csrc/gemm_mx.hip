@@ -6,15 +6,19 @@
 namespace pt {
 
 template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
-    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128, 4 = 256x256 with eight wavefronts
-    // (the eight-wavefront tile measured 2-4 % faster than four wavefronts on MXFP4 at 16384^3 and
-    // 8192 x 28672 x 8192, and 0-9 % slower on MXFP8)
+    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128, 4 = 256x256 with eight wavefronts (MXFP4: 1 as well)
+    // (256x256 with four wavefronts, us, against eight: MXFP4 8192^3 285 / 257, 4096 x 28672 x 8192 471 / 455.
+    // MXFP8 on codes that were not scaled by block 8192^3 420 / 402, but a training step of 8192 x 7168 x 2048 on
+    // quantized activations 376 / 390: there the chip's clock follows the codes, and four wavefronts do less
+    // besides the products.)
     if (tile_cfg == 0)
-        tile_cfg = (a.M >= 2048 && a.N >= 2048) ? (FA == 4 ? 4 : 1) : 3;
-    if (tile_cfg == 4)
+        tile_cfg = dense_tile<SCALE_MX, FA == 4>(a.M, a.N, a.K / KSTEP, FA != 4);
+    if (tile_cfg == 4 || (FA == 4 && tile_cfg == 1))
         return launch_gemm_mx8<FA, FB>(a, stream);
-    if (tile_cfg == 1)
-        return launch_gemm_cfg<8, 8, SCALE_MX, false, FA, FB>(a, stream);
+    if constexpr (FA != 4) {
+        if (tile_cfg == 1)
+            return launch_gemm_cfg<8, 8, SCALE_MX, false, FA, FB>(a, stream);
+    }
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_MX, false, FA, FB>(a, stream);
     if constexpr (FA != 4) {
