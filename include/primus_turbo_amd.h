@@ -666,10 +666,11 @@ PT_API int pt_shuffle_e8m0_scale(const void *in, void *out, int64_t batch, int64
  *   [T + pad_multiple, 2 E + 1] (row of a token: [2E] = n routed experts, [0, n) = 1-based destination
  *   rows in ascending expert order, [E, E + n) = expert id, or the top-k slot when
  *   topk_aligned_probs; rows T + i: negative 1-based rows of the i-th zero pad row of every expert that
- *   has one; other entries are left as they are), tokens_per_expert [E] (padded to pad_multiple,
+ *   has one; other entries are zero), tokens_per_expert [E] (padded to pad_multiple,
  *   clipped at num_permuted_tokens when that is > 0), overflow_flag (1 when rows were dropped for
  *   that limit), num_dispatched_tokens (tokens routed to at least one local expert). E <= 240.
- *   workspace: pt_moe_permute_workspace_bytes(T, E) bytes, contents irrelevant. Three launches, no host
+ *   workspace: pt_moe_permute_workspace_bytes(T, E) bytes, contents irrelevant. One launch for top-k
+ *   indices of at most 4096 tokens, 16 choices and 128 experts, three otherwise; no host
  *   synchronisation, no inter-block waiting.
  * pt_moe_permute: copies token rows (hidden_bytes each, a multiple of 16) to their destination rows
  *   and writes the zero pad rows; optional per-token scale factors (scale_bytes_per_token raw bytes)

@@ -15,7 +15,8 @@
 // The reference finds each token's rank with a single-pass decoupled look-back scan whose blocks
 // spin on each other's tile states. Here the scan is three short launches (per-block counts,
 // one-block prefix, row map) without any inter-block waiting: the maps are a few MB against the
-// GBs the permute moves, and no launch can hang on another block's progress.
+// GBs the permute moves, and no launch can hang on another block's progress. The top-k indices of a
+// micro-batch take one launch (moe_map_small_kernel).
 // Differences: rows of `tokens` are real for every t < T (the reference treats rows at and after
 // the number of routed tokens as padding, which agrees when every token is routed, the case its
 // tests cover), and unpermute writes zeros for tokens routed nowhere instead of leaving them unwritten.
@@ -91,6 +92,31 @@ __device__ __forceinline__ void wave_counts(const uint8_t *s_flag, int *s_wcnt, 
     __syncthreads();
 }
 
+// [first, first + rows) of the map, all zero: entries that no token uses read as zero. (A workgroup clears the rows
+// that it fills itself and meets at a barrier before it does.)
+__device__ __forceinline__ void clear_rows(int *row_id_map, int64_t first, int64_t rows, int E) {
+    int          *p = row_id_map + first * (2 * E + 1);
+    const int64_t n = rows * (2 * E + 1);
+    for (int64_t i = threadIdx.x; i < n; i += 256)
+        p[i] = 0;
+}
+
+// row i of the zero rows: the i-th padding row of every expert that has one
+__device__ __forceinline__ void pad_row(int *row, int i, int E, const int *tot, const int *first, const int *npad, int64_t npt) {
+    int n = 0;
+    for (int e = 0; e < E; ++e) {
+        if (i >= npad[e])
+            continue;
+        const int64_t off = static_cast<int64_t>(tot[e]) + first[e] + i + 1;
+        if (off > npt)
+            continue;
+        row[n]     = -static_cast<int>(off);
+        row[E + n] = e;
+        ++n;
+    }
+    row[2 * E] = n;
+}
+
 template <typename MapT>
 __global__ __launch_bounds__(256) void moe_count_kernel(const MapT *__restrict__ map, int64_t T, int E, int K,
                                                         int *__restrict__ counts) {
@@ -112,6 +138,7 @@ __global__ __launch_bounds__(256) void moe_scan_kernel(int *__restrict__ counts,
                                                        int *__restrict__ row_id_map, int *__restrict__ overflow_flag,
                                                        int *__restrict__ num_dispatched) {
     __shared__ int s_tot[MAX_E + 1], s_pref[MAX_E + 1], s_npad[MAX_E + 1];
+    clear_rows(row_id_map, T, pad_multiple, E);
     for (int e = threadIdx.x; e <= E; e += 256) {
         int run = 0;
         for (int b = 0; b < nb; ++b) {
@@ -140,21 +167,8 @@ __global__ __launch_bounds__(256) void moe_scan_kernel(int *__restrict__ counts,
     }
     __syncthreads();
     const int stride = 2 * E + 1;
-    for (int i = threadIdx.x; i < pad_multiple; i += 256) {
-        int *row = row_id_map + (T + i) * stride;
-        int  n   = 0;
-        for (int e = 0; e < E; ++e) {
-            if (i >= s_npad[e])
-                continue;
-            const int64_t off = static_cast<int64_t>(s_tot[e]) + s_pref[e] + i + 1;
-            if (off > npt)
-                continue;
-            row[n]     = -static_cast<int>(off);
-            row[E + n] = e;
-            ++n;
-        }
-        row[2 * E] = n;
-    }
+    for (int i = threadIdx.x; i < pad_multiple; i += 256)
+        pad_row(row_id_map + (T + i) * stride, i, E, s_tot, s_pref, s_npad, npt);
 }
 
 // Bound by the chain of its loop over the experts. With top-k aligned slots the slot comes with the flag
@@ -170,6 +184,7 @@ __global__ __launch_bounds__(256) void moe_rowmap_kernel(const MapT *__restrict_
     int     *s_wcnt = reinterpret_cast<int *>(lds + TOK * E);
     const int64_t tok0 = blockIdx.x * static_cast<int64_t>(TOK);
     const bool    slots = sizeof(MapT) != 1 && topk_aligned && K <= 255;
+    clear_rows(row_id_map, tok0, T - tok0 < TOK ? T - tok0 : TOK, E);
     if (slots)
         fill_slots(s_flag, map, tok0, T, E, K);
     else
@@ -208,6 +223,137 @@ __global__ __launch_bounds__(256) void moe_rowmap_kernel(const MapT *__restrict_
         row[n]     = static_cast<int>(dest);
         row[E + n] = aux;
         ++n;
+    }
+    if (gt < T)
+        row[2 * E] = n;
+}
+
+constexpr int SMALL_T = 4096, SMALL_E = 128, SMALL_K = 16;
+
+// The whole map in one launch, for the top-k indices of a micro-batch (up to 4096 tokens, 16 choices, 128 local
+// experts): every workgroup counts all tokens by itself, so none waits for another's counts, and fills the rows of
+// its 256 tokens; those behind the last token's do the padding rows. All of it is latency: count, prefix, map and
+// the clearing of two tensors took five launches and 46 us for 1024 tokens x 8 of 32 experts, one workgroup's
+// counting of 4096 tokens is 16 rounds of LDS atomics. Beyond that the counting is worth splitting (above).
+// Grid: cdiv(T, 256) + cdiv(pad_multiple, 256).
+template <typename MapT>
+__global__ __launch_bounds__(256) void moe_map_small_kernel(const MapT *__restrict__ map, int T, int E, int K, int pad_multiple,
+                                                            int64_t npt, int topk_aligned, int64_t *__restrict__ tokens_per_expert,
+                                                            int *__restrict__ row_id_map, int *__restrict__ overflow_flag,
+                                                            int *__restrict__ num_dispatched) {
+    extern __shared__ uint8_t lds[];
+    uint8_t           *s_flag = lds;
+    int               *s_wcnt = reinterpret_cast<int *>(lds + TOK * E);
+    __shared__ int     s_tot[SMALL_E], s_before[SMALL_E], s_first[SMALL_E], s_npad[SMALL_E], s_any;
+    __shared__ int64_t s_sum[256];
+    const int t = threadIdx.x, tok0 = blockIdx.x * TOK, blocks = (T + TOK - 1) / TOK;
+    const int pad0 = (static_cast<int>(blockIdx.x) - blocks) * 256;
+    if (pad0 < 0)
+        clear_rows(row_id_map, tok0, T - tok0 < TOK ? T - tok0 : TOK, E);
+    else
+        clear_rows(row_id_map, static_cast<int64_t>(T) + pad0, pad_multiple - pad0 < 256 ? pad_multiple - pad0 : 256, E);
+    if (t < E)
+        s_tot[t] = s_before[t] = 0;
+    if (t == 0)
+        s_any = 0;
+    __syncthreads();
+    // ---- tokens of every expert, and those ahead of this workgroup's ----
+    int any = 0;
+    for (int tok = t; tok < T; tok += 256) {
+        int idx[SMALL_K];
+#pragma unroll
+        for (int k = 0; k < SMALL_K; ++k) {
+            idx[k] = -1;
+            if (k < K) {
+                const int64_t e = static_cast<int64_t>(map[static_cast<int64_t>(tok) * K + k]);
+                idx[k]          = e >= 0 && e < E ? static_cast<int>(e) : -1;
+            }
+        }
+        bool routed = false;
+#pragma unroll
+        for (int k = 0; k < SMALL_K; ++k) {
+            bool count = idx[k] >= 0; // (an expert named twice by one token counts once)
+#pragma unroll
+            for (int k2 = 0; k2 < k; ++k2)
+                count = count && idx[k2] != idx[k];
+            if (count) {
+                atomicAdd(&s_tot[idx[k]], 1);
+                if (tok < tok0)
+                    atomicAdd(&s_before[idx[k]], 1);
+            }
+            routed = routed || count;
+        }
+        any += routed;
+    }
+    atomicAdd(&s_any, any);
+    __syncthreads();
+    // ---- first row of every expert ----
+    const int v      = t < E ? s_tot[t] : 0;
+    const int padded = pad_multiple > 0 ? (v + pad_multiple - 1) / pad_multiple * pad_multiple : v;
+    s_sum[t]         = padded;
+    __syncthreads();
+    for (int d = 1; d < E; d <<= 1) {
+        const int64_t add = t >= d ? s_sum[t - d] : 0;
+        __syncthreads();
+        s_sum[t] += add;
+        __syncthreads();
+    }
+    if (t < E) {
+        const int64_t prefix = s_sum[t] - padded;
+        s_first[t]           = static_cast<int>(prefix);
+        s_npad[t]            = padded - v;
+        if (blockIdx.x == 0) {
+            const int64_t over   = s_sum[t] - npt;
+            tokens_per_expert[t] = over < 0 ? padded : (padded - over > 0 ? padded - over : 0);
+            if (t == E - 1)
+                *overflow_flag = s_sum[t] > npt ? 1 : 0;
+            if (t == 0)
+                *num_dispatched = s_any;
+        }
+    }
+    __syncthreads();
+    if (pad0 >= 0) {
+        if (pad0 + t < pad_multiple)
+            pad_row(row_id_map + (static_cast<int64_t>(T) + pad0 + t) * (2 * E + 1), pad0 + t, E, s_tot, s_first, s_npad, npt);
+        return;
+    }
+    // ---- the rows of this workgroup's tokens ----
+    if (topk_aligned)
+        fill_slots(s_flag, map, tok0, T, E, K);
+    else
+        fill_flags(s_flag, map, tok0, T, E, K);
+    wave_counts(s_flag, s_wcnt, E);
+    if (t < E) { // in place: the counts of an expert's wavefronts -> the first row of each
+        int run = s_first[t] + s_before[t];
+        for (int w = 0; w < 4; ++w) {
+            const int c       = s_wcnt[t * 4 + w];
+            s_wcnt[t * 4 + w] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    const int w = t >> 6, lane = t & 63, gt = tok0 + t;
+    int      *row = row_id_map + static_cast<int64_t>(gt < T ? gt : 0) * (2 * E + 1);
+    int       n   = 0;
+    constexpr int STEP = 8; // experts whose flags and first rows are read together
+    for (int e0 = 0; e0 < E; e0 += STEP) {
+        int f[STEP], first[STEP];
+#pragma unroll
+        for (int q = 0; q < STEP; ++q) {
+            const int e = e0 + q < E ? e0 + q : E - 1;
+            f[q]        = e0 + q < E ? s_flag[e * TOK + t] : 0;
+            first[q]    = s_wcnt[e * 4 + w];
+        }
+#pragma unroll
+        for (int q = 0; q < STEP; ++q) {
+            const uint64_t mask = __ballot(f[q]);
+            const int64_t  dest = static_cast<int64_t>(first[q]) + __popcll(mask & ((1ull << lane) - 1ull)) + 1;
+            if (f[q] && dest <= npt) {
+                row[n]     = static_cast<int>(dest);
+                row[E + n] = topk_aligned ? f[q] - 1 : e0 + q;
+                ++n;
+            }
+        }
     }
     if (gt < T)
         row[2 * E] = n;
@@ -362,6 +508,19 @@ int pt_moe_permute_preprocess(const void *expert_map, int map_kind, int64_t num_
     int          *pref   = counts + static_cast<int64_t>(nb) * (E + 1);
     auto          st     = static_cast<hipStream_t>(stream);
     const size_t  lds    = preprocess_lds(E);
+    if (map_kind != 0 && num_tokens <= SMALL_T && E <= SMALL_E && K <= SMALL_K && pad_multiple <= SMALL_T) {
+        const int      T = static_cast<int>(num_tokens), pad = static_cast<int>(pad_multiple);
+        const unsigned blocks = static_cast<unsigned>(nb + cdiv(pad_multiple, 256));
+        if (map_kind == 1)
+            moe_map_small_kernel<int32_t><<<blocks, 256, lds, st>>>(static_cast<const int32_t *>(expert_map), T, E, K, pad, npt,
+                                                                    topk_aligned_probs, tokens_per_expert, row_id_map,
+                                                                    overflow_flag, num_dispatched_tokens);
+        else
+            moe_map_small_kernel<int64_t><<<blocks, 256, lds, st>>>(static_cast<const int64_t *>(expert_map), T, E, K, pad, npt,
+                                                                    topk_aligned_probs, tokens_per_expert, row_id_map,
+                                                                    overflow_flag, num_dispatched_tokens);
+        return check_launch("moe_map_small_kernel");
+    }
 #define PT_MOE_MAP(KERNEL, ...)                                                                                           \
     do {                                                                                                                  \
         if (map_kind == 0)                                                                                                \

@@ -30,11 +30,11 @@ _lib.define(
 
 def _preprocessing_outputs(expert_map, num_local_experts, pad_multiple):
     dev, T = expert_map.device, expert_map.shape[0]
-    # entries that no token uses stay zero (the reference leaves them uninitialised)
-    row_id_map = torch.zeros((T + pad_multiple, 2 * num_local_experts + 1), dtype=torch.int32, device=dev)
+    # entries that no token uses are written as zero (the reference leaves them uninitialised)
+    row_id_map = torch.empty((T + pad_multiple, 2 * num_local_experts + 1), dtype=torch.int32, device=dev)
     tokens_per_expert = torch.empty((num_local_experts,), dtype=torch.int64, device=dev)
     overflow_flag = torch.empty((1,), dtype=torch.int32, device=dev)
-    num_dispatched = torch.zeros((1,), dtype=torch.int32, device=dev)
+    num_dispatched = torch.empty((1,), dtype=torch.int32, device=dev)
     return row_id_map, tokens_per_expert, overflow_flag, num_dispatched
 
 

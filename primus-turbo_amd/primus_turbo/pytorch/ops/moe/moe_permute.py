@@ -56,6 +56,8 @@ class _MoEPermute(torch.autograd.Function):
                          out_probs, row_id_map, num_dispatched, pad_multiple, num_local_experts, hidden,
                          scales_per_token, use_fp8, probs is not None, rows, stride)
         ctx.save_for_backward(row_id_map, num_dispatched)
+        ctx.shape = (int(out.shape[0]), tokens.dtype)
+        ctx.set_materialize_grads(False)  # (a fill of each integer output's "gradient", map included, otherwise)
         ctx.mark_non_differentiable(row_id_map, tokens_per_expert, overflow_flag, num_dispatched)
         if out_sf is not None:
             ctx.mark_non_differentiable(out_sf)
@@ -66,10 +68,15 @@ class _MoEPermute(torch.autograd.Function):
         T, hidden, E, use_fp8, with_probs, probs_dtype, stride, row_width = ctx.meta
         assert not use_fp8, "_MoEPermute.backward: FP8 backward not supported"
         row_id_map, num_dispatched = ctx.saved_tensors
+        rows, dtype = ctx.shape
+        if grad_permuted is None:  # only the probabilities were used
+            grad_permuted = torch.zeros((rows, hidden), dtype=dtype, device=row_id_map.device)
         grad_permuted = grad_permuted.contiguous()
         grad_tokens = torch.empty((T, hidden), dtype=grad_permuted.dtype, device=grad_permuted.device)
         grad_probs = None
-        if with_probs and grad_permuted_probs is not None:
+        if with_probs:
+            if grad_permuted_probs is None:
+                grad_permuted_probs = torch.zeros((rows,), dtype=probs_dtype, device=row_id_map.device)
             grad_permuted_probs = grad_permuted_probs.contiguous()
             grad_probs = torch.empty((T, row_width), dtype=probs_dtype, device=grad_permuted.device)
         else:

@@ -227,3 +227,35 @@ def test_half_precision_probs(layout):
                                         permuted_probs=out_p, probs_topk_stride=stride, pad_multiple=pad)
     _, want_back = P.unpermute(np.zeros((int(tpe.sum()), 1), np.float32), rmap, E, T, want_p, stride if stride else E)
     assert back_p.dtype == torch.bfloat16 and np.array_equal(_bits(back_p), want_back)
+
+
+@pytest.mark.parametrize("T,E,K,pad", [(1, 1, 1, 0), (1, 128, 16, 300), (255, 7, 3, 1), (256, 128, 16, 128), (257, 33, 8, 32),
+                                       (1024, 32, 8, 128), (4096, 128, 16, 256), (4096, 129, 2, 16), (4097, 128, 2, 16), (64, 16, 17, 8)])
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("aligned", [False, True])
+@pytest.mark.parametrize("limit", [-1, 100])
+def test_map_in_one_launch(T, E, K, pad, dtype, aligned, limit):
+    """The launch that makes the whole map, up to 4096 tokens, 128 experts and 16 choices, and one beyond each;
+    with repeated and out-of-range choices and a cap on the rows. No entry is left as the allocation had it."""
+    emap = np.random.default_rng(T + K).integers(-2, E + 2, (T, K)).astype(dtype)
+    junk = torch.full((4 * (T + pad) * (2 * E + 1),), 0x7F, dtype=torch.uint8, device="cuda")
+    del junk  # (the map is likely to take its memory)
+    got = ext.permute_preprocessing(torch.from_numpy(emap).cuda(), E, K, pad, limit, K if aligned else 0)
+    rmap, tpe, overflow, nd = P.preprocess(emap, E, pad, topk_aligned_probs=aligned, num_permuted_tokens=limit)
+    assert np.array_equal(got[0].cpu().numpy(), rmap)
+    assert np.array_equal(got[1].cpu().numpy(), tpe)
+    assert int(got[2].item()) == overflow and int(got[3].item()) == nd
+
+
+@pytest.mark.parametrize("use", ["tokens", "probs", "both"])
+def test_gradients_of_unused_outputs(use):
+    """An output that the loss does not use sends a zero gradient back, not none."""
+    T, E, K, H = 37, 4, 2, 64
+    emap = torch.from_numpy(_topk(_routing(T, E, K, 1), K, np.int64, 2)).cuda()
+    tokens = torch.randn(T, H, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    probs = torch.rand(T, K, device="cuda", requires_grad=True)
+    out, *_, out_p = turbo.ops.moe_permute(tokens, emap, num_local_experts=E, num_topk=K, probs=probs, probs_layout="topk")
+    loss = (out.float().sum() if use != "probs" else 0) + (out_p.sum() if use != "tokens" else 0)
+    loss.backward()
+    assert torch.equal(tokens.grad, torch.full_like(tokens, 0.0 if use == "probs" else K))
+    assert torch.equal(probs.grad, torch.full_like(probs, 0.0 if use == "tokens" else 1.0))
