@@ -225,9 +225,9 @@ constexpr int        DIRECT_COUNT   = sizeof(DIRECT_TILES) / sizeof(DIRECT_TILES
 //   cost 2 (16 rows) 17.4 -> 6.5, 4 (64 rows) 18.0 -> 10.0, 6 (128 rows) 18.3 -> 14.4, 8 (256 rows) 18.5 -> 18.2
 // (64 x 64 tiles; the tiled kernel with four stages: 15.4). Short products pay for the tiled kernel's long
 // start as well: 300 x 2880 x 512, cost 8, 6.2 -> 5.9. Block scales fold each product in the VALU, which the
-// tiled kernel cannot hide with one wavefront per SIMD: there cost 8 pays at any length (24.9 -> 19.0, and
-// 1024 x 1024 x 16384 84.8 -> 60.6). MXFP4 has half the matrix time for the same bytes (16 slabs 19.9 -> 18.8,
-// but 64 slabs 50.5 -> 59.7). Cost 16 loses everywhere (512 rows: 19.4 against 33.6).
+// tiled kernel hides with its two teams only in part: there cost 8 pays at any length (20.6 -> 19.8, a scale per
+// column 22.2 -> 20.8, 1024 x 1024 x 16384 61.4 -> 61.0). MXFP4 has half the matrix time for the same bytes (16
+// slabs 13.6 -> 13.2, but 32 slabs 21.1 -> 21.8). Cost 16 loses everywhere (512 rows: 19.4 against 33.6).
 static inline int direct_tile(int64_t M, int64_t N, int64_t slabs, int mode, bool fp4) {
     int     best = -1;
     int64_t least = 0;
@@ -240,7 +240,7 @@ static inline int direct_tile(int64_t M, int64_t N, int64_t slabs, int mode, boo
             least = cost;
         }
     }
-    const bool cost8_pays = mode == SCALE_BLOCK || slabs <= (fp4 ? 32 : 8);
+    const bool cost8_pays = mode == SCALE_BLOCK || slabs <= (fp4 ? 16 : 8);
     return least <= 6 || (least <= 8 && cost8_pays) ? best : -1;
 }
 

@@ -20,13 +20,11 @@ static int launch_block_tiles(const GemmArgs &a, int tile_cfg, hipStream_t strea
     if (tile_cfg == 1 || tile_cfg == 4)
         return launch_gemm_block8<FA, FB, GROUP_NONE, SB_VEC>(a, stream);
     if constexpr (!SB_VEC) {
-        if (tile_cfg == 3 && one_tile_per_cu(a.M, a.N))
-            return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB, GROUP_NONE, 4>(a, stream);
-    }
-    if constexpr (!SB_VEC) {
         if (tile_cfg == 2)
             return launch_gemm_cfg<8, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
     }
+    if (two_teams(SCALE_BLOCK, a.M, a.N, a.K / KSTEP))
+        return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB, GROUP_NONE, 2, 2>(a, stream);
     return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
 }
 

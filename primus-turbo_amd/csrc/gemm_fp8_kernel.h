@@ -821,8 +821,13 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 //   * tile boundaries do not drain the pipeline: while a tile's result is written out, the
 //     fragments of the next tile's first slab are already in registers and its second slab is
 //     in flight.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE>
-__global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
+//
+// KS = 2: eight wavefronts, the slabs shared out to two teams of four in turn, each with stages of its own; at the
+// end the teams exchange half their sums through the LDS, and each writes half the tile. For dense products of at
+// most one tile a CU, where no second workgroup could hide the waits (see two_teams).
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS>
+__global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a) {
+    static_assert(KS == 1 || (KS == 2 && GMODE == GROUP_NONE), "teams: dense products, one tile for each workgroup");
     static_assert(TN % 4 == 0 && TM % 4 == 0, "sub-tiles are multiples of 64 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -866,8 +871,10 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
 
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int team = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wave = __builtin_amdgcn_readfirstlane(KS == 1 ? tid >> 6 : (tid >> 6) & 3);
     const int wm = wave >> 1, wn = wave & 1; // wavefront position in the 2 x 2 grid
+    uint8_t *const stages = KS == 1 ? smem : smem + team * (NSTAGE * STAGE);
     const int lm = lane & 15, lg = lane >> 4;
 
     // byte offsets of this lane's two 16-byte fragment reads within a 16-row group
@@ -989,26 +996,30 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
     };
     TileCtx nxt_t     = cur_t; // tile after the MFMAs' tile (the same tile after the last one)
     auto    loader_to = [&](const TileCtx &t) {
-        ld_ga = t.Ag;
-        ld_gb = t.Bg;
-        ld_na = t.rows_a * static_cast<uint32_t>(a.lda);
-        ld_nb = t.rows_b * static_cast<uint32_t>(a.ldb);
-        ld_kt = 0;
+        ld_ga = t.Ag + team * KSTEP;
+        ld_gb = t.Bg + team * KSTEP;
+        ld_na = t.rows_a * static_cast<uint32_t>(a.lda) - team * KSTEP;
+        ld_nb = t.rows_b * static_cast<uint32_t>(a.ldb) - team * KSTEP;
+        ld_kt = team;
         ld_KT = t.KT;
         scales_to(t);
+        if constexpr (LDS_SC && KS > 1) {
+            ld_sa += team * sa_step;
+            ld_sb += team * sb_step;
+        }
     };
     // bytes a scale copy may read: none for a slab of zero padding beyond the K blocks the
     // arrays hold (whatever lies there must not meet the matrix core: an E8M0 NaN would stick)
     [[maybe_unused]] auto bytes_left = [&](const uint8_t *p, const uint8_t *end, int h) {
         const int64_t n     = end - p;
-        const bool    valid = GMODE == GROUP_K || (MODE == SCALE_MX ? (ld_kt * NW + h) * 4 : ld_kt) < a.kb_valid;
+        const bool    valid = (KS == 1 || ld_kt < KT_ALL) && (GMODE == GROUP_K || (MODE == SCALE_MX ? (ld_kt * NW + h) * 4 : ld_kt) < a.kb_valid);
         return (n <= 0 || !valid) ? 0u : (n > 0x7fffffff ? 0x7fffffffu : static_cast<uint32_t>(n));
     };
     // copy number L of the loader's slab into stage `b`: [0, LA) A rows, [LA, NLD) B rows,
     // [NLD, NL) scale words
     auto issue_copy = [&](auto lc, int b) {
         constexpr int L   = lc;
-        uint8_t      *dst = smem + b * STAGE;
+        uint8_t      *dst = stages + b * STAGE;
 #if defined(__HIP_DEVICE_COMPILE__) // the buffer resource type only exists in the device pass
         constexpr uint32_t RSRC_FLAGS = 0x00020000; // raw buffer, 32-bit data format
         if constexpr (L >= NLD) {
@@ -1034,7 +1045,20 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
         issue_copy(std::integral_constant<int, (C < LB ? LA + C : NLD + (C - LB))>{}, b);
     };
     auto advance_loader = [&]() {
-        if constexpr (XPIPE) {
+        if constexpr (KS > 1) {
+            // behind the last slab nothing is read: the stages fill with zeros (as they do for the slab that a
+            // team has more than the other)
+            ld_kt += KS;
+            const bool in = ld_kt < KT_ALL;
+            ld_ga += KS * KSTEP;
+            ld_gb += KS * KSTEP;
+            ld_na = in ? ld_na - KS * KSTEP : 0;
+            ld_nb = in ? ld_nb - KS * KSTEP : 0;
+            if constexpr (LDS_SC) {
+                ld_sa += KS * sa_step;
+                ld_sb += KS * sb_step;
+            }
+        } else if constexpr (XPIPE) {
             const bool wrap = ld_kt + 1 == KT_ALL;
             ld_kt = wrap ? 0 : ld_kt + 1;
             ld_ga = wrap ? nxt_t.Ag : ld_ga + KSTEP;
@@ -1138,13 +1162,13 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AHEAD - 1) * NL) : "memory");
         __builtin_amdgcn_s_barrier();
         buf = 0;
-        read_scales(smem);
+        read_scales(stages);
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            fb[j] = ldfrag(smem + b_part, j);
+            fb[j] = ldfrag(stages + b_part, j);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-            fa[i] = ldfrag(smem + a_part, i);
+            fa[i] = ldfrag(stages + a_part, i);
     };
     // Stores of the result tile a wavefront has just written that may still be in flight (0, or the
     // count of the straight-line epilogue for 16-bit / fp32 outputs). They are younger than the
@@ -1174,7 +1198,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
         nxt_t               = cur_t;
         if (next_tile < total)
             nxt_t = make_tile<BM, BN, GMODE, FA == 4>(a, next_tile, prefix, g_nxt);
-        const int KT = XPIPE ? KT_ALL : cur_t.KT;
+        const int KT = XPIPE ? (KT_ALL + KS - 1) / KS : cur_t.KT;
         if constexpr (!XPIPE) {
             if (KT > 0)
                 take_first_slab(); // requested before the loop or before the previous tile's epilogue
@@ -1186,7 +1210,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
         auto run_slabs = [&](const int n_slabs) {
         for (int kt = 0; kt < n_slabs; ++kt) {
             const int      buf_n = buf + 1 == NSTAGE ? 0 : buf + 1;
-            const uint8_t *nxt   = smem + buf_n * STAGE;
+            const uint8_t *nxt   = stages + buf_n * STAGE;
             // where the slab two steps ahead goes: the current stage (after barrier X), or with
             // three stages the one that was current a slab ago
             const int      buf_w = NSTAGE == 2 ? buf : (buf == 0 ? NSTAGE - 1 : buf - 1);
@@ -1351,7 +1375,36 @@ __global__ __launch_bounds__(256) void gemm_fp8_nt_kernel(const GemmArgs a) {
         }
         };
         const int64_t wm_base = cur_t.m0 + wm * (TM * 16), wn_base = cur_t.n0 + wn * (TN * 16);
-        if constexpr (XPIPE) {
+        if constexpr (KS > 1) {
+            static_assert(8 * TM / 2 * TN * 1024 <= KS * NSTAGE * STAGE, "the exchanged sums fit the stages");
+            run_slabs(KT);
+            if constexpr (MODE != SCALE_BLOCK)
+                asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // (copies of slabs that do not exist, too)
+            __builtin_amdgcn_s_barrier();
+            // team 0 finishes the upper rows of every wavefront's sub-tile, team 1 the lower ones
+            constexpr int HM = TM / 2;
+            f32x4         sum[HM][TN];
+            f32x4        *give = reinterpret_cast<f32x4 *>(smem) + (team * 4 + wave) * (HM * TN * 64) + lane;
+            const f32x4  *take = reinterpret_cast<const f32x4 *>(smem) + ((team ^ 1) * 4 + wave) * (HM * TN * 64) + lane;
+#pragma unroll
+            for (int i = 0; i < HM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const f32x4 up = read_acc<MODE != SCALE_BLOCK>(acc[i][j]), low = read_acc<MODE != SCALE_BLOCK>(acc[HM + i][j]);
+                    give[(i * TN + j) * 64] = team ? up : low;
+                    sum[i][j]               = team ? low : up;
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+#pragma unroll
+            for (int i = 0; i < HM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    sum[i][j] += take[(i * TN + j) * 64];
+            epilogue<HM, TN, MODE, false, true, MODE != SCALE_BLOCK, PIECES_APART>(a, sum, cur_t.C, cur_t.sA, cur_t.sB, cur_t.m_end,
+                                                                                  wm_base + team * (HM * 16), wn_base, lane);
+        } else if constexpr (XPIPE) {
             run_slabs(KT);
             PT_GEMM_TRACE_POINT(4);
             // the epilogue reads the accumulators with hand-written instructions the compiler's
@@ -1429,10 +1482,10 @@ static inline int vk_pick_chunks(int64_t positions, int64_t grid, int64_t groups
 
 // Upper bound on the number of tiles (exact for the ungrouped case): GROUP_ROWS cannot know
 // the per-group row counts on the host, but every group adds at most one partial tile row.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4)>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4), int KS = 1>
 static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
-    constexpr int STAGES  = NSTAGE * gemm_stage_bytes(TM, TN, MODE, FA == 4);
+    constexpr int STAGES  = KS * NSTAGE * gemm_stage_bytes(TM, TN, MODE, FA == 4);
     // groups whose tile prefix sums fit into the LDS next to the stages
     constexpr int MAX_G   = (160 * 1024 - STAGES) / 4 - 2 < 2048 ? 1024 : 2048;
     constexpr int LDS_MAX = STAGES + (GMODE == GROUP_ROWS ? (MAX_G + 2) * 4 : GMODE == GROUP_K ? (VK_MAX_CHUNKS + 2) * 4 : 0);
@@ -1450,7 +1503,7 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
                              (a.sb_wpitch == 0 && a.sb_n % 4 != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
                              reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
-    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE>;
+    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE, KS>;
     // the attribute belongs to the (kernel, device) pair: one bit per device, set once
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
@@ -1477,24 +1530,36 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     } else {
         total = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
     }
-    if (grid > total)
+    if (grid > total || KS > 1) // (teams: a tile for each workgroup)
         grid = total;
     if (grid <= 0)
         return PT_OK;
-    kern<<<static_cast<unsigned>(grid), 256, lds, stream>>>(a);
+    kern<<<static_cast<unsigned>(grid), 256 * KS, lds, stream>>>(a);
     return check_launch("gemm_fp8_nt_kernel");
 }
 
 // ---- host helpers shared by the translation units that instantiate the kernel ----
 // 128 x 128 tiles, at most one for each CU: the second workgroup that would share a CU, and hide this one's
-// waits, does not exist, so the LDS it would have held goes into four stages and the copies run three slabs
-// ahead instead of two. 777 x 4096 x 7168 (224 tiles, 56 slabs), vector scales: 42.6 us with two stages, 28.8
-// with four; 256 x 4096 x 4096 18.5 -> 15.4. With more tiles than CUs two workgroups on two stages each are the
-// better use of the LDS: 1400 x 4096 x 4096 (352 tiles) 28.7 us, with four stages 31.6. MXFP8 777 x 4096 x 7168
-// 54.3 -> 45.1, block scales 46.2 -> 41.5; no gain, and two stages, for vectors of scales on both operands (51.2
-// against 50.0) and MXFP4 (1024 x 1024 x 16384 50.3 against 52.9), whose slabs take longer to issue than to fetch.
+// waits, does not exist. With vector scales the LDS it would have held goes into four stages and the copies run
+// three slabs ahead instead of two: 777 x 4096 x 7168 (224 tiles, 56 slabs) 42.0 -> 29.8 us, 256 x 4096 x 4096 18.2
+// -> 15.3. With more tiles than CUs two workgroups on two stages each are the better use of the LDS: 1400 x 4096 x
+// 4096 (352 tiles) 28.7 us, with four stages 31.6.
 static inline bool one_tile_per_cu(int64_t M, int64_t N) {
     return (M + 127) / 128 * ((N + 127) / 128) <= device_cu_count();
+}
+// Where a slab takes a SIMD's one wavefront longer to issue than to fetch, two teams of four wavefronts share out
+// the slabs (KS = 2 of the kernel) and work while the other waits, each on two stages of its own. us, 777 x 4096 x
+// 7168 / 2048 x 2048 x 8192 / 256 x 4096 x 4096 / 1000 x 2048 x 2048:
+//    block scales             four stages 42.7 / 48.4 / 24.6 / 15.1    teams 34.4 / 38.9 / 19.7 / 12.8
+//      a scale per column      two stages 50.6 / 56.6 / 30.3 / 17.7          38.5 / 43.2 / 22.4 / 14.4
+//    MXFP8                    four stages 36.8 / 38.3 / 20.6 / 13.0          35.4 / 34.5 / 18.6 / 12.3
+//    MXFP4                     two stages 24.4 / 26.4 / 15.0 / 10.0          21.0 / 23.6 / 13.6 /  9.9
+//    vector scales            four stages 29.8 / 33.2 / 15.3 / 10.9          32.2 / 34.4 / 15.5 / 11.2
+// The exchange of the sums at the end costs what it saves where K is short (MXFP8 1024 x 4096 x 1024, two stages /
+// teams 9.4 / 9.7, MXFP4 8.0 / 8.5; block scales, whose sums cost more to make, gain from K = 512 on: 10.4 / 9.8).
+// The error against 64 bits is that of one sum: 777 x 4096 x 7168 1.500e-5 rms either way, the matrix core's own.
+static inline bool two_teams(int mode, int64_t M, int64_t N, int64_t slabs) {
+    return mode != SCALE_VECTOR && one_tile_per_cu(M, N) && (mode == SCALE_BLOCK || slabs >= 16);
 }
 // The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128. A large tile multiplies more for each
 // byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
