@@ -189,6 +189,36 @@ def test_grouped_mx_eight_wavefront_tile(kind, G_, M, N, K, padded):
     assert torch.equal(got, auto)
 
 
+@pytest.mark.parametrize("rows", [383, 384, 447, 448])  # where the tile changes (MXFP8, MXFP4)
+@pytest.mark.parametrize("N", [1000, 1024, 1184])
+@pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
+def test_tile_of_mid_size_groups(fmt, rows, N):
+    """The automatic tile gives the bits of the pinned ones, uneven groups and an empty one included."""
+    from primus_turbo.pytorch.kernels.grouped_gemm import grouped_gemm_fp4_impl as gimpl4
+
+    K, lens = 768, np.array([0, 3 * rows - 130, 130, rows], dtype=np.int64)
+    gl, offs = _offs(lens)
+    x, w = bf16_randn((int(lens.sum()), K), seed=146).cuda(), bf16_randn((4, N, K), seed=147).cuda()
+    quant = qimpl.quantize_mxfp8_impl if fmt == "e4m3" else qimpl.quantize_mxfp4_impl
+    dt = torch.float8_e4m3fn if fmt == "e4m3" else torch.float4_e2m1fn_x2
+    wq, ws = quant(w, dt, 2, 32, scaling_recipe=ScalingRecipe(use_2d_block=True))
+    if fmt == "e4m3":
+        xq, xs, _, orow = qimpl.grouped_quantize_mxfp8_impl(x, dt, 1, 32, gl, offs)
+    else:
+        xq, xs, _, orow = qimpl.grouped_quantize_mxfp4_impl(x, dt, 1, 32, gl, offs)
+    outs = []
+    for tile in (0, 1, 3):
+        gimpl.MX_TILE_CFG = tile
+        try:
+            outs.append(gimpl.grouped_gemm_fp8_impl(xq, wq, xs, ws, gl, orow, False, True, torch.bfloat16, G.MX_BLOCKWISE.value,
+                                                    None, 0, False, offs) if fmt == "e4m3" else
+                        gimpl4.grouped_gemm_fp4_impl(xq, wq, xs, ws, gl, orow, False, True, torch.bfloat16, G.MX_BLOCKWISE.value,
+                                                     None, 0, False, offs))
+        finally:
+            gimpl.MX_TILE_CFG = 0
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @pytest.mark.parametrize("kind,G_,M,N,K", GCASES)
 @pytest.mark.parametrize("trans_c", [False, True])
 def test_grouped_mx_variable_k_product(kind, G_, M, N, K, trans_c):
