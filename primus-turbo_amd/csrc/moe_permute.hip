@@ -233,8 +233,9 @@ constexpr int SMALL_T = 4096, SMALL_E = 128, SMALL_K = 16;
 // The whole map in one launch, for the top-k indices of a micro-batch (up to 4096 tokens, 16 choices, 128 local
 // experts): every workgroup counts all tokens by itself, so none waits for another's counts, and fills the rows of
 // its 256 tokens; those behind the last token's do the padding rows. All of it is latency: count, prefix, map and
-// the clearing of two tensors took five launches and 46 us for 1024 tokens x 8 of 32 experts, one workgroup's
-// counting of 4096 tokens is 16 rounds of LDS atomics. Beyond that the counting is worth splitting (above).
+// the clearing of two tensors took five launches and 46 us for 1024 tokens x 8 of 32 experts, this one takes 19 (24
+// with a second read of the choices for the flags). One workgroup's counting of 4096 tokens is 16 rounds of LDS
+// atomics; beyond that it is worth splitting (above).
 // Grid: cdiv(T, 256) + cdiv(pad_multiple, 256).
 template <typename MapT>
 __global__ __launch_bounds__(256) void moe_map_small_kernel(const MapT *__restrict__ map, int T, int E, int K, int pad_multiple,
@@ -256,34 +257,37 @@ __global__ __launch_bounds__(256) void moe_map_small_kernel(const MapT *__restri
         s_tot[t] = s_before[t] = 0;
     if (t == 0)
         s_any = 0;
+    for (int i = t; i < TOK / 4 * E; i += 256)
+        reinterpret_cast<uint32_t *>(s_flag)[i] = 0;
     __syncthreads();
-    // ---- tokens of every expert, and those ahead of this workgroup's ----
+    // ---- tokens of every expert, and those ahead of this workgroup's; the flags of its own (1, or with top-k
+    // aligned slots 1 + the first slot), each in its thread's column ----
     int any = 0;
     for (int tok = t; tok < T; tok += 256) {
-        int idx[SMALL_K];
+        const MapT *src     = map + static_cast<int64_t>(tok) * K;
+        uint64_t    seen[2] = {0, 0}; // (an expert named twice by one token counts once)
+        for (int k0 = 0; k0 < K; k0 += 8) {
+            MapT v[8];
 #pragma unroll
-        for (int k = 0; k < SMALL_K; ++k) {
-            idx[k] = -1;
-            if (k < K) {
-                const int64_t e = static_cast<int64_t>(map[static_cast<int64_t>(tok) * K + k]);
-                idx[k]          = e >= 0 && e < E ? static_cast<int>(e) : -1;
+            for (int q = 0; q < 8; ++q)
+                v[q] = src[k0 + q < K ? k0 + q : K - 1];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const bool     in  = k0 + q < K && v[q] >= 0 && v[q] < E;
+                const int      e   = in ? static_cast<int>(v[q]) : 0;
+                const uint64_t bit = in ? 1ull << (e & 63) : 0;
+                uint64_t      &had = e < 64 ? seen[0] : seen[1];
+                if ((bit & ~had) != 0) {
+                    had |= bit;
+                    atomicAdd(&s_tot[e], 1);
+                    if (tok < tok0)
+                        atomicAdd(&s_before[e], 1);
+                    if (tok == tok0 + t)
+                        s_flag[e * TOK + t] = static_cast<uint8_t>(topk_aligned ? k0 + q + 1 : 1);
+                }
             }
         }
-        bool routed = false;
-#pragma unroll
-        for (int k = 0; k < SMALL_K; ++k) {
-            bool count = idx[k] >= 0; // (an expert named twice by one token counts once)
-#pragma unroll
-            for (int k2 = 0; k2 < k; ++k2)
-                count = count && idx[k2] != idx[k];
-            if (count) {
-                atomicAdd(&s_tot[idx[k]], 1);
-                if (tok < tok0)
-                    atomicAdd(&s_before[idx[k]], 1);
-            }
-            routed = routed || count;
-        }
-        any += routed;
+        any += (seen[0] | seen[1]) != 0;
     }
     atomicAdd(&s_any, any);
     __syncthreads();
@@ -318,11 +322,21 @@ __global__ __launch_bounds__(256) void moe_map_small_kernel(const MapT *__restri
         return;
     }
     // ---- the rows of this workgroup's tokens ----
-    if (topk_aligned)
-        fill_slots(s_flag, map, tok0, T, E, K);
-    else
-        fill_flags(s_flag, map, tok0, T, E, K);
-    wave_counts(s_flag, s_wcnt, E);
+    const int w = t >> 6, lane = t & 63, gt = tok0 + t;
+    constexpr int STEP = 8; // experts whose flags and first rows are read together
+    for (int e0 = 0; e0 < E; e0 += STEP) {
+        int f[STEP];
+#pragma unroll
+        for (int q = 0; q < STEP; ++q)
+            f[q] = e0 + q < E ? s_flag[(e0 + q) * TOK + t] : 0;
+#pragma unroll
+        for (int q = 0; q < STEP; ++q) {
+            const int c = __popcll(__ballot(f[q]));
+            if (lane == 0 && e0 + q < E)
+                s_wcnt[(e0 + q) * 4 + w] = c;
+        }
+    }
+    __syncthreads();
     if (t < E) { // in place: the counts of an expert's wavefronts -> the first row of each
         int run = s_first[t] + s_before[t];
         for (int w = 0; w < 4; ++w) {
@@ -332,10 +346,8 @@ __global__ __launch_bounds__(256) void moe_map_small_kernel(const MapT *__restri
         }
     }
     __syncthreads();
-    const int w = t >> 6, lane = t & 63, gt = tok0 + t;
-    int      *row = row_id_map + static_cast<int64_t>(gt < T ? gt : 0) * (2 * E + 1);
-    int       n   = 0;
-    constexpr int STEP = 8; // experts whose flags and first rows are read together
+    int *row = row_id_map + static_cast<int64_t>(gt < T ? gt : 0) * (2 * E + 1);
+    int  n   = 0;
     for (int e0 = 0; e0 < E; e0 += STEP) {
         int f[STEP], first[STEP];
 #pragma unroll
