@@ -33,7 +33,7 @@ from primus_turbo.pytorch.core.quantized_tensor import (
     check_quantized_tensor,
     transpose_last_two,
 )
-from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_accum_impl, gemm_fp8_impl
+from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_accum_impl, gemm_fp8_impl, get_gemm_logical_shape
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_t_impl,
     quant_fp8_blockwise_kmajor_impl,
@@ -96,6 +96,8 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         # (rows are padded to whole slabs of the products where both operands of a product are made here, in
         # one launch each: codes in 16-byte groups along K and N)
         plain = not any(isinstance(t, QuantizedTensor) for t in (a, b, a_t, b_t)) and b.shape[0] % 16 == 0 and b.shape[1] % 16 == 0
+        if plain:
+            get_gemm_logical_shape(a, b, trans_a, trans_b)  # (padded to the same length different ones look alike)
 
         def operand(x, x_t):
             want_t = need_bwd and nt_bwd and not isinstance(x_t, QuantizedTensor)
@@ -149,6 +151,8 @@ class FP8GemmRowFunction(torch.autograd.Function):
         # operands made here have rows of whole slabs: no product copies them to pad them
         plain = trans_b and not any(isinstance(t, QuantizedTensor) for t in (a, b))
         K = a.shape[1]
+        if plain:
+            get_gemm_logical_shape(a, b, trans_a, trans_b)  # (padded to the same length different ones look alike)
 
         def along_rows(x, axis):
             if not plain or K % 128 == 0:
