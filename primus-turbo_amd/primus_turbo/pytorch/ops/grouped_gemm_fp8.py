@@ -160,8 +160,9 @@ class FP8GroupedGemmBlockFunc(torch.autograd.Function):
             a_fp8_row, a_fp8_col_t, a_scale_row, a_scale_col, var_k_lens, var_k_offs = (
                 quant_fp8_blockwise_segment_m_row_col_t_impl(a.contiguous(), a_dtype, bs, group_lens, group_offs))
         else:
-            if not all(t.dtype == torch.int64 and t.is_contiguous() for t in (group_lens, group_offs)):
-                raise RuntimeError("group_lens / group_offs must be contiguous int64")
+            if not all(t.dtype == torch.int64 and t.is_contiguous() and t.device.type == a.device.type
+                       for t in (group_lens, group_offs)):
+                raise RuntimeError("group_lens / group_offs must be contiguous int64 on the device of a")
             a_fp8_row, a_scale_row, _, _ = quant_fp8_blockwise_kmajor_impl(a.contiguous(), a_dtype, bs, False)
         out, saved_b, b_ready = _block_forward_product(a_fp8_row, a_scale_row, b, group_lens, group_offs, trans_b, out_dtype,
                                                        config, num_cu, need_bwd)
