@@ -29,7 +29,7 @@ def test_same_bytes_as_two_steps(native_lib, R, C, dtype, fp8, pad):
         assert torch.equal(got_t.view(torch.uint8)[:, :R], q.view(torch.uint8).t()) and not got_t.view(torch.uint8)[:, R:].any()
 
 
-@pytest.mark.parametrize("M,N", [(1, 32), (33, 200), (257, 2880), (40, 9000)])
+@pytest.mark.parametrize("M,N", [(1, 32), (33, 200), (5, 256), (257, 2880), (40, 9000)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_rowwise_rows_are_padded(native_lib, M, N, dtype):
     from primus_turbo.pytorch.kernels.quantization import quantization_impl as impl
