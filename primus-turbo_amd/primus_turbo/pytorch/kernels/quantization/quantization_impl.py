@@ -1622,14 +1622,17 @@ def grouped_quantize_mxfp8_impl(x, out_dtype, axis, block_size, group_lens, grou
     return cq, cs, lc, ocol
 
 
-def grouped_quantize_mx_operands(x, out_dtype, group_lens, group_offs, recipe, recipe_t, what, with_col=True, known=None):
+def grouped_quantize_mx_operands(x, out_dtype, group_lens, group_offs, recipe, recipe_t, what, with_col=True, known=None,
+                                 col_like=None):
     """:func:`quantize_mx_operands` for the packed rows of groups: the eight outputs of
     ``grouped_quantize_mxfp8_impl`` / ``grouped_quantize_mxfp4_impl`` with ``with_trans`` (the column pair None
     without ``with_col``), scales word-major. ``known``: the last four of an earlier call for the same groups,
-    which are then not computed again."""
+    which are then not computed again. ``col_like``: the scales of the operand that the column direction meets; its own
+    come in that layout (the variable-K product reads one layout for both, the others each operand's)."""
     r, rt = _mx_recipes(True, recipe, recipe_t, what)
+    col_words = _MX_WORDS if col_like is None or col_like.dtype == torch.int32 else 0
     return _grouped_mx_quantize(x, out_dtype, group_lens, group_offs, True, with_col, _mx_flags(r) | _MX_WORDS,
-                                _mx_flags(rt) | _MX_WORDS, known)
+                                _mx_flags(rt) | col_words, known)
 
 
 def grouped_dequantize_mxfp8_impl(x, out_dtype, axis, block_size, scale_inv, group_offs, group_offs_padded,

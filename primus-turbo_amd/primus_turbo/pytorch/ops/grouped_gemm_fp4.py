@@ -103,7 +103,7 @@ def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens,
     known = None if offs_col is None else (None, None, lens_col, offs_col)
     g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
         grad_out, float4_e2m1fn_x2, group_lens, group_offs, ScalingRecipe(use_sr=config.use_gradient_sr),
-        ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), "MXFP4", known=known)
+        ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), "MXFP4", known=known, col_like=a_col_s)
     # dgrad: grad_a = grad_out @ b as an NT product with the transposed weight quantization [G, K, N]
     grad_a = grouped_gemm_fp4_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
                                    gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
