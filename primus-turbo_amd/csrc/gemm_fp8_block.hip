@@ -23,7 +23,7 @@ static int launch_block_tiles(const GemmArgs &a, int tile_cfg, hipStream_t strea
         if (tile_cfg == 2)
             return launch_gemm_cfg<8, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
     }
-    if (two_teams(SCALE_BLOCK, a.M, a.N, a.K / KSTEP))
+    if (two_teams(SCALE_BLOCK, SB_VEC, a.M, a.N, a.K / KSTEP))
         return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB, GROUP_NONE, 2, 2>(a, stream);
     return launch_gemm_cfg<4, 4, SCALE_BLOCK, SB_VEC, FA, FB>(a, stream);
 }

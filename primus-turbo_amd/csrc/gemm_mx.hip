@@ -21,7 +21,7 @@ template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile
     }
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_MX, false, FA, FB>(a, stream);
-    if (two_teams(SCALE_MX, a.M, a.N, a.K / KSTEP))
+    if (two_teams(SCALE_MX, false, a.M, a.N, a.K / KSTEP))
         return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB, GROUP_NONE, 2, 2>(a, stream);
     return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB>(a, stream);
 }
