@@ -1565,32 +1565,44 @@ static inline bool two_teams(int mode, bool sb_vec, int64_t M, int64_t N, int64_
 }
 // The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128. A large tile multiplies more for each
 // byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
-// how the tiles divide among the CUs. The time of a round for one slab, in 64ths of what a 256 x 256 tile takes:
-//                     256x256   256x128   2 of 128x128   1 of 128x128     (256 x 256: us)
-//   vector scales        64        36          42             23                1.50
-//   MXFP8                64        37          42             23                1.64
-//   MXFP4                64        38          40             26                2.1 (256 codes)
-//   block scales         64        40          41             27                1.75 (a scale per column 2.0)
-// and a tile spends about the time of two slabs on its first copies and its result, the 256 x 256 one, whose CU has
-// nothing else to do meanwhile, that of three or four. (Medians over products of 26 sizes with every tile, 512 to
-// 28672 wide, K 512 to 8192.) Taking 256 x 256 wherever both sides reach 2048, and 128 x 128 elsewhere, lost 6 to
-// 13 % against the best tile on average: vector scales 2048 x 2048 x 8192 72 us, 128 x 128 32 (MXFP8 82 / 40);
-// 4096 x 2048 x 4096 43.8, 256 x 128 31.1; 16384 x 1024 x 4096 61.5, 256 x 256 51.9. This rule loses 0.3 %, at
-// most 5 %, and nowhere to that one.
-// middle: 256 x 128 may be taken (for MXFP4 and a scale per column it is nowhere more than 3 % ahead).
+// how the tiles divide among the CUs. The time of a launch is taken to be, in 64ths of what a 256 x 256 tile takes for a
+// slab (1.1 us with vector scales, MXFP8 1.25, MXFP4 1.5 for 256 codes, block scales 1.6, a scale per column 1.8),
+//   256 x 256  64 (rounds (slabs + own) + launch)       256 x 128  half rounds (slabs + half_own)
+//   128 x 128  (pair (rounds of two a CU) + single (a last round of at most one a CU)) (slabs + pair_own)
+// with the time of a tile's first copies and result as slabs of its own. The constants are fitted: they are those
+// that lose least against the best tile, measured with every tile for 330 sizes (96 to 28672 wide, K 512 to 16384, odd
+// ones among them) on weights that come from HBM, as a layer's do, and stand for no one time by themselves. Loss on average
+// / products that lose more than 3 %: see the table; "before" is one set of costs for all modes, fitted to weights
+// in the caches, "old" 256 x 256 wherever both sides reach 2048 and 128 x 128 elsewhere.
+//                      now             before            old
+//   vector scales   0.2 %,  9 of 280  0.7 %, 20       5.3 %, 83
+//   MXFP8           0.3 %, 12 of 278  0.5 %, 17       5.0 %, 79
+//   MXFP4           0.2 %,  4 of 258  0.4 %,  9       2.7 %, 37
+//   block scales    0.1 %,  2 of 249  0.6 %, 20       4.2 %, 59
+//   one per column  0.0 %,  0 of 248  0.9 %, 25       3.6 %, 38
+// On 200 sizes that the fit has not seen, all modes, products that take more than 2 % longer than with the old rule and
+// its kernels went from 42 to 13 of 1000, more than 5 % from 20 to 3. MXFP4 and a scale per column have no 256 x 128 tile
+// (it is nowhere more than 3 % ahead).
+struct DenseCost {
+    int own, launch, half, half_own, pair, single, pair_own; // *own, launch: in half slabs
+};
+constexpr DenseCost dense_cost(int mode, bool fp4, bool middle) {
+    return mode == SCALE_VECTOR ? DenseCost{9, 0, 40, 7, 49, 29, 3}
+           : mode == SCALE_MX   ? (fp4 ? DenseCost{12, 3, 0, 0, 54, 20, 7} : DenseCost{9, 1, 42, 6, 53, 24, 3})
+           : middle             ? DenseCost{5, 2, 40, 5, 44, 18, 4}
+                                : DenseCost{13, 5, 0, 0, 45, 18, 11};
+}
+// middle: 256 x 128 may be taken
 template <int MODE, bool F4 = false> static inline int dense_tile(int64_t M, int64_t N, int64_t slabs, bool middle) {
-    constexpr int64_t PAIR = MODE == SCALE_VECTOR ? 42 : 41, SINGLE = MODE == SCALE_VECTOR ? 28 : 27;
-    constexpr int64_t HALF_SLABS = MODE == SCALE_VECTOR ? 8 : MODE == SCALE_MX && !F4 ? 7 : 6; // half slabs beside the K loop
-    const int64_t cus = device_cu_count();
-    auto up = [](int64_t x, int64_t m) { return (x + m - 1) / m; };
-    const int64_t m2 = up(M, 256), n2 = up(N, 256), m1 = up(M, 128), n1 = up(N, 128);
-    const int64_t pairs = m1 * n1 / (2 * cus), rest = m1 * n1 % (2 * cus);
-    const int64_t t3 = (PAIR * pairs + (rest == 0 ? 0 : rest <= cus ? SINGLE : PAIR)) * (slabs + 2);
-    const int64_t t2 = PAIR * up(m2 * n1, cus) * (slabs + 2);
-    const int64_t t1 = 32 * up(m2 * n2, cus) * (2 * slabs + HALF_SLABS);
+    const DenseCost c   = dense_cost(MODE, F4, middle);
+    const int64_t   cus = device_cu_count(), m2 = cdiv(M, 256), n2 = cdiv(N, 256), m1 = cdiv(M, 128), n1 = cdiv(N, 128);
+    const int64_t   pairs = m1 * n1 / (2 * cus), rest = m1 * n1 % (2 * cus);
+    const int64_t   t3 = (c.pair * pairs + (rest == 0 ? 0 : rest <= cus ? c.single : c.pair)) * (2 * slabs + c.pair_own);
+    const int64_t   t2 = c.half * cdiv(m2 * n1, cus) * (2 * slabs + c.half_own);
+    const int64_t   t1 = 64 * (cdiv(m2 * n2, cus) * (2 * slabs + c.own) + c.launch);
     if (t1 <= t3 && (!middle || t1 <= t2))
         return 1;
-    return middle && t2 <= t3 ? 2 : 3;
+    return middle && t2 < t3 ? 2 : 3;
 }
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;
