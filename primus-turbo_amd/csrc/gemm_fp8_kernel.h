@@ -1558,10 +1558,11 @@ static inline bool one_tile_per_cu(int64_t M, int64_t N) {
 // The exchange of the sums at the end costs what it saves where K is short (MXFP8 1024 x 4096 x 1024, two stages /
 // teams 9.4 / 9.7, MXFP4 8.0 / 8.5). Sums with block scales cost more to make: they gain from eight slabs on (K = 1024:
 // 768 x 928 9.7 / 9.3, 1458 x 896 10.1 / 9.7, 1112 x 1536 12.9 / 12.3, and below 896 x 1984 x 640 8.2 / 8.7, 512 x 7968 x
-// 544 9.2 / 10.3, 378 x 3264 x 864 9.4 / 9.7), with a scale per column from four (4 to 5 slabs 1 % on average, 6 to 7 6 %).
+// 544 9.2 / 10.3, 378 x 3264 x 864 9.4 / 9.7), with a scale per column from six (512 x 1504 x 672 9.9 / 8.2, and below 1946
+// x 608 x 576 9.3 / 9.0 but 256 x 15040 x 608 10.7 / 11.7, 512 x 7968 x 544 10.6 / 11.5).
 // The error against 64 bits is that of one sum: 777 x 4096 x 7168 1.500e-5 rms either way, the matrix core's own.
 static inline bool two_teams(int mode, bool sb_vec, int64_t M, int64_t N, int64_t slabs) {
-    return mode != SCALE_VECTOR && one_tile_per_cu(M, N) && slabs >= (mode == SCALE_MX ? 16 : sb_vec ? 4 : 8);
+    return mode != SCALE_VECTOR && one_tile_per_cu(M, N) && slabs >= (mode == SCALE_MX ? 16 : sb_vec ? 6 : 8);
 }
 // The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128. A large tile multiplies more for each
 // byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
