@@ -25,6 +25,12 @@ def test_edges(recipe, M, N, K, tile):
     few._check(recipe, M, N, K // 32 * 32)
 
 
+@pytest.mark.parametrize("special", ["zero", "nan"])
+@pytest.mark.parametrize("recipe", few.RECIPES)
+def test_special_values(recipe, special, tile):
+    few._check(recipe, 510, 1002, 1216, torch.float32, special=special)
+
+
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("recipe", ["vectors", "blockwise", "mxfp8"])

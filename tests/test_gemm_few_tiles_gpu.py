@@ -22,11 +22,14 @@ def _impl(native_lib):
     from primus_turbo.pytorch.kernels.gemm import gemm_fp8_impl as impl
 
 
-def _check(recipe, M, N, K, out_dtype=torch.bfloat16, accumulate=False, dtypes=None):
+def _check(recipe, M, N, K, out_dtype=torch.bfloat16, accumulate=False, dtypes=None, special=None):
     a, sa, av = _exact_operand("blockwise" if recipe == "vectors" else recipe, M, K, 0, True)
     b, sb, bv = _exact_operand("blockwise" if recipe == "vectors" else recipe, N, K, 1, True, weight=recipe == "blockwise")
     if dtypes:  # (the whole numbers are exact in either format)
         a, b = a.float().to(dtypes[0]), b.float().to(dtypes[1])
+    if special:
+        _make_special(special, a, sa, av)
+        _make_special(special, b, sb, bv)
     if recipe == "vectors":
         sa, sb = sa.t().contiguous(), sb.t().contiguous()
     if recipe.startswith("mx"):  # rows of whole words, as the quantizers leave them
@@ -37,7 +40,22 @@ def _check(recipe, M, N, K, out_dtype=torch.bfloat16, accumulate=False, dtypes=N
     impl._launch(a, sa, False, b, sb, True, out, False, gran, accumulate)
     want = av.double() @ bv.double().T
     want = (want + old.double() if accumulate else want).float().to(out_dtype)
-    assert torch.equal(out, want), f"{(out != want).sum().item()} of {out.numel()} differ"
+    wrong = (out != want) & ~(out.isnan() & want.isnan())
+    assert not wrong.any(), f"{wrong.sum().item()} of {out.numel()} differ"
+
+
+def _make_special(special, codes, scales, values):
+    """"zero": every code 0. "nan" / "inf": such a code in two rows, the last one among them (MXFP4 has none: a NaN scale)."""
+    rows, k = [codes.shape[0] // 3, codes.shape[0] - 1], values.shape[1] // 2
+    if special == "zero":
+        codes.view(torch.uint8).zero_()
+        values.zero_()
+    elif codes.shape[1] == values.shape[1]:
+        codes.view(torch.uint8)[rows, k] = 0x7F if special == "nan" else 0x7C
+        values[rows, k] = float(special)
+    else:
+        scales.view(torch.uint8)[rows, -1] = 0xFF
+        values[rows, -32:] = float(special)
 
 
 @pytest.mark.parametrize("K", [32, 512, 1024, 992])
@@ -73,3 +91,13 @@ def test_formats(recipe, da, db):
 @pytest.mark.parametrize("recipe", RECIPES)
 def test_one_large_tile_per_cu(recipe, M, N, K):
     _check(recipe, M, N, K)
+
+
+# the direct kernel, four stages or two teams, with edges in every direction; rows that are not special stay exact
+@pytest.mark.parametrize("special", ["zero", "nan", "inf"])
+@pytest.mark.parametrize("M,N,K", [(13, 1020, 992), (61, 4091, 640), (700, 1032, 2176)])
+@pytest.mark.parametrize("recipe", RECIPES)
+def test_special_values(recipe, M, N, K, special):
+    if special == "inf" and recipe == "mxfp4":
+        pytest.skip("E2M1 and E8M0 have no infinity")
+    _check(recipe, M, N, K, torch.float32, dtypes=(torch.float8_e5m2,) * 2 if special == "inf" else None, special=special)

@@ -76,7 +76,8 @@ def test_mxfp4_gemm_matches_dequantized_matmul(M, N, K):
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2", "e2m1"])
 def test_mx_gemm_eight_wavefront_tile(M, N, K, fmt):
     """tile_cfg 4 (256 x 256 tile, eight wavefronts, gemm_mx8.h) against the oracle and against the
-    automatic configuration: the same products added in the same order, so the bits are the same.
+    256 x 128 tile: the same products added in the same order, so the bits are the same. The automatic
+    configuration may split K over wavefronts, another order: the oracle's gate holds it.
     Exact-integer operands on the same path in the next test."""
     if fmt == "e2m1" and FP4 is None:
         pytest.skip("torch has no float4_e2m1fn_x2")
@@ -91,17 +92,19 @@ def test_mx_gemm_eight_wavefront_tile(M, N, K, fmt):
         aq, as_ = qi.quantize_mxfp8_impl(a, dt, 1, 32)
         bq, bs = qi.quantize_mxfp8_impl(b, torch.float8_e4m3fn, 1, 32, scaling_recipe=ScalingRecipe(use_2d_block=True))
         run = lambda: gi.gemm_fp8_impl(aq, as_, False, bq, bs, True, torch.bfloat16, False, G.MX_BLOCKWISE.value, 0)  # noqa: E731
-    auto = run()
-    gi.TILE_CFG = 4
+    outs = {}
     try:
-        got = run()
+        for gi.TILE_CFG in (0, 2, 4):
+            outs[gi.TILE_CFG] = run()
     finally:
         gi.TILE_CFG = 0
     torch.cuda.synchronize()
-    assert torch.equal(got, auto), "tile configurations differ"
+    got = outs[4]
+    assert torch.equal(got, outs[2]), "tile configurations differ"
     ref = OG.gemm_dequantized(Q.mx_dequant(codes_np(aq), codes_np(as_), fmt),
                               Q.mx_dequant(codes_np(bq), codes_np(bs), "e2m1" if fmt == "e2m1" else "e4m3"))
     _gate(ref, to_f32_np(got), f"mx8 {fmt} {M}x{N}x{K}")
+    _gate(ref, to_f32_np(outs[0]), f"automatic {fmt} {M}x{N}x{K}")
 
 
 def test_mx_gemm_without_workspace_reads_scales_in_place():

@@ -50,6 +50,25 @@ def test_dense_scales(shape, dtype, recipe):
         _same(plain, _bytes(words))
 
 
+# zeros, an infinity and a NaN; stochastic rounding from one seed
+@pytest.mark.parametrize("recipe", [{}, {"use_sr": True}, {"use_sr": True, "use_rht": True}])
+@pytest.mark.parametrize("values", [(0.0,), (float("inf"),), (float("nan"), float("-inf"))])
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, FP4])
+def test_special_values_and_stochastic_rounding(dtype, values, recipe, monkeypatch):
+    if recipe and dtype != FP4:
+        pytest.skip("belongs to the MXFP4 recipe")
+    monkeypatch.setattr(Q, "_next_sr_seed", lambda *flags: 12345)
+    what, r = "MXFP4" if dtype == FP4 else "MXFP8", Recipe(**recipe)
+    x = _x(130, 160)
+    x[32:64, 32:64] = 0
+    for i, v in enumerate(values):
+        x[129 - i, 159 - i] = v
+    q, s, qt, st = Q._quantize_mx_impl(x, dtype, None, 32, True, r, r, what)
+    wq, ws, wqt, wst = Q.quantize_mx_operands(x, dtype, r, r, what)
+    for plain, words in ((q, wq), (qt, wqt), (s, _bytes(ws)), (st, _bytes(wst))):
+        _same(plain, words)
+
+
 @pytest.mark.parametrize("N", [96, 384])
 @pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, FP4])
 @pytest.mark.parametrize("glu", [False, True])

@@ -54,3 +54,26 @@ def test_one_launch_needs_an_aligned_tensor(native_lib):
     q, q_t, _ = impl.quantize_fp8_tensorwise_t_impl(x, torch.float8_e4m3fn, 64, 64)
     assert torch.equal(q.view(torch.uint8), impl._quantize_fp8_tensorwise(x, torch.float8_e4m3fn)[0].view(torch.uint8))
     assert torch.equal(q_t.view(torch.uint8), q.view(torch.uint8).t())
+
+
+# 0, an infinity and a NaN, in one tile or alone, with rows and columns that are padded
+@pytest.mark.parametrize("R,C", [(144, 272), (3001, 1056)])
+@pytest.mark.parametrize("values", [(), (float("inf"),), (float("nan"),), (float("-inf"), float("nan"))])
+@pytest.mark.parametrize("zeros", [False, True])
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_special_values(native_lib, R, C, values, zeros, fp8):
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as impl
+
+    x = torch.randn(R, C, generator=torch.Generator(device="cuda").manual_seed(R), device="cuda", dtype=torch.bfloat16) * (not zeros)
+    for i, v in enumerate(values):
+        x[R - 1 - i, C - 1 - i] = v
+    u8 = lambda t: t.view(torch.uint8)  # noqa: E731
+    q, scale_inv = impl._quantize_fp8_tensorwise(x, fp8)
+    got, got_t, got_scale = impl.quantize_fp8_tensorwise_t_impl(x, fp8, *(-(-n // 128) * 128 for n in (C, R)))
+    assert torch.equal(got_scale.view(torch.int32), scale_inv.view(torch.int32))
+    assert torch.equal(u8(got)[:, :C], u8(q)) and not u8(got)[:, C:].any()
+    assert torch.equal(u8(got_t)[:, :R], u8(q).t()) and not u8(got_t)[:, R:].any()
+    q, s = impl._quantize_fp8_rowwise(x[:, : C - 8].contiguous(), fp8, 1)
+    got, got_s = impl.quant_fp8_rowwise_padded_impl(x[:, : C - 8].contiguous(), fp8, -(-C // 128) * 128)
+    assert torch.equal(got_s.view(torch.int32), s.view(torch.int32))
+    assert torch.equal(u8(got)[:, : C - 8], u8(q)) and not u8(got)[:, C - 8 :].any()
