@@ -21,7 +21,13 @@ template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile
     }
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_MX, false, FA, FB>(a, stream);
-    if (two_teams(SCALE_MX, false, a.M, a.N, a.K / KSTEP))
+    // MXFP4 with both scale arrays row-major (a serving product of fewer than 1024 rows, whose scales are not copied):
+    // the scale copies of two teams, 64 cache lines each, get in each other's way. Over 34 products of 16 slabs or more
+    // teams took 4 % longer on average, in 27 of them (124 x 5568 x 15072 81 us, teams 91, with word-major scales 52 and
+    // 43; 240 x 14240 x 4512 26.3 / 29.5; but 777 x 4096 x 7168 35.5 / 32.9); one operand word-major: 4 % shorter, both 12 %.
+    // MXFP8 gains either way (124 x 5568 x 15072 120 / 117, 777 x 4096 x 7168 56 / 48).
+    const bool words = a.sa_wpitch != 0 || a.sb_wpitch != 0;
+    if ((FA != 4 || words) && two_teams(SCALE_MX, false, a.M, a.N, a.K / KSTEP))
         return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB, GROUP_NONE, 2, 2>(a, stream);
     return launch_gemm_cfg<4, 4, SCALE_MX, false, FA, FB>(a, stream);
 }

@@ -66,7 +66,7 @@ def test_rule(recipe, M, N, K):
 @pytest.mark.parametrize("out_dtype,accumulate", [(torch.bfloat16, False), (torch.float16, True), (torch.float32, False), (torch.float32, True)])
 @pytest.mark.parametrize("K", [512, 640, 896, 1024, 2048, 2176, 4096, 4352])
 @pytest.mark.parametrize("M,N", [(600, 2056), (513, 2047)])
-@pytest.mark.parametrize("recipe", ["vectors", "blockwise", "mxfp8", "mxfp4"])
+@pytest.mark.parametrize("recipe", ["vectors", "blockwise", "mxfp8", "mxfp4", "mxfp8 words", "mxfp4 words"])
 def test_teams(recipe, M, N, K, out_dtype, accumulate):
     few._check(recipe, M, N, K, out_dtype, accumulate)
 

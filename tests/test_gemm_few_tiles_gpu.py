@@ -23,6 +23,8 @@ def _impl(native_lib):
 
 
 def _check(recipe, M, N, K, out_dtype=torch.bfloat16, accumulate=False, dtypes=None, special=None):
+    """``recipe`` of RECIPES, or mxfp8 / mxfp4 with " words": scales word-major."""
+    recipe, words = recipe.split()[0], recipe.endswith(" words")
     a, sa, av = _exact_operand("blockwise" if recipe == "vectors" else recipe, M, K, 0, True)
     b, sb, bv = _exact_operand("blockwise" if recipe == "vectors" else recipe, N, K, 1, True, weight=recipe == "blockwise")
     if dtypes:  # (the whole numbers are exact in either format)
@@ -34,6 +36,8 @@ def _check(recipe, M, N, K, out_dtype=torch.bfloat16, accumulate=False, dtypes=N
         sa, sb = sa.t().contiguous(), sb.t().contiguous()
     if recipe.startswith("mx"):  # rows of whole words, as the quantizers leave them
         sa, sb = (torch.nn.functional.pad(s, (0, -s.shape[1] % 4)) for s in (sa, sb))
+    if words:
+        sa, sb = (s.contiguous().view(torch.int32).t().contiguous() for s in (sa, sb))
     gran = {"rowwise": G.ROWWISE, "blockwise": G.BLOCKWISE, "vectors": G.BLOCKWISE}.get(recipe, G.MX_BLOCKWISE)
     old = torch.randint(-8, 9, (M, N), device="cuda").to(out_dtype)
     out = old.clone()
