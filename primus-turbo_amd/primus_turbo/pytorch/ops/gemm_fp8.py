@@ -163,17 +163,17 @@ class FP8GemmRowFunction(torch.autograd.Function):
         qb, qb_s, b_hp = along_rows(b, b_axis)
         cols = K if qa.shape[1] != K else None
 
-        def other_axis(q, q_s, hp_dtype, from_axis, given, axis, pad):
+        def other_axis(q, q_s, hp_dtype, from_axis, given, axis):
             # the operand as backward reads it: what the forward codes stand for, quantized again
             # along the other axis -> (codes, scales, whether the codes are stored transposed, i.e.
             # contiguous along the axis that the backward product reduces over)
             if given is not None:
                 assert isinstance(given, QuantizedTensor)
                 return given.qdata, given.scale_inv, False
-            if axis == -2 and pad is not None:
-                return (*quant_fp8_rowwise_t_impl(q, q_s, hp_dtype, q.dtype, pad, cols), True)
-            if cols is not None:
-                q = q[:, :cols].contiguous()
+            # (a transposed operand carries the padding of the product's reduction: tokens in wgrad, N in dgrad;
+            # the other one has not been padded)
+            if axis == -2:
+                return (*quant_fp8_rowwise_t_impl(q, q_s, hp_dtype, q.dtype, 128, cols), True)
             hp = dequantize_fp8(q, hp_dtype, gran, axis=from_axis % q.ndim, scale_inv=q_s, block_size=config.block_size)
             return (*quantize_fp8(hp, q.dtype, gran, axis=axis % q.ndim, block_size=config.block_size), False)
 
@@ -182,9 +182,8 @@ class FP8GemmRowFunction(torch.autograd.Function):
         # input asks for a gradient (same outputs, two quantizer passes less)
         a_t_ready = b_t_ready = False
         if any(ctx.needs_input_grad[:2]):
-            # (both operands of a product carry the padding of its reduction: tokens in wgrad, N in dgrad)
-            a_c, a_cs, a_t_ready = other_axis(qa, qa_s, a_hp, -1, a_t, -2, 128)
-            b_c, b_cs, b_t_ready = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1, 128)
+            a_c, a_cs, a_t_ready = other_axis(qa, qa_s, a_hp, -1, a_t, -2)
+            b_c, b_cs, b_t_ready = other_axis(qb, qb_s, b_hp, b_axis, b_t, -2 if trans_b else -1)
             ctx.save_for_backward(a_c, a_cs, b_c, b_cs)
         ctx.meta = (trans_a, trans_b, out_dtype, config, a_t_ready, b_t_ready)
         return out
