@@ -424,7 +424,10 @@ PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const v
  * copies then read (faster; with a smaller workspace, or none when no row copy is needed, the
  * scales are read in place).
  * accumulate != 0 adds into C (beta = 1). tile_cfg as for pt_gemm_fp8; 4 = 256 x 256 tile with
- * eight wavefronts (MXFP4: 1 as well). The results of these tiles are the same bit for bit. */
+ * eight wavefronts (MXFP4: 1 as well). Tiles 1, 2 and 4 add along K in one order and give the same bits;
+ * 3 may share K out to two teams of wavefronts and 0 to the wavefronts of small tiles as well, fp32 sums in
+ * another order (which, follows from M, N, K, the scales' layout and the device's CUs: the same call gives the same
+ * bits). */
 PT_API size_t pt_gemm_mx_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                          int fp4);
 PT_API int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_scale,
