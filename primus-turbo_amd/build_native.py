@@ -1,4 +1,5 @@
-"""Build libprimus_turbo_amd.so (the C-ABI library) with hipcc for gfx950.
+"""Build libprimus_turbo_amd.so (the C-ABI library) with hipcc for gfx950, and libprimus_turbo_torch.so (the host side of
+the dense torch operators, csrc/torch_ops.cpp) with the host compiler against the installed torch.
 
 Usage:  python primus-turbo_amd/build_native.py [--force] [-j N]
 
@@ -22,6 +23,7 @@ CSRC = ROOT / "csrc"
 BUILD = ROOT / "build"
 LIBDIR = ROOT / "lib"
 LIBNAME = "libprimus_turbo_amd.so"
+TORCH_LIBNAME = "libprimus_turbo_torch.so"
 HEADER = ROOT.parent / "include" / "primus_turbo_amd.h"
 
 ARCH = "gfx950"
@@ -50,6 +52,31 @@ def hipcc_path() -> str:
 
 def lib_path() -> Path:
     return LIBDIR / LIBNAME
+
+
+def torch_lib_path() -> Path:
+    return LIBDIR / TORCH_LIBNAME
+
+
+def _build_torch_ops(force: bool, verbose: bool) -> Path:
+    """One host translation unit on torch's headers; the HIP runtime is the one that torch ships."""
+    src, out = CSRC / "torch_ops.cpp", torch_lib_path()
+    if not force and out.exists() and out.stat().st_mtime >= max(src.stat().st_mtime, HEADER.stat().st_mtime):
+        return out
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-isystem", str(root / "include"), "-isystem", str(rocm / "include"), str(src), "-o", str(out),
+           f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-lamdhip64", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{src.name} failed:\n{res.stderr}")
+    return out
 
 
 def sources() -> list[Path]:
@@ -98,7 +125,9 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = False) -
         raise RuntimeError(f"no .hip sources under {CSRC}")
     jobs = jobs or min(8, len(srcs))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        torch_ops = ex.submit(_build_torch_ops, force, verbose)
         objs = list(ex.map(lambda s: _compile_one(hipcc, s, force, verbose), srcs))
+        torch_ops.result()
     out = lib_path()
     cmd = [hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", str(out)] + [str(o) for o in objs]
     if verbose:
@@ -110,9 +139,9 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = False) -
 
 
 def ensure_built() -> Path:
-    """Return the library path, building it only when no library exists yet."""
+    """Return the library path, building the libraries only when one does not exist yet."""
     out = lib_path()
-    if not out.exists():
+    if not out.exists() or not torch_lib_path().exists():
         build()
     return out
 

@@ -18,6 +18,8 @@ import torch
 
 _PKG_ROOT = Path(__file__).resolve().parent.parent  # .../primus-turbo_amd
 LIB_PATH = Path(os.environ.get("PRIMUS_TURBO_AMD_LIB", _PKG_ROOT / "lib" / "libprimus_turbo_amd.so"))
+#: the CUDA kernels of the dense operators (csrc/torch_ops.cpp), which call the entry points of LIB_PATH
+TORCH_LIB_PATH = _PKG_ROOT / "lib" / "libprimus_turbo_torch.so"
 
 # element type codes of include/primus_turbo_amd.h
 DT_BF16, DT_F16, DT_F32, DT_E4M3, DT_E5M2, DT_E2M1X2, DT_E8M0 = range(7)
@@ -261,8 +263,36 @@ def lib() -> ctypes.CDLL:
             fn = getattr(handle, name)  # AttributeError if the build is stale
             fn.restype = res
             fn.argtypes = args
+        load_torch_ops()
+        torch.ops.primus_turbo._bind_native(str(LIB_PATH))
         _lib = handle
     return _lib
+
+
+_torch_ops_loaded = False
+_tensorwise_mode = 0
+
+
+def load_torch_ops() -> None:
+    """Register the CUDA kernels of the dense operators. Done when the package is imported, so that tracing and
+    calls see the same operators from the start, or by ``lib()`` if they were built after that."""
+    global _torch_ops_loaded
+    if _torch_ops_loaded:
+        return
+    if not TORCH_LIB_PATH.exists():
+        raise RuntimeError(f"primus_turbo: native library {TORCH_LIB_PATH} is missing. Build it with "
+                           f"`python {_PKG_ROOT / 'build_native.py'}`. There is no CPU fallback.")
+    torch.ops.load_library(str(TORCH_LIB_PATH))
+    _torch_ops_loaded = True
+    torch.ops.primus_turbo._native_tensorwise_mode(_tensorwise_mode)
+
+
+def set_tensorwise_mode(mode: int) -> None:
+    """0 automatic, 1 fused, 2 two passes, for the operators' C++ side (see ``quantization_impl``)."""
+    global _tensorwise_mode
+    _tensorwise_mode = mode
+    if _torch_ops_loaded:
+        torch.ops.primus_turbo._native_tensorwise_mode(mode)
 
 
 def dtype_code(dtype: torch.dtype) -> int:

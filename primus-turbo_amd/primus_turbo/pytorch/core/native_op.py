@@ -6,6 +6,11 @@ from typing import Callable, Optional
 
 import torch
 
+from primus_turbo import _native
+
+if _native.TORCH_LIB_PATH.exists():
+    _native.load_torch_ops()
+
 _lib = torch.library.Library("primus_turbo", "FRAGMENT")
 _below_autograd = torch._C._AutoDispatchBelowAutograd
 _is_compiling = torch.compiler.is_compiling
@@ -34,7 +39,7 @@ def _wants_gradient(args, kwargs) -> bool:
     return torch.is_grad_enabled() and torch._C._any_requires_grad(*args, **kwargs)
 
 
-def native_op(qualname: str, device_types: Optional[str] = None) -> Callable:
+def native_op(qualname: str, device_types: Optional[str] = None, cpp: bool = False) -> Callable:
     """``torch.library.custom_op(qualname, mutates_args=(), device_types=...)`` for functions that allocate
     their results, launch on the current stream and return: the same operator for tracing (schema from the
     annotations, ``register_fake`` on the returned function) and for autograd (a backward pass through it raises),
@@ -44,13 +49,21 @@ def native_op(qualname: str, device_types: Optional[str] = None) -> Callable:
     functions call these operators with gradients off: the returned function sees that and steps over the
     autograd kernel (0.9 us), which everything else that reaches the operator passes through. Results are fresh tensors,
     and a tracer sees the operator through its fake. Operators that write into an argument stay with ``custom_op``,
-    which advances that tensor's version."""
+    which advances that tensor's version.
+
+    ``cpp``: the operator's CUDA kernel is in csrc/torch_ops.cpp; the function is the body for every other
+    device and, as the operator ``<name>_general``, for the forms which that kernel does not handle itself."""
     namespace, name = qualname.split("::")
     assert namespace == "primus_turbo"
 
     def wrap(fn: Callable) -> Callable:
-        _lib.define(name + torch.library.infer_schema(fn, mutates_args=()), tags=(torch.Tag.pt2_compliant_tag,))
-        _lib.impl(name, fn, "CUDA" if device_types == "cuda" else "CompositeExplicitAutograd")
+        schema, key = torch.library.infer_schema(fn, mutates_args=()), "CUDA" if device_types == "cuda" else "CompositeExplicitAutograd"
+        _lib.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
+        if cpp:
+            _lib.define(name + "_general" + schema)
+            _lib.impl(name + "_general", fn, key)
+        if not cpp or key != "CUDA":
+            _lib.impl(name, fn, key)
         op = getattr(torch.ops.primus_turbo, name).default
 
         def autograd_kernel(*args, **kwargs):

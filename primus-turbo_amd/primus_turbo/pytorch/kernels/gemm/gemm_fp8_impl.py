@@ -168,8 +168,8 @@ def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, gran
     return out
 
 
-@native_op("primus_turbo::gemm_fp8_impl", device_types="cuda")
-def gemm_fp8_impl(
+@native_op("primus_turbo::gemm_fp8_impl", device_types="cuda", cpp=True)
+def _gemm_fp8_op(
     a: torch.Tensor,
     a_scale_inv: torch.Tensor,
     trans_a: bool,
@@ -189,7 +189,26 @@ def gemm_fp8_impl(
     return _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, ScalingGranularity(granularity), False)
 
 
-@gemm_fp8_impl.register_fake
+def gemm_fp8_impl(
+    a: torch.Tensor,
+    a_scale_inv: torch.Tensor,
+    trans_a: bool,
+    b: torch.Tensor,
+    b_scale_inv: torch.Tensor,
+    trans_b: bool,
+    out_dtype: torch.dtype,
+    trans_c: bool,
+    granularity: int,
+    default_backend: int,
+) -> torch.Tensor:
+    op = torch.ops.primus_turbo.gemm_fp8_impl_general if TILE_CFG else _gemm_fp8_op  # (a pinned tile: the Python body)
+    return op(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out_dtype, trans_c, granularity, default_backend)
+
+
+gemm_fp8_impl.__doc__ = _gemm_fp8_op.__doc__
+
+
+@_gemm_fp8_op.register_fake
 def _gemm_fp8_impl_fake(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out_dtype, trans_c, granularity, default_backend):
     M, Nn, _ = get_gemm_logical_shape(a, b, trans_a, trans_b)
     if trans_c:
@@ -212,6 +231,10 @@ def gemm_fp8_accum_impl(
     default_backend: int,
 ) -> None:
     """``out += op(a) @ op(b)``: the accumulation is folded into the GEMM epilogue (beta = 1)."""
+    N.lib()
+    if TILE_CFG == 0 and torch.ops.primus_turbo._gemm_fp8_into(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, trans_c,
+                                                               granularity, out):
+        return
     _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, ScalingGranularity(granularity), True)
 
 

@@ -25,6 +25,12 @@ _FP8_DTYPES = (torch.float8_e4m3fn, torch.float8_e5m2)
 _ext = torch.library.Library("primus_turbo_cpp_extension", "DEF")
 
 
+def _define_cpp(name: str, schema: str) -> None:
+    """An operator whose CUDA kernel is in csrc/torch_ops.cpp: what that does not handle goes to ``<name>_general``."""
+    _ext.define(name + schema)
+    _ext.define(name + "_general" + schema)
+
+
 def _check(cond: bool, msg: str) -> None:
     if not cond:
         raise RuntimeError(msg)
@@ -53,7 +59,7 @@ def _bmn(shape, axis: int) -> Tuple[int, int, int]:
 # ---------------------------------------------------------------------------
 # quantize_fp8_tensorwise(Tensor input, ScalarType dest_dtype, Tensor? scale_opt=None) -> Tensor[]
 # ---------------------------------------------------------------------------
-_ext.define("quantize_fp8_tensorwise(Tensor input, ScalarType dest_dtype, Tensor? scale_opt=None) -> Tensor[]")
+_define_cpp("quantize_fp8_tensorwise", "(Tensor input, ScalarType dest_dtype, Tensor? scale_opt=None) -> Tensor[]")
 
 
 # Which launch structure the dynamic tensorwise quantizer takes.
@@ -68,6 +74,7 @@ _TENSORWISE_MODES = ("auto", "fused", "two_pass")
 _tensorwise_mode = os.environ.get("PRIMUS_TURBO_TENSORWISE_MODE", "auto")
 if _tensorwise_mode not in _TENSORWISE_MODES:
     raise RuntimeError(f"PRIMUS_TURBO_TENSORWISE_MODE must be one of {_TENSORWISE_MODES}")
+N.set_tensorwise_mode(_TENSORWISE_MODES.index(_tensorwise_mode))
 
 
 def set_tensorwise_mode(mode: str) -> str:
@@ -77,6 +84,7 @@ def set_tensorwise_mode(mode: str) -> str:
     global _tensorwise_mode
     _check(mode in _TENSORWISE_MODES, f"mode must be one of {_TENSORWISE_MODES}")
     prev, _tensorwise_mode = _tensorwise_mode, mode
+    N.set_tensorwise_mode(_TENSORWISE_MODES.index(mode))
     return prev
 
 
@@ -128,12 +136,12 @@ def _quantize_fp8_tensorwise_meta(input, dest_dtype, scale_opt=None):
     ]
 
 
-_ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise, "CUDA")
+_ext.impl("quantize_fp8_tensorwise_general", _quantize_fp8_tensorwise, "CUDA")
 _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise, "CPU")  # raises: no CPU path
 _ext.impl("quantize_fp8_tensorwise", _quantize_fp8_tensorwise_meta, "Meta")
 
 
-@native_op("primus_turbo::quantize_fp8_tensorwise_t")
+@native_op("primus_turbo::quantize_fp8_tensorwise_t", cpp=True)
 def quantize_fp8_tensorwise_t_impl(x: torch.Tensor, dtype: torch.dtype, width: int, width_t: int
                                    ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """TENSORWISE quantization of a contiguous matrix ``x [R, C]`` with the codes emitted transposed as well:
@@ -180,7 +188,7 @@ def _quantize_fp8_tensorwise_t_impl_fake(x, dtype, width, width_t):
 # ---------------------------------------------------------------------------
 # dequantize_fp8_tensorwise(Tensor input, Tensor scale_inv, ScalarType dest_dtype) -> Tensor
 # ---------------------------------------------------------------------------
-_ext.define("dequantize_fp8_tensorwise(Tensor input, Tensor scale_inv, ScalarType dest_dtype) -> Tensor")
+_define_cpp("dequantize_fp8_tensorwise", "(Tensor input, Tensor scale_inv, ScalarType dest_dtype) -> Tensor")
 
 
 def _dequantize_fp8_tensorwise(input: torch.Tensor, scale_inv: torch.Tensor, dest_dtype: torch.dtype):
@@ -204,14 +212,14 @@ def _dequantize_fp8_tensorwise_meta(input, scale_inv, dest_dtype):
     return torch.empty_like(input, dtype=dest_dtype)
 
 
-_ext.impl("dequantize_fp8_tensorwise", _dequantize_fp8_tensorwise, "CUDA")
+_ext.impl("dequantize_fp8_tensorwise_general", _dequantize_fp8_tensorwise, "CUDA")
 _ext.impl("dequantize_fp8_tensorwise", _dequantize_fp8_tensorwise, "CPU")
 _ext.impl("dequantize_fp8_tensorwise", _dequantize_fp8_tensorwise_meta, "Meta")
 
 # ---------------------------------------------------------------------------
 # quantize_fp8_rowwise(Tensor input, ScalarType dest_dtype, int axis, Tensor? scale_opt=None) -> Tensor[]
 # ---------------------------------------------------------------------------
-_ext.define("quantize_fp8_rowwise(Tensor input, ScalarType dest_dtype, int axis, Tensor? scale_opt=None) -> Tensor[]")
+_define_cpp("quantize_fp8_rowwise", "(Tensor input, ScalarType dest_dtype, int axis, Tensor? scale_opt=None) -> Tensor[]")
 
 
 def _valid_axis(axis: int, ndim: int) -> int:
@@ -270,7 +278,7 @@ def _quantize_fp8_rowwise_meta(input, dest_dtype, axis, scale_opt=None):
     ]
 
 
-_ext.impl("quantize_fp8_rowwise", _quantize_fp8_rowwise, "CUDA")
+_ext.impl("quantize_fp8_rowwise_general", _quantize_fp8_rowwise, "CUDA")
 _ext.impl("quantize_fp8_rowwise", _quantize_fp8_rowwise, "CPU")
 _ext.impl("quantize_fp8_rowwise", _quantize_fp8_rowwise_meta, "Meta")
 
@@ -340,7 +348,7 @@ def _padded_rows(M: int, pad: int) -> int:
     return -(-M // pad) * pad
 
 
-@native_op("primus_turbo::quant_fp8_rowwise_t_impl")
+@native_op("primus_turbo::quant_fp8_rowwise_t_impl", cpp=True)
 def quant_fp8_rowwise_t_impl(
     x: torch.Tensor, row_scale_inv: Optional[torch.Tensor], hp_dtype: torch.dtype, dtype: torch.dtype, pad: int,
     cols: Optional[int] = None,
@@ -386,7 +394,7 @@ def _quant_fp8_rowwise_t_impl_fake(x, row_scale_inv, hp_dtype, dtype, pad, cols=
     )
 
 
-@native_op("primus_turbo::quant_fp8_rowwise_padded_impl")
+@native_op("primus_turbo::quant_fp8_rowwise_padded_impl", cpp=True)
 def quant_fp8_rowwise_padded_impl(x: torch.Tensor, dtype: torch.dtype, width: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """ROWWISE quantization of a contiguous matrix ``x [M, N]`` along its rows with zero codes behind them:
     ``(x_fp8 [M, width], scale_inv [M, 1])``, rows that a product reads without a padding copy. (No counterpart in
@@ -537,7 +545,7 @@ def _quant_fp8_blockwise_dual_t_impl_fake(x, dtype, block_size=128):
     )
 
 
-@native_op("primus_turbo::quant_fp8_blockwise_kmajor_impl")
+@native_op("primus_turbo::quant_fp8_blockwise_kmajor_impl", cpp=True)
 def quant_fp8_blockwise_kmajor_impl(
     x: torch.Tensor, dtype: torch.dtype, block_size: int, with_col_t: bool
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -1265,7 +1273,7 @@ def _mx_quantize(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, want_c
     return rq, rs, cq, cs
 
 
-@native_op("primus_turbo::quantize_mx")
+@native_op("primus_turbo::quantize_mx", cpp=True)
 def _quantize_mx_op(x: torch.Tensor, out_dtype: torch.dtype, want_row: bool, want_col: bool, row_flags: int,
                     col_flags: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """The four outputs of ``_mx_quantize`` with an empty tensor for an unwanted direction (an
