@@ -387,7 +387,8 @@ PT_API int pt_dequantize_mx(const void *q, int q_dtype, const void *scale, int64
  *     sa_block / sb_block are 1 (1 x 128 activation blocks) or 128 (128 x 128 tiles).
  * accumulate != 0 adds into C (beta = 1) instead of overwriting it.
  * tile_cfg: 0 = automatic, 1 = 256x256, 2 = 256x128, 3 = 128x128 workgroup tile, 4 = 256x256
- *           with eight wavefronts (block scales; 1 is the same there; vector scales: as 1).
+ *           with eight wavefronts (block scales; 1 is the same there; vector scales: as 1),
+ *           5 = 192x256 (vector scales only).
  *           Per-column block scales have no 256x128 tile: 2 is 128x128.
  * For large problems the workspace also holds a [K / 128, M] copy of per-row block scales that
  * arrive as [M, K / 128] (sa_block == 1, sa_k == 1): the kernel's scale copies then read
@@ -424,7 +425,7 @@ PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const v
  * copies then read (faster; with a smaller workspace, or none when no row copy is needed, the
  * scales are read in place).
  * accumulate != 0 adds into C (beta = 1). tile_cfg as for pt_gemm_fp8; 4 = 256 x 256 tile with
- * eight wavefronts (MXFP4: 1 as well). Tiles 1, 2 and 4 add along K in one order and give the same bits;
+ * eight wavefronts (MXFP4: 1 as well), 5 = 192 x 256 (MXFP8 only). Tiles 1, 2, 4 and 5 add along K in one order and give the same bits;
  * 3 may share K out to two teams of wavefronts and 0 to the wavefronts of small tiles as well, fp32 sums in
  * another order (which, follows from M, N, K, the scales' layout and the device's CUs: the same call gives the same
  * bits). */

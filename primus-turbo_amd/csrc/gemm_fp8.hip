@@ -174,9 +174,11 @@ int launch_transpose_words(const uint32_t *in, uint32_t *out, int64_t R, int64_t
 
 template <int FA, int FB>
 static int launch_vector_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
-    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128
+    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128, 5 = 192x256
     if (tile_cfg == 0)
         tile_cfg = dense_tile<SCALE_VECTOR>(a.M, a.N, a.K / KSTEP, true);
+    if (tile_cfg == 5)
+        return launch_gemm_cfg<6, 8, SCALE_VECTOR, false, FA, FB>(a, stream);
     if (tile_cfg == 1 || tile_cfg == 4)
         return launch_gemm_cfg<8, 8, SCALE_VECTOR, false, FA, FB>(a, stream);
     if (tile_cfg == 2)
@@ -305,7 +307,7 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     PT_REQUIRE(scale_mode == SCALE_VECTOR || scale_mode == SCALE_BLOCK, "unknown scale mode");
     PT_REQUIRE(scale_mode != SCALE_BLOCK || ((sa_block == 1 || sa_block == 128) && (sb_block == 1 || sb_block == 128)),
                "sa_block / sb_block must be 1 or 128");
-    PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= 4, "tile_cfg must be 0..4");
+    PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= (scale_mode == SCALE_VECTOR ? 5 : 4), "tile_cfg must be 0..4, vector scales 0..5");
     if (M == 0 || N == 0)
         return PT_OK;
     PT_REQUIRE(a && b && c && a_scale && b_scale, "NULL tensor pointer");

@@ -101,8 +101,12 @@ constexpr int GEMM_MIN_SLABS = 4;
 // BLOCK and MX modes: the scales of a slab travel with it through the LDS stages; every
 // wavefront keeps a private copy of the scale words (one per slab, two for MXFP4) of its
 // 16 * TM rows and 16 * TN columns.
+// (A copy fetches 64 words: the words of the rows take whole copies of room, those behind the last row are not read.)
+constexpr int gemm_scale_rows(int T) {
+    return (T + 3) / 4 * 64;
+}
 constexpr int gemm_scale_bytes(int TM, int TN, int MODE, bool F4) {
-    return MODE == 0 ? 0 : GEMM_WAVES * (TM * 16 + TN * 16) * 4 * (F4 ? 2 : 1);
+    return MODE == 0 ? 0 : GEMM_WAVES * (gemm_scale_rows(TM) + gemm_scale_rows(TN)) * 4 * (F4 ? 2 : 1);
 }
 constexpr int gemm_stage_bytes(int TM, int TN, int MODE, bool F4) {
     return (2 * TM * 16 + 2 * TN * 16) * KSTEP + gemm_scale_bytes(TM, TN, MODE, F4);
@@ -828,7 +832,7 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS>
 __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a) {
     static_assert(KS == 1 || (KS == 2 && GMODE == GROUP_NONE), "teams: dense products, one tile for each workgroup");
-    static_assert(TN % 4 == 0 && TM % 4 == 0, "sub-tiles are multiples of 64 x 64");
+    static_assert(TN % 4 == 0 && TM % 2 == 0, "sub-tiles are multiples of 32 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
     constexpr int AHEAD = NSTAGE < 4 ? 2 : NSTAGE - 1; // slabs the copies run ahead of the MFMAs
@@ -849,7 +853,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     // scale, or the E8M0 bytes of four 32-wide K blocks (two words for MXFP4) -- fetched 64 rows
     // per copy instruction into an area of the stage that is private to the wavefront.
     constexpr bool LDS_SC  = MODE != SCALE_VECTOR;
-    constexpr int  SC_A    = TM * 16, SC_B = TN * 16, SC_ROWS = SC_A + SC_B;
+    constexpr int  SC_A    = gemm_scale_rows(TM), SC_B = gemm_scale_rows(TN), SC_ROWS = SC_A + SC_B;
     constexpr int  NW      = MODE == SCALE_MX ? NH : 1;       // scale words per row and slab
     constexpr int  NSC     = LDS_SC ? NW * SC_ROWS / 64 : 0;  // scale copies per wave and slab
     constexpr int  SC_WAVE = NW * SC_ROWS * 4;                // bytes of a wavefront's scale area
@@ -963,10 +967,10 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         for (int q = 0; q < NSC; ++q) {
             const int e = (q % (SC_ROWS / 64)) * 64 + lane;
             if (e < SC_A)
-                off[NLD + q] = static_cast<uint32_t>((wm * SC_A + e) >> a.sa_shift) * sa_rowp +
+                off[NLD + q] = static_cast<uint32_t>((wm * (TM * 16) + e) >> a.sa_shift) * sa_rowp +
                                (q / (SC_ROWS / 64)) * sa_wordp; // (+ the second scale word of an MXFP4 slab)
             else
-                off[NLD + q] = static_cast<uint32_t>((wn * SC_B + e - SC_A) >> a.sb_shift) * sb_rowp +
+                off[NLD + q] = static_cast<uint32_t>((wn * (TN * 16) + e - SC_A) >> a.sb_shift) * sb_rowp +
                                (q / (SC_ROWS / 64)) * sb_wordp;
         }
     }
@@ -1564,12 +1568,13 @@ static inline bool one_tile_per_cu(int64_t M, int64_t N) {
 static inline bool two_teams(int mode, bool sb_vec, int64_t M, int64_t N, int64_t slabs) {
     return mode != SCALE_VECTOR && one_tile_per_cu(M, N) && slabs >= (mode == SCALE_MX ? 16 : sb_vec ? 6 : 8);
 }
-// The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128. A large tile multiplies more for each
-// byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
+// The tile of a dense product: 1 = 256 x 256, 2 = 256 x 128, 3 = 128 x 128, 5 = 192 x 256. A large tile multiplies more for
+// each byte that it fetches, a small one leaves less of the chip idle in the last round, and how these weigh depends on
 // how the tiles divide among the CUs. The time of a launch is taken to be, in 64ths of what a 256 x 256 tile takes for a
 // slab (1.1 us with vector scales, MXFP8 1.25, MXFP4 1.5 for 256 codes, block scales 1.6, a scale per column 1.8),
 //   256 x 256  64 (rounds (slabs + own) + launch)       256 x 128  half rounds (slabs + half_own)
 //   128 x 128  (pair (rounds of two a CU) + single (a last round of at most one a CU)) (slabs + pair_own)
+//   192 x 256  three rounds (slabs + three_own)
 // with the time of a tile's first copies and result as slabs of its own. The constants are fitted: they are those
 // that lose least against the best tile, measured with every tile for 330 sizes (96 to 28672 wide, K 512 to 16384, odd
 // ones among them) on weights that come from HBM, as a layer's do, and stand for no one time by themselves. Loss on average
@@ -1584,14 +1589,20 @@ static inline bool two_teams(int mode, bool sb_vec, int64_t M, int64_t N, int64_
 // On 200 sizes that the fit has not seen, all modes, products that take more than 2 % longer than with the old rule and
 // its kernels went from 42 to 13 of 1000, more than 5 % from 20 to 3. MXFP4 and a scale per column have no 256 x 128 tile
 // (it is nowhere more than 3 % ahead).
+// 192 x 256 came later, for products of a little more than half a round of 256 x 256 tiles, and fills it: 3001 x
+// 2880 x 4096 (144 tiles of 256 rows, 192 of 192) 47.9 -> 42.5 us, MXFP8 53.4 -> 44.0. (96 rows a wavefront: 48 MFMAs a slab
+// instead of 64 for 56 KB instead of 64.) Its two constants are fitted to 320 other sizes (300 to 16384 wide), the others
+// kept. With it the rule loses, against the best of the four, 0.2 % (8 of 320 more than 3 %) with vector scales and 0.1 % (5) with
+// MXFP8, without it 1.8 % (53) and 2.3 % (54); of the 68 and 55 products that take it, 6 and 2 got slower by more than 2 %, the
+// worst by 6, the best faster by 24 %.
 struct DenseCost {
-    int own, launch, half, half_own, pair, single, pair_own; // *own, launch: in half slabs
+    int own, launch, half, half_own, pair, single, pair_own, three, three_own; // *own, launch: in half slabs
 };
 constexpr DenseCost dense_cost(int mode, bool fp4, bool middle) {
-    return mode == SCALE_VECTOR ? DenseCost{9, 0, 40, 7, 49, 29, 3}
-           : mode == SCALE_MX   ? (fp4 ? DenseCost{12, 3, 0, 0, 54, 20, 7} : DenseCost{9, 1, 42, 6, 53, 24, 3})
-           : middle             ? DenseCost{5, 2, 40, 5, 44, 18, 4}
-                                : DenseCost{13, 5, 0, 0, 45, 18, 11};
+    return mode == SCALE_VECTOR ? DenseCost{9, 0, 40, 7, 49, 29, 3, 50, 10}
+           : mode == SCALE_MX   ? (fp4 ? DenseCost{12, 3, 0, 0, 54, 20, 7, 0, 0} : DenseCost{9, 1, 42, 6, 53, 24, 3, 62, 6})
+           : middle             ? DenseCost{5, 2, 40, 5, 44, 18, 4, 0, 0}
+                                : DenseCost{13, 5, 0, 0, 45, 18, 11, 0, 0};
 }
 // middle: 256 x 128 may be taken
 template <int MODE, bool F4 = false> static inline int dense_tile(int64_t M, int64_t N, int64_t slabs, bool middle) {
@@ -1601,10 +1612,12 @@ template <int MODE, bool F4 = false> static inline int dense_tile(int64_t M, int
     const int64_t   t3 = (c.pair * pairs + (rest == 0 ? 0 : rest <= cus ? c.single : c.pair)) * (2 * slabs + c.pair_own);
     const int64_t   t2 = c.half * cdiv(m2 * n1, cus) * (2 * slabs + c.half_own);
     const int64_t   t1 = 64 * (cdiv(m2 * n2, cus) * (2 * slabs + c.own) + c.launch);
-    if (t1 <= t3 && (!middle || t1 <= t2))
-        return 1;
-    return middle && t2 < t3 ? 2 : 3;
+    const int64_t   t5 = c.three * cdiv(cdiv(M, 192) * n2, cus) * (2 * slabs + c.three_own);
+    const int       best = t1 <= t3 && (!middle || t1 <= t2) ? 1 : middle && t2 < t3 ? 2 : 3;
+    return c.three != 0 && t5 < (best == 1 ? t1 : best == 2 ? t2 : t3) ? 5 : best;
 }
+// (Row groups do not take it: at 320 rows a group on average it gains 4 to 17 % over 128 x 128 tiles where the groups' sizes are
+// any numbers, and loses 2 % of a whole expert layer's step where they are padded to 128, since it pads them again.)
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;
 }

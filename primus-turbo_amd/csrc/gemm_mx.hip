@@ -6,7 +6,7 @@
 namespace pt {
 
 template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
-    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128, 4 = 256x256 with eight wavefronts (MXFP4: 1 as well)
+    // tile_cfg: 0 = auto, 1 = 256x256, 2 = 256x128, 3 = 128x128, 4 = 256x256 with eight wavefronts (MXFP4: 1 as well), 5 = 192x256 (MXFP8)
     // (256x256 with four wavefronts, us, against eight: MXFP4 8192^3 285 / 257, 4096 x 28672 x 8192 471 / 455.
     // MXFP8 on codes that were not scaled by block 8192^3 420 / 402, but a training step of 8192 x 7168 x 2048 on
     // quantized activations 376 / 390: there the chip's clock follows the codes, and four wavefronts do less
@@ -18,6 +18,8 @@ template <int FA, int FB> static int launch_mx_tiles(const GemmArgs &a, int tile
     if constexpr (FA != 4) {
         if (tile_cfg == 1)
             return launch_gemm_cfg<8, 8, SCALE_MX, false, FA, FB>(a, stream);
+        if (tile_cfg == 5)
+            return launch_gemm_cfg<6, 8, SCALE_MX, false, FA, FB>(a, stream);
     }
     if (tile_cfg == 2)
         return launch_gemm_cfg<8, 4, SCALE_MX, false, FA, FB>(a, stream);
@@ -73,7 +75,7 @@ int pt_gemm_mx(const void *a, const void *a_scale, const void *b, const void *b_
     PT_REQUIRE(fp4 || ab_dtype == PT_DTYPE_E4M3 || ab_dtype == PT_DTYPE_E5M2, "operands must be fp8 or e2m1x2");
     PT_REQUIRE(is_hp_dtype(c_dtype), "output must be bf16, fp16 or fp32");
     PT_REQUIRE(M >= 0 && N >= 0 && K > 0 && K % 32 == 0, "K must be a positive multiple of 32");
-    PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= 4, "tile_cfg must be 0..4");
+    PT_REQUIRE(tile_cfg >= 0 && tile_cfg <= (fp4 ? 4 : 5), "tile_cfg must be 0..4, MXFP8 0..5");
     const int64_t kbytes = fp4 ? K / 2 : K, kblocks = K / 32;
     const bool    words_a = sa_ld == 0, words_b = sb_ld == 0; // word-major scales
     PT_REQUIRE(lda >= kbytes && ldb >= kbytes && (words_a || sa_ld >= kblocks) && (words_b || sb_ld >= kblocks), "row pitches too small");
