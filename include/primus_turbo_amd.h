@@ -397,6 +397,11 @@ PT_API int pt_dequantize_mx(const void *q, int q_dtype, const void *scale, int64
  */
 PT_API size_t pt_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K, int trans_a,
                                           int trans_b);
+/* 1 if pt_gemm_fp8 (block scales, sa_block 1, sb_block 128, trans_a 0, tile_cfg 0) reads a B stored [K, N] (trans_b 0) where it
+ * lies on the current device: such a product needs the workspace of trans_b 1, and its weight no transposed copy.
+ * pt_grouped_gemm_fp8_nn_in_place says the same of pt_grouped_gemm_fp8, for any group sizes. */
+PT_API int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K);
+PT_API int pt_grouped_gemm_fp8_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K);
 PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b, int b_dtype,
                        const float *b_scale, void *c, int c_dtype, int64_t M, int64_t N, int64_t K,
                        int trans_a, int trans_b, int scale_mode, int64_t sa_m, int64_t sa_k,

@@ -1,7 +1,7 @@
 // Scaled FP8 GEMM entry points: operand preparation (transposes / K padding), the
 // VECTOR-scale (tensorwise, rowwise) kernel instantiations and the C ABI. The BLOCK-scale
 // instantiations live in gemm_fp8_block.hip, which is compiled with MFMA results in VGPRs.
-#include "gemm_fp8_kernel.h"
+#include "gemm_fp8_block8.h"
 
 namespace pt {
 
@@ -281,6 +281,17 @@ static bool block_scale_copy_pays(int64_t M, int64_t N, int64_t K) {
     return M >= 1024 && N >= 1024 && K >= 1024;
 }
 
+// B stored [K, N] with 128 x 128 blocks is read as it is by the 256 x 256 tile; the others want it transposed in the workspace.
+static bool block_nn_in_place(int64_t M, int64_t N, int64_t K, int tile_cfg) {
+    if (!b8_reads_kn(N, K))
+        return false;
+    return tile_cfg == 0 ? gemm_direct_tile(M, N, K, SCALE_BLOCK, false) < 0 && dense_tile<SCALE_BLOCK>(M, N, K / KSTEP, true) == 1
+                         : tile_cfg == 1 || tile_cfg == 4;
+}
+int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K) {
+    return M > 0 && N > 0 && K > 0 && block_nn_in_place(M, N, K, 0);
+}
+
 size_t pt_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
     // An operand is copied into the workspace when its reduction axis is not contiguous
     // (transpose) or when K is not a multiple of 128 (zero padding of the K tail).
@@ -330,11 +341,14 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     const int      direct    = tile_cfg == 0 ? gemm_direct_tile(M, N, K, scale_mode, false) : -1;
     const bool     unpadded  = direct >= 0 && !trans_a && trans_b && K % 16 == 0;
     const bool     pad       = Kp != K;
+    const bool     nn        = scale_mode == SCALE_BLOCK && !trans_a && !trans_b && sa_block == 1 && sb_block == 128 &&
+                    block_nn_in_place(M, N, K, tile_cfg);
+    const bool     copies    = trans_a || (!trans_b && !nn) || pad;
     const uint8_t *A   = static_cast<const uint8_t *>(a);
     const uint8_t *B   = static_cast<const uint8_t *>(b);
     // workspace layout: [scale area of block_scale_copy_pays problems][operand copies]
     const int64_t KB         = cdiv(K, 128);
-    const size_t  full       = pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, trans_b);
+    const size_t  full       = pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, trans_b || nn);
     const bool    have_ws    = workspace != nullptr && aligned_to(workspace, 16) && workspace_bytes >= full;
     const size_t  scale_area = block_scale_copy_pays(M, N, K) ? static_cast<size_t>(round_up(M * KB * 4, 256)) : 0;
     // per-row A scales stored [M, K / 128] (sa_k == 1): hand the kernel a [K / 128, M] copy
@@ -345,11 +359,11 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
         sa_m    = 1;
         sa_k    = M;
     }
-    if (trans_a || !trans_b || pad) {
+    if (copies) {
         if (!have_ws)
             return fail(PT_ERR_WORKSPACE, "pt_gemm_fp8: workspace missing, too small or misaligned");
     }
-    if ((trans_a || !trans_b || pad) && !unpadded) {
+    if (copies && !unpadded) {
         uint8_t *ws = static_cast<uint8_t *>(workspace) + scale_area;
         if (trans_a || pad) {
             if (M * Kp > 0) {
@@ -382,7 +396,8 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     g.N = N;
     g.K = Kp;
     g.lda = Kp;
-    g.ldb = Kp;
+    g.ldb = nn ? N : Kp;
+    g.b_kn = nn;
     g.sa_m = sa_m;
     g.sa_k = sa_k;
     g.sb_n = sb_n;

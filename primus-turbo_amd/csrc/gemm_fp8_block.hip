@@ -15,6 +15,10 @@ static int launch_block_tiles(const GemmArgs &a, int tile_cfg, hipStream_t strea
     // 256x128 / 128x128: 8192^3 522 / 651 / 661, 4096 x 7168 x 4096 127 / 164 / 144, 2048 x 2048 x 8192 106 / 81
     // / 59, 5120 x 4096 x 2048 66 / 68 / 54; 128 x 128 B blocks: 454 / 566 / 574, 112 / 142 / 131, 87 / 64 / 48,
     // 57 / 56 / 49.)
+    if constexpr (!SB_VEC) {
+        if (a.b_kn) // (block_nn_in_place has looked at the tile)
+            return launch_gemm_block8<FA, FB, GROUP_NONE, false, true>(a, stream);
+    }
     if (tile_cfg == 0)
         tile_cfg = dense_tile<SCALE_BLOCK>(a.M, a.N, a.K / KSTEP, !SB_VEC);
     if (tile_cfg == 1 || tile_cfg == 4)

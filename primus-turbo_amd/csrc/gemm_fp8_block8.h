@@ -28,7 +28,11 @@
 //     for each value (bound by it: 8192^3 takes 522 us, without the multiply 434) and the 24 scales are read as
 //     the slab starts, for want of registers. Still a fifth faster than 256 x 128 with four wavefronts (651 us);
 //   * the slab sequence runs across tile boundaries (persistent grid), the loader changing
-//     tile by swapping uniform values as in the four-wavefront kernel.
+//     tile by swapping uniform values as in the four-wavefront kernel;
+//   * BT: B is stored [K, N] (read_transposed): the backward product of a layer reads the weight's codes as the forward
+//     product does, and the weight's cast writes no transposed copy. A slab takes eight LDS reads and twelve scalar
+//     instructions more: 8192^3 541 us against 527, 32 experts of 4096 x 7168 on 32768 tokens 998 against 972; the cast
+//     takes 36 us instead of 44 and 462 instead of 681, and the scales need no transposition of their own (4.6).
 #pragma once
 #include "gemm_fp8_kernel.h"
 
@@ -50,7 +54,13 @@ constexpr int B8_LA = B8_BM / 8 / B8_WAVES, B8_LB = B8_BN / 8 / B8_WAVES; // row
 constexpr int B8_NL = B8_LA + B8_LB + 1;                                  // + one scale copy
 constexpr int B8_P1 = B8_LB + 1; // copies of a slab issued in row groups 6, 7 (B rows, scales)
 
-template <int FA, int FB, int GMODE, bool SB_VEC>
+// Whether the kernel can read a B stored [K, N] where it is: whole slabs (nothing behind K may meet the matrix core), rows of
+// whole 16-byte groups, byte offsets of 32 bits.
+static inline bool b8_reads_kn(int64_t N, int64_t K) {
+    return K % KSTEP == 0 && K >= GEMM_MIN_SLABS * KSTEP && N % 16 == 0 && K * N < (1LL << 31);
+}
+
+template <int FA, int FB, int GMODE, bool SB_VEC, bool BT>
 __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmArgs a) {
     static_assert(GMODE == GROUP_NONE || GMODE == GROUP_ROWS, "row groups or none");
     static_assert(!SB_VEC || GMODE == GROUP_NONE, "a scale per column: dense products");
@@ -97,7 +107,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     if (tile >= total || KT_ALL < 2)
         return;
     int     g_cur = 0, g_nxt = 0;
-    TileCtx cur_t = make_tile<BM, BN, GMODE>(a, tile, prefix, g_cur);
+    TileCtx cur_t = make_tile<BM, BN, GMODE, false, BT>(a, tile, prefix, g_cur);
     g_nxt         = g_cur;
     TileCtx nxt_t = cur_t;
 
@@ -111,6 +121,10 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
             const bool isA = j < LA;
             const int  row = ((isA ? j : j - LA) * B8_WAVES + wave) * 8 + lrow;
             off[j] = static_cast<uint32_t>(row * (isA ? a.lda : a.ldb)) + ((pchk ^ swz(row)) << 4);
+            if (BT && !isA) { // 1 KB = four K rows of the tile's 256 columns
+                const int k = ((j - LA) * B8_WAVES + wave) * 4 + (lane >> 4);
+                off[j]      = static_cast<uint32_t>(k * a.ldb) + (((lane & 15) ^ swz_t(k)) << 4);
+            }
         }
         if (wave < 4) // scale of tile row 64 wave + lane
             off[NL - 1] = static_cast<uint32_t>((wave * 64 + lane) >> a.sa_shift) * static_cast<uint32_t>(a.sa_m) * 4u;
@@ -133,16 +147,50 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
                        : as_bytes(t.sB) + ((t.n0 >> a.sb_shift) * a.sb_n) * 4;
     };
     auto scale_end = [&](const TileCtx &t) { return sc_is_a ? as_bytes(t.sA) + sa_extent : as_bytes(t.sB) + sb_extent; };
+    // BT: to the end of the matrix (a column behind N reads the next row's, or zero: it is never stored)
+    const uint32_t kn_bytes = opaque_uniform(static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.ldb));
+    auto bytes_b = [&](const TileCtx &t) {
+        return BT ? kn_bytes - static_cast<uint32_t>(t.n0) : t.rows_b * static_cast<uint32_t>(a.ldb);
+    };
+    // (in a register and opaque: where the compiler can work it out anew it does so behind a branch, and the slab has to
+    // stay one basic block)
+    uint32_t step_b = BT ? KSTEP * static_cast<uint32_t>(a.ldb) : KSTEP;
+    if constexpr (BT)
+        step_b = opaque_uniform(step_b);
     auto loader_to = [&](const TileCtx &t) {
         ld_ga     = t.Ag;
         ld_gb     = t.Bg;
         ld_na     = t.rows_a * static_cast<uint32_t>(a.lda);
-        ld_nb     = t.rows_b * static_cast<uint32_t>(a.ldb);
+        ld_nb     = bytes_b(t);
         ld_kt     = 0;
         ld_sc     = scale_src(t);
         ld_sc_end = scale_end(t);
     };
+    // BT: where the loader goes at the end of its tile, worked out ahead of the K loop (as step_b is)
+    const uint8_t *to_ga = nullptr, *to_gb = nullptr, *to_sc = nullptr, *to_sc_end = nullptr;
+    uint32_t       to_na = 0, to_nb = 0;
+    auto set_next = [&]() {
+        if constexpr (BT) {
+            to_ga     = opaque_uniform(nxt_t.Ag);
+            to_gb     = opaque_uniform(nxt_t.Bg);
+            to_na     = opaque_uniform(nxt_t.rows_a * static_cast<uint32_t>(a.lda));
+            to_nb     = opaque_uniform(bytes_b(nxt_t));
+            to_sc     = opaque_uniform(scale_src(nxt_t));
+            to_sc_end = opaque_uniform(scale_end(nxt_t));
+        }
+    };
     auto advance_loader = [&]() {
+        if constexpr (BT) {
+            const bool wrap = ld_kt + 1 == KT_ALL;
+            ld_kt     = wrap ? 0 : ld_kt + 1;
+            ld_ga     = wrap ? to_ga : ld_ga + KSTEP;
+            ld_gb     = wrap ? to_gb : ld_gb + step_b;
+            ld_na     = wrap ? to_na : ld_na - KSTEP;
+            ld_nb     = wrap ? to_nb : ld_nb - step_b;
+            ld_sc     = wrap ? to_sc : ld_sc + sc_step;
+            ld_sc_end = wrap ? to_sc_end : ld_sc_end;
+            return;
+        }
         const bool wrap = ld_kt + 1 == KT_ALL;
         ld_kt     = wrap ? 0 : ld_kt + 1;
         ld_ga     = wrap ? nxt_t.Ag : ld_ga + KSTEP;
@@ -158,10 +206,20 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         uint8_t      *dst = smem + b * STAGE;
 #if defined(__HIP_DEVICE_COMPILE__) // the buffer resource type only exists in the device pass
         constexpr uint32_t RSRC_FLAGS = 0x00020000; // raw buffer, 32-bit data format
-        if constexpr (L == NL - 1) {
-            // nothing is read for a slab of zero padding beyond the K blocks the arrays hold
-            const int64_t  n     = ld_sc_end - ld_sc;
-            const uint32_t bytes = (n <= 0 || ld_kt >= a.kb_valid) ? 0u : (n > 0x7fffffff ? 0x7fffffffu : static_cast<uint32_t>(n));
+        // nothing is read for a slab of zero padding beyond the K blocks the arrays hold
+        auto scale_bytes = [&]() {
+            const int64_t n = ld_sc_end - ld_sc;
+            return (n <= 0 || ld_kt >= a.kb_valid) ? 0u : (n > 0x7fffffff ? 0x7fffffffu : static_cast<uint32_t>(n));
+        };
+        if constexpr (BT) {
+            if constexpr (L == NL - 1)
+                copy_to_lds<4, B8_SC_A>(dst + wave * 256, ld_sc, scale_bytes(), off[L]);
+            else if constexpr (L < LA)
+                copy_to_lds<16, L * B8_WAVES * 1024>(dst + wave * 1024, ld_ga, ld_na, off[L]);
+            else
+                copy_to_lds<16, A_BYTES + (L - LA) * B8_WAVES * 1024>(dst + wave * 1024, ld_gb, ld_nb, off[L]);
+        } else if constexpr (L == NL - 1) {
+            const uint32_t bytes = scale_bytes();
             __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(ld_sc), 0, bytes, RSRC_FLAGS);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(dst + B8_SC_A + wave * 256), 4, off[L], 0, 0, 0);
         } else if constexpr (L < LA) {
@@ -205,11 +263,19 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     };
     const uint32_t a_part = wm * (TM * 16) * KSTEP;
     const uint32_t b_part = A_BYTES + wn * (TN * 16) * KSTEP;
+    [[maybe_unused]] const uint32_t t_off = A_BYTES + transposed_offset<BN>(lane, wn * TN);
+    auto ldfrag_b = [&](const uint8_t *stage, int j) {
+        if constexpr (BT)
+            return read_transposed<BN>(stage + (t_off ^ (j << 4))); // (A_BYTES and wn * TN leave the bits of j free)
+        else
+            return ldfrag(stage + b_part, j);
+    };
 
     // ---- pipeline start: slabs 0 and 1 ----
     // (the loader steps past slab 1 here: with two slabs per tile that is the next tile already)
     if (tile + static_cast<int>(gridDim.x) < total)
-        nxt_t = make_tile<BM, BN, GMODE>(a, tile + gridDim.x, prefix, g_nxt);
+        nxt_t = make_tile<BM, BN, GMODE, false, BT>(a, tile + gridDim.x, prefix, g_nxt);
+    set_next();
     loader_to(cur_t);
     static_for<0, NL>([&](auto c) { issue_nth(c, 0); });
     advance_loader();
@@ -227,7 +293,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         read_scales(smem);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-        fb[j] = ldfrag(smem + b_part, j);
+        fb[j] = ldfrag_b(smem, j);
     fa[0] = ldfrag(smem + a_part, 0);
     fa[1] = ldfrag(smem + a_part, 1);
 
@@ -241,7 +307,8 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
         const int next_tile = tile + gridDim.x;
         nxt_t               = cur_t;
         if (next_tile < total)
-            nxt_t = make_tile<BM, BN, GMODE>(a, next_tile, prefix, g_nxt);
+            nxt_t = make_tile<BM, BN, GMODE, false, BT>(a, next_tile, prefix, g_nxt);
+        set_next();
 
         // one K slab per iteration; the body stays a single basic block
         for (int kt = 0; kt < KT_ALL; ++kt) {
@@ -313,7 +380,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
                         fold(t - DEPTH);
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (i == TM - 1)
-                        fb[j] = ldfrag(nxt + b_part, j); // dead from here on: refill from the next slab
+                        fb[j] = ldfrag_b(nxt, j); // dead from here on: refill from the next slab
                     // all copies of the slab after next: row groups 6 and 7, into the stage the
                     // barrier has just freed (nine copies in eight MFMA slots)
                     if constexpr (i >= 6) {
@@ -348,7 +415,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int FA, int FB, int GMODE = GROUP_NONE, bool SB_VEC = false>
+template <int FA, int FB, int GMODE = GROUP_NONE, bool SB_VEC = false, bool BT = false>
 static int launch_gemm_block8(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int STAGES  = B8_NSTAGE * B8_STAGE;
     constexpr int MAX_G   = 2048;
@@ -364,7 +431,7 @@ static int launch_gemm_block8(const GemmArgs &args_in, hipStream_t stream) {
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_fp8: unsupported block-scale layout for the 256x256 tile");
     if (a.K / KSTEP < 2)
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_fp8: K too short for the 256x256 tile");
-    auto kern = gemm_fp8_block8_kernel<FA, FB, GMODE, SB_VEC>;
+    auto kern = gemm_fp8_block8_kernel<FA, FB, GMODE, SB_VEC, BT>;
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)

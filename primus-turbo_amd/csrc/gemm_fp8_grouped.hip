@@ -13,16 +13,29 @@
 
 namespace pt {
 
+// The tile of a row-grouped product with block scales
+static int grouped_rows_tile(int64_t G, int64_t M, int64_t N) {
+    // 256-row tiles once the average group fills a couple of them
+    return G > 0 && M / G >= 512 && N >= 1024 ? (N >= 2048 ? 4 : 2) : 3;
+}
+// B stored [G, K, N] is read as it is by the 256 x 256 tile; the others want it transposed in the workspace
+static bool grouped_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K, int tile_cfg) {
+    return (tile_cfg == 0 ? grouped_rows_tile(G, M, N) : tile_cfg) == 4 && G > 0 && G <= 2048 && M > 0 && b8_reads_kn(N, K);
+}
+
 template <int GMODE, bool SB_VEC, int FA, int FB>
 static int launch_grouped_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
     // tile_cfg: 0 = auto, 1 / 2 = 256x128, 3 = 128x128 (two workgroups per CU), 4 = 256x256 with
     // eight wavefronts (row groups: gemm_fp8_block8.h; variable K: gemm_fp8_block8_vk.h)
     // (the 256x128 tile leaves LDS for the tile prefix sums of 1024 groups only)
-    if (tile_cfg == 0) { // 256-row tiles once the average group fills a couple of them
-        tile_cfg = ((GMODE == GROUP_K ? a.M >= 1024 : (a.G > 0 && a.M / a.G >= 512)) && a.N >= 1024) ? 2 : 3;
-        if (GMODE == GROUP_ROWS && !SB_VEC && tile_cfg == 2 && a.N >= 2048)
-            tile_cfg = 4;
-        if (GMODE == GROUP_K && SB_VEC && a.M >= 1024 && a.N >= 1024)
+    static_assert((GMODE == GROUP_ROWS) == !SB_VEC, "row groups with 128 x 128 B blocks, variable K with a scale per column");
+    if constexpr (GMODE == GROUP_ROWS) {
+        if (a.b_kn) // (grouped_nn_in_place has looked at the tile)
+            return launch_gemm_block8<FA, FB, GROUP_ROWS, false, true>(a, stream);
+    }
+    if (tile_cfg == 0) {
+        tile_cfg = GMODE == GROUP_ROWS ? grouped_rows_tile(a.G, a.M, a.N) : 3;
+        if (GMODE == GROUP_K && a.M >= 1024 && a.N >= 1024)
             tile_cfg = 4; // measured 15-20 % faster than the 256x128 tile on 4096 x 7168 and 7168 x 2048 outputs
     }
     if (tile_cfg == 4) {
@@ -79,6 +92,10 @@ size_t pt_grouped_gemm_fp8_workspace_bytes(int64_t G, int64_t M, int64_t N, int6
     return b;
 }
 
+int pt_grouped_gemm_fp8_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K) {
+    return grouped_nn_in_place(G, M, N, K, 0);
+}
+
 int pt_grouped_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b, int b_dtype,
                         const float *b_scale, void *c, int c_dtype, const int64_t *group_offs, int64_t G,
                         int64_t M, int64_t out_rows, int64_t N, int64_t K, int trans_b, void *workspace,
@@ -101,7 +118,8 @@ int pt_grouped_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const 
     const bool     pad = Kp != K;
     const uint8_t *A   = static_cast<const uint8_t *>(a);
     const uint8_t *B   = static_cast<const uint8_t *>(b);
-    if (!trans_b || pad) {
+    const bool     nn  = !trans_b && grouped_nn_in_place(G, M, N, K, tile_cfg);
+    if ((!trans_b && !nn) || pad) {
         const size_t need = pt_grouped_gemm_fp8_workspace_bytes(G, M, N, K, trans_b);
         if (workspace == nullptr || workspace_bytes < need || !aligned_to(workspace, 16))
             return fail(PT_ERR_WORKSPACE, "pt_grouped_gemm_fp8: workspace missing, too small or misaligned");
@@ -132,7 +150,8 @@ int pt_grouped_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const 
     g.N          = N;
     g.K          = Kp;
     g.lda        = Kp;
-    g.ldb        = Kp;
+    g.ldb        = nn ? N : Kp;
+    g.b_kn       = nn;
     g.sa_m       = 1;
     g.sa_k       = M;
     g.sb_n       = trans_b ? kb : 1;

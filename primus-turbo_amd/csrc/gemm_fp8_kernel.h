@@ -54,7 +54,8 @@ struct GemmArgs {
     const float   *sA;
     const float   *sB;
     int64_t        M, N, K;     // K is a multiple of 128 here (the host pads)
-    int64_t        lda, ldb;    // row pitch of A and B in bytes (>= K)
+    int64_t        lda, ldb;    // row pitch of A and B in bytes (>= K; b_kn: N)
+    bool           b_kn;        // B is stored [K, N] (block8 kernel, 128 x 128 B blocks)
     // VECTOR: sA[m * sa_m], sB[n * sb_n]                      (stride 0 = one scalar)
     // BLOCK : sA[(m >> sa_shift) * sa_m + kb * sa_k], sB[(n >> sb_shift) * sb_n + kb * sb_k]
     // MX    : sA / sB point at E8M0 bytes, byte[m * sa_m + kb] and byte[n * sb_n + kb];
@@ -130,6 +131,52 @@ typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 // wavefront's sub-tile uses the same two lane addresses plus an immediate offset. The reads
 // are ordinary loads: with buffer-load copies the compiler's wait-count pass does not treat an
 // outstanding direct-to-LDS copy as aliasing them.
+
+// A weight that the forward product reads along its rows is reduced over its columns' axis in the backward product: its codes
+// lie [K, N] there, N contiguous. Instead of a transposed copy from the quantizer (a quarter of the bytes of a weight's cast)
+// the tile is copied as it lies, KSTEP rows of BN bytes, and transposed as it is read: ds_read_b64_tr_b8 gives lane i of
+// each 16 lanes the i-th byte of the eight 16-byte rows whose halves those lanes address. A fragment (16 columns, the K bytes of
+// a lane group as above) takes four such reads instead of two of 16 bytes.
+// The 16-byte chunk c of stage row k sits at chunk c ^ swz_t(k): eight consecutive rows, and the rows 16 further that the
+// next lane group reads at the same time, hit all 64 banks once (256-byte rows).
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) i32x2 *lds_i32x2_t;
+__device__ __forceinline__ int swz_t(int k) {
+    return (k & 7) | ((k >> 4 & 1) << 3);
+}
+// lane's byte offset of fragment `f` of a stage of ROW-byte rows; its reads lie 8, 64 and 72 rows further
+template <int ROW> __device__ __forceinline__ uint32_t transposed_offset(int lane, int f) {
+    const int k = 16 * (lane >> 4) + ((lane & 15) >> 1);
+    return static_cast<uint32_t>(k * ROW + ((f ^ swz_t(k)) << 4) + (lane & 1) * 8);
+}
+template <int ROW> __device__ __forceinline__ i32x8 read_transposed(const uint8_t *p) {
+    i32x8 r{};
+#if defined(__HIP_DEVICE_COMPILE__)
+    auto at = [&](int row) { return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2_t)(p + row * ROW)); };
+    const i32x2 a = at(0), b = at(8), c = at(64), d = at(72);
+    r[0] = a.x; r[1] = a.y; r[2] = b.x; r[3] = b.y;
+    r[4] = c.x; r[5] = c.y; r[6] = d.x; r[7] = d.y;
+#endif
+    return r;
+}
+
+// A copy of 16 (4) bytes a lane to the 64 x 16 (64 x 4) bytes at `dst` + AT, from `src` + the lane's `off`, zeros where that is not within
+// `bytes`. As an instruction of our own: the compiler knows its builtin for one that writes the LDS, and makes the builtin
+// of the transposed read wait for every copy in flight (vmcnt(0) before each fragment), which the kernels' own waits have
+// seen to. (One wait state from the write of M0; no result register, so nothing for the compiler to reuse early.)
+template <int SIZE, int AT>
+__device__ __forceinline__ void copy_to_lds(uint8_t *dst, const uint8_t *src, uint32_t bytes, uint32_t off) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+    const uint64_t   p    = reinterpret_cast<uint64_t>(src);
+    const u32x4s     rsrc = {static_cast<uint32_t>(p), static_cast<uint32_t>(p >> 32) & 0xffffu, bytes, 0x00020000u};
+    const uint32_t   lds  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)dst));
+    if constexpr (SIZE == 16)
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
+    else
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
+#endif
+}
 
 template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
     if constexpr (I < N) {
@@ -691,6 +738,13 @@ __device__ __forceinline__ void uniform_load_pair(const int64_t *p, int64_t &v0,
     v1 = p[1];
 #endif
 }
+// The value in a scalar register, unknown to the compiler from here on.
+template <typename T> __device__ __forceinline__ T opaque_uniform(T v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(v));
+#endif
+    return v;
+}
 __device__ __forceinline__ int64_t uniform_load(const int64_t *p) {
     int64_t v;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -732,8 +786,8 @@ struct TileCtx {
 };
 
 // GROUP_ROWS: prefix[g] = number of tiles of the groups before g (in LDS), `g` is a search
-// hint that only moves forward as a workgroup walks its tiles.
-template <int BM, int BN, int GMODE, bool F4 = false>
+// hint that only moves forward as a workgroup walks its tiles. BT: B is stored [K, N] (see read_transposed).
+template <int BM, int BN, int GMODE, bool F4 = false, bool BT = false>
 __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const int *prefix, int &g) {
     TileCtx t;
     t.g0 = t.g1 = 0;
@@ -798,7 +852,7 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
     t.n0     = static_cast<int64_t>(tn) * BN;
     t.rows_a = (t.m_end - t.m0) < BM ? static_cast<int>(t.m_end - t.m0) : BM;
     t.rows_b = (a.N - t.n0) < BN ? static_cast<int>(a.N - t.n0) : BN;
-    t.Bg += t.n0 * a.ldb;
+    t.Bg += BT ? t.n0 : t.n0 * a.ldb;
     return t;
 }
 

@@ -140,6 +140,8 @@ _SIGNATURES = {
          c_void_p, c_void_p],
     ),
     "pt_gemm_fp8_workspace_bytes": (c_size_t, [c_i64, c_i64, c_i64, c_int, c_int]),
+    "pt_gemm_fp8_nn_in_place": (c_int, [c_i64, c_i64, c_i64]),
+    "pt_grouped_gemm_fp8_nn_in_place": (c_int, [c_i64, c_i64, c_i64, c_i64]),
     "pt_gemm_fp8": (
         c_int,
         [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_i64, c_i64, c_i64, c_int, c_int,

@@ -118,6 +118,12 @@ def launch_mx(a, a_scale, b, b_scale, out, trans_c, accumulate):
     return out
 
 
+def reads_kn_in_place(M: int, Nn: int, K: int) -> bool:
+    """Whether the block-scaled product reads a ``b`` stored ``[K, N]`` where it lies, so that a weight needs no
+    transposed copy for it."""
+    return bool(N.lib().pt_gemm_fp8_nn_in_place(M, Nn, K))
+
+
 def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, granularity, accumulate):
     if granularity == ScalingGranularity.MX_BLOCKWISE:
         _check(not trans_a and trans_b, "MX_BLOCKWISE GEMM supports the NT layout only (trans_a=False, trans_b=True)")
@@ -153,7 +159,8 @@ def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, gran
     _check(tuple(out.shape) == (M, Nn) and out.is_contiguous(), f"out must be a contiguous {(M, Nn)} tensor")
     lib = N.lib()
     ws = None
-    ws_bytes = lib.pt_gemm_fp8_workspace_bytes(M, Nn, K, int(trans_a), int(trans_b))
+    in_place = (mode, sa_blk, sb_blk, trans_a, trans_b, TILE_CFG) == (1, 1, 128, False, False, 0) and reads_kn_in_place(M, Nn, K)
+    ws_bytes = lib.pt_gemm_fp8_workspace_bytes(M, Nn, K, int(trans_a), int(trans_b or in_place))
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
     N.check(

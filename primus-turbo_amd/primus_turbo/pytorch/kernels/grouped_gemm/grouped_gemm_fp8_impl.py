@@ -242,6 +242,12 @@ def _variable_k_mx(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans
     return out
 
 
+def reads_kn_in_place(G: int, M: int, Nn: int, K: int) -> bool:
+    """Whether the block-scaled product over ``M`` rows reads a ``b`` stored ``[G, K, N]`` where it lies, so that the
+    weights need no transposed copy for it."""
+    return bool(N.lib().pt_grouped_gemm_fp8_nn_in_place(G, M, Nn, K))
+
+
 @native_op("primus_turbo::grouped_gemm_fp8_impl", device_types="cuda")
 def grouped_gemm_fp8_impl(
     a: torch.Tensor,
@@ -289,7 +295,8 @@ def grouped_gemm_fp8_impl(
     out = torch.empty((M, Nn), dtype=out_dtype, device=a.device)
     lib = N.lib()
     ws = None
-    ws_bytes = lib.pt_grouped_gemm_fp8_workspace_bytes(G, M, Nn, K, int(trans_b))
+    in_place = not trans_b and TILE_CFG == 0 and reads_kn_in_place(G, M, Nn, K)
+    ws_bytes = lib.pt_grouped_gemm_fp8_workspace_bytes(G, M, Nn, K, int(trans_b or in_place))
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
     N.check(

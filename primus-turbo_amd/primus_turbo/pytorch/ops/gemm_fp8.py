@@ -33,7 +33,12 @@ from primus_turbo.pytorch.core.quantized_tensor import (
     check_quantized_tensor,
     transpose_last_two,
 )
-from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import gemm_fp8_accum_impl, gemm_fp8_impl, get_gemm_logical_shape
+from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import (
+    gemm_fp8_accum_impl,
+    gemm_fp8_impl,
+    get_gemm_logical_shape,
+    reads_kn_in_place,
+)
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_t_impl,
     quant_fp8_blockwise_kmajor_impl,
@@ -244,7 +249,9 @@ class FP8GemmBlockFunction(torch.autograd.Function):
         if isinstance(b, QuantizedTensor):
             check_quantized_tensor(b, config, scaling_recipe=w_recipe)
             b_q, b_s = b.qdata, b.scale_inv
-        elif (need_bwd or not trans_b) and b.dim() == 2 and b.size(0) % 16 == 0:
+        elif ((need_bwd or not trans_b) and b.dim() == 2 and b.size(0) % 16 == 0
+              and not (trans_b and a.dim() == 2 and not torch.compiler.is_compiling() and b.is_cuda
+                       and reads_kn_in_place(a.shape[0], b.shape[1], b.shape[0]))):
             b_q, b_q_t, b_s = quant_fp8_blockwise_for_weight_dual_impl(b, fdt, bs)
         else:
             b_q, b_s = quantize_fp8(b, fdt, gran, block_size=bs, scaling_recipe=w_recipe)

@@ -37,6 +37,7 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import (
     grouped_gemm_fp8_impl,
     grouped_gemm_fp8_variable_k_accum_impl,
     grouped_gemm_fp8_variable_k_impl,
+    reads_kn_in_place,
 )
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
@@ -80,7 +81,7 @@ def _grouped_gemm_fp8_variable_k_impl_wrapper(a, b, a_scales, b_scales, group_le
 
 def _block_forward_product(a_fp8_row, a_scale_row, b, group_lens, group_offs, trans_b, out_dtype, config, num_cu, need_bwd):
     """Quantize the BLOCKWISE weight (2-D blocks; with the transposed copy for the backward product
-    when it is needed and possible) and multiply -> ``(out, (weight codes, scales) for dgrad,
+    when it is needed and possible: the large tile reads the forward operand as it lies) and multiply -> ``(out, (weight codes, scales) for dgrad,
     whether those are K-contiguous for dgrad already)``."""
     bs = config.block_size
     b_dtype = _get_fp8_dtype(config.format, True)
@@ -89,7 +90,9 @@ def _block_forward_product(a_fp8_row, a_scale_row, b, group_lens, group_offs, tr
     if isinstance(b, QuantizedTensor):
         check_quantized_tensor(b, config, scaling_recipe=b_recipe)
         b_fp8, b_scale = b.qdata, b.scale_inv
-    elif (need_bwd or not trans_b) and b.size(-2) % 16 == 0:
+    elif ((need_bwd or not trans_b) and b.size(-2) % 16 == 0
+          and not (trans_b and not torch.compiler.is_compiling() and b.is_cuda
+                   and reads_kn_in_place(b.shape[0], a_fp8_row.shape[0], b.shape[2], b.shape[1]))):
         b_fp8, b_fp8_t, b_scale = quant_fp8_blockwise_for_weight_dual_impl(b, b_dtype, block_size=bs)
     else:
         b_fp8, b_scale = quant_fp8_blockwise_for_weight_impl(b, b_dtype, block_size=bs)

@@ -1,0 +1,125 @@
+"""Block-scaled products that read a weight stored [K, N] where it lies (256 x 256 tile, transposed reads from the LDS): the bits
+of the product of the transposed copy, at the edges of the tile and of the matrix, and the same gradients of the layers."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import bf16_randn
+
+pytestmark = pytest.mark.gpu
+E4M3, E5M2 = torch.float8_e4m3fn, torch.float8_e5m2
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _turbo(native_lib):
+    global turbo, G, impl, gimpl, Q, LP
+    import primus_turbo.pytorch as turbo
+    from primus_turbo.pytorch.core import low_precision as LP
+    from primus_turbo.pytorch.core.low_precision import ScalingGranularity as G
+    from primus_turbo.pytorch.kernels.gemm import gemm_fp8_impl as impl
+    from primus_turbo.pytorch.kernels.grouped_gemm import grouped_gemm_fp8_impl as gimpl
+    from primus_turbo.pytorch.kernels.quantization import quantization_impl as Q
+
+
+def _operands(M, N, K, da=E4M3, db=E4M3, lead=()):
+    x, w = bf16_randn((M, K), seed=1).cuda(), bf16_randn((*lead, K, N), seed=2).cuda()
+    a, sa, _, _ = Q.quant_fp8_blockwise_kmajor_impl(x, da, 128, False)
+    b, sb = Q.quant_fp8_blockwise_for_weight_impl(w, db, 128)
+    return a, sa, b, sb
+
+
+def _dense(a, sa, b, sb, out, accumulate=False):
+    """(read in place, on the transposed copy)"""
+    outs = [out.clone(), out.clone()]
+    impl._launch(a, sa, False, b, sb, False, outs[0], False, G.BLOCKWISE, accumulate)
+    impl._launch(a, sa, False, b.t().contiguous(), sb.t().contiguous(), True, outs[1], False, G.BLOCKWISE, accumulate)
+    return outs
+
+
+@pytest.fixture
+def pinned():
+    impl.TILE_CFG = 4
+    yield
+    impl.TILE_CFG = 0
+
+
+# one tile; columns that end inside a tile, a fragment's and a copy's width before its end; rows of less than a tile
+@pytest.mark.parametrize("N", [16, 112, 128, 240, 256, 272, 528, 1008])
+@pytest.mark.parametrize("M,K", [(256, 512), (300, 640), (1, 1152)])
+def test_edges(M, N, K, pinned):
+    a, sa, b, sb = _operands(M, N, K)
+    got, want = _dense(a, sa.t(), b, sb, torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"))
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("da", [E4M3, E5M2])
+@pytest.mark.parametrize("db", [E4M3, E5M2])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_forms(da, db, out_dtype, accumulate, pinned):
+    a, sa, b, sb = _operands(520, 784, 1024, da, db)
+    old = torch.randn(520, 784, device="cuda").to(out_dtype)
+    for scales in (sa.t(), sa.t().contiguous()):  # block-major, row-major
+        got, want = _dense(a, scales, b, sb, old, accumulate)
+        assert torch.equal(got, want)
+
+
+def test_special_values_stay_in_their_column(pinned):
+    a, sa, b, sb = _operands(300, 528, 640)
+    b.view(torch.uint8)[639, 5] = 0x7F
+    b.view(torch.uint8)[0, 527] = 0x7F
+    got, want = _dense(a, sa.t(), b, sb, torch.zeros(300, 528, dtype=torch.float32, device="cuda"))
+    assert torch.equal(got.nan_to_num(nan=7e9), want.nan_to_num(nan=7e9))
+    assert got.isnan().any(0).nonzero().flatten().tolist() == [5, 527]
+
+
+# reductions and widths that the tile does not read in place take the copy
+@pytest.mark.parametrize("M,N,K", [(300, 520, 640), (300, 528, 600), (300, 528, 384), (4096, 4096, 512), (8192, 4080, 1024)])
+def test_rule(M, N, K):
+    a, sa, b, sb = _operands(M, N, K)
+    assert impl.reads_kn_in_place(M, N, K) == (M > 300)
+    got, want = _dense(a, sa.t(), b, sb, torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"))
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("lens", [[256, 0, 255, 1, 257], [700, 513, 0, 300]])
+@pytest.mark.parametrize("N", [256, 400, 2064])
+@pytest.mark.parametrize("da", [E4M3, E5M2])
+@pytest.mark.parametrize("tile", [0, 4])
+def test_grouped(lens, N, da, tile):
+    M, K = sum(lens), 640
+    a, sa, b, sb = _operands(M + 70, N, K, da, E4M3, (len(lens),))  # (rows behind the last group read as zero)
+    gl = torch.from_numpy(np.array(lens, dtype=np.int64)).cuda()
+    offs = torch.ops.primus_turbo_cpp_extension.grouped_gemm_compute_offs(gl)
+    outs = []
+    for w, s, tb in ((b, sb, False), (b.transpose(1, 2).contiguous(), sb.transpose(1, 2).contiguous(), True)):
+        gimpl.TILE_CFG = tile
+        try:
+            outs.append(gimpl.grouped_gemm_fp8_impl(a, w, sa, s, gl, offs, False, tb, torch.bfloat16, G.BLOCKWISE.value, None, 0))
+        finally:
+            gimpl.TILE_CFG = 0
+    assert torch.equal(*outs)
+    assert not outs[0][M:].any()
+
+
+@pytest.mark.parametrize("hybrid", [False, True])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_layer_gradients(grouped, hybrid, monkeypatch):
+    import importlib
+
+    ops = importlib.import_module("primus_turbo.pytorch.ops." + ("grouped_gemm_fp8" if grouped else "gemm_fp8"))
+    config = LP.Float8QuantConfig(granularity=G.BLOCKWISE, block_size=128, format=LP.Format.HYBRID if hybrid else LP.Format.E4M3)
+    lens = torch.tensor([1500, 0, 700, 1896], device="cuda")
+    k = 2064 if grouped else 4080
+    x = bf16_randn((4096, k), seed=1).cuda().requires_grad_()
+    w = bf16_randn((4, 2176, k) if grouped else (4224, k), seed=2).cuda().requires_grad_()
+    g = bf16_randn((4096, w.shape[-2]), seed=3).cuda()
+    used, grads = [], []
+    for on in (True, False):
+        real = (gimpl if grouped else impl).reads_kn_in_place
+        monkeypatch.setattr(ops, "reads_kn_in_place", lambda *a: used.append(real(*a)) or (on and used[-1]))
+        out = ops.grouped_gemm_fp8(x, w, lens, trans_b=True, config=config) if grouped else ops.gemm_fp8(x, w, trans_b=True, config=config)
+        grads.append((out, *torch.autograd.grad(out, (x, w), g)))
+    assert used == [True, True]
+    assert all(torch.equal(p, q) for p, q in zip(*grads))
