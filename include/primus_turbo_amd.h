@@ -356,6 +356,8 @@ PT_API int pt_dequantize_fp8_block(const void *q, int q_dtype, int64_t B, int64_
  *   y[r, c] = T(float(q[r, c]) * bits_to_f32(scale[r, c / 32] << 23))
  * over q [rows, cols] (cols % 32 == 0; FP4 packed), written as y [rows, cols] or, for
  * column-direction data, transposed back as y [cols, rows]. */
+/* (One exception to codes and scales coming in pairs: with 2-D blocks in the row direction and col_flags 9, col_scale may be given
+ * without col_q, for a product that reads the row codes along the other axis, pt_grouped_gemm_mx_kn.) */
 PT_API int pt_quantize_mx(const void *x, int x_dtype, int64_t B, int64_t M, int64_t N, int q_dtype,
                           void *row_q, void *row_scale, int row_flags, void *col_q, void *col_scale,
                           int col_flags, uint32_t sr_seed, void *stream);
@@ -606,6 +608,13 @@ PT_API int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, i
                               const int64_t *group_offs, const int64_t *group_offs_out, int64_t G,
                               int64_t a_rows, int64_t out_rows, int64_t N, int64_t K, void *workspace,
                               size_t workspace_bytes, int tile_cfg, void *stream);
+/* pt_grouped_gemm_mx for weights stored [G, K, N] (MXFP8; what a layer's backward product reads of the forward
+ * quantization of its weights, whose blocks are 32 x 32): scales word-major for both operands, a_words [K / 128, a_rows],
+ * b_words [G, K / 128, N]. K a multiple of 128, at least 512, N of 16, K * N below 2^31. Nothing is copied: no workspace. */
+PT_API int pt_grouped_gemm_mx_kn(const void *a, int a_dtype, const void *a_words, const void *b, int b_dtype,
+                                 const void *b_words, void *c, int c_dtype, const int64_t *group_offs,
+                                 const int64_t *group_offs_out, int64_t G, int64_t a_rows, int64_t out_rows,
+                                 int64_t N, int64_t K, void *stream);
 PT_API size_t pt_grouped_gemm_mx_workspace_bytes(int64_t G, int64_t a_rows, int64_t N, int64_t K);
 PT_API size_t pt_grouped_gemm_mx_variable_k_workspace_bytes(int64_t Ml, int64_t Nr, int64_t ld);
 PT_API int pt_grouped_gemm_mx_variable_k(const void *lhs, int lhs_dtype, const void *lhs_scale,

@@ -1,7 +1,7 @@
 // Scaled FP8 GEMM entry points: operand preparation (transposes / K padding), the
 // VECTOR-scale (tensorwise, rowwise) kernel instantiations and the C ABI. The BLOCK-scale
 // instantiations live in gemm_fp8_block.hip, which is compiled with MFMA results in VGPRs.
-#include "gemm_fp8_block8.h"
+#include "gemm_fp8_kernel.h"
 
 namespace pt {
 
@@ -283,7 +283,7 @@ static bool block_scale_copy_pays(int64_t M, int64_t N, int64_t K) {
 
 // B stored [K, N] with 128 x 128 blocks is read as it is by the 256 x 256 tile; the others want it transposed in the workspace.
 static bool block_nn_in_place(int64_t M, int64_t N, int64_t K, int tile_cfg) {
-    if (!b8_reads_kn(N, K))
+    if (!reads_kn(N, K))
         return false;
     return tile_cfg == 0 ? gemm_direct_tile(M, N, K, SCALE_BLOCK, false) < 0 && dense_tile<SCALE_BLOCK>(M, N, K / KSTEP, true) == 1
                          : tile_cfg == 1 || tile_cfg == 4;

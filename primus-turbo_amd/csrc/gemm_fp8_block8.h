@@ -54,12 +54,6 @@ constexpr int B8_LA = B8_BM / 8 / B8_WAVES, B8_LB = B8_BN / 8 / B8_WAVES; // row
 constexpr int B8_NL = B8_LA + B8_LB + 1;                                  // + one scale copy
 constexpr int B8_P1 = B8_LB + 1; // copies of a slab issued in row groups 6, 7 (B rows, scales)
 
-// Whether the kernel can read a B stored [K, N] where it is: whole slabs (nothing behind K may meet the matrix core), rows of
-// whole 16-byte groups, byte offsets of 32 bits.
-static inline bool b8_reads_kn(int64_t N, int64_t K) {
-    return K % KSTEP == 0 && K >= GEMM_MIN_SLABS * KSTEP && N % 16 == 0 && K * N < (1LL << 31);
-}
-
 template <int FA, int FB, int GMODE, bool SB_VEC, bool BT>
 __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmArgs a) {
     static_assert(GMODE == GROUP_NONE || GMODE == GROUP_ROWS, "row groups or none");
@@ -123,7 +117,7 @@ __global__ __launch_bounds__(B8_THREADS) void gemm_fp8_block8_kernel(const GemmA
             off[j] = static_cast<uint32_t>(row * (isA ? a.lda : a.ldb)) + ((pchk ^ swz(row)) << 4);
             if (BT && !isA) { // 1 KB = four K rows of the tile's 256 columns
                 const int k = ((j - LA) * B8_WAVES + wave) * 4 + (lane >> 4);
-                off[j]      = static_cast<uint32_t>(k * a.ldb) + (((lane & 15) ^ swz_t(k)) << 4);
+                off[j]      = static_cast<uint32_t>(k * a.ldb) + (((lane & 15) ^ swz_t<BN>(k)) << 4);
             }
         }
         if (wave < 4) // scale of tile row 64 wave + lane

@@ -20,7 +20,7 @@ static int grouped_rows_tile(int64_t G, int64_t M, int64_t N) {
 }
 // B stored [G, K, N] is read as it is by the 256 x 256 tile; the others want it transposed in the workspace
 static bool grouped_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K, int tile_cfg) {
-    return (tile_cfg == 0 ? grouped_rows_tile(G, M, N) : tile_cfg) == 4 && G > 0 && G <= 2048 && M > 0 && b8_reads_kn(N, K);
+    return (tile_cfg == 0 ? grouped_rows_tile(G, M, N) : tile_cfg) == 4 && G > 0 && G <= 2048 && M > 0 && reads_kn(N, K);
 }
 
 template <int GMODE, bool SB_VEC, int FA, int FB>

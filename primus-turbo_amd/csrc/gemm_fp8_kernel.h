@@ -138,16 +138,17 @@ typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 // each 16 lanes the i-th byte of the eight 16-byte rows whose halves those lanes address. A fragment (16 columns, the K bytes of
 // a lane group as above) takes four such reads instead of two of 16 bytes.
 // The 16-byte chunk c of stage row k sits at chunk c ^ swz_t(k): eight consecutive rows, and the rows 16 further that the
-// next lane group reads at the same time, hit all 64 banks once (256-byte rows).
+// next lane group reads at the same time, hit all 64 banks once (rows of 256 bytes, or two of 128).
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i32x2 *lds_i32x2_t;
-__device__ __forceinline__ int swz_t(int k) {
-    return (k & 7) | ((k >> 4 & 1) << 3);
+template <int ROW> __device__ __forceinline__ int swz_t(int k) {
+    static_assert(ROW == 128 || ROW == 256, "rows of a tile of 128 or 256 columns");
+    return ROW == 256 ? (k & 7) | ((k >> 4 & 1) << 3) : (k >> 1 & 3) | ((k >> 4 & 1) << 2);
 }
 // lane's byte offset of fragment `f` of a stage of ROW-byte rows; its reads lie 8, 64 and 72 rows further
 template <int ROW> __device__ __forceinline__ uint32_t transposed_offset(int lane, int f) {
     const int k = 16 * (lane >> 4) + ((lane & 15) >> 1);
-    return static_cast<uint32_t>(k * ROW + ((f ^ swz_t(k)) << 4) + (lane & 1) * 8);
+    return static_cast<uint32_t>(k * ROW + ((f ^ swz_t<ROW>(k)) << 4) + (lane & 1) * 8);
 }
 template <int ROW> __device__ __forceinline__ i32x8 read_transposed(const uint8_t *p) {
     i32x8 r{};
@@ -883,9 +884,10 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 // KS = 2: eight wavefronts, the slabs shared out to two teams of four in turn, each with stages of its own; at the
 // end the teams exchange half their sums through the LDS, and each writes half the tile. For dense products of at
 // most one tile a CU, where no second workgroup could hide the waits (see two_teams).
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS, bool BT>
 __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a) {
     static_assert(KS == 1 || (KS == 2 && GMODE == GROUP_NONE), "teams: dense products, one tile for each workgroup");
+    static_assert(!BT || (GMODE != GROUP_K && KS == 1 && FA != 4 && MODE == SCALE_MX), "B stored [K, N]: MXFP8, one team, one K range");
     static_assert(TN % 4 == 0 && TM % 2 == 0, "sub-tiles are multiples of 32 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -987,7 +989,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     if (tile >= total || (XPIPE && KT_ALL <= AHEAD))
         return;
     int     g_cur = 0, g_nxt = 0;
-    TileCtx cur_t = make_tile<BM, BN, GMODE, FA == 4>(a, tile, prefix, g_cur);
+    TileCtx cur_t = make_tile<BM, BN, GMODE, FA == 4, BT>(a, tile, prefix, g_cur);
     g_nxt         = g_cur;
 
     // ---- loader: two slabs ahead of the MFMAs ----
@@ -1013,6 +1015,12 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
             const bool isA = j < LA;
             const int  row = ((isA ? j : j - LA) * GEMM_WAVES + wave) * 8 + lrow;
             off[j] = static_cast<uint32_t>(row * (isA ? a.lda : a.ldb)) + ((pchk ^ swz(row)) << 4);
+            if constexpr (BT)
+                if (!isA) { // 1 KB = four or eight K rows of the tile's columns
+                    constexpr int CH = BN / 16;
+                    const int     k  = ((j - LA) * GEMM_WAVES + wave) * (64 / CH) + lane / CH;
+                    off[j]           = static_cast<uint32_t>(k * a.ldb) + ((lane % CH ^ swz_t<BN>(k)) << 4);
+                }
         }
         // scale copies: lane l of copy q fetches the word of the wavefront's row (or column)
         // 64 q + l, at an offset relative to the scale of the tile's first row / column (exact,
@@ -1052,12 +1060,20 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
             ld_sb_end = as_bytes(GMODE == GROUP_K ? a.sB : t.sB) + sb_extent;
         }
     };
+    // BT: to the end of the matrix (a column behind N reads the next row's, or zero: it is never stored)
+    [[maybe_unused]] const uint32_t kn_bytes = BT ? opaque_uniform(static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.ldb)) : 0;
+    [[maybe_unused]] auto bytes_b = [&](const TileCtx &t) {
+        return BT ? kn_bytes - static_cast<uint32_t>(t.n0) : t.rows_b * static_cast<uint32_t>(a.ldb);
+    };
+    // (in a register and opaque: where the compiler can work it out anew it does so behind a branch, and the slab has to
+    // stay one basic block)
+    [[maybe_unused]] const uint32_t step_b = BT ? opaque_uniform(KSTEP * static_cast<uint32_t>(a.ldb)) : KSTEP;
     TileCtx nxt_t     = cur_t; // tile after the MFMAs' tile (the same tile after the last one)
     auto    loader_to = [&](const TileCtx &t) {
         ld_ga = t.Ag + team * KSTEP;
         ld_gb = t.Bg + team * KSTEP;
         ld_na = t.rows_a * static_cast<uint32_t>(a.lda) - team * KSTEP;
-        ld_nb = t.rows_b * static_cast<uint32_t>(a.ldb) - team * KSTEP;
+        ld_nb = bytes_b(t) - team * KSTEP;
         ld_kt = team;
         ld_KT = t.KT;
         scales_to(t);
@@ -1080,7 +1096,16 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         uint8_t      *dst = stages + b * STAGE;
 #if defined(__HIP_DEVICE_COMPILE__) // the buffer resource type only exists in the device pass
         constexpr uint32_t RSRC_FLAGS = 0x00020000; // raw buffer, 32-bit data format
-        if constexpr (L >= NLD) {
+        if constexpr (BT && L >= NLD) {
+            constexpr int  Q = L - NLD, H = Q / (SC_ROWS / 64), QQ = Q % (SC_ROWS / 64);
+            constexpr bool isA = QQ * 64 < SC_A;
+            copy_to_lds<4, A_BYTES + B_BYTES + Q * 256>(dst + wave * SC_WAVE, isA ? ld_sa : ld_sb,
+                                                        isA ? bytes_left(ld_sa, ld_sa_end, H) : bytes_left(ld_sb, ld_sb_end, H), off[L]);
+        } else if constexpr (BT) {
+            constexpr bool isA = L < LA;
+            copy_to_lds<16, isA ? L * GEMM_WAVES * 1024 : A_BYTES + (L - LA) * GEMM_WAVES * 1024>(dst + wave * 1024, isA ? ld_ga : ld_gb,
+                                                                                                 isA ? ld_na : ld_nb, off[L]);
+        } else if constexpr (L >= NLD) {
             constexpr int  Q = L - NLD, H = Q / (SC_ROWS / 64), QQ = Q % (SC_ROWS / 64);
             constexpr bool isA = QQ * 64 < SC_A;
             __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
@@ -1102,8 +1127,34 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         constexpr int C = cc;
         issue_copy(std::integral_constant<int, (C < LB ? LA + C : NLD + (C - LB))>{}, b);
     };
+    // BT: where the loader goes at the end of its tile, worked out ahead of the K loop (as step_b is)
+    [[maybe_unused]] const uint8_t *to_ga = nullptr, *to_gb = nullptr, *to_sa = nullptr, *to_sb = nullptr, *to_sa_end = nullptr, *to_sb_end = nullptr;
+    [[maybe_unused]] uint32_t       to_na = 0, to_nb = 0;
+    auto set_next = [&]() {
+        if constexpr (BT) {
+            to_ga     = opaque_uniform(nxt_t.Ag);
+            to_gb     = opaque_uniform(nxt_t.Bg);
+            to_na     = opaque_uniform(nxt_t.rows_a * static_cast<uint32_t>(a.lda));
+            to_nb     = opaque_uniform(bytes_b(nxt_t));
+            to_sa     = opaque_uniform(as_bytes(nxt_t.sA) + (nxt_t.m0 >> a.sa_shift) * sa_rowp);
+            to_sb     = opaque_uniform(as_bytes(nxt_t.sB) + (nxt_t.n0 >> a.sb_shift) * sb_rowp);
+            to_sa_end = opaque_uniform(as_bytes(nxt_t.sA) + sa_extent);
+            to_sb_end = opaque_uniform(as_bytes(nxt_t.sB) + sb_extent);
+        }
+    };
     auto advance_loader = [&]() {
-        if constexpr (KS > 1) {
+        if constexpr (BT) {
+            const bool wrap = ld_kt + 1 == KT_ALL;
+            ld_kt     = wrap ? 0 : ld_kt + 1;
+            ld_ga     = wrap ? to_ga : ld_ga + KSTEP;
+            ld_gb     = wrap ? to_gb : ld_gb + step_b;
+            ld_na     = wrap ? to_na : ld_na - KSTEP;
+            ld_nb     = wrap ? to_nb : ld_nb - step_b;
+            ld_sa     = wrap ? to_sa : ld_sa + sa_step;
+            ld_sb     = wrap ? to_sb : ld_sb + sb_step;
+            ld_sa_end = wrap ? to_sa_end : ld_sa_end;
+            ld_sb_end = wrap ? to_sb_end : ld_sb_end;
+        } else if constexpr (KS > 1) {
             // behind the last slab nothing is read: the stages fill with zeros (as they do for the slab that a
             // team has more than the other)
             ld_kt += KS;
@@ -1201,6 +1252,14 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     };
     const uint32_t a_part = wm * (TM * 16) * KSTEP;
     const uint32_t b_part = A_BYTES + wn * (TN * 16) * KSTEP;
+    // (A_BYTES and wn * TN leave the bits of j free)
+    [[maybe_unused]] const uint32_t t_off = BT ? A_BYTES + transposed_offset<BT ? BN : 256>(lane, wn * TN) : 0;
+    auto ldfrag_b = [&](const uint8_t *stage, int j) {
+        if constexpr (BT)
+            return read_transposed<BN>(stage + (t_off ^ (j << 4)));
+        else
+            return ldfrag(stage + b_part, j);
+    };
 
     // pipeline start at tile t, in two steps: the first two slabs are requested (stages 0 and 1,
     // which nobody may still be reading) ...
@@ -1223,7 +1282,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         read_scales(stages);
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-            fb[j] = ldfrag(stages + b_part, j);
+            fb[j] = ldfrag_b(stages, j);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
             fa[i] = ldfrag(stages + a_part, i);
@@ -1255,7 +1314,8 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         const int next_tile = tile + gridDim.x;
         nxt_t               = cur_t;
         if (next_tile < total)
-            nxt_t = make_tile<BM, BN, GMODE, FA == 4>(a, next_tile, prefix, g_nxt);
+            nxt_t = make_tile<BM, BN, GMODE, FA == 4, BT>(a, next_tile, prefix, g_nxt);
+        set_next();
         const int KT = XPIPE ? (KT_ALL + KS - 1) / KS : cur_t.KT;
         if constexpr (!XPIPE) {
             if (KT > 0)
@@ -1420,7 +1480,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
                     pending = 0; // from the next slab on every wait is for copies younger than the stores
                     __builtin_amdgcn_s_barrier();
                 }
-                fb[j] = ldfrag(nxt + b_part, j); // column j is done: refill from the next slab
+                fb[j] = ldfrag_b(nxt, j); // column j is done: refill from the next slab
                 __builtin_amdgcn_sched_barrier(0);
             });
             if constexpr (MODE == SCALE_BLOCK) {
@@ -1540,7 +1600,7 @@ static inline int vk_pick_chunks(int64_t positions, int64_t grid, int64_t groups
 
 // Upper bound on the number of tiles (exact for the ungrouped case): GROUP_ROWS cannot know
 // the per-group row counts on the host, but every group adds at most one partial tile row.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4), int KS = 1>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4), int KS = 1, bool BT = false>
 static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int STAGES  = KS * NSTAGE * gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -1561,7 +1621,7 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
                              (a.sb_wpitch == 0 && a.sb_n % 4 != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
                              reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
-    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE, KS>;
+    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE, KS, BT>;
     // the attribute belongs to the (kernel, device) pair: one bit per device, set once
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
@@ -1672,6 +1732,20 @@ template <int MODE, bool F4 = false> static inline int dense_tile(int64_t M, int
 }
 // (Row groups do not take it: at 320 rows a group on average it gains 4 to 17 % over 128 x 128 tiles where the groups' sizes are
 // any numbers, and loses 2 % of a whole expert layer's step where they are padded to 128, since it pads them again.)
+// The tile of a row-grouped MX product: 1 = 256 x 256, 3 = 128 x 128. The larger tile fetches half the bytes from the L2 for each
+// product and multiplies more padding at a group's end, so the rows of a group decide (on average, as allocated; how uneven they are
+// is only known on the device). us of the forward product, 128x128 / 256x256, 32 groups, N = K = 4096, even
+// and uneven (two idle, the largest a fifth of all):
+//   MXFP8  256 rows a group 199 / 181, 220 / 228;  384: 267 / 250, 298 / 248;  448: 336 / 253, 333 / 302
+//   MXFP4  256              106 /  95, 125 / 144;  384: 156 / 161, 180 / 156;  448: 204 / 164, 189 / 184
+static inline int mx_rows_tile(const GemmArgs &a, bool fp4) {
+    return a.G > 0 && a.M / a.G >= (fp4 ? 448 : 384) && a.N >= 1024 ? 1 : 3;
+}
+// Whether the 32-bit byte offsets and whole slabs of a kernel that reads B where it lies, [K, N], fit it (nothing behind K may
+// meet the matrix core, rows are whole 16-byte groups).
+static inline bool reads_kn(int64_t N, int64_t K) {
+    return K % KSTEP == 0 && K >= GEMM_MIN_SLABS * KSTEP && N % 16 == 0 && K * N < (1LL << 31);
+}
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;
 }

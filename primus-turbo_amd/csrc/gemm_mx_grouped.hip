@@ -19,18 +19,8 @@ namespace pt {
 template <int GMODE, int FA, int FB> static int launch_mxg_tiles(const GemmArgs &a, int tile_cfg, hipStream_t stream) {
     // tile_cfg: 0 = auto, 1 = 256x256, 3 = 128x128 (two workgroups per CU), 4 = 256x256 with eight
     // wavefronts (row groups only)
-    if (tile_cfg == 0) {
-        // Row groups: the larger tile fetches half the bytes from the L2 for each product and multiplies more
-        // padding at a group's end, so the rows of a group decide (on average, as allocated; how uneven they are
-        // is only known on the device). us of the forward product, 128x128 / 256x256, 32 groups, N = K = 4096, even
-        // and uneven (two idle, the largest a fifth of all):
-        //   MXFP8  256 rows a group 199 / 181, 220 / 228;  384: 267 / 250, 298 / 248;  448: 336 / 253, 333 / 302
-        //   MXFP4  256              106 /  95, 125 / 144;  384: 156 / 161, 180 / 156;  448: 204 / 164, 189 / 184
-        constexpr int64_t ROWS = FA == 4 ? 448 : 384;
-        const bool big = GMODE == GROUP_K ? (a.M >= 1024 && a.N >= 1024)
-                                          : (a.G > 0 && a.M / a.G >= ROWS && a.N >= 1024);
-        tile_cfg       = big ? 1 : 3;
-    }
+    if (tile_cfg == 0)
+        tile_cfg = GMODE == GROUP_ROWS ? mx_rows_tile(a, FA == 4) : a.M >= 1024 && a.N >= 1024 ? 1 : 3;
     if constexpr (GMODE == GROUP_ROWS) {
         if (tile_cfg == 4)
             return launch_gemm_mx8<FA, FB, GROUP_ROWS>(a, stream);

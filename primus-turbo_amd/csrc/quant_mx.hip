@@ -162,7 +162,7 @@ struct MxArgs {
     int64_t     B, M, N, Mpad, Npad;
     uint8_t    *row_q; // [B, M, Npad] (FP4: Npad / 2 bytes per row) or NULL
     uint8_t    *row_s; // [B, M, Npad / 32] or NULL; word-major: [B, Npad / 128, rows, 4]
-    uint8_t    *col_q; // [B, N, Mpad] (FP4: Mpad / 2) or NULL
+    uint8_t    *col_q; // [B, N, Mpad] (FP4: Mpad / 2) or NULL (with 2-D blocks: col_s may be wanted by itself)
     uint8_t    *col_s; // [B, N, Mpad / 32] or NULL; word-major: [B, Mpad / 128, N, 4]
     // Bytes from the scale word of a row (column) to the next one's, and to the row's next word. Word-major
     // scales are what the GEMM reads (gemm_fp8_kernel.h): a tile's 128 words leave side by side, 512 bytes,
@@ -542,6 +542,14 @@ __global__ __launch_bounds__(256) void mx_quant_kernel(const MxArgs a) {
         if (tid < MX_TILE && tid < row_cnt)
             *reinterpret_cast<uint32_t *>(a.row_s + b * a.M * (a.Npad >> 5) + (row_dst0 - b * a.M + tid) * a.row_s_row + (n0 >> 7) * a.row_s_word) =
                 *reinterpret_cast<const uint32_t *>(&sbytes[tid * 4]);
+        if constexpr (ROW2D && !COL) // a column's word: its blocks of the four 32-row strips, which both directions share
+            if (a.col_s != nullptr && tid < MX_TILE && n0 + tid < a.N) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb)
+                    w |= static_cast<uint32_t>(sbytes[rb * 32 * 4 + (tid >> 5)]) << (8 * rb);
+                *reinterpret_cast<uint32_t *>(a.col_s + b * a.N * (a.Mpad >> 5) + (n0 + tid) * a.col_s_row + (m0 >> 7) * a.col_s_word) = w;
+            }
     }
 
     PT_MX_TRACE(3);
@@ -1022,7 +1030,10 @@ int pt_quantize_mx(const void *x, int x_dtype, int64_t B, int64_t M, int64_t N, 
     const int fmt = mx_fmt_of(q_dtype);
     PT_REQUIRE(fmt >= 0, "q_dtype must be e4m3, e5m2 or e2m1x2");
     PT_REQUIRE(B >= 0 && M >= 0 && N >= 0, "dimensions must be non-negative");
-    PT_REQUIRE((row_q != nullptr) == (row_scale != nullptr) && (col_q != nullptr) == (col_scale != nullptr),
+    // (2-D blocks are the same in both directions: a product that reads the row codes along the other axis
+    // needs the column scales alone)
+    const bool words_alone = row_q && !col_q && col_scale && (row_flags & 1) && col_flags == 9;
+    PT_REQUIRE((row_q != nullptr) == (row_scale != nullptr) && ((col_q != nullptr) == (col_scale != nullptr) || words_alone),
                "codes and scales come in pairs");
     PT_REQUIRE(row_q || col_q, "nothing to produce");
     if (const int rc = check_mx_flags(fmt, row_q ? row_flags : 0, col_q ? col_flags : 0))

@@ -195,6 +195,51 @@ def _grouped_mx(a, b, a_scales, b_scales, group_offs, group_offs_out, trans_a, t
     return out
 
 
+def mx_reads_kn(Nn: int, K: int) -> bool:
+    """Whether ``grouped_gemm_mx_kn_impl`` takes weights of ``K`` x ``Nn`` that were quantized in whole blocks of 128."""
+    return K % 128 == 0 and K >= 512 and Nn % 128 == 0 and K * Nn < 1 << 31
+
+
+@native_op("primus_turbo::grouped_gemm_mx_kn_impl", device_types="cuda")
+def grouped_gemm_mx_kn_impl(
+    a: torch.Tensor,
+    b: torch.Tensor,
+    a_words: torch.Tensor,
+    b_words: torch.Tensor,
+    group_offs: torch.Tensor,
+    group_offs_out: torch.Tensor,
+    out_dtype: torch.dtype,
+) -> torch.Tensor:
+    """The MXFP8 row-group product of ``grouped_gemm_fp8_impl`` with the weights as the forward product reads them: ``a [rows, K]``,
+    ``b [G, K, N]``, scales word-major, ``[K / 128, rows]`` and ``[G, K / 128, N]`` (``quantize_mx_weight_impl``). The layers'
+    backward product. (No counterpart in the reference.)"""
+    N.require_cuda(a, b, a_words, b_words, group_offs, group_offs_out)
+    _check(a.dim() == 2 and b.dim() == 3 and a.is_contiguous() and b.is_contiguous(), "a must be 2-D, b 3-D, both contiguous")
+    _check(a.dtype in _FP8 and b.dtype in _FP8, "operands must be float8_e4m3fn / float8_e5m2")
+    _check(out_dtype in (torch.float16, torch.bfloat16, torch.float32), "out_dtype must be float16, bfloat16 or float32")
+    G, K, Nn = b.shape
+    rows = a.shape[0]
+    _check(a.shape[1] == K, f"reduction dims differ: {a.shape[1]} vs {K}")
+    for t, shape in ((a_words, (K // 128, rows)), (b_words, (G, K // 128, Nn))):
+        _check(t.dtype == torch.int32 and tuple(t.shape) == shape and t.is_contiguous(), f"word-major scales must be {shape}")
+    for o in (group_offs, group_offs_out):
+        _check(o.dtype == torch.int64 and o.numel() == G + 1, "group offsets must be int64 [G + 1]")
+    out = torch.empty((rows, Nn), dtype=out_dtype, device=a.device)
+    N.check(
+        N.lib().pt_grouped_gemm_mx_kn(
+            N.ptr(a), N.dtype_code(a.dtype), N.ptr(a_words), N.ptr(b), N.dtype_code(b.dtype), N.ptr(b_words), N.ptr(out),
+            N.dtype_code(out_dtype), N.ptr(group_offs.contiguous()), N.ptr(group_offs_out.contiguous()), G, rows, rows, Nn, K,
+            N.stream_of(a),
+        )
+    )
+    return out
+
+
+@grouped_gemm_mx_kn_impl.register_fake
+def _grouped_gemm_mx_kn_impl_fake(a, b, a_words, b_words, group_offs, group_offs_out, out_dtype):
+    return torch.empty((a.shape[0], b.shape[2]), device=a.device, dtype=out_dtype)
+
+
 def _variable_k_mx(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans_c, out, accumulate):
     """MX variable K: ``out[g] = a[:, p[g]:p[g+1]] @ b[:, p[g]:p[g+1]]^T`` over the transposed
     column-direction outputs of the grouped quantizer (both K-contiguous already); ``p`` counts

@@ -1325,6 +1325,38 @@ def _quantize_mx_op_fake(x, out_dtype, want_row, want_col, row_flags, col_flags)
             mk(shapes[2], out_dtype), _mx_scales(lead, Nn, Mp, col_flags, x.device) if want_col else mk((0,), _E8M0))
 
 
+@native_op("primus_turbo::quantize_mx_weight")
+def quantize_mx_weight_impl(w: torch.Tensor, out_dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """MXFP8 weights ``w [G, N, K]`` in 32 x 32 blocks as the products of a layer read them, ``(codes [G, N, K],
+    words [G, K / 128, N], words_t [G, N / 128, K])``: the row direction of ``quantize_mx_operands`` and the scales of the other
+    one, whose codes are these, read along the other axis. N and K are multiples of 128. (No counterpart in the
+    reference, which writes the codes of both directions.)"""
+    N.require_cuda(w)
+    _check(w.dtype in (torch.bfloat16, torch.float16), "Input must be BFloat16 or Half")
+    _check(w.dim() == 3 and w.is_contiguous(), "Input must be contiguous, [G, N, K]")
+    _check(out_dtype in (torch.float8_e4m3fn, torch.float8_e5m2), "Output must be Float8_e4m3fn or Float8_e5m2")
+    G, M, Nn = w.shape
+    _check(M % 128 == 0 and Nn % 128 == 0, "N and K must be multiples of 128")
+    q = torch.empty(w.shape, dtype=out_dtype, device=w.device)
+    words = torch.empty((G, Nn // 128, M), dtype=torch.int32, device=w.device)
+    words_t = torch.empty((G, M // 128, Nn), dtype=torch.int32, device=w.device)
+    N.check(
+        N.lib().pt_quantize_mx(
+            N.ptr(w), N.dtype_code(w.dtype), G, M, Nn, N.dtype_code(out_dtype), N.ptr(q), N.ptr(words), 1 | _MX_WORDS, None,
+            N.ptr(words_t), 1 | _MX_WORDS, 0, N.stream_of(w),
+        )
+    )
+    return q, words, words_t
+
+
+@quantize_mx_weight_impl.register_fake
+def _quantize_mx_weight_impl_fake(w, out_dtype):
+    G, M, Nn = w.shape
+    return (torch.empty(w.shape, dtype=out_dtype, device=w.device),
+            torch.empty((G, Nn // 128, M), dtype=torch.int32, device=w.device),
+            torch.empty((G, M // 128, Nn), dtype=torch.int32, device=w.device))
+
+
 def _quantize_mx_impl(x, out_dtype, axis, block_size, with_trans, scaling_recipe, scaling_recipe_for_trans, what):
     assert block_size == 32, f"The block size must be 32 for {what} quantization"
     r, rt = _mx_recipes(with_trans, scaling_recipe, scaling_recipe_for_trans, what)

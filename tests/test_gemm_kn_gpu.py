@@ -123,3 +123,68 @@ def test_layer_gradients(grouped, hybrid, monkeypatch):
         grads.append((out, *torch.autograd.grad(out, (x, w), g)))
     assert used == [True, True]
     assert all(torch.equal(p, q) for p, q in zip(*grads))
+
+
+def _mx_weight(G_, n, k, fmt=E4M3, special=True):
+    w = bf16_randn((G_, n, k), seed=4).cuda() * torch.rand(G_, n // 32, k // 32, device="cuda").exp2().repeat_interleave(32, 1).repeat_interleave(32, 2)
+    w = w.to(torch.bfloat16)
+    if special:
+        w[0, :32, :64], w[-1, n - 1, k - 1], w[0, 40, 3] = 0, float("nan"), float("inf")
+    return w
+
+
+@pytest.mark.parametrize("shape", [(1, 128, 128), (3, 256, 640), (2, 1152, 384)])
+@pytest.mark.parametrize("fmt", [E4M3, E5M2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mx_weight_quantizer(shape, fmt, dtype):
+    """The codes of both directions are each other's transposition, and the scales those of the two-direction quantizer."""
+    w, recipe = _mx_weight(*shape).to(dtype), LP.ScalingRecipe(use_2d_block=True)
+    q, words, words_t = Q.quantize_mx_weight_impl(w, fmt)
+    rq, rs, cq, cs = Q.quantize_mx_operands(w, fmt, recipe, recipe, "MXFP8")
+    u8 = lambda t: t.contiguous().view(torch.uint8)  # noqa: E731
+    assert torch.equal(u8(q), u8(rq)) and torch.equal(u8(q.transpose(1, 2)), u8(cq))
+    assert torch.equal(words, rs) and torch.equal(words_t, cs)
+
+
+# rows of less than a tile, of a whole one, one over; columns that end inside a tile; both tiles (128 x 128 and 256 x 256)
+@pytest.mark.parametrize("lens", [[128, 0, 127, 1, 129], [700, 513, 0, 460], [33, 95, 256]])
+@pytest.mark.parametrize("n,k", [(128, 512), (1152, 640), (1408, 768)])
+@pytest.mark.parametrize("da", [E4M3, E5M2])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_mx_grouped(lens, n, k, da, out_dtype):
+    """grad [rows, k] x weight [G, k, n] as it lies against the product on the transposed quantization."""
+    w, recipe = _mx_weight(len(lens), k, n, special=False), LP.ScalingRecipe(use_2d_block=True)
+    x = bf16_randn((sum(lens), k), seed=5).cuda()
+    gl = torch.from_numpy(np.array(lens, dtype=np.int64)).cuda()
+    offs = torch.ops.primus_turbo_cpp_extension.grouped_gemm_compute_offs(gl)
+    xq, xs, _, _, _, orow, _, _ = Q.grouped_quantize_mx_operands(x, da, gl, offs, None, None, "MXFP8")
+    q, _, words_t = Q.quantize_mx_weight_impl(w, E4M3)
+    _, _, cq, cs = Q.quantize_mx_operands(w, E4M3, recipe, recipe, "MXFP8")
+    got = gimpl.grouped_gemm_mx_kn_impl(xq, q, xs, words_t, orow, offs, out_dtype)
+    want = gimpl.grouped_gemm_fp8_impl(xq, cq, xs, cs, gl, orow, False, True, out_dtype, G.MX_BLOCKWISE.value, None, 0, False, offs)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("hybrid", [False, True])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("n,k", [(640, 384), (512, 400)])  # (the second: blocks of 32, not of 128)
+def test_mx_layer_gradients(glu, hybrid, n, k, monkeypatch):
+    import importlib
+
+    ops = importlib.import_module("primus_turbo.pytorch.ops.grouped_gemm_fp8")
+    config = LP.Float8QuantConfig(granularity=G.MX_BLOCKWISE, block_size=32, scale_dtype=LP.ScaleDtype.E8M0,
+                                  format=LP.Format.HYBRID if hybrid else LP.Format.E4M3)
+    k = k // 32 * 32
+    lens = torch.tensor([300, 0, 213, 87], device="cuda")
+    x = bf16_randn((600, 2 * k if glu else k), seed=1).cuda().requires_grad_()
+    w = bf16_randn((4, n, k), seed=2).cuda().requires_grad_()
+    p = torch.rand(600, device="cuda").requires_grad_()
+    g = bf16_randn((600, n), seed=3).cuda()
+    used, grads = [], []
+    for on in (True, False):
+        monkeypatch.setattr(ops, "mx_reads_kn", lambda *a: used.append(gimpl.mx_reads_kn(*a)) or (on and used[-1]))
+        out = (ops.glu_grouped_gemm_fp8(x, p, w, lens, trans_b=True, config=config, act_type="silu") if glu else
+               ops.grouped_gemm_fp8(x, w, lens, trans_b=True, config=config))
+        grads.append((out, *torch.autograd.grad(out, (x, w, p) if glu else (x, w), g)))
+    assert used == ([True, True] if k % 128 == 0 else [])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
