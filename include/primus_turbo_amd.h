@@ -403,6 +403,8 @@ PT_API size_t pt_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K, int t
  * lies on the current device: such a product needs the workspace of trans_b 1, and its weight no transposed copy.
  * pt_grouped_gemm_fp8_nn_in_place says the same of pt_grouped_gemm_fp8, for any group sizes. */
 PT_API int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K);
+/* The same with vector scales, for trans_b 0 and either trans_a; such a product needs no workspace. */
+PT_API int pt_gemm_fp8_vec_in_place(int64_t M, int64_t N, int64_t K, int trans_a);
 PT_API int pt_grouped_gemm_fp8_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K);
 PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b, int b_dtype,
                        const float *b_scale, void *c, int c_dtype, int64_t M, int64_t N, int64_t K,

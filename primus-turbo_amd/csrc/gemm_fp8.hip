@@ -288,6 +288,16 @@ static bool block_nn_in_place(int64_t M, int64_t N, int64_t K, int tile_cfg) {
     return tile_cfg == 0 ? gemm_direct_tile(M, N, K, SCALE_BLOCK, false) < 0 && dense_tile<SCALE_BLOCK>(M, N, K / KSTEP, true) == 1
                          : tile_cfg == 1 || tile_cfg == 4;
 }
+// With vector scales the 256 x 256 tile reads B stored [K, N], and A stored [K, M] beside it.
+static bool vector_kn_in_place(int64_t M, int64_t N, int64_t K, bool at, int tile_cfg) {
+    if (!reads_kn(N, K) || (at && !reads_kn(M, K)))
+        return false;
+    return tile_cfg == 0 ? gemm_direct_tile(M, N, K, SCALE_VECTOR, false) < 0 && dense_tile<SCALE_VECTOR>(M, N, K / KSTEP, true) == 1
+                         : tile_cfg == 1 || tile_cfg == 4;
+}
+int pt_gemm_fp8_vec_in_place(int64_t M, int64_t N, int64_t K, int trans_a) {
+    return M > 0 && N > 0 && K > 0 && vector_kn_in_place(M, N, K, trans_a != 0, 0);
+}
 int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K) {
     return M > 0 && N > 0 && K > 0 && block_nn_in_place(M, N, K, 0);
 }
@@ -343,12 +353,13 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     const bool     pad       = Kp != K;
     const bool     nn        = scale_mode == SCALE_BLOCK && !trans_a && !trans_b && sa_block == 1 && sb_block == 128 &&
                     block_nn_in_place(M, N, K, tile_cfg);
-    const bool     copies    = trans_a || (!trans_b && !nn) || pad;
+    const bool     kn        = scale_mode == SCALE_VECTOR && !trans_b && vector_kn_in_place(M, N, K, trans_a != 0, tile_cfg);
+    const bool     copies    = (trans_a && !kn) || (!trans_b && !nn && !kn) || pad;
     const uint8_t *A   = static_cast<const uint8_t *>(a);
     const uint8_t *B   = static_cast<const uint8_t *>(b);
     // workspace layout: [scale area of block_scale_copy_pays problems][operand copies]
     const int64_t KB         = cdiv(K, 128);
-    const size_t  full       = pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, trans_b || nn);
+    const size_t  full       = pt_gemm_fp8_workspace_bytes(M, N, K, trans_a && !kn, trans_b || nn || kn);
     const bool    have_ws    = workspace != nullptr && aligned_to(workspace, 16) && workspace_bytes >= full;
     const size_t  scale_area = block_scale_copy_pays(M, N, K) ? static_cast<size_t>(round_up(M * KB * 4, 256)) : 0;
     // per-row A scales stored [M, K / 128] (sa_k == 1): hand the kernel a [K / 128, M] copy
@@ -395,9 +406,9 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
     g.M = M;
     g.N = N;
     g.K = Kp;
-    g.lda = Kp;
-    g.ldb = nn ? N : Kp;
-    g.b_kn = nn;
+    g.lda = kn && trans_a ? M : Kp;
+    g.ldb = nn || kn ? N : Kp;
+    g.b_kn = nn || kn;
     g.sa_m = sa_m;
     g.sa_k = sa_k;
     g.sb_n = sb_n;
@@ -414,6 +425,8 @@ int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b,
             g.lda = g.ldb = K;
         return launch_gemm_direct_mode(g, scale_mode, sb_block == 1, fa, fb, direct, st);
     }
+    if (kn)
+        return launch_gemm_vector_kn(g, fa, fb, trans_a != 0, st);
     if (scale_mode == SCALE_VECTOR)
         return launch_gemm_vector(g, fa, fb, tile_cfg, st);
     return launch_gemm_block(g, fa, fb, sb_block == 1, tile_cfg, st);

@@ -787,8 +787,9 @@ struct TileCtx {
 };
 
 // GROUP_ROWS: prefix[g] = number of tiles of the groups before g (in LDS), `g` is a search
-// hint that only moves forward as a workgroup walks its tiles. BT: B is stored [K, N] (see read_transposed).
-template <int BM, int BN, int GMODE, bool F4 = false, bool BT = false>
+// hint that only moves forward as a workgroup walks its tiles. BT: B is stored [K, N], AT: A is stored [K, M] (see
+// read_transposed).
+template <int BM, int BN, int GMODE, bool F4 = false, bool BT = false, bool AT = false>
 __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const int *prefix, int &g) {
     TileCtx t;
     t.g0 = t.g1 = 0;
@@ -797,7 +798,7 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
         tile_coords(tile, a.tiles_m, a.tiles_n, tm, tn);
         t.m0    = static_cast<int64_t>(tm) * BM;
         t.m_end = a.M;
-        t.Ag    = a.A + t.m0 * a.lda;
+        t.Ag    = a.A + (AT ? t.m0 : t.m0 * a.lda);
         t.Bg    = a.B;
         t.sA    = a.sA;
         t.sB    = a.sB;
@@ -884,10 +885,11 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 // KS = 2: eight wavefronts, the slabs shared out to two teams of four in turn, each with stages of its own; at the
 // end the teams exchange half their sums through the LDS, and each writes half the tile. For dense products of at
 // most one tile a CU, where no second workgroup could hide the waits (see two_teams).
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS, bool BT>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS, bool BT, bool AT>
 __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a) {
     static_assert(KS == 1 || (KS == 2 && GMODE == GROUP_NONE), "teams: dense products, one tile for each workgroup");
-    static_assert(!BT || (GMODE != GROUP_K && KS == 1 && FA != 4 && MODE == SCALE_MX), "B stored [K, N]: MXFP8, one team, one K range");
+    static_assert(!BT || (GMODE != GROUP_K && KS == 1 && FA != 4 && MODE != SCALE_BLOCK), "B stored [K, N]: FP8, one team, one K range");
+    static_assert(!AT || (BT && GMODE == GROUP_NONE), "A stored [K, M]: with B, dense products");
     static_assert(TN % 4 == 0 && TM % 2 == 0, "sub-tiles are multiples of 32 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -989,7 +991,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     if (tile >= total || (XPIPE && KT_ALL <= AHEAD))
         return;
     int     g_cur = 0, g_nxt = 0;
-    TileCtx cur_t = make_tile<BM, BN, GMODE, FA == 4, BT>(a, tile, prefix, g_cur);
+    TileCtx cur_t = make_tile<BM, BN, GMODE, FA == 4, BT, AT>(a, tile, prefix, g_cur);
     g_nxt         = g_cur;
 
     // ---- loader: two slabs ahead of the MFMAs ----
@@ -1015,11 +1017,18 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
             const bool isA = j < LA;
             const int  row = ((isA ? j : j - LA) * GEMM_WAVES + wave) * 8 + lrow;
             off[j] = static_cast<uint32_t>(row * (isA ? a.lda : a.ldb)) + ((pchk ^ swz(row)) << 4);
+            // 1 KB = four or eight K rows of the tile's columns
             if constexpr (BT)
-                if (!isA) { // 1 KB = four or eight K rows of the tile's columns
+                if (!isA) {
                     constexpr int CH = BN / 16;
                     const int     k  = ((j - LA) * GEMM_WAVES + wave) * (64 / CH) + lane / CH;
                     off[j]           = static_cast<uint32_t>(k * a.ldb) + ((lane % CH ^ swz_t<BN>(k)) << 4);
+                }
+            if constexpr (AT)
+                if (isA) {
+                    constexpr int CH = BM / 16;
+                    const int     k  = (j * GEMM_WAVES + wave) * (64 / CH) + lane / CH;
+                    off[j]           = static_cast<uint32_t>(k * a.lda) + ((lane % CH ^ swz_t<BM>(k)) << 4);
                 }
         }
         // scale copies: lane l of copy q fetches the word of the wavefront's row (or column)
@@ -1068,11 +1077,16 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     // (in a register and opaque: where the compiler can work it out anew it does so behind a branch, and the slab has to
     // stay one basic block)
     [[maybe_unused]] const uint32_t step_b = BT ? opaque_uniform(KSTEP * static_cast<uint32_t>(a.ldb)) : KSTEP;
+    [[maybe_unused]] const uint32_t km_bytes = AT ? opaque_uniform(static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.lda)) : 0;
+    [[maybe_unused]] auto bytes_a = [&](const TileCtx &t) {
+        return AT ? km_bytes - static_cast<uint32_t>(t.m0) : t.rows_a * static_cast<uint32_t>(a.lda);
+    };
+    [[maybe_unused]] const uint32_t step_a = AT ? opaque_uniform(KSTEP * static_cast<uint32_t>(a.lda)) : KSTEP;
     TileCtx nxt_t     = cur_t; // tile after the MFMAs' tile (the same tile after the last one)
     auto    loader_to = [&](const TileCtx &t) {
         ld_ga = t.Ag + team * KSTEP;
         ld_gb = t.Bg + team * KSTEP;
-        ld_na = t.rows_a * static_cast<uint32_t>(a.lda) - team * KSTEP;
+        ld_na = bytes_a(t) - team * KSTEP;
         ld_nb = bytes_b(t) - team * KSTEP;
         ld_kt = team;
         ld_KT = t.KT;
@@ -1134,26 +1148,30 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         if constexpr (BT) {
             to_ga     = opaque_uniform(nxt_t.Ag);
             to_gb     = opaque_uniform(nxt_t.Bg);
-            to_na     = opaque_uniform(nxt_t.rows_a * static_cast<uint32_t>(a.lda));
+            to_na     = opaque_uniform(bytes_a(nxt_t));
             to_nb     = opaque_uniform(bytes_b(nxt_t));
-            to_sa     = opaque_uniform(as_bytes(nxt_t.sA) + (nxt_t.m0 >> a.sa_shift) * sa_rowp);
-            to_sb     = opaque_uniform(as_bytes(nxt_t.sB) + (nxt_t.n0 >> a.sb_shift) * sb_rowp);
-            to_sa_end = opaque_uniform(as_bytes(nxt_t.sA) + sa_extent);
-            to_sb_end = opaque_uniform(as_bytes(nxt_t.sB) + sb_extent);
+            if constexpr (LDS_SC) {
+                to_sa     = opaque_uniform(as_bytes(nxt_t.sA) + (nxt_t.m0 >> a.sa_shift) * sa_rowp);
+                to_sb     = opaque_uniform(as_bytes(nxt_t.sB) + (nxt_t.n0 >> a.sb_shift) * sb_rowp);
+                to_sa_end = opaque_uniform(as_bytes(nxt_t.sA) + sa_extent);
+                to_sb_end = opaque_uniform(as_bytes(nxt_t.sB) + sb_extent);
+            }
         }
     };
     auto advance_loader = [&]() {
         if constexpr (BT) {
             const bool wrap = ld_kt + 1 == KT_ALL;
             ld_kt     = wrap ? 0 : ld_kt + 1;
-            ld_ga     = wrap ? to_ga : ld_ga + KSTEP;
+            ld_ga     = wrap ? to_ga : ld_ga + step_a;
             ld_gb     = wrap ? to_gb : ld_gb + step_b;
-            ld_na     = wrap ? to_na : ld_na - KSTEP;
+            ld_na     = wrap ? to_na : ld_na - step_a;
             ld_nb     = wrap ? to_nb : ld_nb - step_b;
-            ld_sa     = wrap ? to_sa : ld_sa + sa_step;
-            ld_sb     = wrap ? to_sb : ld_sb + sb_step;
-            ld_sa_end = wrap ? to_sa_end : ld_sa_end;
-            ld_sb_end = wrap ? to_sb_end : ld_sb_end;
+            if constexpr (LDS_SC) {
+                ld_sa     = wrap ? to_sa : ld_sa + sa_step;
+                ld_sb     = wrap ? to_sb : ld_sb + sb_step;
+                ld_sa_end = wrap ? to_sa_end : ld_sa_end;
+                ld_sb_end = wrap ? to_sb_end : ld_sb_end;
+            }
         } else if constexpr (KS > 1) {
             // behind the last slab nothing is read: the stages fill with zeros (as they do for the slab that a
             // team has more than the other)
@@ -1260,6 +1278,13 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         else
             return ldfrag(stage + b_part, j);
     };
+    [[maybe_unused]] const uint32_t ta_off = AT ? transposed_offset<AT ? BM : 256>(lane, wm * TM) : 0;
+    auto ldfrag_a = [&](const uint8_t *stage, int i) {
+        if constexpr (AT)
+            return read_transposed<BM>(stage + (ta_off ^ (i << 4)));
+        else
+            return ldfrag(stage + a_part, i);
+    };
 
     // pipeline start at tile t, in two steps: the first two slabs are requested (stages 0 and 1,
     // which nobody may still be reading) ...
@@ -1285,7 +1310,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
             fb[j] = ldfrag_b(stages, j);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-            fa[i] = ldfrag(stages + a_part, i);
+            fa[i] = ldfrag_a(stages, i);
     };
     // Stores of the result tile a wavefront has just written that may still be in flight (0, or the
     // count of the straight-line epilogue for 16-bit / fp32 outputs). They are younger than the
@@ -1314,7 +1339,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         const int next_tile = tile + gridDim.x;
         nxt_t               = cur_t;
         if (next_tile < total)
-            nxt_t = make_tile<BM, BN, GMODE, FA == 4, BT>(a, next_tile, prefix, g_nxt);
+            nxt_t = make_tile<BM, BN, GMODE, FA == 4, BT, AT>(a, next_tile, prefix, g_nxt);
         set_next();
         const int KT = XPIPE ? (KT_ALL + KS - 1) / KS : cur_t.KT;
         if constexpr (!XPIPE) {
@@ -1411,7 +1436,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
                     mma(i, j, h);
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (j == TN - 1 && h == NH - 1)
-                        fa[i] = ldfrag(nxt + a_part, i); // dead from here on: refill from the next slab
+                        fa[i] = ldfrag_a(nxt, i); // dead from here on: refill from the next slab
                     if constexpr (s >= S_B0 && s < S_B1)
                         static_for<(s - S_B0) * NB / (S_B1 - S_B0), (s + 1 - S_B0) * NB / (S_B1 - S_B0)>(
                             [&](auto c) { issue_part_b(c, buf_w); });
@@ -1600,7 +1625,7 @@ static inline int vk_pick_chunks(int64_t positions, int64_t grid, int64_t groups
 
 // Upper bound on the number of tiles (exact for the ungrouped case): GROUP_ROWS cannot know
 // the per-group row counts on the host, but every group adds at most one partial tile row.
-template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4), int KS = 1, bool BT = false>
+template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE = GROUP_NONE, int NSTAGE = gemm_stages(TM, TN, FA == 4), int KS = 1, bool BT = false, bool AT = false>
 static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int STAGES  = KS * NSTAGE * gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -1621,7 +1646,7 @@ static int launch_gemm_cfg(const GemmArgs &args_in, hipStream_t stream) {
                              (a.sb_wpitch == 0 && a.sb_n % 4 != 0) || a.sa_wpitch % 4 != 0 || a.sb_wpitch % 4 != 0 ||
                              reinterpret_cast<uintptr_t>(a.sA) % 4 != 0 || reinterpret_cast<uintptr_t>(a.sB) % 4 != 0))
         return fail(PT_ERR_INVALID_ARGUMENT, "gemm_mx: scale rows must be 4-byte aligned");
-    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE, KS, BT>;
+    auto kern            = gemm_fp8_nt_kernel<TM, TN, MODE, SB_VEC, FA, FB, GMODE, NSTAGE, KS, BT, AT>;
     // the attribute belongs to the (kernel, device) pair: one bit per device, set once
     static std::atomic<unsigned long long> attr_set{0};
     int                                    dev = 0;
@@ -1766,6 +1791,8 @@ int launch_zero_rows(void *c, const int64_t *offs, int64_t G, int64_t rows, int6
 // out[b][w * R + r] = in[b][r * pitch + w] for w < W (32-bit words): scale arrays made contiguous along their rows
 int launch_transpose_words(const uint32_t *in, uint32_t *out, int64_t R, int64_t W, int64_t pitch, hipStream_t st,
                             int64_t batch = 1);
+// The dense product with vector scales on 256 x 256 tiles with B stored [K, N], and A [K, M] if `at` (gemm_fp8_kn.hip)
+int  launch_gemm_vector_kn(const GemmArgs &a, int fa, int fb, bool at, hipStream_t stream);
 int  launch_gemm_block(const GemmArgs &a, int fa, int fb, bool sb_vec, int tile_cfg, hipStream_t stream);
 // The GEMM for few output tiles (gemm_direct.hip): its tile for an M x N product over rows of row_bytes, or -1
 // where the tiled kernel is the faster one; rows need whole 16-byte groups and pitches below 2^24, no padding.

@@ -29,6 +29,7 @@ struct Api {
 #define PT_FN(name) decltype(&::name) name
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
+    PT_FN(pt_gemm_fp8_vec_in_place);
     PT_FN(pt_gemm_mx);
     PT_FN(pt_gemm_mx_workspace_bytes);
     PT_FN(pt_quantize_fp8_tensorwise_static);
@@ -56,6 +57,7 @@ void bind_native(std::string path) {
     TORCH_CHECK(a.name != nullptr, "primus_turbo: ", path, " does not export " #name)
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
+    PT_FN(pt_gemm_fp8_vec_in_place);
     PT_FN(pt_gemm_mx);
     PT_FN(pt_gemm_mx_workspace_bytes);
     PT_FN(pt_quantize_fp8_tensorwise_static);
@@ -130,7 +132,7 @@ template <typename... Args> torch::jit::Stack general(const char *name, Args &&.
 // ---- products -------------------------------------------------------------------------------------------------------
 enum : int64_t { TENSORWISE = 1, ROWWISE = 2, BLOCKWISE = 3, MX_BLOCKWISE = 4 }; // ScalingGranularity
 
-// An NT product C[M, N] = A[M, K] . B[N, K]^T into `out`; false: a form for the Python body.
+// A product into `out` (MX: NT); false: a form for the Python body.
 bool launch_mx(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor &b_s, Tensor &out, bool accumulate) {
     const bool fp4 = a.scalar_type() == at::kFloat4_e2m1fn_x2;
     if (fp4 ? b.scalar_type() != at::kFloat4_e2m1fn_x2 : !is_fp8(a.scalar_type()) || !is_fp8(b.scalar_type()))
@@ -146,13 +148,13 @@ bool launch_mx(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor
                           code_of(out.scalar_type()), M, N, K, ld, ld, 0, 0, accumulate, nullptr, 0, 0, stream_of(a)) == PT_OK;
 }
 
-bool launch_scaled(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor &b_s, Tensor &out, bool trans_c,
-                   int64_t granularity, bool accumulate) {
+bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b, Tensor &out,
+                   bool trans_c, int64_t granularity, bool accumulate) {
     if (!is_fp8(a.scalar_type()) || !is_fp8(b.scalar_type()) || a_s.scalar_type() != at::kFloat || b_s.scalar_type() != at::kFloat)
         return false;
-    int64_t M = a.size(0), N = b.size(0);
-    const int64_t K = a.size(1), kb = cdiv(K, 128);
-    if (b.size(1) != K)
+    int64_t M = a.size(trans_a), N = b.size(!trans_b);
+    const int64_t K = a.size(!trans_a), kb = cdiv(K, 128);
+    if (b.size(trans_b) != K)
         return false;
     int     mode = 0, sa_blk = 1, sb_blk = 1;
     int64_t sa_m = 0, sa_k = 0, sb_n = 0, sb_k = 0;
@@ -164,6 +166,8 @@ bool launch_scaled(const Tensor &a, const Tensor &a_s, const Tensor &b, const Te
             return false;
         sa_m = sb_n = 1;
     } else if (granularity == BLOCKWISE) {
+        if (trans_a || !trans_b)
+            return false;
         if (a_s.dim() != 2 || b_s.dim() != 2 || !b_s.is_contiguous())
             return false;
         mode = 1;
@@ -189,36 +193,42 @@ bool launch_scaled(const Tensor &a, const Tensor &a_s, const Tensor &b, const Te
         std::swap(sa_m, sb_n);
         std::swap(sa_k, sb_k);
         std::swap(sa_blk, sb_blk);
+        const bool was_a = trans_a;
+        trans_a          = !trans_b;
+        trans_b          = !was_a;
     }
-    const size_t ws_bytes = api.pt_gemm_fp8_workspace_bytes(M, N, K, 0, 1);
+    const bool   in_place = mode == 0 && !trans_b && api.pt_gemm_fp8_vec_in_place(M, N, K, trans_a);
+    const size_t ws_bytes = in_place ? 0 : api.pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, trans_b);
     Tensor       ws;
     if (ws_bytes)
         ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, a);
     return api.pt_gemm_fp8(pa->data_ptr(), code_of(pa->scalar_type()), static_cast<const float *>(psa->data_ptr()), pb->data_ptr(),
                            code_of(pb->scalar_type()), static_cast<const float *>(psb->data_ptr()), out.data_ptr(),
-                           code_of(out.scalar_type()), M, N, K, 0, 1, mode, sa_m, sa_k, sb_n, sb_k, sa_blk, sb_blk, accumulate,
+                           code_of(out.scalar_type()), M, N, K, trans_a, trans_b, mode, sa_m, sa_k, sb_n, sb_k, sa_blk, sb_blk, accumulate,
                            ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, 0, stream_of(a)) == PT_OK;
 }
 
-bool launch_product(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor &b_s, Tensor &out, bool trans_c,
-                    int64_t granularity, bool accumulate) {
+bool launch_product(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b, Tensor &out,
+                    bool trans_c, int64_t granularity, bool accumulate) {
     if (granularity == MX_BLOCKWISE)
-        return trans_c ? launch_mx(b, b_s, a, a_s, out, accumulate) : launch_mx(a, a_s, b, b_s, out, accumulate);
-    return launch_scaled(a, a_s, b, b_s, out, trans_c, granularity, accumulate);
+        return !trans_a && trans_b && trans_c ? launch_mx(b, b_s, a, a_s, out, accumulate)
+               : !trans_a && trans_b          ? launch_mx(a, a_s, b, b_s, out, accumulate)
+                                              : false;
+    return launch_scaled(a, a_s, trans_a, b, b_s, trans_b, out, trans_c, granularity, accumulate);
 }
 
-bool product_form(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b) {
-    return !trans_a && trans_b && on_current_device(a) && a.dim() == 2 && b.dim() == 2 && plain(a, a) && plain(b, a) &&
+bool product_form(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor &b_s) {
+    return on_current_device(a) && a.dim() == 2 && b.dim() == 2 && plain(a, a) && plain(b, a) &&
            a_s.is_cuda() && b_s.is_cuda() && a_s.get_device() == a.get_device() && b_s.get_device() == a.get_device();
 }
 
 Tensor gemm_fp8(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b,
                 ScalarType out_dtype, bool trans_c, int64_t granularity, int64_t backend) {
-    if (product_form(a, a_s, trans_a, b, b_s, trans_b) && is_hp(out_dtype)) {
-        const int64_t M = a.size(0), N = b.size(0);
+    if (product_form(a, a_s, b, b_s) && is_hp(out_dtype)) {
+        const int64_t M = a.size(trans_a), N = b.size(!trans_b);
         Tensor        out = trans_c ? empty({N, M}, out_dtype, a) : empty({M, N}, out_dtype, a);
         if ((granularity != MX_BLOCKWISE || (plain(a_s, a) && plain(b_s, a))) &&
-            launch_product(a, a_s, b, b_s, out, trans_c, granularity, false))
+            launch_product(a, a_s, trans_a, b, b_s, trans_b, out, trans_c, granularity, false))
             return out;
     }
     return general("primus_turbo::gemm_fp8_impl_general", a, a_s, trans_a, b, b_s, trans_b, out_dtype, trans_c, granularity,
@@ -228,12 +238,12 @@ Tensor gemm_fp8(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &
 // out += the product; false: nothing was done
 bool gemm_fp8_into(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b,
                    bool trans_c, int64_t granularity, Tensor out) {
-    if (!product_form(a, a_s, trans_a, b, b_s, trans_b) || !is_hp(out.scalar_type()) || out.dim() != 2 || !plain(out, a) ||
-        out.size(0) != (trans_c ? b : a).size(0) || out.size(1) != (trans_c ? a : b).size(0))
+    if (!product_form(a, a_s, b, b_s) || !is_hp(out.scalar_type()) || out.dim() != 2 || !plain(out, a) ||
+        out.size(trans_c) != a.size(trans_a) || out.size(!trans_c) != b.size(!trans_b))
         return false;
     if (granularity == MX_BLOCKWISE && (!plain(a_s, a) || !plain(b_s, a)))
         return false;
-    return launch_product(a, a_s, b, b_s, out, trans_c, granularity, true);
+    return launch_product(a, a_s, trans_a, b, b_s, trans_b, out, trans_c, granularity, true);
 }
 
 // ---- quantizers -----------------------------------------------------------------------------------------------------

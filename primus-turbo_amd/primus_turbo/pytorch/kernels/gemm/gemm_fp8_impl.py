@@ -124,6 +124,11 @@ def reads_kn_in_place(M: int, Nn: int, K: int) -> bool:
     return bool(N.lib().pt_gemm_fp8_nn_in_place(M, Nn, K))
 
 
+def vec_reads_in_place(M: int, Nn: int, K: int, trans_a: bool) -> bool:
+    """The same of the products with vector scales, and of an ``a`` stored ``[K, M]`` beside it with ``trans_a``."""
+    return bool(N.lib().pt_gemm_fp8_vec_in_place(M, Nn, K, int(trans_a)))
+
+
 def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, granularity, accumulate):
     if granularity == ScalingGranularity.MX_BLOCKWISE:
         _check(not trans_a and trans_b, "MX_BLOCKWISE GEMM supports the NT layout only (trans_a=False, trans_b=True)")
@@ -161,6 +166,8 @@ def _launch(a, a_scale_inv, trans_a, b, b_scale_inv, trans_b, out, trans_c, gran
     ws = None
     in_place = (mode, sa_blk, sb_blk, trans_a, trans_b, TILE_CFG) == (1, 1, 128, False, False, 0) and reads_kn_in_place(M, Nn, K)
     ws_bytes = lib.pt_gemm_fp8_workspace_bytes(M, Nn, K, int(trans_a), int(trans_b or in_place))
+    if ws_bytes and mode == 0 and not trans_b and TILE_CFG == 0 and vec_reads_in_place(M, Nn, K, trans_a):
+        ws_bytes = 0
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
     N.check(

@@ -38,6 +38,7 @@ from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import (
     gemm_fp8_impl,
     get_gemm_logical_shape,
     reads_kn_in_place,
+    vec_reads_in_place,
 )
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quant_fp8_blockwise_dual_t_impl,
@@ -103,6 +104,13 @@ class FP8GemmTensorFunction(torch.autograd.Function):
         plain = not any(isinstance(t, QuantizedTensor) for t in (a, b, a_t, b_t)) and b.shape[0] % 16 == 0 and b.shape[1] % 16 == 0
         if plain:
             get_gemm_logical_shape(a, b, trans_a, trans_b)  # (padded to the same length different ones look alike)
+
+        # (the large tile reads the forward codes as they lie in both backward products: no transposed copies)
+        # (where the forward product needs no padding of its rows)
+        if (nt_bwd and plain and need_bwd and b.shape[1] % 128 == 0 and not torch.compiler.is_compiling() and a.is_cuda
+                and vec_reads_in_place(a.shape[0], b.shape[1], b.shape[0], False)
+                and vec_reads_in_place(b.shape[0], b.shape[1], a.shape[0], True)):
+            nt_bwd = False
 
         def operand(x, x_t):
             want_t = need_bwd and nt_bwd and not isinstance(x_t, QuantizedTensor)

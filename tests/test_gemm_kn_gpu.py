@@ -188,3 +188,55 @@ def test_mx_layer_gradients(glu, hybrid, n, k, monkeypatch):
         grads.append((out, *torch.autograd.grad(out, (x, w, p) if glu else (x, w), g)))
     assert used == ([True, True] if k % 128 == 0 else [])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 256, 512), (272, 528, 640), (16, 1008, 1152), (528, 112, 768)])
+@pytest.mark.parametrize("trans_a,trans_c", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("granularity", ["TENSORWISE", "ROWWISE"])
+@pytest.mark.parametrize("out_dtype,accumulate", [(torch.bfloat16, False), (torch.float16, True), (torch.float32, False), (torch.float32, True)])
+def test_vector_scales(M, N, K, trans_a, trans_c, granularity, out_dtype, accumulate, pinned):
+    a, b = bf16_randn((M, K), seed=1).cuda().to(E4M3), bf16_randn((N, K), seed=2).cuda().to(E5M2)
+    one = torch.full((), 0.5, device="cuda")
+    sa, sb = (torch.rand(M, 1, device="cuda"), torch.rand(N, 1, device="cuda")) if granularity == "ROWWISE" else (one, one)
+    old = torch.randn((N, M) if trans_c else (M, N), device="cuda").to(out_dtype)
+    got, want = old.clone(), old.clone()
+    impl._launch(a.t().contiguous() if trans_a else a, sa, trans_a, b.t().contiguous(), sb, False, got, trans_c, G[granularity], accumulate)
+    impl._launch(a, sa, False, b, sb, True, want, trans_c, G[granularity], accumulate)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("da", [E4M3, E5M2])
+@pytest.mark.parametrize("db", [E4M3, E5M2])
+def test_vector_scales_by_the_rule(da, db):
+    """Taken at a whole round of 256 x 256 tiles; in the operator as in its Python body."""
+    a, b = bf16_randn((4096, 1024), seed=1).cuda().to(da), bf16_randn((4096, 1024), seed=2).cuda().to(db)
+    one = torch.full((), 0.5, device="cuda")
+    assert impl.vec_reads_in_place(4096, 4096, 1024, True) and impl.vec_reads_in_place(4096, 4096, 1024, False)
+    args = (torch.bfloat16, False, G.TENSORWISE.value, 1)
+    want = impl.gemm_fp8_impl(a, one, False, b, one, True, *args)
+    bt = b.t().contiguous()
+    for op in (impl.gemm_fp8_impl, torch.ops.primus_turbo.gemm_fp8_impl_general):
+        assert torch.equal(op(a, one, False, bt, one, False, *args), want)
+        assert torch.equal(op(a.t().contiguous(), one, True, bt, one, False, *args), want)
+
+
+@pytest.mark.parametrize("hybrid", [False, True])
+@pytest.mark.parametrize("main_grad", [False, True])
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 4096), (4096, 4096, 4080)])  # (the second: rows that are no whole slabs)
+def test_tensorwise_layer_gradients(M, N, K, main_grad, hybrid, monkeypatch):
+    import importlib
+
+    ops = importlib.import_module("primus_turbo.pytorch.ops.gemm_fp8")
+    config = LP.Float8QuantConfig(format=LP.Format.HYBRID if hybrid else LP.Format.E4M3)
+    x, g = bf16_randn((M, K), seed=1).cuda().requires_grad_(), bf16_randn((M, N), seed=3).cuda()
+    used, grads = [], []
+    for on in (True, False):
+        monkeypatch.setattr(ops, "vec_reads_in_place", lambda *a: used.append(impl.vec_reads_in_place(*a)) or (on and used[-1]))
+        w = torch.nn.Parameter(bf16_randn((N, K), seed=2).cuda())
+        if main_grad:
+            w.main_grad, w.grad_added_to_main_grad = torch.full(w.shape, 0.25, device="cuda"), False
+        out = ops.gemm_fp8(x, w, trans_b=True, config=config, fuse_bgrad_accum_pattern="megatron" if main_grad else None)
+        gx, gw = torch.autograd.grad(out, (x, w), g)
+        grads.append((out, gx, w.main_grad if main_grad else gw))
+    assert used == ([True, True, True] if K % 128 == 0 else [])  # (the patched rule is asked once, and says no)
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
