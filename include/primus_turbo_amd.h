@@ -610,9 +610,10 @@ PT_API int pt_grouped_gemm_mx(const void *a, int a_dtype, const void *a_scale, i
                               const int64_t *group_offs, const int64_t *group_offs_out, int64_t G,
                               int64_t a_rows, int64_t out_rows, int64_t N, int64_t K, void *workspace,
                               size_t workspace_bytes, int tile_cfg, void *stream);
-/* pt_grouped_gemm_mx for weights stored [G, K, N] (MXFP8; what a layer's backward product reads of the forward
+/* pt_grouped_gemm_mx for weights stored [G, K, N] (what a layer's backward product reads of the forward
  * quantization of its weights, whose blocks are 32 x 32): scales word-major for both operands, a_words [K / 128, a_rows],
- * b_words [G, K / 128, N]. K a multiple of 128, at least 512, N of 16, K * N below 2^31. Nothing is copied: no workspace. */
+ * b_words [G, K / 128, N]. K a multiple of 128, at least 512, N of 16, K * N below 2^31 (e2m1x2: 256, 1024, 32, 2^32).
+ * Nothing is copied: no workspace. */
 PT_API int pt_grouped_gemm_mx_kn(const void *a, int a_dtype, const void *a_words, const void *b, int b_dtype,
                                  const void *b_words, void *c, int c_dtype, const int64_t *group_offs,
                                  const int64_t *group_offs_out, int64_t G, int64_t a_rows, int64_t out_rows,

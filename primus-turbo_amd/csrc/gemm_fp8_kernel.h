@@ -141,20 +141,31 @@ typedef const __attribute__((address_space(1))) void *glb_ptr_t;
 // next lane group reads at the same time, hit all 64 banks once (rows of 256 bytes, or two of 128).
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) i32x2 *lds_i32x2_t;
-template <int ROW> __device__ __forceinline__ int swz_t(int k) {
-    static_assert(ROW == 128 || ROW == 256, "rows of a tile of 128 or 256 columns");
+// MXFP4 (F4): a row holds two columns a byte, a slab 256 rows, and ds_read_b64_tr_b4 gives lane i of sixteen the i-th code of the
+// sixteen 8-byte pieces that those lanes address. A lane group's two reads for an MFMA's K lie 16 rows apart. (Sixteen rows
+// hit 32 banks once; the next lane group's, 32 further, the same ones: a chunk holds two pieces, which its place cannot part.)
+template <int ROW, bool F4 = false> __device__ __forceinline__ int swz_t(int k) {
+    static_assert(F4 ? ROW == 64 || ROW == 128 : ROW == 128 || ROW == 256, "rows of a tile of 128 or 256 columns");
+    if constexpr (F4)
+        return ROW == 128 ? k >> 1 & 7 : k >> 2 & 3;
     return ROW == 256 ? (k & 7) | ((k >> 4 & 1) << 3) : (k >> 1 & 3) | ((k >> 4 & 1) << 2);
 }
-// lane's byte offset of fragment `f` of a stage of ROW-byte rows; its reads lie 8, 64 and 72 rows further
-template <int ROW> __device__ __forceinline__ uint32_t transposed_offset(int lane, int f) {
-    const int k = 16 * (lane >> 4) + ((lane & 15) >> 1);
-    return static_cast<uint32_t>(k * ROW + ((f ^ swz_t<ROW>(k)) << 4) + (lane & 1) * 8);
+// lane's byte offset of fragment `f` of a stage of ROW-byte rows; its reads lie 8, 64 and 72 (F4: 16, 128, 144) rows further
+template <int ROW, bool F4 = false> __device__ __forceinline__ uint32_t transposed_offset(int lane, int f) {
+    const int k = F4 ? 32 * (lane >> 4) + (lane & 15) : 16 * (lane >> 4) + ((lane & 15) >> 1);
+    return static_cast<uint32_t>(k * ROW + (F4 ? (f << 3) ^ (swz_t<ROW, F4>(k) << 4) : ((f ^ swz_t<ROW, F4>(k)) << 4) + (lane & 1) * 8));
 }
-template <int ROW> __device__ __forceinline__ i32x8 read_transposed(const uint8_t *p) {
+template <int ROW, bool F4 = false> __device__ __forceinline__ i32x8 read_transposed(const uint8_t *p) {
     i32x8 r{};
 #if defined(__HIP_DEVICE_COMPILE__)
-    auto at = [&](int row) { return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2_t)(p + row * ROW)); };
-    const i32x2 a = at(0), b = at(8), c = at(64), d = at(72);
+    constexpr int S = F4 ? 2 : 1;
+    auto at = [&](int row) {
+        if constexpr (F4)
+            return __builtin_amdgcn_ds_read_tr4_b64_v2i32((lds_i32x2_t)(p + row * ROW));
+        else
+            return __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2_t)(p + row * ROW));
+    };
+    const i32x2 a = at(0), b = at(8 * S), c = at(64 * S), d = at(72 * S);
     r[0] = a.x; r[1] = a.y; r[2] = b.x; r[3] = b.y;
     r[4] = c.x; r[5] = c.y; r[6] = d.x; r[7] = d.y;
 #endif
@@ -854,7 +865,7 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
     t.n0     = static_cast<int64_t>(tn) * BN;
     t.rows_a = (t.m_end - t.m0) < BM ? static_cast<int>(t.m_end - t.m0) : BM;
     t.rows_b = (a.N - t.n0) < BN ? static_cast<int>(a.N - t.n0) : BN;
-    t.Bg += BT ? t.n0 : t.n0 * a.ldb;
+    t.Bg += BT ? (F4 ? t.n0 / 2 : t.n0) : t.n0 * a.ldb;
     return t;
 }
 
@@ -888,8 +899,8 @@ __device__ __forceinline__ TileCtx make_tile(const GemmArgs &a, int tile, const 
 template <int TM, int TN, int MODE, bool SB_VEC, int FA, int FB, int GMODE, int NSTAGE, int KS, bool BT, bool AT>
 __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a) {
     static_assert(KS == 1 || (KS == 2 && GMODE == GROUP_NONE), "teams: dense products, one tile for each workgroup");
-    static_assert(!BT || (GMODE != GROUP_K && KS == 1 && FA != 4 && MODE != SCALE_BLOCK), "B stored [K, N]: FP8, one team, one K range");
-    static_assert(!AT || (BT && GMODE == GROUP_NONE), "A stored [K, M]: with B, dense products");
+    static_assert(!BT || (GMODE != GROUP_K && KS == 1 && MODE != SCALE_BLOCK), "B stored [K, N]: one team, one K range");
+    static_assert(!AT || (BT && GMODE == GROUP_NONE && FA != 4), "A stored [K, M]: with B, dense products");
     static_assert(TN % 4 == 0 && TM % 2 == 0, "sub-tiles are multiples of 32 x 64");
     constexpr int BM = 2 * TM * 16, BN = 2 * TN * 16;
     constexpr int A_BYTES = BM * KSTEP, B_BYTES = BN * KSTEP, STAGE = gemm_stage_bytes(TM, TN, MODE, FA == 4);
@@ -906,6 +917,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     constexpr bool F4 = FA == 4;
     static_assert((FA == 4) == (FB == 4), "FP4 operands come in pairs");
     constexpr int NH = F4 ? 2 : 1; // MFMAs per fragment pair
+    constexpr int B_ROW = F4 ? BN / 2 : BN; // BT: bytes of a stage row of B
     // BLOCK and MX modes: the scales of a slab travel with it through the stages. Per row
     // (column) of the wavefront's sub-tile and slab that is one 32-bit word -- an fp32 block
     // scale, or the E8M0 bytes of four 32-wide K blocks (two words for MXFP4) -- fetched 64 rows
@@ -1017,12 +1029,12 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
             const bool isA = j < LA;
             const int  row = ((isA ? j : j - LA) * GEMM_WAVES + wave) * 8 + lrow;
             off[j] = static_cast<uint32_t>(row * (isA ? a.lda : a.ldb)) + ((pchk ^ swz(row)) << 4);
-            // 1 KB = four or eight K rows of the tile's columns
+            // 1 KB = four K rows of the tile's columns, or eight or sixteen
             if constexpr (BT)
                 if (!isA) {
-                    constexpr int CH = BN / 16;
+                    constexpr int CH = B_ROW / 16;
                     const int     k  = ((j - LA) * GEMM_WAVES + wave) * (64 / CH) + lane / CH;
-                    off[j]           = static_cast<uint32_t>(k * a.ldb) + ((lane % CH ^ swz_t<BN>(k)) << 4);
+                    off[j]           = static_cast<uint32_t>(k * a.ldb) + ((lane % CH ^ swz_t<B_ROW, F4>(k)) << 4);
                 }
             if constexpr (AT)
                 if (isA) {
@@ -1070,13 +1082,13 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
         }
     };
     // BT: to the end of the matrix (a column behind N reads the next row's, or zero: it is never stored)
-    [[maybe_unused]] const uint32_t kn_bytes = BT ? opaque_uniform(static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.ldb)) : 0;
+    [[maybe_unused]] const uint32_t kn_bytes = BT ? opaque_uniform((F4 ? 2 : 1) * static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.ldb)) : 0;
     [[maybe_unused]] auto bytes_b = [&](const TileCtx &t) {
-        return BT ? kn_bytes - static_cast<uint32_t>(t.n0) : t.rows_b * static_cast<uint32_t>(a.ldb);
+        return BT ? kn_bytes - static_cast<uint32_t>(F4 ? t.n0 / 2 : t.n0) : t.rows_b * static_cast<uint32_t>(a.ldb);
     };
     // (in a register and opaque: where the compiler can work it out anew it does so behind a branch, and the slab has to
     // stay one basic block)
-    [[maybe_unused]] const uint32_t step_b = BT ? opaque_uniform(KSTEP * static_cast<uint32_t>(a.ldb)) : KSTEP;
+    [[maybe_unused]] const uint32_t step_b = BT ? opaque_uniform((F4 ? 2 : 1) * KSTEP * static_cast<uint32_t>(a.ldb)) : KSTEP;
     [[maybe_unused]] const uint32_t km_bytes = AT ? opaque_uniform(static_cast<uint32_t>(a.K) * static_cast<uint32_t>(a.lda)) : 0;
     [[maybe_unused]] auto bytes_a = [&](const TileCtx &t) {
         return AT ? km_bytes - static_cast<uint32_t>(t.m0) : t.rows_a * static_cast<uint32_t>(a.lda);
@@ -1271,10 +1283,10 @@ __global__ __launch_bounds__(256 * KS) void gemm_fp8_nt_kernel(const GemmArgs a)
     const uint32_t a_part = wm * (TM * 16) * KSTEP;
     const uint32_t b_part = A_BYTES + wn * (TN * 16) * KSTEP;
     // (A_BYTES and wn * TN leave the bits of j free)
-    [[maybe_unused]] const uint32_t t_off = BT ? A_BYTES + transposed_offset<BT ? BN : 256>(lane, wn * TN) : 0;
+    [[maybe_unused]] const uint32_t t_off = BT ? A_BYTES + transposed_offset<B_ROW, F4>(lane, wn * TN) : 0;
     auto ldfrag_b = [&](const uint8_t *stage, int j) {
         if constexpr (BT)
-            return read_transposed<BN>(stage + (t_off ^ (j << 4)));
+            return read_transposed<B_ROW, F4>(stage + (t_off ^ (j << (F4 ? 3 : 4))));
         else
             return ldfrag(stage + b_part, j);
     };
@@ -1768,8 +1780,9 @@ static inline int mx_rows_tile(const GemmArgs &a, bool fp4) {
 }
 // Whether the 32-bit byte offsets and whole slabs of a kernel that reads B where it lies, [K, N], fit it (nothing behind K may
 // meet the matrix core, rows are whole 16-byte groups).
-static inline bool reads_kn(int64_t N, int64_t K) {
-    return K % KSTEP == 0 && K >= GEMM_MIN_SLABS * KSTEP && N % 16 == 0 && K * N < (1LL << 31);
+static inline bool reads_kn(int64_t N, int64_t K, bool fp4 = false) {
+    const int64_t codes = fp4 ? 2 : 1; // a byte
+    return K % (KSTEP * codes) == 0 && K >= GEMM_MIN_SLABS * KSTEP * codes && N % (16 * codes) == 0 && K * N / codes < (1LL << 31);
 }
 static inline int64_t round_up(int64_t x, int64_t m) {
     return (x + m - 1) / m * m;

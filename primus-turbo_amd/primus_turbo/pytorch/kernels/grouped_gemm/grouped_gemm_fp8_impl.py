@@ -195,9 +195,10 @@ def _grouped_mx(a, b, a_scales, b_scales, group_offs, group_offs_out, trans_a, t
     return out
 
 
-def mx_reads_kn(Nn: int, K: int) -> bool:
+def mx_reads_kn(Nn: int, K: int, fp4: bool = False) -> bool:
     """Whether ``grouped_gemm_mx_kn_impl`` takes weights of ``K`` x ``Nn`` that were quantized in whole blocks of 128."""
-    return K % 128 == 0 and K >= 512 and Nn % 128 == 0 and K * Nn < 1 << 31
+    pack = 2 if fp4 else 1
+    return K % (128 * pack) == 0 and K >= 512 * pack and Nn % 128 == 0 and K * Nn // pack < 1 << 31
 
 
 @native_op("primus_turbo::grouped_gemm_mx_kn_impl", device_types="cuda")
@@ -210,16 +211,18 @@ def grouped_gemm_mx_kn_impl(
     group_offs_out: torch.Tensor,
     out_dtype: torch.dtype,
 ) -> torch.Tensor:
-    """The MXFP8 row-group product of ``grouped_gemm_fp8_impl`` with the weights as the forward product reads them: ``a [rows, K]``,
-    ``b [G, K, N]``, scales word-major, ``[K / 128, rows]`` and ``[G, K / 128, N]`` (``quantize_mx_weight_impl``). The layers'
+    """The MX row-group product of ``grouped_gemm_fp8_impl`` with the weights as the forward product reads them: ``a [rows, K]``,
+    ``b [G, K, N]`` (MXFP4: half as many bytes a row), scales word-major, ``[K / 128, rows]`` and ``[G, K / 128, N]`` (``quantize_mx_weight_impl``). The layers'
     backward product. (No counterpart in the reference.)"""
     N.require_cuda(a, b, a_words, b_words, group_offs, group_offs_out)
     _check(a.dim() == 2 and b.dim() == 3 and a.is_contiguous() and b.is_contiguous(), "a must be 2-D, b 3-D, both contiguous")
-    _check(a.dtype in _FP8 and b.dtype in _FP8, "operands must be float8_e4m3fn / float8_e5m2")
+    fp4 = _FP4X2 is not None and a.dtype == _FP4X2
+    _check(b.dtype == _FP4X2 if fp4 else (a.dtype in _FP8 and b.dtype in _FP8), "operands must both be fp8 or both fp4")
     _check(out_dtype in (torch.float16, torch.bfloat16, torch.float32), "out_dtype must be float16, bfloat16 or float32")
-    G, K, Nn = b.shape
+    pack = 2 if fp4 else 1
+    G, K, Nn = b.shape[0], b.shape[1], b.shape[2] * pack
     rows = a.shape[0]
-    _check(a.shape[1] == K, f"reduction dims differ: {a.shape[1]} vs {K}")
+    _check(a.shape[1] * pack == K, f"reduction dims differ: {a.shape[1] * pack} vs {K}")
     for t, shape in ((a_words, (K // 128, rows)), (b_words, (G, K // 128, Nn))):
         _check(t.dtype == torch.int32 and tuple(t.shape) == shape and t.is_contiguous(), f"word-major scales must be {shape}")
     for o in (group_offs, group_offs_out):
@@ -237,7 +240,7 @@ def grouped_gemm_mx_kn_impl(
 
 @grouped_gemm_mx_kn_impl.register_fake
 def _grouped_gemm_mx_kn_impl_fake(a, b, a_words, b_words, group_offs, group_offs_out, out_dtype):
-    return torch.empty((a.shape[0], b.shape[2]), device=a.device, dtype=out_dtype)
+    return torch.empty((a.shape[0], b.shape[2] * (2 if a.dtype == _FP4X2 else 1)), device=a.device, dtype=out_dtype)
 
 
 def _variable_k_mx(a, b, a_scales, b_scales, group_offs, trans_a, trans_b, trans_c, out, accumulate):

@@ -1327,17 +1327,19 @@ def _quantize_mx_op_fake(x, out_dtype, want_row, want_col, row_flags, col_flags)
 
 @native_op("primus_turbo::quantize_mx_weight")
 def quantize_mx_weight_impl(w: torch.Tensor, out_dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """MXFP8 weights ``w [G, N, K]`` in 32 x 32 blocks as the products of a layer read them, ``(codes [G, N, K],
-    words [G, K / 128, N], words_t [G, N / 128, K])``: the row direction of ``quantize_mx_operands`` and the scales of the other
+    """MXFP8 / MXFP4 weights ``w [G, N, K]`` in 32 x 32 blocks as the products of a layer read them, ``(codes [G, N, K]
+    (MXFP4: K / 2), words [G, K / 128, N], words_t [G, N / 128, K])``: the row direction of ``quantize_mx_operands`` and the scales of the other
     one, whose codes are these, read along the other axis. N and K are multiples of 128. (No counterpart in the
     reference, which writes the codes of both directions.)"""
     N.require_cuda(w)
     _check(w.dtype in (torch.bfloat16, torch.float16), "Input must be BFloat16 or Half")
     _check(w.dim() == 3 and w.is_contiguous(), "Input must be contiguous, [G, N, K]")
-    _check(out_dtype in (torch.float8_e4m3fn, torch.float8_e5m2), "Output must be Float8_e4m3fn or Float8_e5m2")
+    fp4 = _FP4X2 is not None and out_dtype == _FP4X2
+    _check(fp4 or out_dtype in (torch.float8_e4m3fn, torch.float8_e5m2),
+           "Output must be Float8_e4m3fn, Float8_e5m2 or Float4_e2m1fn_x2")
     G, M, Nn = w.shape
     _check(M % 128 == 0 and Nn % 128 == 0, "N and K must be multiples of 128")
-    q = torch.empty(w.shape, dtype=out_dtype, device=w.device)
+    q = torch.empty((G, M, Nn // 2 if fp4 else Nn), dtype=torch.uint8, device=w.device).view(out_dtype)
     words = torch.empty((G, Nn // 128, M), dtype=torch.int32, device=w.device)
     words_t = torch.empty((G, M // 128, Nn), dtype=torch.int32, device=w.device)
     N.check(
@@ -1352,7 +1354,8 @@ def quantize_mx_weight_impl(w: torch.Tensor, out_dtype: torch.dtype) -> Tuple[to
 @quantize_mx_weight_impl.register_fake
 def _quantize_mx_weight_impl_fake(w, out_dtype):
     G, M, Nn = w.shape
-    return (torch.empty(w.shape, dtype=out_dtype, device=w.device),
+    fp4 = _FP4X2 is not None and out_dtype == _FP4X2
+    return (torch.empty((G, M, Nn // 2 if fp4 else Nn), dtype=torch.uint8, device=w.device).view(out_dtype),
             torch.empty((G, Nn // 128, M), dtype=torch.int32, device=w.device),
             torch.empty((G, M // 128, Nn), dtype=torch.int32, device=w.device))
 

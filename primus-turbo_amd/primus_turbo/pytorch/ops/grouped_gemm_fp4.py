@@ -38,12 +38,14 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp4_impl import (
     grouped_gemm_fp4_variable_k_accum_impl,
     grouped_gemm_fp4_variable_k_impl,
 )
+from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import grouped_gemm_mx_kn_impl, mx_reads_kn
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     _MX_WORDS,
     glu_grouped_quantize_mx_impl,
     grouped_quantize_mx_operands,
     quantize_mx_operands,
+    quantize_mx_weight_impl,
     quantize_mxfp4_impl,
 )
 from primus_turbo.pytorch.ops.utils import (
@@ -87,6 +89,10 @@ def _fp4_weight_operands(b, b_t, config, need_bwd):
                                                scaling_recipe=w_recipe)
             assert isinstance(b_t, QuantizedTensor)
             b_col, b_col_s = b_t.qdata, b_t.scale_inv
+    elif need_bwd and b.shape[2] % 128 == 0 and mx_reads_kn(b.shape[2], b.shape[1], True) and b.dtype in (torch.bfloat16, torch.float16):
+        # backward reads the same codes along the other axis: no transposed copy (None), its scales alone
+        assert bs == 32, "The block size must be 32 for MXFP4 quantization"
+        b_row, b_row_s, b_col_s = quantize_mx_weight_impl(b.contiguous(), float4_e2m1fn_x2)
     elif need_bwd:
         assert bs == 32, "The block size must be 32 for MXFP4 quantization"
         b_row, b_row_s, b_col, b_col_s = quantize_mx_operands(b.contiguous(), float4_e2m1fn_x2, w_recipe, w_recipe, "MXFP4")
@@ -95,18 +101,23 @@ def _fp4_weight_operands(b, b_t, config, need_bwd):
     return b_row, b_row_s, b_col, b_col_s
 
 
-def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col, offs_col, config,
-                           dgrad_dtype, wgrad_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad):
+def _fp4_backward_products(grad_out, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col, offs_col, b_as_forward,
+                           config, dgrad_dtype, wgrad_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad):
     """dgrad and wgrad of the MXFP4 grouped product from the saved column-direction operands; the padded
-    offsets are the forward quantizer's (None: the caller quantized the activation)."""
+    offsets are the forward quantizer's (None: the caller quantized the activation). ``b_as_forward``: ``b_col`` are the
+    forward codes, ``b_col_s`` their other direction's scales."""
     gran = config.granularity
     known = None if offs_col is None else (None, None, lens_col, offs_col)
     g_row, g_row_s, g_col, g_col_s, _, offs_row, lens_col, offs_col = grouped_quantize_mx_operands(
         grad_out, float4_e2m1fn_x2, group_lens, group_offs, ScalingRecipe(use_sr=config.use_gradient_sr),
         ScalingRecipe(use_sr=config.use_gradient_sr, use_rht=True), "MXFP4", known=known, col_like=a_col_s)
-    # dgrad: grad_a = grad_out @ b as an NT product with the transposed weight quantization [G, K, N]
-    grad_a = grouped_gemm_fp4_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
-                                   gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
+    # dgrad: grad_a = grad_out @ b with the forward codes [G, N, K] as they lie, or as an NT product with the transposed
+    # weight quantization [G, K, N]
+    if b_as_forward:
+        grad_a = grouped_gemm_mx_kn_impl(g_row, b_col, g_row_s, b_col_s, offs_row, group_offs, dgrad_dtype)[:total_m]
+    else:
+        grad_a = grouped_gemm_fp4_impl(g_row, b_col, g_row_s, b_col_s, group_lens, offs_row, False, True, dgrad_dtype,
+                                       gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
     # wgrad: grad_b[g] = grad_out_g^T @ a_g over the 256-padded token ranges -> [G, N, K]
     grad_b = _bgrad_grouped_gemm_fp4_impl_wrapper(
         g_col, a_col, g_col_s, a_col_s, lens_col, offs_col, False, False, False, wgrad_dtype, gran.value, num_cu,
@@ -163,16 +174,17 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
 
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
                                     gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
+        b_as_forward = b_col is None
         if need_bwd:
-            ctx.save_for_backward(a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col, offs_col)
-        ctx.meta = (config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad)
+            ctx.save_for_backward(a_col, a_col_s, b_row if b_as_forward else b_col, b_col_s, group_lens, group_offs, lens_col, offs_col)
+        ctx.meta = (b_as_forward, config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad)
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
         grad_out = _ensure_contiguous_grad_out(grad_out)
-        config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad = ctx.meta
-        grad_a, grad_b = _fp4_backward_products(grad_out, *ctx.saved_tensors, config, out_dtype, out_dtype, num_cu, total_m,
+        b_as_forward, config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad = ctx.meta
+        grad_a, grad_b = _fp4_backward_products(grad_out, *ctx.saved_tensors, b_as_forward, config, out_dtype, out_dtype, num_cu, total_m,
                                                 fuse_bgrad_accum, main_grad)
         return grad_a, grad_b, None, None, None, None, None, None, None, None, None
 
@@ -206,10 +218,11 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
         b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, None, config, need_bwd)
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, group_offs, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]
+        b_as_forward = b_col is None
         if need_bwd:
-            ctx.save_for_backward(x2, p1, row_mask, a_col, a_col_s, b_col, b_col_s, group_lens, group_offs, lens_col,
-                                  offs_col)
-        ctx.meta = (config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs.shape)
+            ctx.save_for_backward(x2, p1, row_mask, a_col, a_col_s, b_row if b_as_forward else b_col, b_col_s, group_lens,
+                                  group_offs, lens_col, offs_col)
+        ctx.meta = (b_as_forward, config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs.shape)
         return out
 
     @staticmethod
@@ -218,8 +231,8 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
 
         grad_out = _ensure_contiguous_grad_out(grad_out)
         x2, p1, row_mask, *operands = ctx.saved_tensors
-        config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs_shape = ctx.meta
-        grad_act, grad_b = _fp4_backward_products(grad_out, *operands, config, x2.dtype, out_dtype, num_cu, total_m,
+        b_as_forward, config, out_dtype, num_cu, total_m, fuse_bgrad_accum, main_grad, act_type, probs_shape = ctx.meta
+        grad_act, grad_b = _fp4_backward_products(grad_out, *operands, b_as_forward, config, x2.dtype, out_dtype, num_cu, total_m,
                                                   fuse_bgrad_accum, main_grad)
         grad_x, grad_probs = glu_bwd_with_probs(grad_act.contiguous(), x2, p1, row_mask,
                                                 ACT_SILU if act_type == "silu" else ACT_GELU)

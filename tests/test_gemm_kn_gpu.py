@@ -240,3 +240,62 @@ def test_tensorwise_layer_gradients(M, N, K, main_grad, hybrid, monkeypatch):
         grads.append((out, gx, w.main_grad if main_grad else gw))
     assert used == ([True, True, True] if K % 128 == 0 else [])  # (the patched rule is asked once, and says no)
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+F4 = torch.float4_e2m1fn_x2
+
+
+def _nibbles(q):
+    """Codes of ``[.., rows, cols / 2]`` packed bytes, one a byte."""
+    u = q.contiguous().view(torch.uint8)
+    return torch.stack((u & 15, u >> 4), -1).flatten(-2)
+
+
+@pytest.mark.parametrize("shape", [(1, 128, 128), (3, 256, 640), (2, 1152, 384)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mxfp4_weight_quantizer(shape, dtype):
+    w, recipe = _mx_weight(*shape).to(dtype), LP.ScalingRecipe(use_2d_block=True)
+    q, words, words_t = Q.quantize_mx_weight_impl(w, F4)
+    rq, rs, cq, cs = Q.quantize_mx_operands(w, F4, recipe, recipe, "MXFP4")
+    assert torch.equal(_nibbles(q), _nibbles(rq)) and torch.equal(_nibbles(q).transpose(1, 2), _nibbles(cq))
+    assert torch.equal(words, rs) and torch.equal(words_t, cs)
+
+
+@pytest.mark.parametrize("lens", [[128, 0, 127, 1, 129], [900, 513, 0, 460], [33, 95, 256]])
+@pytest.mark.parametrize("n,k", [(128, 1024), (1152, 1280), (1408, 1536)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_mxfp4_grouped(lens, n, k, out_dtype):
+    from primus_turbo.pytorch.kernels.grouped_gemm import grouped_gemm_fp4_impl as gimpl4
+
+    w, recipe = _mx_weight(len(lens), k, n, special=False), LP.ScalingRecipe(use_2d_block=True)
+    x = bf16_randn((sum(lens), k), seed=5).cuda()
+    gl = torch.from_numpy(np.array(lens, dtype=np.int64)).cuda()
+    offs = torch.ops.primus_turbo_cpp_extension.grouped_gemm_compute_offs(gl)
+    xq, xs, _, _, _, orow, _, _ = Q.grouped_quantize_mx_operands(x, F4, gl, offs, LP.ScalingRecipe(), LP.ScalingRecipe(), "MXFP4")
+    q, _, words_t = Q.quantize_mx_weight_impl(w, F4)
+    _, _, cq, cs = Q.quantize_mx_operands(w, F4, recipe, recipe, "MXFP4")
+    got = gimpl.grouped_gemm_mx_kn_impl(xq, q, xs, words_t, orow, offs, out_dtype)
+    want = gimpl4.grouped_gemm_fp4_impl(xq, cq, xs, cs, gl, orow, False, True, out_dtype, G.MX_BLOCKWISE.value, None, 0, False, offs)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("n,k", [(1280, 384), (1152, 384)])  # (the second: an odd number of half slabs)
+def test_mxfp4_layer_gradients(glu, n, k, monkeypatch):
+    import importlib
+
+    ops = importlib.import_module("primus_turbo.pytorch.ops.grouped_gemm_fp4")
+    config, lens = LP.Float4QuantConfig(), torch.tensor([300, 0, 213, 87], device="cuda")
+    x = bf16_randn((600, 2 * k if glu else k), seed=1).cuda().requires_grad_()
+    w = bf16_randn((4, n, k), seed=2).cuda().requires_grad_()
+    p = torch.rand(600, device="cuda").requires_grad_()
+    g = bf16_randn((600, n), seed=3).cuda()
+    used, grads = [], []
+    monkeypatch.setattr(Q, "_next_sr_seed", lambda *flags: 12345)
+    for on in (True, False):
+        monkeypatch.setattr(ops, "mx_reads_kn", lambda *a: used.append(gimpl.mx_reads_kn(*a)) or (on and used[-1]))
+        out = (ops.glu_grouped_gemm_fp4(x, p, w, lens, trans_b=True, config=config, act_type="silu") if glu else
+               ops.grouped_gemm_fp4(x, w, lens, trans_b=True, config=config))
+        grads.append((out, *torch.autograd.grad(out, (x, w, p) if glu else (x, w), g)))
+    assert used == [n % 256 == 0] * 2
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
