@@ -48,7 +48,7 @@ class _MoEPermute(torch.autograd.Function):
         else:
             row_id_map, tokens_per_expert, overflow_flag, num_dispatched = _ops.permute_preprocessing(
                 expert_map, num_local_experts, num_topk, pad_multiple, num_permuted_tokens, stride)
-            rows = int(num_permuted_tokens) if num_permuted_tokens > 0 else int(tokens_per_expert.sum().item())
+            rows = int(num_permuted_tokens) if num_permuted_tokens > 0 else sum(tokens_per_expert.tolist())
             out = torch.empty((rows, hidden), dtype=tokens.dtype, device=dev)
             out_sf = torch.empty((rows, scales_per_token), dtype=scaling_factor.dtype, device=dev) if with_sf else None
             out_probs = torch.empty((rows,), dtype=probs.dtype, device=dev) if probs is not None else None
