@@ -132,20 +132,36 @@ template <typename... Args> torch::jit::Stack general(const char *name, Args &&.
 // ---- products -------------------------------------------------------------------------------------------------------
 enum : int64_t { TENSORWISE = 1, ROWWISE = 2, BLOCKWISE = 3, MX_BLOCKWISE = 4 }; // ScalingGranularity
 
+// Bytes from one row's scales to the next row's, 0 for word-major ones; -1: not the scales of `rows` rows of K values.
+int64_t mx_scale_pitch(const Tensor &s, int64_t rows, int64_t K) {
+    if (s.dim() != 2 || !s.is_contiguous())
+        return -1;
+    if (s.scalar_type() == at::kInt)
+        return K % 128 == 0 && s.size(0) == K / 128 && s.size(1) == rows ? 0 : -1;
+    return s.element_size() == 1 && s.size(0) == rows && s.size(1) >= K / 32 && s.size(1) > 0 ? s.size(1) : -1;
+}
+
 // A product into `out` (MX: NT); false: a form for the Python body.
 bool launch_mx(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor &b_s, Tensor &out, bool accumulate) {
     const bool fp4 = a.scalar_type() == at::kFloat4_e2m1fn_x2;
     if (fp4 ? b.scalar_type() != at::kFloat4_e2m1fn_x2 : !is_fp8(a.scalar_type()) || !is_fp8(b.scalar_type()))
         return false;
     const int64_t pack = fp4 ? 2 : 1, M = a.size(0), N = b.size(0), ld = a.size(1), K = ld * pack;
-    // word-major scales of both operands and rows of whole slabs: nothing is copied
-    if (a_s.scalar_type() != at::kInt || b_s.scalar_type() != at::kInt || b.size(1) != ld || K % 128 != 0 || ld % 128 != 0 || ld < 512)
+    if (b.size(1) != ld || K % 32 != 0)
         return false;
-    if (a_s.dim() != 2 || b_s.dim() != 2 || a_s.size(0) != K / 128 || a_s.size(1) != M || b_s.size(0) != K / 128 || b_s.size(1) != N)
+    const int64_t sa_ld = mx_scale_pitch(a_s, M, K), sb_ld = mx_scale_pitch(b_s, N, K);
+    if (sa_ld < 0 || sb_ld < 0)
         return false;
+    // (word-major scales of both operands and rows of whole slabs: nothing is copied)
+    const bool   ready    = sa_ld == 0 && sb_ld == 0 && ld % 128 == 0 && ld >= 512;
+    const size_t ws_bytes = ready ? 0 : api.pt_gemm_mx_workspace_bytes(M, N, K, ld, ld, fp4);
+    Tensor       ws;
+    if (ws_bytes)
+        ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, a);
     return api.pt_gemm_mx(a.data_ptr(), a_s.data_ptr(), b.data_ptr(), b_s.data_ptr(), code_of(a.scalar_type()),
                           a.scalar_type() == at::kFloat8_e5m2, b.scalar_type() == at::kFloat8_e5m2, out.data_ptr(),
-                          code_of(out.scalar_type()), M, N, K, ld, ld, 0, 0, accumulate, nullptr, 0, 0, stream_of(a)) == PT_OK;
+                          code_of(out.scalar_type()), M, N, K, ld, ld, sa_ld, sb_ld, accumulate, ws_bytes ? ws.data_ptr() : nullptr,
+                          ws_bytes, 0, stream_of(a)) == PT_OK;
 }
 
 bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b, Tensor &out,
@@ -360,19 +376,35 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> quant_fp8_blockwise_kmajor(const Tens
     return {r[0].toTensor(), r[1].toTensor(), r[2].toTensor(), r[3].toTensor()};
 }
 
-// Both directions with word-major scales (8): what the layers' products read. Stochastic rounding (4) takes its
-// seed in the Python body.
+// The codes and scales of one direction, `rows` rows of `width` values each (both a multiple of what the kernel pads
+// to): E8M0 bytes [rows, width / 32] or, word-major (8), words [width / 128, rows]. Empty tensors for one not wanted.
+std::pair<Tensor, Tensor> mx_direction(const Tensor &x, ScalarType dtype, bool wanted, int64_t flags, int64_t rows, int64_t width) {
+    if (!wanted)
+        return {empty({0}, dtype, x), empty({0}, at::kFloat8_e8m0fnu, x)};
+    const int64_t        pack = dtype == at::kFloat4_e2m1fn_x2 ? 2 : 1;
+    std::vector<int64_t> q(x.sizes().begin(), x.sizes().end() - 2), s = q;
+    q.insert(q.end(), {rows, width / pack});
+    if (flags & 8) {
+        s.insert(s.end(), {width / 128, rows});
+        return {empty(q, dtype, x), empty(s, at::kInt, x)};
+    }
+    s.insert(s.end(), {rows, width / 32});
+    return {empty(q, dtype, x), empty(s, at::kFloat8_e8m0fnu, x)};
+}
+
+// Stochastic rounding (4) takes its seed in the Python body.
 std::tuple<Tensor, Tensor, Tensor, Tensor> quantize_mx(const Tensor &x, ScalarType dtype, bool row, bool col, int64_t row_flags,
                                                        int64_t col_flags) {
-    const bool fp4 = dtype == at::kFloat4_e2m1fn_x2;
-    if (row && col && (row_flags & 12) == 8 && (col_flags & 12) == 8 && on_current_device(x) && x.is_contiguous() && x.dim() == 2 &&
-        (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && (fp4 || is_fp8(dtype)) && x.size(1) % 32 == 0) {
-        const int64_t M = x.size(0), N = x.size(1), Mp = round_up(M, 128), Np = round_up(N, 128), pack = fp4 ? 2 : 1;
-        Tensor        rq = empty({M, Np / pack}, dtype, x), rs = empty({Np / 128, M}, at::kInt, x);
-        Tensor        cq = empty({N, Mp / pack}, dtype, x), cs = empty({Mp / 128, N}, at::kInt, x);
-        if (api.pt_quantize_mx(x.data_ptr(), code_of(x.scalar_type()), 1, M, N, code_of(dtype), rq.data_ptr(),
-                               static_cast<uint8_t *>(rs.data_ptr()), static_cast<int>(row_flags), cq.data_ptr(),
-                               static_cast<uint8_t *>(cs.data_ptr()), static_cast<int>(col_flags), 0, stream_of(x)) == PT_OK)
+    if ((row || col) && (row_flags & 4) == 0 && (col_flags & 4) == 0 && on_current_device(x) && x.is_contiguous() &&
+        (x.dim() == 2 || x.dim() == 3) && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) &&
+        (dtype == at::kFloat4_e2m1fn_x2 || is_fp8(dtype)) && x.size(-1) % 32 == 0) {
+        const int64_t B = x.dim() == 3 ? x.size(0) : 1, M = x.size(-2), N = x.size(-1);
+        auto [rq, rs] = mx_direction(x, dtype, row, row_flags, M, round_up(N, 128));
+        auto [cq, cs] = mx_direction(x, dtype, col, col_flags, N, round_up(M, 128));
+        if (api.pt_quantize_mx(x.data_ptr(), code_of(x.scalar_type()), B, M, N, code_of(dtype), row ? rq.data_ptr() : nullptr,
+                               row ? static_cast<uint8_t *>(rs.data_ptr()) : nullptr, static_cast<int>(row_flags),
+                               col ? cq.data_ptr() : nullptr, col ? static_cast<uint8_t *>(cs.data_ptr()) : nullptr,
+                               static_cast<int>(col_flags), 0, stream_of(x)) == PT_OK)
             return {rq, rs, cq, cs};
     }
     auto r = general("primus_turbo::quantize_mx_general", x, dtype, row, col, row_flags, col_flags);

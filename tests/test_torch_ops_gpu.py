@@ -97,6 +97,17 @@ def test_quantizer_modes_and_codes():
             _same(ext, "dequantize_fp8_tensorwise", q.t(), scale, hp)
 
 
+@pytest.mark.parametrize("shape", [(1, 32), (97, 160), (128, 128), (130, 1024), (1, 33, 96), (3, 96, 160), (0, 64)])
+@pytest.mark.parametrize("to", [E4M3, E5M2, F4])
+def test_mx_directions(shape, to):
+    """Each direction alone and both, scales of either layout, also batched."""
+    x = bf16_randn(shape, seed=2).cuda()
+    for row, col in ((True, False), (False, True), (True, True), (False, False)):
+        for flags in ((0, 0), (8, 8), (1, 9), (0, 8), (2, 2)):
+            _same("primus_turbo", "quantize_mx", x, to, row, col, *flags)
+            _same("primus_turbo", "quantize_mx", x.half(), to, row, col, *flags)
+
+
 @pytest.mark.parametrize("out_dtype", [BF16, F16, F32, torch.float64])
 @pytest.mark.parametrize("trans_c", [False, True])
 @pytest.mark.parametrize("M,N,K", [(16, 256, 512), (300, 520, 640), (1, 1, 128), (129, 128, 129), (5, 640, 640), (0, 64, 128), (1100, 1040, 1056)])
@@ -136,6 +147,10 @@ def test_products(M, N, K, trans_c, out_dtype):
         fa, ga, _, _ = torch.ops.primus_turbo.quantize_mx(a, F4, True, True, 8, 8)
         fb, gb, _, _ = torch.ops.primus_turbo.quantize_mx(b, F4, True, True, 8, 8)
         product(fa, ga, False, fb, gb, True, G.MX_BLOCKWISE)
+        for to in (E4M3, F4):  # row-major scales of both, which a user's own calls have
+            ua, ta, _, _ = torch.ops.primus_turbo.quantize_mx(a, to, True, False, 0, 0)
+            ub, tb, _, _ = torch.ops.primus_turbo.quantize_mx(b, to, True, False, 1, 0)
+            product(ua, ta, False, ub, tb, True, G.MX_BLOCKWISE)
 
 
 @pytest.mark.parametrize("bad", ["reduction", "scale shape", "scale type", "half operands", "3-D", "device"])
