@@ -124,6 +124,16 @@ def reads_kn_in_place(M: int, Nn: int, K: int) -> bool:
     return bool(N.lib().pt_gemm_fp8_nn_in_place(M, Nn, K))
 
 
+def kn_layer_pays(rows: int, mx: bool = False) -> bool:
+    """Whether a layer with block or MX scales and so many rows a weight leaves the weight's transposed codes out. Writing
+    them costs the cast a fixed time, the product that reads ``[K, N]`` is 1 to 3 % slower on every row. A training step of
+    M x N x K, copies / in place, blocks: 2048 x 8192 x 8192 469 / 459 us, 4096 851 / 829, 6144 1230 / 1206, 8192 1612 / 1610
+    (1609 / 1615 on another card), 16384 x 8192 x 4096 1646 / 1672; four experts of 4096 x 4096: 16384 rows 972 / 950, 32768
+    1777 / 1775. MXFP8 there 832 / 822 and 1511 / 1519, MXFP4 608 / 598 and 1063 / 1073. (The products with vector scales gain
+    at any size: 16384 x 8192 x 4096 1365 / 1330.)"""
+    return rows < (5120 if mx else 8192)
+
+
 def vec_reads_in_place(M: int, Nn: int, K: int, trans_a: bool) -> bool:
     """The same of the products with vector scales, and of an ``a`` stored ``[K, M]`` beside it with ``trans_a``."""
     return bool(N.lib().pt_gemm_fp8_vec_in_place(M, Nn, K, int(trans_a)))

@@ -2,8 +2,9 @@
 
 Which quantizer feeds which GEMM layout, per granularity (same recipes as the reference):
 
-  TENSORWISE  fwd  C = Aq . Bq            one scale per tensor; backward runs NT GEMMs on
-                   physically transposed fp8 copies when the forward is NT (ref :96-276)
+  TENSORWISE  fwd  C = Aq . Bq            one scale per tensor; both backward products read the forward
+                   codes along their other axis in place where the kernels can, else they are
+                   NT products on physically transposed fp8 copies (ref :96-276)
   ROWWISE     fwd  A, B quantized along K; backward re-quantizes the de-quantized
                    operands along the other axis and quantizes grad_out twice (ref :278-426)
   BLOCKWISE   fwd  A 1x128 (+128x1 for wgrad from the same read), B 128x128 tiles;
@@ -37,6 +38,7 @@ from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import (
     gemm_fp8_accum_impl,
     gemm_fp8_impl,
     get_gemm_logical_shape,
+    kn_layer_pays,
     reads_kn_in_place,
     vec_reads_in_place,
 )
@@ -226,8 +228,9 @@ class FP8GemmBlockFunction(torch.autograd.Function):
     """BLOCKWISE (128): activations and gradients in 1 x 128 blocks along the reduction of each
     product, the weight in 128 x 128 tiles that serve forward and backward. When a gradient is
     wanted the quantizers also emit, from the same read, the operands of the backward products with
-    their reduction axis contiguous (the transposed 128 x 1 column codes of ``a`` and ``grad_out``,
-    the transposed weight codes), so that every product is an NT product read in place."""
+    their reduction axis contiguous (the transposed 128 x 1 column codes of ``a`` and ``grad_out``).
+    The input gradient reads the forward weight codes ``[N, K]`` in place; where its product cannot
+    (``reads_kn_in_place``) or that does not pay (``kn_layer_pays``) the weight's quantizer writes transposed codes too."""
 
     @staticmethod
     def forward(ctx, a, b, a_t, b_t, trans_a, trans_b, out_dtype, config):
@@ -259,7 +262,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
             b_q, b_s = b.qdata, b.scale_inv
         elif ((need_bwd or not trans_b) and b.dim() == 2 and b.size(0) % 16 == 0
               and not (trans_b and a.dim() == 2 and not torch.compiler.is_compiling() and b.is_cuda
-                       and reads_kn_in_place(a.shape[0], b.shape[1], b.shape[0]))):
+                       and kn_layer_pays(a.shape[0]) and reads_kn_in_place(a.shape[0], b.shape[1], b.shape[0]))):
             b_q, b_q_t, b_s = quant_fp8_blockwise_for_weight_dual_impl(b, fdt, bs)
         else:
             b_q, b_s = quantize_fp8(b, fdt, gran, block_size=bs, scaling_recipe=w_recipe)

@@ -38,6 +38,7 @@ from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp4_impl import (
     grouped_gemm_fp4_variable_k_accum_impl,
     grouped_gemm_fp4_variable_k_impl,
 )
+from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import kn_layer_pays
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import grouped_gemm_mx_kn_impl, mx_reads_kn
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_utils import group_offs_from_lens
 from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
@@ -73,10 +74,10 @@ def _bgrad_grouped_gemm_fp4_impl_wrapper(a, b, a_scales, b_scales, group_lens, g
     return _get_dummy_wgrad(out.shape, out_dtype)
 
 
-def _fp4_weight_operands(b, b_t, config, need_bwd):
+def _fp4_weight_operands(b, b_t, config, need_bwd, rows):
     """The expert weights ``[G, N, K]`` as MXFP4 operands with 32 x 32 blocks: ``(row codes, row scales,
-    column codes, column scales)``, the column pair (the transposed quantization dgrad reads) only
-    when a backward pass will follow."""
+    column codes, column scales)``, the column pair (the transposed quantization) only when a
+    backward pass will follow whose input gradient cannot read the row codes."""
     gran, bs = config.granularity, config.block_size
     w_recipe = ScalingRecipe(use_2d_block=True)
     b_col = b_col_s = None
@@ -89,7 +90,8 @@ def _fp4_weight_operands(b, b_t, config, need_bwd):
                                                scaling_recipe=w_recipe)
             assert isinstance(b_t, QuantizedTensor)
             b_col, b_col_s = b_t.qdata, b_t.scale_inv
-    elif need_bwd and b.shape[2] % 128 == 0 and mx_reads_kn(b.shape[2], b.shape[1], True) and b.dtype in (torch.bfloat16, torch.float16):
+    elif (need_bwd and b.shape[2] % 128 == 0 and b.dtype in (torch.bfloat16, torch.float16)
+          and mx_reads_kn(b.shape[2], b.shape[1], True) and kn_layer_pays(rows // max(1, b.shape[0]), True)):
         # backward reads the same codes along the other axis: no transposed copy (None), its scales alone
         assert bs == 32, "The block size must be 32 for MXFP4 quantization"
         b_row, b_row_s, b_col_s = quantize_mx_weight_impl(b.contiguous(), float4_e2m1fn_x2)
@@ -170,7 +172,7 @@ class FP4GroupedGemmMXFunc(torch.autograd.Function):
             a_row, a_row_s, a_col, a_col_s, _, offs_row, _, _ = grouped_quantize_mx_operands(
                 a.contiguous(), float4_e2m1fn_x2, group_lens, group_offs, a_recipe, a_t_recipe, "MXFP4", with_col=False)
 
-        b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, b_t, config, need_bwd)
+        b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, b_t, config, need_bwd, total_m)
 
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
                                     gran.value, num_cu, _NATIVE, False, group_offs)[:total_m]
@@ -215,7 +217,7 @@ class FP4GluGroupedGemmMXFunc(torch.autograd.Function):
         x2, p1 = x.contiguous(), probs.reshape(-1).contiguous()
         a_row, a_row_s, a_col, a_col_s, _, _, lens_col, offs_col = glu_grouped_quantize_mx_impl(
             x2, p1, row_mask, act_type, float4_e2m1fn_x2, group_lens, group_offs, need_bwd, 2 | _MX_WORDS)
-        b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, None, config, need_bwd)
+        b_row, b_row_s, b_col, b_col_s = _fp4_weight_operands(b, None, config, need_bwd, total_m)
         out = grouped_gemm_fp4_impl(a_row, b_row, a_row_s, b_row_s, group_lens, group_offs, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]
         b_as_forward = b_col is None

@@ -33,6 +33,7 @@ from primus_turbo.pytorch.core.quantized_tensor import (
     QuantizedTensorPair,
     check_quantized_tensor,
 )
+from primus_turbo.pytorch.kernels.gemm.gemm_fp8_impl import kn_layer_pays
 from primus_turbo.pytorch.kernels.grouped_gemm.grouped_gemm_fp8_impl import (
     grouped_gemm_fp8_impl,
     grouped_gemm_fp8_variable_k_accum_impl,
@@ -95,7 +96,8 @@ def _block_forward_product(a_fp8_row, a_scale_row, b, group_lens, group_offs, tr
         b_fp8, b_scale = b.qdata, b.scale_inv
     elif ((need_bwd or not trans_b) and b.size(-2) % 16 == 0
           and not (trans_b and not torch.compiler.is_compiling() and b.is_cuda
-                   and reads_kn_in_place(b.shape[0], a_fp8_row.shape[0], b.shape[2], b.shape[1]))):
+                   and reads_kn_in_place(b.shape[0], a_fp8_row.shape[0], b.shape[2], b.shape[1])
+                   and kn_layer_pays(a_fp8_row.shape[0] // b.shape[0]))):
         b_fp8, b_fp8_t, b_scale = quant_fp8_blockwise_for_weight_dual_impl(b, b_dtype, block_size=bs)
     else:
         b_fp8, b_scale = quant_fp8_blockwise_for_weight_impl(b, b_dtype, block_size=bs)
@@ -322,10 +324,10 @@ class FP8GroupedGemmTensorFunc(torch.autograd.Function):
         return grad_a, grad_b, None, None, None, None, None, None, None, None, None
 
 
-def _mx_weight_operands(b, b_t, config, need_bwd):
+def _mx_weight_operands(b, b_t, config, need_bwd, rows):
     """The expert weights ``[G, N, K]`` as MXFP8 operands with 32 x 32 blocks: ``(row codes, row scales,
-    column codes, column scales)``, the column pair (the transposed quantization dgrad reads) only
-    when a backward pass will follow."""
+    column codes, column scales)``, the column pair (the transposed quantization) only when a
+    backward pass will follow whose input gradient cannot read the row codes."""
     fdt, bs, gran = _get_fp8_dtype(config.format, True), config.block_size, config.granularity
     w_recipe = ScalingRecipe(use_2d_block=True)
     b_col = b_col_s = None
@@ -338,7 +340,8 @@ def _mx_weight_operands(b, b_t, config, need_bwd):
                                                scaling_recipe=w_recipe)
             assert isinstance(b_t, QuantizedTensor)
             b_col, b_col_s = b_t.qdata, b_t.scale_inv
-    elif need_bwd and b.shape[2] % 128 == 0 and mx_reads_kn(b.shape[2], b.shape[1]) and b.dtype in (torch.bfloat16, torch.float16):
+    elif (need_bwd and b.shape[2] % 128 == 0 and b.dtype in (torch.bfloat16, torch.float16)
+          and mx_reads_kn(b.shape[2], b.shape[1]) and kn_layer_pays(rows // max(1, b.shape[0]), True)):
         # backward reads the same codes along the other axis: no transposed copy (None), its scales alone
         assert bs == 32, "The block size must be 32 for MXFP8 quantization"
         b_row, b_row_s, b_col_s = quantize_mx_weight_impl(b.contiguous(), fdt)
@@ -411,7 +414,7 @@ class FP8GroupedGemmMXFunc(torch.autograd.Function):
             assert bs == 32, "The block size must be 32 for MXFP8 quantization"
             a_row, a_row_s, _, _, _, offs_row, _, _ = grouped_quantize_mx_operands(
                 a.contiguous(), fdt, group_lens, group_offs, None, None, "MXFP8", with_col=False)
-        b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, b_t, config, need_bwd)
+        b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, b_t, config, need_bwd, total_m)
         # the padded row layout is read through offs_row, the result is packed by group_offs
         # into an output over-allocated to the padded rows
         out = grouped_gemm_fp8_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
@@ -451,7 +454,7 @@ class FP8GluGroupedGemmMXFunc(torch.autograd.Function):
         x2, p1 = x.contiguous(), probs.reshape(-1).contiguous()
         a_row, a_row_s, a_col, a_col_s, _, offs_row, lens_col, offs_col = glu_grouped_quantize_mx_impl(
             x2, p1, row_mask, act_type, _get_fp8_dtype(config.format, True), group_lens, group_offs, need_bwd, _MX_WORDS)
-        b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, None, config, need_bwd)
+        b_row, b_row_s, b_col, b_col_s = _mx_weight_operands(b, None, config, need_bwd, total_m)
         out = grouped_gemm_fp8_impl(a_row, b_row, a_row_s, b_row_s, group_lens, offs_row, False, True, out_dtype,
                                     config.granularity.value, num_cu, _NATIVE, False, group_offs)[:total_m]
         b_as_forward = b_col is None

@@ -299,3 +299,27 @@ def test_mxfp4_layer_gradients(glu, n, k, monkeypatch):
         grads.append((out, *torch.autograd.grad(out, (x, w, p) if glu else (x, w), g)))
     assert used == [n % 256 == 0] * 2
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+# both sides of the line at which a bank's weight gets its transposed copy again: the same bits, and the copy's path where it pays
+@pytest.mark.parametrize("recipe,rows", [("MX_BLOCKWISE", 2 * 5120 - 1), ("MX_BLOCKWISE", 2 * 5120), ("BLOCKWISE", 2 * 8192 - 1), ("BLOCKWISE", 2 * 8192)])
+def test_rows_a_weight(recipe, rows, monkeypatch):
+    import importlib
+
+    ops = importlib.import_module("primus_turbo.pytorch.ops.grouped_gemm_fp8")
+    mx = recipe == "MX_BLOCKWISE"
+    more = dict(block_size=32, scale_dtype=LP.ScaleDtype.E8M0) if mx else dict(block_size=128)
+    config = LP.Float8QuantConfig(granularity=G[recipe], **more)
+    lens = torch.tensor([700, rows - 700], device="cuda")
+    x, g = bf16_randn((rows, 2048), seed=1).cuda().requires_grad_(), bf16_randn((rows, 512), seed=3).cuda()
+    w = bf16_randn((2, 512, 2048), seed=2).cuda().requires_grad_()
+    name = "quantize_mx_weight_impl" if mx else "quant_fp8_blockwise_for_weight_impl"
+    calls, real, pays = [], getattr(ops, name), ops.kn_layer_pays
+    monkeypatch.setattr(ops, name, lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    grads = []
+    for on in (True, False):
+        monkeypatch.setattr(ops, "kn_layer_pays", lambda *a: on and pays(*a))
+        out = ops.grouped_gemm_fp8(x, w, lens, trans_b=True, config=config)
+        grads.append((out, *torch.autograd.grad(out, (x, w), g)))
+    assert len(calls) == (rows // 2 < (5120 if mx else 8192))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
