@@ -27,6 +27,7 @@ using at::Tensor;
 // Entry points of the library that Python loaded (by path: there is one of them in the process).
 struct Api {
 #define PT_FN(name) decltype(&::name) name
+    PT_FN(pt_last_error);
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
     PT_FN(pt_gemm_fp8_vec_in_place);
@@ -55,6 +56,7 @@ void bind_native(std::string path) {
 #define PT_FN(name)                                                                                                       \
     a.name = reinterpret_cast<decltype(a.name)>(dlsym(lib, #name));                                                       \
     TORCH_CHECK(a.name != nullptr, "primus_turbo: ", path, " does not export " #name)
+    PT_FN(pt_last_error);
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
     PT_FN(pt_gemm_fp8_vec_in_place);
@@ -76,6 +78,18 @@ void bind_native(std::string path) {
 
 void set_tensorwise_mode(int64_t mode) {
     tensorwise_mode.store(mode, std::memory_order_relaxed);
+}
+
+// Whether a call of the C library was carried out. What it refuses (arguments, a form, a workspace), it refuses before it
+// launches the kernel that writes the results: the Python body then refuses as well, or finds another way. Any other status
+// raises here: a failed launch is found by the error that HIP holds after it, which may be one that an earlier call of
+// this thread left while this kernel runs, and an accumulating product that is issued again adds twice.
+bool carried_out(int status) {
+    if (status == PT_OK)
+        return true;
+    TORCH_CHECK(status == PT_ERR_INVALID_ARGUMENT || status == PT_ERR_UNSUPPORTED || status == PT_ERR_WORKSPACE,
+                "primus_turbo native error ", status, ": ", api.pt_last_error());
+    return false;
 }
 
 bool is_fp8(ScalarType t) {
@@ -158,10 +172,10 @@ bool launch_mx(const Tensor &a, const Tensor &a_s, const Tensor &b, const Tensor
     Tensor       ws;
     if (ws_bytes)
         ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, a);
-    return api.pt_gemm_mx(a.data_ptr(), a_s.data_ptr(), b.data_ptr(), b_s.data_ptr(), code_of(a.scalar_type()),
-                          a.scalar_type() == at::kFloat8_e5m2, b.scalar_type() == at::kFloat8_e5m2, out.data_ptr(),
-                          code_of(out.scalar_type()), M, N, K, ld, ld, sa_ld, sb_ld, accumulate, ws_bytes ? ws.data_ptr() : nullptr,
-                          ws_bytes, 0, stream_of(a)) == PT_OK;
+    return carried_out(api.pt_gemm_mx(a.data_ptr(), a_s.data_ptr(), b.data_ptr(), b_s.data_ptr(), code_of(a.scalar_type()),
+                                      a.scalar_type() == at::kFloat8_e5m2, b.scalar_type() == at::kFloat8_e5m2, out.data_ptr(),
+                                      code_of(out.scalar_type()), M, N, K, ld, ld, sa_ld, sb_ld, accumulate, ws_bytes ? ws.data_ptr() : nullptr,
+                                      ws_bytes, 0, stream_of(a)));
 }
 
 bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b, Tensor &out,
@@ -218,10 +232,10 @@ bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tenso
     Tensor       ws;
     if (ws_bytes)
         ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, a);
-    return api.pt_gemm_fp8(pa->data_ptr(), code_of(pa->scalar_type()), static_cast<const float *>(psa->data_ptr()), pb->data_ptr(),
-                           code_of(pb->scalar_type()), static_cast<const float *>(psb->data_ptr()), out.data_ptr(),
-                           code_of(out.scalar_type()), M, N, K, trans_a, trans_b, mode, sa_m, sa_k, sb_n, sb_k, sa_blk, sb_blk, accumulate,
-                           ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, 0, stream_of(a)) == PT_OK;
+    return carried_out(api.pt_gemm_fp8(pa->data_ptr(), code_of(pa->scalar_type()), static_cast<const float *>(psa->data_ptr()), pb->data_ptr(),
+                                       code_of(pb->scalar_type()), static_cast<const float *>(psb->data_ptr()), out.data_ptr(),
+                                       code_of(out.scalar_type()), M, N, K, trans_a, trans_b, mode, sa_m, sa_k, sb_n, sb_k, sa_blk, sb_blk, accumulate,
+                                       ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, 0, stream_of(a)));
 }
 
 bool launch_product(const Tensor &a, const Tensor &a_s, bool trans_a, const Tensor &b, const Tensor &b_s, bool trans_b, Tensor &out,
@@ -272,8 +286,8 @@ std::vector<Tensor> quantize_fp8_tensorwise(const Tensor &x, ScalarType dtype, c
         const hipStream_t st = stream_of(x);
         if (!capturing(st)) {
             Tensor q = at::empty_like(x, x.options().dtype(dtype)), scale_inv = empty({}, at::kFloat, x);
-            if (api.pt_quantize_fp8_tensorwise_static(x.data_ptr(), code_of(x.scalar_type()), x.numel(), q.data_ptr(), code_of(dtype),
-                                                      nullptr, static_cast<float *>(scale_inv.data_ptr()), nullptr, st) == PT_OK)
+            if (carried_out(api.pt_quantize_fp8_tensorwise_static(x.data_ptr(), code_of(x.scalar_type()), x.numel(), q.data_ptr(), code_of(dtype),
+                                                                  nullptr, static_cast<float *>(scale_inv.data_ptr()), nullptr, st)))
                 return {q, scale_inv};
         }
     }
@@ -288,9 +302,9 @@ std::tuple<Tensor, Tensor, Tensor> quantize_fp8_tensorwise_t(const Tensor &x, Sc
             (width_t == R || width_t == round_up(R, 128)) && x.numel() > 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
             !capturing(st)) {
             Tensor q = empty({R, width}, dtype, x), q_t = empty({C, width_t}, dtype, x), scale_inv = empty({}, at::kFloat, x);
-            if (api.pt_quantize_fp8_tensorwise_t(x.data_ptr(), code_of(x.scalar_type()), R, C, q.data_ptr(), width, q_t.data_ptr(),
-                                                 width_t, code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), nullptr, 0,
-                                                 st) == PT_OK)
+            if (carried_out(api.pt_quantize_fp8_tensorwise_t(x.data_ptr(), code_of(x.scalar_type()), R, C, q.data_ptr(), width, q_t.data_ptr(),
+                                                             width_t, code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), nullptr, 0,
+                                                             st)))
                 return {q, q_t, scale_inv};
         }
     }
@@ -302,9 +316,9 @@ Tensor dequantize_fp8_tensorwise(const Tensor &x, const Tensor &scale_inv, Scala
     if (on_current_device(x) && is_fp8(x.scalar_type()) && x.is_contiguous() && is_hp(dtype) && scale_inv.is_cuda() &&
         scale_inv.get_device() == x.get_device() && scale_inv.numel() == 1 && scale_inv.scalar_type() == at::kFloat) {
         Tensor out = at::empty_like(x, x.options().dtype(dtype));
-        if (api.pt_dequantize_fp8_tensorwise(x.data_ptr(), code_of(x.scalar_type()), x.numel(),
-                                             static_cast<const float *>(scale_inv.data_ptr()), out.data_ptr(), code_of(dtype),
-                                             stream_of(x)) == PT_OK)
+        if (carried_out(api.pt_dequantize_fp8_tensorwise(x.data_ptr(), code_of(x.scalar_type()), x.numel(),
+                                                         static_cast<const float *>(scale_inv.data_ptr()), out.data_ptr(), code_of(dtype),
+                                                         stream_of(x))))
             return out;
     }
     return general("primus_turbo_cpp_extension::dequantize_fp8_tensorwise_general", x, scale_inv, dtype)[0].toTensor();
@@ -320,8 +334,8 @@ std::vector<Tensor> quantize_fp8_rowwise(const Tensor &x, ScalarType dtype, int6
         auto shape   = x.sizes().vec();
         shape.back() = 1;
         Tensor q = at::empty_like(x, x.options().dtype(dtype)), scale_inv = empty(shape, at::kFloat, x);
-        if (api.pt_quantize_fp8_rowwise(x.data_ptr(), code_of(x.scalar_type()), B, M, 1, q.data_ptr(), code_of(dtype), nullptr,
-                                        static_cast<float *>(scale_inv.data_ptr()), stream_of(x)) == PT_OK)
+        if (carried_out(api.pt_quantize_fp8_rowwise(x.data_ptr(), code_of(x.scalar_type()), B, M, 1, q.data_ptr(), code_of(dtype), nullptr,
+                                                    static_cast<float *>(scale_inv.data_ptr()), stream_of(x))))
             return {q, scale_inv};
     }
     return general("primus_turbo_cpp_extension::quantize_fp8_rowwise_general", x, dtype, axis, scale)[0].toTensorVector();
@@ -330,8 +344,8 @@ std::vector<Tensor> quantize_fp8_rowwise(const Tensor &x, ScalarType dtype, int6
 std::tuple<Tensor, Tensor> quant_fp8_rowwise_padded(const Tensor &x, ScalarType dtype, int64_t width) {
     if (castable(x, dtype) && x.dim() == 2 && width >= x.size(1)) {
         Tensor q = empty({x.size(0), width}, dtype, x), scale_inv = empty({x.size(0), 1}, at::kFloat, x);
-        if (api.pt_quantize_fp8_rowwise_padded(x.data_ptr(), code_of(x.scalar_type()), x.size(0), x.size(1), q.data_ptr(), width,
-                                               code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), stream_of(x)) == PT_OK)
+        if (carried_out(api.pt_quantize_fp8_rowwise_padded(x.data_ptr(), code_of(x.scalar_type()), x.size(0), x.size(1), q.data_ptr(), width,
+                                                           code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), stream_of(x))))
             return {q, scale_inv};
     }
     auto s = general("primus_turbo::quant_fp8_rowwise_padded_impl_general", x, dtype, width);
@@ -349,10 +363,10 @@ std::tuple<Tensor, Tensor> quant_fp8_rowwise_t(const Tensor &x, const std::optio
         const int64_t M = x.size(0), N = cols.value_or(x.size(1)), Mp = round_up(M, pad);
         Tensor        q_t = empty({N, Mp}, dtype, x), scale_inv = empty({1, N}, at::kFloat, x);
         Tensor        ws  = empty({static_cast<int64_t>(api.pt_quantize_fp8_rowwise_outer_workspace_bytes(1, M, N))}, at::kByte, x);
-        if (api.pt_quantize_fp8_rowwise_outer_ld(
+        if (carried_out(api.pt_quantize_fp8_rowwise_outer_ld(
                 x.data_ptr(), codes ? x.size(1) : N, code_of(x.scalar_type()),
                 codes ? static_cast<const float *>(row_scale->data_ptr()) : nullptr, code_of(hp), 1, M, N, nullptr, q_t.data_ptr(),
-                Mp, code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), ws.data_ptr(), ws.numel(), stream_of(x)) == PT_OK)
+                Mp, code_of(dtype), static_cast<float *>(scale_inv.data_ptr()), ws.data_ptr(), ws.numel(), stream_of(x))))
             return {q_t, scale_inv};
     }
     auto s = general("primus_turbo::quant_fp8_rowwise_t_impl_general", x, row_scale, hp, dtype, pad, cols);
@@ -366,10 +380,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> quant_fp8_blockwise_kmajor(const Tens
         Tensor        q = empty({M, N}, dtype, x), s = empty({cdiv(N, block), M}, at::kFloat, x);
         Tensor        q_t = with_col_t ? empty({N, Mp}, dtype, x) : empty({0}, dtype, x);
         Tensor        s_t = with_col_t ? empty({cdiv(M, block), N}, at::kFloat, x) : empty({0}, at::kFloat, x);
-        if (api.pt_quantize_fp8_blockwise_kmajor(x.data_ptr(), code_of(x.scalar_type()), M, N, code_of(dtype), q.data_ptr(),
-                                                 static_cast<float *>(s.data_ptr()), with_col_t ? q_t.data_ptr() : nullptr,
-                                                 with_col_t ? Mp : 0, with_col_t ? static_cast<float *>(s_t.data_ptr()) : nullptr,
-                                                 stream_of(x)) == PT_OK)
+        if (carried_out(api.pt_quantize_fp8_blockwise_kmajor(x.data_ptr(), code_of(x.scalar_type()), M, N, code_of(dtype), q.data_ptr(),
+                                                             static_cast<float *>(s.data_ptr()), with_col_t ? q_t.data_ptr() : nullptr,
+                                                             with_col_t ? Mp : 0, with_col_t ? static_cast<float *>(s_t.data_ptr()) : nullptr,
+                                                             stream_of(x))))
             return {q, s, q_t, s_t};
     }
     auto r = general("primus_turbo::quant_fp8_blockwise_kmajor_impl_general", x, dtype, block, with_col_t);
@@ -401,10 +415,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> quantize_mx(const Tensor &x, ScalarTy
         const int64_t B = x.dim() == 3 ? x.size(0) : 1, M = x.size(-2), N = x.size(-1);
         auto [rq, rs] = mx_direction(x, dtype, row, row_flags, M, round_up(N, 128));
         auto [cq, cs] = mx_direction(x, dtype, col, col_flags, N, round_up(M, 128));
-        if (api.pt_quantize_mx(x.data_ptr(), code_of(x.scalar_type()), B, M, N, code_of(dtype), row ? rq.data_ptr() : nullptr,
-                               row ? static_cast<uint8_t *>(rs.data_ptr()) : nullptr, static_cast<int>(row_flags),
-                               col ? cq.data_ptr() : nullptr, col ? static_cast<uint8_t *>(cs.data_ptr()) : nullptr,
-                               static_cast<int>(col_flags), 0, stream_of(x)) == PT_OK)
+        if (carried_out(api.pt_quantize_mx(x.data_ptr(), code_of(x.scalar_type()), B, M, N, code_of(dtype), row ? rq.data_ptr() : nullptr,
+                                           row ? static_cast<uint8_t *>(rs.data_ptr()) : nullptr, static_cast<int>(row_flags),
+                                           col ? cq.data_ptr() : nullptr, col ? static_cast<uint8_t *>(cs.data_ptr()) : nullptr,
+                                           static_cast<int>(col_flags), 0, stream_of(x))))
             return {rq, rs, cq, cs};
     }
     auto r = general("primus_turbo::quantize_mx_general", x, dtype, row, col, row_flags, col_flags);

@@ -172,3 +172,83 @@ def test_refusals(bad):
     args = (a, sa, False, b, sb, True, BF16, False, G.ROWWISE.value, 1)
     assert isinstance(_run(torch.ops.primus_turbo.gemm_fp8_impl_general, args), str)
     _same("primus_turbo", "gemm_fp8_impl", *args)
+
+
+# What the C library answers: every entry point returns `status` and counts the call, none launches anything.
+_STUB = """
+int status, calls;
+const char *pt_last_error(void) { return "stub"; }
+unsigned long pt_gemm_fp8_workspace_bytes(void) { return 0; }
+unsigned long pt_gemm_mx_workspace_bytes(void) { return 0; }
+unsigned long pt_quantize_fp8_rowwise_outer_workspace_bytes(void) { return 256; }
+int pt_gemm_fp8_vec_in_place(void) { return 0; }
+int pt_gemm_fp8_nn_in_place(void) { return 0; }
+""" + "".join(f"int {n}(void) {{ ++calls; return status; }}\n" for n in (
+    "pt_gemm_fp8", "pt_gemm_mx", "pt_quantize_fp8_tensorwise_static", "pt_quantize_fp8_tensorwise_t", "pt_dequantize_fp8_tensorwise",
+    "pt_quantize_fp8_rowwise", "pt_quantize_fp8_rowwise_padded", "pt_quantize_fp8_rowwise_outer_ld",
+    "pt_quantize_fp8_blockwise_kmajor", "pt_quantize_mx"))
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    import ctypes
+    import subprocess
+
+    d = tmp_path_factory.mktemp("stub")
+    (d / "stub.c").write_text(_STUB)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(d / "stub.so"), str(d / "stub.c")], check=True)
+    return ctypes.CDLL(str(d / "stub.so")), str(d / "stub.so")
+
+
+@pytest.mark.parametrize("status", ["LAUNCH", "INVALID_ARGUMENT", "UNSUPPORTED", "WORKSPACE"])
+def test_status_of_the_library(stub, status):
+    """A call that the library refuses goes to the Python body. One whose launch failed raises and is not issued again:
+    the error may be one that an earlier call left, found after a kernel that did run, and an accumulating product would
+    add twice."""
+    import ctypes
+
+    from primus_turbo import _native as N
+
+    x = bf16_randn((64, 256), seed=1).cuda()
+    q, one = x.to(E4M3), torch.full((), 0.5, device="cuda")
+    qt, s, qmx, smx = *torch.ops.primus_turbo.quant_fp8_rowwise_padded_impl(x, E4M3, 256), *torch.ops.primus_turbo.quantize_mx(x, E4M3, True, False, 8, 8)[:2]
+    own, ext = torch.ops.primus_turbo, torch.ops.primus_turbo_cpp_extension
+    product = (q, one, False, q, one, True)
+    out = torch.zeros(64, 64, device="cuda")
+    calls = {
+        "gemm": lambda: own.gemm_fp8_impl(*product, F32, False, G.TENSORWISE.value, 1),
+        "gemm mx": lambda: own.gemm_fp8_impl(qmx, smx, False, qmx, smx, True, F32, False, G.MX_BLOCKWISE.value, 1),
+        "accumulating": lambda: own.gemm_fp8_accum_impl(*product, F32, False, G.TENSORWISE.value, out, 1),
+        "accumulating mx": lambda: own.gemm_fp8_accum_impl(qmx, smx, False, qmx, smx, True, F32, False, G.MX_BLOCKWISE.value, out, 1),
+        "tensorwise": lambda: ext.quantize_fp8_tensorwise(x, E4M3, None),
+        "tensorwise t": lambda: own.quantize_fp8_tensorwise_t(x, E4M3, 256, 128),
+        "dequantize": lambda: ext.dequantize_fp8_tensorwise(q, one, BF16),
+        "rowwise": lambda: ext.quantize_fp8_rowwise(x, E4M3, -1, None),
+        "rowwise padded": lambda: own.quant_fp8_rowwise_padded_impl(x, E4M3, 384),
+        "rowwise t": lambda: own.quant_fp8_rowwise_t_impl(qt, s, BF16, E4M3, 128, None),
+        "kmajor": lambda: own.quant_fp8_blockwise_kmajor_impl(x, E4M3, 128, True),
+        "mx": lambda: own.quantize_mx(x, E4M3, True, True, 8, 8),
+    }
+    lib, path = stub
+    code, counter = ctypes.c_int.in_dll(lib, "status"), ctypes.c_int.in_dll(lib, "calls")
+
+    def results(call):
+        out.zero_()
+        r = call()
+        r = out.clone() if r is None else r
+        return [t.contiguous().flatten().view(torch.uint8) for t in (r if isinstance(r, (list, tuple)) else [r])]
+
+    code.value, want = getattr(N, "PT_ERR_" + status), {name: results(call) for name, call in calls.items()}
+    own._bind_native(path)
+    try:
+        for name, call in calls.items():
+            counter.value = 0
+            if status == "LAUNCH":
+                with pytest.raises(RuntimeError, match="native error -4: stub"):
+                    results(call)
+                assert not out.any(), name  # (a second launch would have been the real library's)
+            else:
+                assert all(torch.equal(g, w) for g, w in zip(results(call), want[name])), name
+            assert counter.value == 1, name
+    finally:
+        own._bind_native(str(N.LIB_PATH))
