@@ -52,7 +52,7 @@ from primus_turbo.pytorch.kernels.quantization.quantization_impl import (
     quantize_mx_operands,
 )
 from primus_turbo.pytorch.ops.quantization import dequantize_fp8, quantize_fp8, quantize_fp8_with_trans
-from primus_turbo.pytorch.ops.utils import _get_dummy_wgrad, _get_fp8_dtype, _setup_fused_grad_accum
+from primus_turbo.pytorch.ops.utils import _get_dummy_wgrad, _get_fp8_dtype, _setup_fused_grad_accum, _traced
 
 __all__ = ["gemm_fp8"]
 
@@ -109,7 +109,7 @@ class FP8GemmTensorFunction(torch.autograd.Function):
 
         # (the large tile reads the forward codes as they lie in both backward products: no transposed copies)
         # (where the forward product needs no padding of its rows)
-        if (nt_bwd and plain and need_bwd and b.shape[1] % 128 == 0 and not torch.compiler.is_compiling() and a.is_cuda
+        if (nt_bwd and plain and need_bwd and b.shape[1] % 128 == 0 and not _traced(a, b) and a.is_cuda
                 and vec_reads_in_place(a.shape[0], b.shape[1], b.shape[0], False)
                 and vec_reads_in_place(b.shape[0], b.shape[1], a.shape[0], True)):
             nt_bwd = False
@@ -261,7 +261,7 @@ class FP8GemmBlockFunction(torch.autograd.Function):
             check_quantized_tensor(b, config, scaling_recipe=w_recipe)
             b_q, b_s = b.qdata, b.scale_inv
         elif ((need_bwd or not trans_b) and b.dim() == 2 and b.size(0) % 16 == 0
-              and not (trans_b and a.dim() == 2 and not torch.compiler.is_compiling() and b.is_cuda
+              and not (trans_b and a.dim() == 2 and not _traced(a, b) and b.is_cuda
                        and kn_layer_pays(a.shape[0]) and reads_kn_in_place(a.shape[0], b.shape[1], b.shape[0]))):
             b_q, b_q_t, b_s = quant_fp8_blockwise_for_weight_dual_impl(b, fdt, bs)
         else:

@@ -62,6 +62,7 @@ from primus_turbo.pytorch.ops.utils import (
     _get_dummy_wgrad,
     _get_fp8_dtype,
     _setup_fused_grad_accum,
+    _traced,
 )
 
 __all__ = ["grouped_gemm_fp8", "glu_grouped_gemm_fp8"]
@@ -95,7 +96,7 @@ def _block_forward_product(a_fp8_row, a_scale_row, b, group_lens, group_offs, tr
         check_quantized_tensor(b, config, scaling_recipe=b_recipe)
         b_fp8, b_scale = b.qdata, b.scale_inv
     elif ((need_bwd or not trans_b) and b.size(-2) % 16 == 0
-          and not (trans_b and not torch.compiler.is_compiling() and b.is_cuda
+          and not (trans_b and not _traced(a_fp8_row, b) and b.is_cuda
                    and reads_kn_in_place(b.shape[0], a_fp8_row.shape[0], b.shape[2], b.shape[1])
                    and kn_layer_pays(a_fp8_row.shape[0] // b.shape[0]))):
         b_fp8, b_fp8_t, b_scale = quant_fp8_blockwise_for_weight_dual_impl(b, b_dtype, block_size=bs)

@@ -6,6 +6,8 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from torch._subclasses.fake_tensor import FakeTensor
+
 from primus_turbo.pytorch.core.low_precision import Format, float8_e4m3, float8_e5m2
 
 
@@ -18,6 +20,13 @@ def _get_fp8_dtype(format: Format, is_fwd_stage: bool) -> torch.dtype:
     if format == Format.HYBRID:
         return float8_e4m3 if is_fwd_stage else float8_e5m2
     raise ValueError(f"Unsupported FP8 format: {format}")
+
+
+def _traced(*tensors: torch.Tensor) -> bool:
+    """Whether the call is traced, by ``torch.compile`` or otherwise: sizes may be symbolic, and asking the native library
+    about them would pin the graph to the sizes it was traced with (and needs the library, which shapes alone do not)."""
+    return torch.compiler.is_compiling() or any(
+        isinstance(t, FakeTensor) or not all(type(n) is int for n in t.shape) for t in tensors)
 
 
 def _ensure_contiguous_grad_out(grad_out: torch.Tensor) -> torch.Tensor:

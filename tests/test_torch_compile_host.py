@@ -122,3 +122,27 @@ def test_mx_dispatcher_meta_shapes_with_shuffled_scales(turbo):
     assert tuple(s.shape) == (3, 136, 8)
     rq, rs, cq, cs = ext.quantize_mxfp8_dual(x, torch.float8_e4m3fn, 128, False, False, False, False, True, False)
     assert tuple(rs.shape) == (3, 136, 8) and tuple(cq.shape) == (3, 160, 256) and tuple(cs.shape) == (3, 256, 8)
+
+
+# (grouped: no tensorwise products, and MX groups are padded by a number on the host)
+@pytest.mark.parametrize("gran,grouped", [(g, False) for g in GRANS] + [("rowwise", True), ("blockwise", True)])
+def test_symbolic_sizes_stay_symbolic(turbo, gran, grouped):
+    """Tracing without ``torch.compile``: sizes at which backward reads the weight in place as well do not pin the graph."""
+    from torch._subclasses import FakeTensorMode
+    from torch.fx.experimental.symbolic_shapes import DimDynamic, ShapeEnv, StatelessSymbolicContext
+
+    mode = FakeTensorMode(shape_env=ShapeEnv())
+
+    def symbolic(*shape):
+        t = mode.from_tensor(_meta(*shape, grad=False), symbolic_context=StatelessSymbolicContext([DimDynamic.DYNAMIC] * len(shape)))
+        with mode:
+            return torch.empty(t.shape, dtype=t.dtype, device="cuda", requires_grad=True)
+
+    a, b = symbolic(8192, 4096) if grouped else symbolic(4096, 4096), symbolic(4, 4096, 4096) if grouped else symbolic(4096, 4096)
+    with mode:
+        if grouped:
+            lens = torch.empty(4, device="cuda", dtype=torch.int64)
+            out = turbo.ops.grouped_gemm_fp8(a, b, lens, trans_b=True, config=_cfg(gran))
+        else:
+            out = turbo.ops.gemm_fp8(a, b, False, True, torch.bfloat16, _cfg(gran))
+    assert all(isinstance(n, torch.SymInt) and n.node.maybe_as_int() is None for n in out.shape), out.shape
