@@ -25,8 +25,15 @@ def _get_fp8_dtype(format: Format, is_fwd_stage: bool) -> torch.dtype:
 def _traced(*tensors: torch.Tensor) -> bool:
     """Whether the call is traced, by ``torch.compile`` or otherwise: sizes may be symbolic, and asking the native library
     about them would pin the graph to the sizes it was traced with (and needs the library, which shapes alone do not)."""
-    return torch.compiler.is_compiling() or any(
-        isinstance(t, FakeTensor) or not all(type(n) is int for n in t.shape) for t in tensors)
+    if torch.compiler.is_compiling():
+        return True
+    for t in tensors:
+        if isinstance(t, FakeTensor):
+            return True
+        for n in t.shape:
+            if type(n) is not int:
+                return True
+    return False
 
 
 def _ensure_contiguous_grad_out(grad_out: torch.Tensor) -> torch.Tensor:
