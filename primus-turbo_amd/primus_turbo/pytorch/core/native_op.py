@@ -39,6 +39,18 @@ def _wants_gradient(args, kwargs) -> bool:
     return torch.is_grad_enabled() and torch._C._any_requires_grad(*args, **kwargs)
 
 
+def _autograd_kernel(name: str) -> Callable:
+    op, qualname = getattr(torch.ops.primus_turbo, name).default, f"primus_turbo::{name}"
+
+    def kernel(*args, **kwargs):
+        if _wants_gradient(args, kwargs):
+            return _NoBackward.apply(qualname, op, kwargs, *args)
+        with _below_autograd():
+            return op(*args, **kwargs)
+
+    return kernel
+
+
 def native_op(qualname: str, device_types: Optional[str] = None, cpp: bool = False) -> Callable:
     """``torch.library.custom_op(qualname, mutates_args=(), device_types=...)`` for functions that allocate
     their results, launch on the current stream and return: the same operator for tracing (schema from the
@@ -52,27 +64,20 @@ def native_op(qualname: str, device_types: Optional[str] = None, cpp: bool = Fal
     which advances that tensor's version.
 
     ``cpp``: the operator's CUDA kernel is in csrc/torch_ops.cpp; the function is the body for every other
-    device and, as the operator ``<name>_general``, for the forms which that kernel does not handle itself."""
+    device and, as the operator ``<name>_general`` (with the same fake and the same autograd), for the forms which that kernel does
+    not handle itself."""
     namespace, name = qualname.split("::")
     assert namespace == "primus_turbo"
 
     def wrap(fn: Callable) -> Callable:
         schema, key = torch.library.infer_schema(fn, mutates_args=()), "CUDA" if device_types == "cuda" else "CompositeExplicitAutograd"
-        _lib.define(name + schema, tags=(torch.Tag.pt2_compliant_tag,))
-        if cpp:
-            _lib.define(name + "_general" + schema)
-            _lib.impl(name + "_general", fn, key)
-        if not cpp or key != "CUDA":
-            _lib.impl(name, fn, key)
+        names = [name, name + "_general"] if cpp else [name]
+        for n in names:
+            _lib.define(n + schema, tags=(torch.Tag.pt2_compliant_tag,))
+            if not cpp or n != name or key != "CUDA":
+                _lib.impl(n, fn, key)
+            _lib.impl(n, _autograd_kernel(n), "Autograd")
         op = getattr(torch.ops.primus_turbo, name).default
-
-        def autograd_kernel(*args, **kwargs):
-            if _wants_gradient(args, kwargs):
-                return _NoBackward.apply(qualname, op, kwargs, *args)
-            with _below_autograd():
-                return op(*args, **kwargs)
-
-        _lib.impl(name, autograd_kernel, "Autograd")
 
         def call(*args, **kwargs):
             if _is_compiling() or _wants_gradient(args, kwargs) or _is_excluded(_AUTOGRAD):
@@ -84,7 +89,7 @@ def native_op(qualname: str, device_types: Optional[str] = None, cpp: bool = Fal
                 _set_excluded(_AUTOGRAD, False)
 
         call.__name__, call.__doc__, call.__module__ = fn.__name__, fn.__doc__, fn.__module__
-        call.register_fake = lambda fake: torch.library.register_fake(qualname, fake, lib=_lib)
+        call.register_fake = lambda fake: [torch.library.register_fake(f"{namespace}::{n}", fake, lib=_lib) for n in names]
         return call
 
     return wrap

@@ -131,3 +131,20 @@ def test_native_op_traced_and_batched(fill):
 
     with FakeTensorMode():
         assert fill(torch.ones(3), 2, torch.ones(3)).shape == (3,)
+
+
+@pytest.mark.parametrize("pinned", [0, 3])
+def test_product_with_a_pinned_tile(pinned, monkeypatch):
+    """The operator behind ``gemm_fp8_impl`` while a tile is pinned is traced and refuses a backward pass as the other."""
+    from primus_turbo.pytorch.kernels.gemm import gemm_fp8_impl as impl
+
+    monkeypatch.setattr(impl, "TILE_CFG", pinned)
+    scale = _meta(1, dtype=torch.float32)
+    args = (_codes(48, 256), scale, False, _codes(32, 256), _meta(1, dtype=torch.float32, grad=False), True, HP, True, G.TENSORWISE.value, 1)
+    out = impl.gemm_fp8_impl(*args)
+    assert out.shape == (32, 48) and out.dtype == HP
+    with pytest.raises(RuntimeError, match=NO_FORMULA):
+        (out.float().sum() + scale.sum()).backward()
+    torch._dynamo.reset()
+    with torch.no_grad():
+        assert torch.compile(impl.gemm_fp8_impl, backend="aot_eager", fullgraph=True)(*args).shape == (32, 48)
