@@ -1,5 +1,6 @@
-"""Build libprimus_turbo_amd.so (the C-ABI library) with hipcc for gfx950, and libprimus_turbo_torch.so (the host side of
-the dense torch operators, csrc/torch_ops.cpp) with the host compiler against the installed torch.
+"""Build libprimus_turbo_amd.so (the C-ABI library) with hipcc for gfx950, and libprimus_turbo_torch-<torch's version>.so
+(the host side of the dense torch operators, csrc/torch_ops.cpp) with the host compiler against the installed torch. Without
+torch the C library is all that there is to build.
 
 Usage:  python primus-turbo_amd/build_native.py [--force] [-j N]
 
@@ -11,6 +12,7 @@ cross-compiles for gfx950, so no GPU is needed to build.
 from __future__ import annotations
 
 import argparse
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -23,7 +25,6 @@ CSRC = ROOT / "csrc"
 BUILD = ROOT / "build"
 LIBDIR = ROOT / "lib"
 LIBNAME = "libprimus_turbo_amd.so"
-TORCH_LIBNAME = "libprimus_turbo_torch.so"
 HEADER = ROOT.parent / "include" / "primus_turbo_amd.h"
 
 ARCH = "gfx950"
@@ -54,13 +55,20 @@ def lib_path() -> Path:
     return LIBDIR / LIBNAME
 
 
-def torch_lib_path() -> Path:
-    return LIBDIR / TORCH_LIBNAME
+def torch_lib_path() -> Path | None:
+    """The library for the installed torch (its C++ interface is that version's alone), None without one."""
+    if importlib.util.find_spec("torch") is None:
+        return None
+    import torch
+
+    return LIBDIR / f"libprimus_turbo_torch-{torch.__version__}.so"
 
 
-def _build_torch_ops(force: bool, verbose: bool) -> Path:
+def _build_torch_ops(force: bool, verbose: bool) -> Path | None:
     """One host translation unit on torch's headers; the HIP runtime is the one that torch ships."""
     src, out = CSRC / "torch_ops.cpp", torch_lib_path()
+    if out is None:
+        return None
     if not force and out.exists() and out.stat().st_mtime >= max(src.stat().st_mtime, HEADER.stat().st_mtime):
         return out
     import torch
@@ -127,7 +135,6 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = False) -
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         torch_ops = ex.submit(_build_torch_ops, force, verbose)
         objs = list(ex.map(lambda s: _compile_one(hipcc, s, force, verbose), srcs))
-        torch_ops.result()
     out = lib_path()
     cmd = [hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", str(out)] + [str(o) for o in objs]
     if verbose:
@@ -135,13 +142,14 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = False) -
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
+    torch_ops.result()  # (a failure there leaves the C library built)
     return out
 
 
 def ensure_built() -> Path:
     """Return the library path, building the libraries only when one does not exist yet."""
-    out = lib_path()
-    if not out.exists() or not torch_lib_path().exists():
+    out, torch_out = lib_path(), torch_lib_path()
+    if not out.exists() or (torch_out is not None and not torch_out.exists()):
         build()
     return out
 

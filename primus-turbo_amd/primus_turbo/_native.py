@@ -18,8 +18,9 @@ import torch
 
 _PKG_ROOT = Path(__file__).resolve().parent.parent  # .../primus-turbo_amd
 LIB_PATH = Path(os.environ.get("PRIMUS_TURBO_AMD_LIB", _PKG_ROOT / "lib" / "libprimus_turbo_amd.so"))
-#: the CUDA kernels of the dense operators (csrc/torch_ops.cpp), which call the entry points of LIB_PATH
-TORCH_LIB_PATH = _PKG_ROOT / "lib" / "libprimus_turbo_torch.so"
+#: the CUDA kernels of the dense operators (csrc/torch_ops.cpp), which call the entry points of LIB_PATH. Built for one
+#: version of torch: a library of another one's is a missing one.
+TORCH_LIB_PATH = _PKG_ROOT / "lib" / f"libprimus_turbo_torch-{torch.__version__}.so"
 
 # element type codes of include/primus_turbo_amd.h
 DT_BF16, DT_F16, DT_F32, DT_E4M3, DT_E5M2, DT_E2M1X2, DT_E8M0 = range(7)
