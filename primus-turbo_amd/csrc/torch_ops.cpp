@@ -31,6 +31,7 @@ struct Api {
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
     PT_FN(pt_gemm_fp8_vec_in_place);
+    PT_FN(pt_gemm_fp8_nn_in_place);
     PT_FN(pt_gemm_mx);
     PT_FN(pt_gemm_mx_workspace_bytes);
     PT_FN(pt_quantize_fp8_tensorwise_static);
@@ -60,6 +61,7 @@ void bind_native(std::string path) {
     PT_FN(pt_gemm_fp8);
     PT_FN(pt_gemm_fp8_workspace_bytes);
     PT_FN(pt_gemm_fp8_vec_in_place);
+    PT_FN(pt_gemm_fp8_nn_in_place);
     PT_FN(pt_gemm_mx);
     PT_FN(pt_gemm_mx_workspace_bytes);
     PT_FN(pt_quantize_fp8_tensorwise_static);
@@ -196,17 +198,21 @@ bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tenso
             return false;
         sa_m = sb_n = 1;
     } else if (granularity == BLOCKWISE) {
-        if (trans_a || !trans_b)
-            return false;
-        if (a_s.dim() != 2 || b_s.dim() != 2 || !b_s.is_contiguous())
+        if (trans_a || a_s.dim() != 2 || b_s.dim() != 2 || !b_s.is_contiguous())
             return false;
         mode = 1;
-        if (a_s.size(0) == M && a_s.size(1) == kb && b_s.size(0) == cdiv(N, 128) && b_s.size(1) == kb) {
-            // row blocks and tiles: the view of a block-major tensor that the activation's quantizer made
-            if (kb == 1 || a_s.stride(0) != 1 || a_s.stride(1) != M)
+        // row blocks: the view of a block-major tensor that the activation's quantizer made
+        const int64_t nb        = cdiv(N, 128);
+        const bool    row_major = a_s.size(0) == M && a_s.size(1) == kb;
+        const bool    rows      = row_major && kb > 1 && a_s.stride(0) == 1 && a_s.stride(1) == M;
+        if (trans_b && row_major && b_s.size(0) == nb && b_s.size(1) == kb) {
+            if (!rows)
                 return false;
             sa_m = 1, sa_k = M, sb_n = kb, sb_k = 1, sb_blk = 128;
-        } else if (a_s.is_contiguous() && a_s.size(0) == kb && a_s.size(1) == M && b_s.size(0) == kb && b_s.size(1) == N) {
+        } else if (!trans_b && rows && b_s.size(0) == kb && b_s.size(1) == nb) {
+            // the input gradient: the weight's codes and tiles as the forward product reads them
+            sa_m = 1, sa_k = M, sb_n = 1, sb_k = nb, sb_blk = 128;
+        } else if (trans_b && a_s.is_contiguous() && a_s.size(0) == kb && a_s.size(1) == M && b_s.size(0) == kb && b_s.size(1) == N) {
             // both operands transposed 128 x 1 column quantizations: a scale per row of either
             sa_m = 1, sa_k = M, sb_n = 1, sb_k = N;
         } else {
@@ -228,7 +234,8 @@ bool launch_scaled(const Tensor &a, const Tensor &a_s, bool trans_a, const Tenso
         trans_b          = !was_a;
     }
     const bool   in_place = mode == 0 && !trans_b && api.pt_gemm_fp8_vec_in_place(M, N, K, trans_a);
-    const size_t ws_bytes = in_place ? 0 : api.pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, trans_b);
+    const bool   b_as_is  = trans_b || (mode == 1 && !trans_a && sa_blk == 1 && sb_blk == 128 && api.pt_gemm_fp8_nn_in_place(M, N, K));
+    const size_t ws_bytes = in_place ? 0 : api.pt_gemm_fp8_workspace_bytes(M, N, K, trans_a, b_as_is);
     Tensor       ws;
     if (ws_bytes)
         ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, a);

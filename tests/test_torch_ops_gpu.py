@@ -138,6 +138,10 @@ def test_products(M, N, K, trans_c, out_dtype):
     product(qa, km.t().contiguous(), False, qb, tiles, True, G.BLOCKWISE)
     product(qa, km.t(), False, qb, tiles.t().contiguous().t(), True, G.BLOCKWISE)
     product(qa, km, False, qb, torch.rand(kb, N, device="cuda"), True, G.BLOCKWISE)
+    tiles_t, bt = tiles.t().contiguous(), qb.t().contiguous()
+    product(qa, km.t(), False, bt, tiles_t, False, G.BLOCKWISE)
+    product(qa, km.t().contiguous(), False, bt, tiles_t, False, G.BLOCKWISE)
+    _same("primus_turbo", "gemm_fp8_impl", qa, km.t(), False, bt, tiles, False, out_dtype, trans_c, G.BLOCKWISE.value, 1)  # (the wrong way round)
     if M and K % 32 == 0:
         wa, sa, _, _ = torch.ops.primus_turbo.quantize_mx(a, E4M3, True, True, 8, 8)
         wb, sb, _, _ = torch.ops.primus_turbo.quantize_mx(b, E4M3, True, True, 8, 8)
@@ -214,10 +218,13 @@ def test_status_of_the_library(stub, status):
     qt, s, qmx, smx = *torch.ops.primus_turbo.quant_fp8_rowwise_padded_impl(x, E4M3, 256), *torch.ops.primus_turbo.quantize_mx(x, E4M3, True, False, 8, 8)[:2]
     own, ext = torch.ops.primus_turbo, torch.ops.primus_turbo_cpp_extension
     product = (q, one, False, q, one, True)
+    km, tiles, bt = torch.rand(2, 64, device="cuda"), torch.rand(1, 2, device="cuda"), q.t().contiguous()
     out = torch.zeros(64, 64, device="cuda")
     calls = {
         "gemm": lambda: own.gemm_fp8_impl(*product, F32, False, G.TENSORWISE.value, 1),
         "gemm mx": lambda: own.gemm_fp8_impl(qmx, smx, False, qmx, smx, True, F32, False, G.MX_BLOCKWISE.value, 1),
+        "gemm block": lambda: own.gemm_fp8_impl(q, km.t(), False, q, tiles, True, F32, False, G.BLOCKWISE.value, 1),
+        "gemm block, b [K, N]": lambda: own.gemm_fp8_impl(q, km.t(), False, bt, tiles.t().contiguous(), False, F32, False, G.BLOCKWISE.value, 1),
         "accumulating": lambda: own.gemm_fp8_accum_impl(*product, F32, False, G.TENSORWISE.value, out, 1),
         "accumulating mx": lambda: own.gemm_fp8_accum_impl(qmx, smx, False, qmx, smx, True, F32, False, G.MX_BLOCKWISE.value, out, 1),
         "tensorwise": lambda: ext.quantize_fp8_tensorwise(x, E4M3, None),
