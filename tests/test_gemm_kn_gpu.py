@@ -167,14 +167,13 @@ def test_mx_grouped(lens, n, k, da, out_dtype):
 
 @pytest.mark.parametrize("hybrid", [False, True])
 @pytest.mark.parametrize("glu", [False, True])
-@pytest.mark.parametrize("n,k", [(640, 384), (512, 400)])  # (the second: blocks of 32, not of 128)
+@pytest.mark.parametrize("n,k", [(640, 384), (512, 416)])  # (the second: blocks of 32, not of 128)
 def test_mx_layer_gradients(glu, hybrid, n, k, monkeypatch):
     import importlib
 
     ops = importlib.import_module("primus_turbo.pytorch.ops.grouped_gemm_fp8")
     config = LP.Float8QuantConfig(granularity=G.MX_BLOCKWISE, block_size=32, scale_dtype=LP.ScaleDtype.E8M0,
                                   format=LP.Format.HYBRID if hybrid else LP.Format.E4M3)
-    k = k // 32 * 32
     lens = torch.tensor([300, 0, 213, 87], device="cuda")
     x = bf16_randn((600, 2 * k if glu else k), seed=1).cuda().requires_grad_()
     w = bf16_randn((4, n, k), seed=2).cuda().requires_grad_()
@@ -280,7 +279,8 @@ def test_mxfp4_grouped(lens, n, k, out_dtype):
 
 
 @pytest.mark.parametrize("glu", [False, True])
-@pytest.mark.parametrize("n,k", [(1280, 384), (1152, 384)])  # (the second: an odd number of half slabs)
+# (the second: an odd number of half slabs; the third: blocks of 32, not of 128)
+@pytest.mark.parametrize("n,k", [(1280, 384), (1152, 384), (1280, 416)])
 def test_mxfp4_layer_gradients(glu, n, k, monkeypatch):
     import importlib
 
@@ -297,7 +297,7 @@ def test_mxfp4_layer_gradients(glu, n, k, monkeypatch):
         out = (ops.glu_grouped_gemm_fp4(x, p, w, lens, trans_b=True, config=config, act_type="silu") if glu else
                ops.grouped_gemm_fp4(x, w, lens, trans_b=True, config=config))
         grads.append((out, *torch.autograd.grad(out, (x, w, p) if glu else (x, w), g)))
-    assert used == [n % 256 == 0] * 2
+    assert used == ([n % 256 == 0] * 2 if k % 128 == 0 else [])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
 
 
