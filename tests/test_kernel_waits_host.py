@@ -7,8 +7,12 @@ compiler's own wait-count bookkeeping does not see those; if it believes that a 
 the epilogue may still be outstanding when the K loop of the next tile begins (a load and its use
 in two separately guarded blocks are enough), it puts an ``s_waitcnt vmcnt(0)`` in front of the
 first instruction of the loop that overwrites the load's register -- and every slab then begins by
-waiting for all copies in flight (dense MXFP8 16384^3: 3.2 -> 3.7 ms). The test compiles three
-translation units to assembly (no GPU needed) and looks at the MFMA loops of their kernels."""
+waiting for all copies in flight (dense MXFP8 16384^3: 3.2 -> 3.7 ms). The test compiles the
+translation units to assembly (no GPU needed) and looks at the MFMA loops of their kernels.
+
+Kernels that transpose an operand as they read it issue their copies in ``asm`` statements, which the
+compiler's hazard recognizer does not look into: each statement has to keep the wait states in front of
+its load, and M0 has to be its alone."""
 
 import re
 import subprocess
@@ -57,6 +61,45 @@ def _compiler_vmcnt_waits(seg):
     return out
 
 
+def _split_asm(seg):
+    """``(statements, rest)``: the instructions of each ``asm`` statement, and those of the compiler."""
+    statements, rest, inside = [], [], False
+    for x in seg:
+        if "#ASMSTART" in x or "#ASMEND" in x:
+            inside = "#ASMSTART" in x
+            if inside:
+                statements.append([])
+        elif x := x.split(";")[0].strip():
+            (statements[-1] if inside else rest).append(x)
+    return statements, rest
+
+
+def _faults_of_copies(seg):
+    """``(copies, faults)`` of a kernel: the copies to the LDS in its ``asm`` statements, those whose statement has less than
+    five wait states in front of the load (VALU write of a scalar register -> VMEM read of it), and other uses of M0."""
+    statements, rest = _split_asm(seg)
+    copies, faults = 0, []
+    for s in statements:
+        at = next((i for i, x in enumerate(s) if re.match(r"buffer_load_\w+ .* lds\b", x)), None)
+        if at is None:
+            continue
+        copies += 1
+        states = sum(int(x.split()[1], 0) + 1 if x.startswith("s_nop") else 1 for x in s[:at])
+        if states < 5 or not re.match(r"s_\w+ m0\b", s[0]):
+            faults.append("; ".join(s))
+    return copies, faults + ([x for x in rest if re.search(r"\bm0\b", x)] if copies else [])
+
+
+def test_scanner_sees_a_hazard():
+    def copy(nop):
+        return ["\t;;#ASMSTART", "\ts_add_u32 m0, s4, 16", f"\ts_nop {nop}", "\tbuffer_load_dword v1, s[0:3], 0 offen lds", "\t;;#ASMEND"]
+
+    assert _faults_of_copies(copy(3) + ["\tv_readlane_b32 s1, v2, 0"] + copy(4)) == (2, [])
+    assert _faults_of_copies(copy(0) + copy(3)) == (2, ["s_add_u32 m0, s4, 16; s_nop 0; buffer_load_dword v1, s[0:3], 0 offen lds"])
+    assert _faults_of_copies(copy(3) + ["\ts_mov_b32 m0, s7 ; m0"]) == (1, ["s_mov_b32 m0, s7"])
+    assert _faults_of_copies(["\ts_mov_b32 m0, s7", "\tbuffer_load_dword v1, s[0:3], 0 offen lds"]) == (0, [])
+
+
 def test_scanner_sees_a_compiler_wait():
     body = [".LBB0_1:"] + ["\tv_mfma_f32 a, b, c"] * 16 + ["\t;;#ASMSTART", "\ts_waitcnt vmcnt(3)", "\t;;#ASMEND",
                                                           "\ts_waitcnt vmcnt(0)", "\ts_cbranch_scc0 .LBB0_1"]
@@ -67,18 +110,24 @@ def test_scanner_sees_a_compiler_wait():
 # translation unit -> which of its kernels are looked at: the dense MX kernels (gemm_mx8_kernel and
 # gemm_fp8_nt_kernel<TM, TN, 2 = MX, ...>), the block-scaled eight-wavefront kernel of the
 # headline workload (the four-wavefront block kernels of that unit load their scales into
-# registers inside the loop and wait for them legitimately) and the grouped vector-scale kernels
+# registers inside the loop and wait for them legitimately), its grouped form, the grouped vector-scale kernels
+# and those that transpose an operand as they read it; and how many MFMA loops they have at least
 UNITS = {
     "gemm_mx.hip": (lambda n: "gemm_mx8_kernel" in n or re.search(r"gemm_fp8_nt_kernelILi\dELi\dELi2E", n), 8),
     "gemm_fp8_block.hip": (lambda n: "gemm_fp8_block8_kernel" in n, 4),
     # vector scales (tensorwise / rowwise), row groups and variable K: the epilogue loads its scales
     "gemm_fp8_grouped_vec.hip": (lambda n: re.search(r"gemm_fp8_nt_kernelILi\dELi\dELi0E", n), 8),
+    "gemm_fp8_grouped.hip": (lambda n: "gemm_fp8_block8_kernel" in n, 8),
+    "gemm_fp8_kn.hip": (lambda n: "gemm_fp8_nt_kernel" in n, 8),
+    "gemm_mx_grouped_kn.hip": (lambda n: "gemm_fp8_nt_kernel" in n, 10),
 }
+# those of them with copies in asm statements, and in how many kernels
+COPIES = {"gemm_fp8_block.hip": 4, "gemm_fp8_grouped.hip": 4, "gemm_fp8_kn.hip": 8, "gemm_mx_grouped_kn.hip": 10}
 
 
 @pytest.fixture(scope="module")
 def assembly(tmp_path_factory):
-    """Device assembly of the units, compiled side by side (about two minutes of hipcc)."""
+    """Device assembly of the units, compiled side by side (about three minutes of hipcc)."""
     from concurrent.futures import ThreadPoolExecutor
 
     import build_native
@@ -118,3 +167,13 @@ def test_mfma_loops_have_no_compiler_inserted_vmcnt_wait(assembly, unit):
                 bad.append((name, waits))
     assert seen >= least, f"only {seen} MFMA loops found: the scanner no longer matches the compiler's output"
     assert not bad, bad
+
+
+@pytest.mark.parametrize("unit", sorted(COPIES))
+def test_copies_keep_their_wait_states(assembly, unit):
+    lines, kernels = assembly[unit], 0
+    for name, a, b in _functions(lines):
+        copies, faults = _faults_of_copies(lines[a:b])
+        kernels += copies > 0
+        assert not faults, (name, faults[:5])
+    assert kernels == COPIES[unit]
