@@ -17,8 +17,11 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
+
+import check_asm
 
 ROOT = Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
@@ -109,10 +112,16 @@ def _compile_one(hipcc: str, src: Path, force: bool, verbose: bool) -> Path:
     if not force and obj.exists():
         if obj.stat().st_mtime >= max(src.stat().st_mtime, _deps_mtime()):
             return obj
-    cmd = [hipcc, *HIPCC_FLAGS, *_extra_flags(src), "-c", str(src), "-o", str(obj)]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
+    with tempfile.TemporaryDirectory(dir=BUILD) as tmp:  # (for the assembly, which is looked at before the object counts)
+        made = Path(tmp) / obj.name
+        cmd = [hipcc, *HIPCC_FLAGS, *_extra_flags(src), "-save-temps=obj", "-c", str(src), "-o", str(made)]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        if res.returncode == 0:
+            asm = Path(tmp) / f"{src.stem}-hip-amdgcn-amd-amdhsa-{ARCH}.s"
+            check_asm.check(asm.read_text().split("\n"), src.name)
+            made.replace(obj)
     # the host pass warns that it does not know the packed-fp32 feature: harmless
     err = "\n".join(
         l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l and l.strip()

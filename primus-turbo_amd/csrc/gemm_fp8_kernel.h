@@ -175,11 +175,10 @@ template <int ROW, bool F4 = false> __device__ __forceinline__ i32x8 read_transp
 // A copy of 16 (4) bytes a lane to the 64 x 16 (64 x 4) bytes at `dst` + AT, from `src` + the lane's `off`, zeros where that is not within
 // `bytes`. As an instruction of our own: the compiler knows its builtin for one that writes the LDS, and makes the builtin
 // of the transposed read wait for every copy in flight (vmcnt(0) before each fragment), which the kernels' own waits have
-// seen to. The compiler does not see the load's hazards either, so the statement keeps them by itself: one wait state from
-// the write of M0, and five from a VALU instruction that wrote a register of the descriptor (v_readfirstlane, v_readlane of a
-// spilled one) in front of the statement. M0 is the statement's: a kernel that copies with this has no other use for it (the
-// compiler warns that it does not keep a reserved register; test_kernel_waits_host looks for one). No result register, so
-// nothing for the compiler to reuse early.
+// seen to. The statement has the one wait state from the write of M0. The compiler does not see that its load also has to be five
+// behind a VALU instruction that wrote a register of the descriptor, nor that M0 is taken (it warns that it keeps no
+// reserved register): the build looks at both in the assembly (check_asm.py). No result register, so nothing for the compiler to
+// reuse early.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 template <int SIZE, int AT>
@@ -190,9 +189,9 @@ __device__ __forceinline__ void copy_to_lds(uint8_t *dst, const uint8_t *src, ui
     const u32x4s     rsrc = {static_cast<uint32_t>(p), static_cast<uint32_t>(p >> 32) & 0xffffu, bytes, 0x00020000u};
     const uint32_t   lds  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)dst));
     if constexpr (SIZE == 16)
-        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
     else
-        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rsrc), "n"(AT) : "memory", "m0", "scc");
 #endif
 }
 #pragma clang diagnostic pop

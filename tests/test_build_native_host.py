@@ -16,8 +16,10 @@ def _tool(path, body):
     return str(path)
 
 
-# (stands for hipcc and g++: the word behind -o names the file to write)
-_COMPILES = 'while [ "$1" != -o ]; do shift; done; : > "$2"\n'
+# (stands for hipcc and g++: the word behind -o names the file to write, the assembly of a unit beside it)
+_COMPILES = """while [ "$1" != -o ]; do shift; done; : > "$2"
+case "$2" in *.o) cp "$ASM" "${2%.o}-hip-amdgcn-amd-amdhsa-gfx950.s";; esac
+"""
 
 
 @pytest.fixture
@@ -28,6 +30,8 @@ def tree(tmp_path, monkeypatch):
         (src / name).write_text("")
     for name, path in dict(CSRC=src, BUILD=tmp_path / "build", LIBDIR=tmp_path / "lib", HEADER=src / "a.h").items():
         monkeypatch.setattr(build_native, name, path)
+    (tmp_path / "asm").write_text("")
+    monkeypatch.setenv("ASM", str(tmp_path / "asm"))
     monkeypatch.setenv("HIPCC", _tool(tmp_path / "hipcc", _COMPILES))
     monkeypatch.setenv("CXX", _tool(tmp_path / "cxx", _COMPILES))
     return tmp_path
@@ -68,3 +72,12 @@ def test_library_of_another_torch(tree, monkeypatch):
     monkeypatch.setattr(torch, "__version__", "0.0")
     build_native.ensure_built()
     assert _libs(tree) == sorted([build_native.LIBNAME, TORCH_LIB, "libprimus_turbo_torch-0.0.so"])
+
+
+def test_unsafe_assembly(tree):
+    """A copy right behind a VALU write of its descriptor fails the build and leaves no object behind."""
+    (tree / "asm").write_text("_Z1k:\n\tv_readlane_b32 s1, v2, 0\n\t;;#ASMSTART\n\ts_add_u32 m0, s4, 16\n\ts_nop 0\n"
+                              "\tbuffer_load_dword v1, s[0:3], 0 offen lds\n\t;;#ASMEND\n.Lfunc_end0:\n")
+    with pytest.raises(RuntimeError, match="_Z1k: 1 unsafe uses"):
+        build_native.build()
+    assert not list((tree / "build").iterdir()) and not (tree / "lib" / build_native.LIBNAME).exists()

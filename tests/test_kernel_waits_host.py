@@ -10,9 +10,7 @@ first instruction of the loop that overwrites the load's register -- and every s
 waiting for all copies in flight (dense MXFP8 16384^3: 3.2 -> 3.7 ms). The test compiles the
 translation units to assembly (no GPU needed) and looks at the MFMA loops of their kernels.
 
-Kernels that transpose an operand as they read it issue their copies in ``asm`` statements, which the
-compiler's hazard recognizer does not look into: each statement has to keep the wait states in front of
-its load, and M0 has to be its alone."""
+The same assembly goes through what the build looks for in it (check_asm.py)."""
 
 import re
 import subprocess
@@ -23,18 +21,7 @@ import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
 sys.path.insert(0, str(ROOT / "primus-turbo_amd"))
-
-
-def _functions(lines):
-    cur = None
-    for i, line in enumerate(lines):
-        m = re.match(r"^(_Z\w+):", line)
-        if m:
-            cur = [m.group(1), i, None]
-        elif cur is not None and line.startswith(".Lfunc_end"):
-            cur[2] = i
-            yield tuple(cur)
-            cur = None
+import check_asm  # noqa: E402
 
 
 def _innermost_mfma_loops(body):
@@ -61,43 +48,30 @@ def _compiler_vmcnt_waits(seg):
     return out
 
 
-def _split_asm(seg):
-    """``(statements, rest)``: the instructions of each ``asm`` statement, and those of the compiler."""
-    statements, rest, inside = [], [], False
-    for x in seg:
-        if "#ASMSTART" in x or "#ASMEND" in x:
-            inside = "#ASMSTART" in x
-            if inside:
-                statements.append([])
-        elif x := x.split(";")[0].strip():
-            (statements[-1] if inside else rest).append(x)
-    return statements, rest
+def _copy(nop=0, descriptor="s[0:3]"):
+    return ["\t;;#ASMSTART", "\ts_add_u32 m0, s4, 16", f"\ts_nop {nop}", f"\tbuffer_load_dword v1, {descriptor}, 0 offen lds", "\t;;#ASMEND"]
 
 
-def _faults_of_copies(seg):
-    """``(copies, faults)`` of a kernel: the copies to the LDS in its ``asm`` statements, those whose statement has less than
-    five wait states in front of the load (VALU write of a scalar register -> VMEM read of it), and other uses of M0."""
-    statements, rest = _split_asm(seg)
-    copies, faults = 0, []
-    for s in statements:
-        at = next((i for i, x in enumerate(s) if re.match(r"buffer_load_\w+ .* lds\b", x)), None)
-        if at is None:
-            continue
-        copies += 1
-        states = sum(int(x.split()[1], 0) + 1 if x.startswith("s_nop") else 1 for x in s[:at])
-        if states < 5 or not re.match(r"s_\w+ m0\b", s[0]):
-            faults.append("; ".join(s))
-    return copies, faults + ([x for x in rest if re.search(r"\bm0\b", x)] if copies else [])
+@pytest.mark.parametrize("write,caught", [("v_readlane_b32 s3, v2, 0", True), ("v_readlane_b32 s4, v2, 0", False),
+                                          ("v_readfirstlane_b32 s0, v2", True), ("v_cmp_lt_u32_e64 s[2:3], v1, v2", True),
+                                          ("v_add_co_u32_e64 v1, s[0:1], v1, v2", True), ("v_add_u32_e32 v1, s0, v2", False),
+                                          ("s_mov_b32 s0, s7", False)])
+def test_check_sees_a_short_wait(write, caught):
+    three = ["\ts_nop 1", "\ts_mov_b32 s9, s8"]
+    fault = ["less than 5 wait states from a VALU write of the descriptor: buffer_load_dword v1, s[0:3], 0 offen lds"]
+    found = (1, fault if caught else [])
+    assert check_asm.faults_of_copies(["\t" + write] + _copy()) == found
+    assert check_asm.faults_of_copies(["\t" + write] + three[:1] + _copy()) == found  # (four states)
+    assert check_asm.faults_of_copies(["\t" + write] + three + _copy()) == (1, [])  # (five)
+    # on the way of a jump, and behind one that does not come here
+    loop = [".LBB0_1:"] + _copy() + ["\ts_nop 7", "\t" + write, "\ts_cbranch_scc0 .LBB0_1"]
+    assert check_asm.faults_of_copies(loop) == found
+    assert check_asm.faults_of_copies(["\t" + write, "\ts_branch .LBB0_2", ".LBB0_1:"] + _copy()) == (1, [])
 
 
-def test_scanner_sees_a_hazard():
-    def copy(nop):
-        return ["\t;;#ASMSTART", "\ts_add_u32 m0, s4, 16", f"\ts_nop {nop}", "\tbuffer_load_dword v1, s[0:3], 0 offen lds", "\t;;#ASMEND"]
-
-    assert _faults_of_copies(copy(3) + ["\tv_readlane_b32 s1, v2, 0"] + copy(4)) == (2, [])
-    assert _faults_of_copies(copy(0) + copy(3)) == (2, ["s_add_u32 m0, s4, 16; s_nop 0; buffer_load_dword v1, s[0:3], 0 offen lds"])
-    assert _faults_of_copies(copy(3) + ["\ts_mov_b32 m0, s7 ; m0"]) == (1, ["s_mov_b32 m0, s7"])
-    assert _faults_of_copies(["\ts_mov_b32 m0, s7", "\tbuffer_load_dword v1, s[0:3], 0 offen lds"]) == (0, [])
+def test_check_sees_another_use_of_m0():
+    assert check_asm.faults_of_copies(_copy() + ["\ts_mov_b32 m0, s7 ; m0"]) == (1, ["M0 is used besides the copies: s_mov_b32 m0, s7"])
+    assert check_asm.faults_of_copies(["\ts_mov_b32 m0, s7", "\tbuffer_load_dword v1, s[0:3], 0 offen lds"]) == (0, [])
 
 
 def test_scanner_sees_a_compiler_wait():
@@ -156,7 +130,7 @@ def test_mfma_loops_have_no_compiler_inserted_vmcnt_wait(assembly, unit):
     lines = assembly[unit]
     wanted, least = UNITS[unit]
     seen, bad = 0, []
-    for name, a, b in _functions(lines):
+    for name, a, b in check_asm.functions(lines):
         if not wanted(name):
             continue
         body = lines[a:b]
@@ -169,11 +143,11 @@ def test_mfma_loops_have_no_compiler_inserted_vmcnt_wait(assembly, unit):
     assert not bad, bad
 
 
-@pytest.mark.parametrize("unit", sorted(COPIES))
-def test_copies_keep_their_wait_states(assembly, unit):
+@pytest.mark.parametrize("unit", sorted(UNITS))
+def test_copies_are_checked(assembly, unit):
     lines, kernels = assembly[unit], 0
-    for name, a, b in _functions(lines):
-        copies, faults = _faults_of_copies(lines[a:b])
+    for name, a, b in check_asm.functions(lines):
+        copies, faults = check_asm.faults_of_copies(lines[a:b])
         kernels += copies > 0
         assert not faults, (name, faults[:5])
-    assert kernels == COPIES[unit]
+    assert kernels == COPIES.get(unit, 0)
