@@ -406,6 +406,10 @@ PT_API int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K);
 /* The same with vector scales, for trans_b 0 and either trans_a; such a product needs no workspace. */
 PT_API int pt_gemm_fp8_vec_in_place(int64_t M, int64_t N, int64_t K, int trans_a);
 PT_API int pt_grouped_gemm_fp8_nn_in_place(int64_t G, int64_t M, int64_t N, int64_t K);
+/* The tile_cfg that tile_cfg 0 stands for with vector scales on the current device (pt_gemm_mx_tile: of pt_gemm_mx, with rows of whole
+ * slabs), 0 for the kernel of products with few output tiles, -1 for no product. */
+PT_API int pt_gemm_fp8_tile(int64_t M, int64_t N, int64_t K);
+PT_API int pt_gemm_mx_tile(int64_t M, int64_t N, int64_t K, int fp4);
 PT_API int pt_gemm_fp8(const void *a, int a_dtype, const float *a_scale, const void *b, int b_dtype,
                        const float *b_scale, void *c, int c_dtype, int64_t M, int64_t N, int64_t K,
                        int trans_a, int trans_b, int scale_mode, int64_t sa_m, int64_t sa_k,

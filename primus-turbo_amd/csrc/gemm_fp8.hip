@@ -302,6 +302,12 @@ int pt_gemm_fp8_nn_in_place(int64_t M, int64_t N, int64_t K) {
     return M > 0 && N > 0 && K > 0 && block_nn_in_place(M, N, K, 0);
 }
 
+int pt_gemm_fp8_tile(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0)
+        return -1;
+    return gemm_direct_tile(M, N, K, SCALE_VECTOR, false) >= 0 ? 0 : dense_tile<SCALE_VECTOR>(M, N, padded_k(K) / KSTEP, true);
+}
+
 size_t pt_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K, int trans_a, int trans_b) {
     // An operand is copied into the workspace when its reduction axis is not contiguous
     // (transpose) or when K is not a multiple of 128 (zero padding of the K tail).

@@ -55,6 +55,15 @@ static int64_t mx_scale_words(int64_t K) {
     return cdiv(K / 32, 4);
 }
 
+int pt_gemm_mx_tile(int64_t M, int64_t N, int64_t K, int fp4) {
+    if (M <= 0 || N <= 0 || K <= 0)
+        return -1;
+    if (gemm_direct_tile(M, N, fp4 ? K / 2 : K, SCALE_MX, fp4 != 0) >= 0)
+        return 0;
+    const int64_t slabs = mx_row_bytes(K, fp4 != 0) / KSTEP;
+    return fp4 ? dense_tile<SCALE_MX, true>(M, N, slabs, false) : dense_tile<SCALE_MX>(M, N, slabs, true);
+}
+
 size_t pt_gemm_mx_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int fp4) {
     const int64_t need = mx_row_bytes(K, fp4 != 0);
     size_t        b    = 0;

@@ -144,6 +144,8 @@ _SIGNATURES = {
     "pt_gemm_fp8_nn_in_place": (c_int, [c_i64, c_i64, c_i64]),
     "pt_gemm_fp8_vec_in_place": (c_int, [c_i64, c_i64, c_i64, c_int]),
     "pt_grouped_gemm_fp8_nn_in_place": (c_int, [c_i64, c_i64, c_i64, c_i64]),
+    "pt_gemm_fp8_tile": (c_int, [c_i64, c_i64, c_i64]),
+    "pt_gemm_mx_tile": (c_int, [c_i64, c_i64, c_i64, c_int]),
     "pt_gemm_fp8": (
         c_int,
         [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_i64, c_i64, c_i64, c_int, c_int,

@@ -176,3 +176,33 @@ def test_quantize_traces_under_torch_compile_on_meta():
         x = torch.empty(64, 256, dtype=torch.bfloat16, device="cuda")
         q, s = torch.ops.primus_turbo_cpp_extension.quantize_fp8_tensorwise(x, torch.float8_e4m3fn, None)
         assert q.shape == (64, 256) and s.shape == ()
+
+
+# (M, N, K) -> the tile with vector scales, MXFP8, MXFP4, on the 256 CUs that a device that is not there is taken to have
+TILES = {
+    (16, 4096, 4096): (0, 0, 0),  # few tiles
+    (2048, 2048, 8192): (3, 3, 3),  # 128 x 128, one a CU
+    (4096, 2048, 4096): (2, 2, 3),  # 256 x 128, the same
+    (4096, 4096, 4096): (1, 1, 1),  # 256 x 256, the same
+    (8192, 8192, 8192): (1, 1, 1),
+    # more than half a round of 256 x 256 and no whole one: 192 x 256, up to a round of it
+    (3001, 2880, 1024): (5, 5, 3),
+    (3072, 4096, 1024): (5, 5, 3),
+    (3073, 4096, 1024): (1, 1, 1),
+    (2880, 4352, 1024): (5, 5, 1),
+    (2880, 4353, 1024): (1, 1, 1),
+    # two rounds of it
+    (5760, 4096, 544): (3, 5, 3),
+    (5760, 4096, 1056): (5, 5, 3),
+}
+
+
+@pytest.mark.parametrize("M,N,K", TILES)
+def test_tile_of_a_dense_product(native_lib, M, N, K):
+    assert native_lib.pt_device_cu_count() == 256
+    assert (native_lib.pt_gemm_fp8_tile(M, N, K), *(native_lib.pt_gemm_mx_tile(M, N, K, fp4) for fp4 in (0, 1))) == TILES[M, N, K]
+
+
+@pytest.mark.parametrize("M,N,K", [(0, 128, 128), (128, 0, 128), (128, 128, 0)])
+def test_tile_of_no_product(native_lib, M, N, K):
+    assert native_lib.pt_gemm_fp8_tile(M, N, K) == native_lib.pt_gemm_mx_tile(M, N, K, 0) == native_lib.pt_gemm_mx_tile(M, N, K, 1) == -1

@@ -44,8 +44,11 @@ def test_special_values(recipe, special, pinned):
     few._check(recipe, 510, 1002, 1216, torch.float32, special=special)
 
 
-# where the rule takes the tile: 16 x 12, 16 x 16 and 15 x 16 tiles of it on 256 CUs, and more rounds than one
-@pytest.mark.parametrize("M,N,K", [(3001, 2880, 1024), (3001, 4096, 1024), (2880, 4096, 1024), (5760, 4096, 544)])
+# where the rule takes the tile: 16 x 12, 16 x 16 and 15 x 16 tiles of it on 256 CUs, and more rounds than one (with vector scales not
+# of as few slabs)
+@pytest.mark.parametrize("M,N,K", [(3001, 2880, 1024), (3001, 4096, 1024), (2880, 4096, 1024), (5760, 4096, 544), (5760, 4096, 1056)])
 @pytest.mark.parametrize("recipe", ["rowwise", "mxfp8"])
-def test_rule(recipe, M, N, K, _impl):
+def test_rule(recipe, M, N, K, native_lib):
+    assert (native_lib.pt_gemm_mx_tile(M, N, K, 0) if recipe == "mxfp8" else native_lib.pt_gemm_fp8_tile(M, N, K)) == (
+        3 if recipe == "rowwise" and K == 544 else 5)
     few._check(recipe, M, N, K)
