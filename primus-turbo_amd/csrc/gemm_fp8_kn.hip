@@ -2,8 +2,11 @@
 // [K, N], and A stored [K, M] as well. Slabs are copied into the LDS as they lie and transposed as they are read
 // (read_transposed), where other tiles want a transposed copy in memory. What a TENSORWISE layer's backward products read:
 // the forward codes of weight, activation and gradient, whose casts then write one layout (4096^2 17 -> 12 us each). The
-// products take 4 (B) and up to 3 % (both) longer than on transposed copies. A whole training step, with copies / in place, us:
-// 4096^3 206 / 200, 8192 x 2048 x 8192 422 / 411, 4096 x 8192 x 8192 716 / 705, 8192^3 1298 / 1290, 8192 x 4096 x 4096 379 / 374.
+// products take longer than on transposed copies, 3 to 4 % with B in place, 5 to 6 % with both (us, copies / B / both: 4096^3 52.1 /
+// 53.8 / 54.6, 8192 x 4096 x 4096 101.4 / 105.8 / 107.4, 4096 x 8192 x 8192 183.0 / 188.7 / 192.1, 8192^3 365 / 379 / 382): a
+// fragment takes four LDS reads instead of two. A whole training step, copies / in place, us: 4096^3 210.1 / 204.4, 8192 x 8192 x 2048
+// 428 / 414, 4096 x 8192 x 8192 734 / 716, 8192 x 4096 x 4096 397.5 / 392.6, 16384 x 4096 x 8192 1402 / 1363 (7 runs of either in turn, which
+// differ by 1 % or less); adding the weight gradient into fp32 231.3 / 225.4, 450 / 432, 829 / 806, 418.0 / 418.5, 1456 / 1411.
 #include "gemm_fp8_kernel.h"
 
 namespace pt {

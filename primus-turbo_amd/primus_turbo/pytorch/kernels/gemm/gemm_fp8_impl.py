@@ -129,8 +129,10 @@ def kn_layer_pays(rows: int, mx: bool = False) -> bool:
     them costs the cast a fixed time, the product that reads ``[K, N]`` is 1 to 3 % slower on every row. A training step of
     M x N x K, copies / in place, blocks: 2048 x 8192 x 8192 469 / 459 us, 4096 851 / 829, 6144 1230 / 1206, 8192 1612 / 1610
     (1609 / 1615 on another card), 16384 x 8192 x 4096 1646 / 1672; four experts of 4096 x 4096: 16384 rows 972 / 950, 32768
-    1777 / 1775. MXFP8 there 832 / 822 and 1511 / 1519, MXFP4 608 / 598 and 1063 / 1073. (The products with vector scales gain
-    at any size: 16384 x 8192 x 4096 1365 / 1330.)"""
+    1777 / 1775. MX: time in place over time with copies, average (range) of MXFP8 and MXFP4 steps of banks 4 x 4096 x 4096, 4 x 7168 x 2048,
+    2 x 2048 x 7168, 8 x 2048 x 2048: 2048 rows a weight 0.979 (0.968 to 0.996), 4096 0.992 (0.979 to 1.004), 5120 0.997 (0.991 to 1.006), 6144 1.000
+    (0.990 to 1.007), 7168 1.002 (0.995 to 1.010), 8192 1.013 (1.000 to 1.023). (The products with vector scales gain at any size:
+    16384 x 4096 x 8192 1402 / 1363.)"""
     return rows < (5120 if mx else 8192)
 
 
